@@ -597,7 +597,7 @@ __global__ __launch_bounds__((8 + NP) * 64) void spmm_dspp_kernel(SpmmParams p) 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     if (wave < 4) {
         ds_consumer_pp<Cfg, OUT_LAYOUT, false>(p, walk, smem, wave, lane);
@@ -620,7 +620,7 @@ __global__ __launch_bounds__((NC + NP) * 64) void spmm_ds_kernel(SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     if (SPATHA_SKEW_ON(p)) {
         // workgroups of one XCD start up to 7 * skew * 1024 clocks apart (write-out bursts spread over time)

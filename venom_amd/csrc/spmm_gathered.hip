@@ -240,7 +240,8 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
     const int tile = xcd * chunk + local;
     if (local >= chunk || tile >= tiles) return;
-    const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
+    const int place = tile / p.tiles_m, tile_m = tile - place * p.tiles_m;
+    const int tile_n = static_tile_column(place, xcd, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -450,7 +451,8 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
     const int tile = xcd * chunk + local;
     if (local >= chunk || tile >= tiles) return;
-    const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
+    const int place = tile / p.tiles_m, tile_m = tile - place * p.tiles_m;
+    const int tile_n = static_tile_column(place, xcd, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wn = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -686,25 +688,12 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
     const int wm = wave / WN, wn = wave - wm * WN;
     const int S = p.S, N = p.N;
 
-    // ---- this workgroup's tile list: XCD x (= id % 8) owns a contiguous range of tile ids
-    //      (id -> n-tile major, m-tile minor); its workgroups take them round robin.  Tile
-    //      coordinates advance by a fixed (dm, dn) with carry: no division per tile.
-    const int tiles = p.tiles_m * p.tiles_n;
-    const int chunk = (tiles + 7) >> 3;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
-    const int first = xcd * chunk;
-    const int last = (first + chunk) < tiles ? (first + chunk) : tiles;      // exclusive
-    int my_tiles = 0;
-    if (first + slot < last) my_tiles = (last - first - slot + slots - 1) / slots;
+    // ---- this workgroup's tile list (TileWalkT, spmm_device.h)
+    TileWalk walk;
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
+    const int my_tiles = walk.my_tiles;
     if (my_tiles == 0) return;
     const int Q = my_tiles * S;
-    const int step_dn = slots / p.tiles_m, step_dm = slots - step_dn * p.tiles_m;
-    const int tn0 = (first + slot) / p.tiles_m, tm0 = (first + slot) - tn0 * p.tiles_m;
-    auto next_tile = [&](int& tm, int& tn) {
-        tm += step_dm;
-        tn += step_dn;
-        if (tm >= p.tiles_m) { tm -= p.tiles_m; tn += 1; }
-    };
     const int tiles_per_vblock = p.v / BM;           // V % BM == 0 is checked on the host
 
     const i32x4 rsrc_b = make_buffer(p.B, p.b_bytes);
@@ -729,13 +718,13 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
     const uint32_t rt_lane_off = (uint32_t)((wave * NB_LOADS) * RPI + slot_row) * 4;   // + j*RPI*4
 
     // ---- issue state (all scalar except coloff): stage f = next batch to issue
-    int is_tm = tm0, is_tn = tn0, is_step = 0;
+    int is_tm = walk.tm0, is_tn = walk.tn0, is_step = 0;
     uint32_t is_stage = 0;                                   // byte offset of the LDS stage for f
     uint32_t a_soff = (uint32_t)((is_tm * (BM / 64) + wm) * S) * (uint32_t)APACK_BLOCK;
     int issue_left = Q;                                      // batches not yet issued
     uint32_t rt_read = 0;                                    // ring slot (bytes) holding the rows of stage f
     // row-table state: stage f + PA (clamped to the last stage)
-    int rt_tm = tm0, rt_tn = tn0, rt_step = 0, rt_left = Q - 1;   // advances still allowed
+    int rt_tm = walk.tm0, rt_tn = walk.tn0, rt_step = 0, rt_left = Q - 1;   // advances still allowed
     uint32_t rt_soff = (uint32_t)((rt_tm / tiles_per_vblock) * S) * 256u;
     uint32_t coloff[NB_LOADS];
     auto set_coloff = [&]() {
@@ -752,7 +741,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
             rt_soff += 256u;
             if (++rt_step == S) {
                 rt_step = 0;
-                next_tile(rt_tm, rt_tn);
+                walk.next(rt_tm, rt_tn);
                 rt_soff = (uint32_t)((rt_tm / tiles_per_vblock) * S) * 256u;
             }
         }
@@ -785,7 +774,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
         a_soff += (uint32_t)APACK_BLOCK;
         if (++is_step == S) {
             is_step = 0;
-            next_tile(is_tm, is_tn);
+            walk.next(is_tm, is_tn);
             a_soff = (uint32_t)((is_tm * (BM / 64) + wm) * S) * (uint32_t)APACK_BLOCK;
             set_coloff();
         }
@@ -809,14 +798,14 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
     //      flight yet); the row-table cursor starts PA stages ahead of the issue cursor.
     {
         uint32_t rows0[PA][NB_LOADS];
-        int st_tm = tm0, st_tn = tn0, st_step = 0;
+        int st_tm = walk.tm0, st_tn = walk.tn0, st_step = 0;
 #pragma unroll
         for (int t = 0; t < PA; t++) {
             const int64_t base = ((int64_t)(st_tm / tiles_per_vblock) * S + st_step) * 64;
 #pragma unroll
             for (int j = 0; j < NB_LOADS; j++)
                 rows0[t][j] = (t < Q) ? p.rowtab[base + (wave * NB_LOADS + j) * RPI + slot_row] : 0xffffffffu;
-            if (++st_step == S) { st_step = 0; next_tile(st_tm, st_tn); }
+            if (++st_step == S) { st_step = 0; walk.next(st_tm, st_tn); }
         }
 #pragma unroll
         for (int t = 0; t < PA; t++) rt_advance();
@@ -826,7 +815,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
     }
 
     const int j16 = lane & 15, ib = lane >> 4;
-    int c_tm = tm0, c_tn = tn0;
+    int c_tm = walk.tm0, c_tn = walk.tn0;
     int q_left = Q;                 // steps not yet multiplied
     uint32_t c_stage = 0;           // byte offset of the stage multiplied next
     for (int c_tile = 0; c_tile < my_tiles; c_tile++) {
@@ -905,7 +894,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
                 __builtin_amdgcn_wave_barrier();
             }
         }
-        next_tile(c_tm, c_tn);
+        walk.next(c_tm, c_tn);
     }
 }
 

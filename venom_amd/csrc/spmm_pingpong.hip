@@ -315,7 +315,7 @@ __global__ __launch_bounds__(512) void spmm_up_kernel(SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalkT<WALK> walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     // (development builds: the workgroups of an XCD start in four groups, skew * 1024 clocks apart, so that their write-outs
     // no longer fall together)

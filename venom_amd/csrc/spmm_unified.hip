@@ -42,7 +42,7 @@ __global__ __launch_bounds__(512) void spmm_du_kernel(SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     const int S = p.S, N = p.N;
     const int Q = walk.my_tiles * S;

@@ -478,7 +478,7 @@ __global__ __launch_bounds__((WN + NP) * 64) void spmm_wst_kernel(SpmmParams p) 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     if (SPATHA_SKEW_ON(p)) {
         const int units = ((blockIdx.x >> 3) & 7) * p.skew;
@@ -528,7 +528,7 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void spmm_ws_kernel(SpmmParams
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalkT<WALK_GROUP> walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     // Workgroups of one XCD start up to 7 * skew apart, so that tiles do not all finish (and
     // hit HBM with their stores) at the same moment on every CU.
@@ -751,7 +751,7 @@ __global__ __launch_bounds__((8 + NP) * 64) void spmm_wsw_kernel(SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk walk;
-    walk.init(p.tiles_m, p.tiles_n);
+    walk.init(p.tiles_m, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
     if (walk.my_tiles == 0) return;
     if (wave < Cfg::NC) {
         wsw_consumer<Cfg, OUT_LAYOUT>(p, walk, smem, wave, lane);
