@@ -1,0 +1,60 @@
+"""Conversion of a matrix that lives on the GPU (search, encoding and decoding as kernels) against the host builder, which the
+oracle checks: the same arrays bit for bit - narrow and wide tails, groups without a winner, equal magnitudes, every group count
+per workgroup, strided and fp32 inputs, infinities and NaN."""
+import numpy as np
+import pytest
+import torch
+
+from venom_amd import _lib, bert
+from venom_amd import format as F
+from venom_amd.grouped_nmv_tensor import SrNMTensor, nm_vector_mask_sparsify
+
+pytestmark = pytest.mark.gpu
+
+
+def host_matrix(w, m, v):
+    mask, columns = nm_vector_mask_sparsify(w, 2, m, v, gpu=True, exact_ties=False)
+    return SrNMTensor(2, m, v, w, mask, columns, w.device)
+
+
+def same(a, b):
+    assert a.dtype == b.dtype and a.device == b.device and a.shape == b.shape
+    bits = {torch.float16: torch.int16}.get(a.dtype, a.dtype)
+    assert torch.equal(a.view(bits), b.view(bits))
+
+
+@pytest.mark.parametrize("rows,cols,m,v", [(32, 4, 4, 32), (64, 64, 8, 32), (64, 65, 8, 32), (64, 66, 8, 64), (64, 67, 8, 32),
+                                           (128, 70, 8, 128), (64, 300, 7, 32), (256, 1280, 10, 64), (128, 777, 16, 64),
+                                           (64, 6, 16, 32), (64, 3, 8, 32), (64, 2, 8, 64), (32, 600, 40, 32), (64, 1024, 4, 64)])
+@pytest.mark.parametrize("kind", ["gauss", "ties", "sparse", "fp32", "strided", "special"])
+def test_conversion_equals_the_host_path(gpu, rows, cols, m, v, kind):
+    gen = torch.Generator(device="cuda").manual_seed(rows + 3 * cols + m)
+    w = torch.randn((rows, cols), generator=gen, device="cuda").half()
+    if kind == "ties":
+        w = torch.randint(-2, 3, (rows, cols), generator=gen, device="cuda").half()
+    elif kind == "sparse":
+        w = w * (torch.rand((rows, cols), generator=gen, device="cuda") < 0.2)
+        w[:, :m] = 0
+    elif kind == "fp32":
+        w = torch.randn((rows, cols), generator=gen, device="cuda")
+    elif kind == "strided":
+        w = torch.randn((cols, rows + 3), generator=gen, device="cuda").half()[:, 1:rows + 1].t()
+    elif kind == "special":
+        w[::7, ::5] = float("inf")
+        w[::11, 1::9] = float("nan")
+        w[1::3, ::4] = -0.0
+    got = bert.NMVectorSparsifier(2, m, v, magnitude=True)(w).wrapped_tensor
+    want = host_matrix(w, m, v)
+    for name in ("values", "metadata", "columns"):
+        same(getattr(got, name), getattr(want, name))
+    assert (got.nrows, got.ncols, got.nnz, got.device) == (want.nrows, want.ncols, want.nnz, want.device)
+    dense = F.decode(got.values.cpu().numpy(), got.metadata.cpu().numpy().view(np.uint32),
+                     got.columns.cpu().numpy().astype(np.uint32), rows, cols, 2, m, v)
+    same(got.to_dense(), torch.from_numpy(dense).cuda())
+
+
+def test_a_column_offset_beyond_the_group_is_refused(gpu):
+    a = bert.NMVectorSparsifier(2, 8, 32, magnitude=True)(torch.randn(32, 64, device="cuda").half()).wrapped_tensor
+    a.columns[5] = 8
+    with pytest.raises(_lib.SpathaError):
+        a.to_dense()

@@ -12,6 +12,9 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SPATHA_LIBRARY") or os.path.join(_HERE, "lib", "libspatha.so")
 
 
+ERR_BAD_ARGUMENT = 1          # SPATHA_ERR_BAD_ARGUMENT
+
+
 class SpathaError(RuntimeError):
     def __init__(self, status, where):
         self.status = int(status)
@@ -42,6 +45,8 @@ SIGNATURES = {
     "spatha_vnm_decode_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int]),
     "spatha_vnm_select_columns_f32": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int]),
     "spatha_vnm_select_columns_f32_gpu": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p]),
+    "spatha_vnm_convert_gpu": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "spatha_vnm_decode_f16_gpu": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "spatha_vnm_pack_meta_blob": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, POINTER(c_int64), POINTER(c_int64)]),
     "spatha_spmm_plan_create": (c_int, [c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_void_p)]),
     "spatha_spmm_plan_destroy": (c_int, [c_void_p]),

@@ -25,6 +25,14 @@ inline int hip_fail(hipError_t e) {
     return SPATHA_ERR_HIP;
 }
 
+// compute units of the current device (0 where the runtime does not say)
+int device_cus() {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return 0;
+    return cus;
+}
+
 // kernels whose write-out can apply bias and activation ahead of either output layout
 bool variant_has_fused_writeout(int variant) {
     using namespace spatha;
@@ -534,26 +542,55 @@ int spatha_vnm_select_columns_f32_gpu(const float* dense_abs, int rows, int cols
     if (tasks > 0) {
         if ((size_t)v * (size_t)m * sizeof(float) > 150u * 1024u) return SPATHA_ERR_TOO_LARGE;   // one V x m block per workgroup in LDS
         float* d_abs = nullptr;
-        spatha::SelectWinner* d_out = nullptr;
-        std::vector<spatha::SelectWinner> h_out((size_t)tasks);
+        int32_t* d_out = nullptr;
+        std::vector<int32_t> h_out((size_t)tasks * 4);
         const size_t bytes = (size_t)rows * (size_t)cols * sizeof(float);
         hipStream_t s = (hipStream_t)stream;
         hipError_t e = hipMalloc((void**)&d_abs, bytes);
-        if (e == hipSuccess) e = hipMalloc((void**)&d_out, (size_t)tasks * sizeof(spatha::SelectWinner));
+        if (e == hipSuccess) e = hipMalloc((void**)&d_out, h_out.size() * sizeof(int32_t));
         if (e == hipSuccess) e = hipMemcpyAsync(d_abs, dense_abs, bytes, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = spatha::launch_select_winners(d_abs, rows, cols, m, v, d_out, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(h_out.data(), d_out, (size_t)tasks * sizeof(spatha::SelectWinner), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = spatha::launch_select_winners_f32(d_abs, rows, cols, m, v, device_cus(), d_out, per_block, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(h_out.data(), d_out, h_out.size() * sizeof(int32_t), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (d_abs) (void)hipFree(d_abs);
         if (d_out) (void)hipFree(d_out);
         if (e != hipSuccess) return hip_fail(e);
         for (int i = 0; i < tasks; i++) {
-            winners[(size_t)i].any = h_out[(size_t)i].any != 0;
-            for (int k = 0; k < 4; k++) winners[(size_t)i].best[k] = h_out[(size_t)i].best[k];
+            winners[(size_t)i].any = h_out[(size_t)i * 4 + 1] != 0;
+            for (int k = 0; k < 4; k++) winners[(size_t)i].best[k] = h_out[(size_t)i * 4 + k];
         }
     }
     return spatha::select_columns_with_winners(dense_abs, rows, cols, n, m, v, tasks > 0 ? winners.data() : nullptr,
                                                exact_ties != 0, masks, columns, threads);
+}
+
+int spatha_vnm_convert_gpu(const void* dense_dev, int value_bits, int rows, int cols, int n, int m, int v, uint16_t* values_dev,
+                           uint32_t* metadata_dev, uint32_t* columns_dev, void* stream) {
+    spatha_vnm_geometry geo;
+    int st = spatha::geometry_init(rows, cols, n, m, v, &geo);
+    if (st) return st;
+    if (!dense_dev || !values_dev || !metadata_dev || !columns_dev || (value_bits != 16 && value_bits != 32)) return SPATHA_ERR_BAD_ARGUMENT;
+    const int tasks = spatha::select_task_count(rows, cols, m, v, nullptr);
+    if (tasks > 0 && (size_t)v * (size_t)m * sizeof(float) > 150u * 1024u) return SPATHA_ERR_TOO_LARGE;
+    hipStream_t s = (hipStream_t)stream;
+    int32_t* columns = (int32_t*)columns_dev;
+    hipError_t e = value_bits == 16
+                       ? spatha::launch_select_winners_f16((const uint16_t*)dense_dev, rows, cols, m, v, device_cus(), columns, geo.ksp / 2, s)
+                       : spatha::launch_select_winners_f32((const float*)dense_dev, rows, cols, m, v, device_cus(), columns, geo.ksp / 2, s);
+    if (e == hipSuccess)
+        e = spatha::launch_encode_winners(dense_dev, value_bits, rows, cols, m, v, geo.ksp, values_dev, metadata_dev, columns, s);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_vnm_decode_f16_gpu(const uint16_t* values_dev, const uint32_t* metadata_dev, const uint32_t* columns_dev, int rows, int cols,
+                              int n, int m, int v, uint16_t* dense_dev, uint32_t* bad_dev, void* stream) {
+    spatha_vnm_geometry geo;
+    int st = spatha::geometry_init(rows, cols, n, m, v, &geo);
+    if (st) return st;
+    if (!values_dev || !metadata_dev || !columns_dev || !dense_dev || !bad_dev) return SPATHA_ERR_BAD_ARGUMENT;
+    const hipError_t e = spatha::launch_decode_f16(values_dev, metadata_dev, columns_dev, rows, cols, m, v, geo.ksp, dense_dev, bad_dev,
+                                                   (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 
 int spatha_vnm_pack_meta_blob(const uint32_t* metadata, int64_t n_metadata, const uint32_t* columns,

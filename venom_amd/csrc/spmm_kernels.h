@@ -90,14 +90,20 @@ hipError_t launch_onehalf(int variant, int out_layout, const SpmmParams& p, hipS
 hipError_t launch_pack(const uint16_t* values, const uint32_t* metadata, const uint32_t* columns, int rows, int cols,
                        int m, int v, int ksp, int S, int half_tiles, uint16_t* apack, uint32_t* rowtab, hipStream_t stream);
 
-// Search phase of the magnitude selector on the GPU (select_gpu.hip): one entry per (V-row block, group) task,
-// block-major, groups in the order full groups then the tail group (if it has three or more columns).
-struct SelectWinner {
-    int best[4];    // winning column subset, ascending; zeros when no subset has a positive total
-    int any;
-};
-hipError_t launch_select_winners(const float* dense_abs_dev, int rows, int cols, int m, int v, SelectWinner* out_dev,
-                                 hipStream_t stream);
+// Search phase of the magnitude selector on the GPU (select_gpu.hip): per V-row block and group (full groups, then the tail group
+// if it has three or more columns) the winning column subset, four int32, ascending; zeros when no subset has a positive total
+// (a winner's second column is at least 1).  out_pitch: entries of four per V-row block.  dense: the signed matrix or |A|.
+hipError_t launch_select_winners_f32(const float* dense_dev, int rows, int cols, int m, int v, int cus, int32_t* out_dev,
+                                     int64_t out_pitch, hipStream_t stream);
+hipError_t launch_select_winners_f16(const uint16_t* dense_dev, int rows, int cols, int m, int v, int cus, int32_t* out_dev,
+                                     int64_t out_pitch, hipStream_t stream);
+
+// Encoding of the selector's choice and decoding on the GPU (format_gpu.hip); column-loc holds the search's winners on entry to
+// the encoder, which completes it (narrow tail, padding groups).  decode: *bad is set to 1 if a column offset is not below m.
+hipError_t launch_encode_winners(const void* dense_dev, int value_bits, int rows, int cols, int m, int v, int ksp, uint16_t* values,
+                                 uint32_t* metadata, int32_t* columns, hipStream_t stream);
+hipError_t launch_decode_f16(const uint16_t* values, const uint32_t* metadata, const uint32_t* columns, int rows, int cols, int m,
+                             int v, int ksp, uint16_t* dense, uint32_t* bad, hipStream_t stream);
 
 // words of 32 bits set to zero by a kernel (tickets of a k-split launch; a kernel, so that the launch can be recorded into a graph)
 hipError_t launch_clear_words(uint32_t* words, int count, hipStream_t stream);

@@ -7,6 +7,7 @@ time: all work is done by libspatha.so through the C ABI."""
 import numpy as np
 import torch
 
+from . import _lib
 from . import format as F
 
 
@@ -63,7 +64,50 @@ class SrNMTensor:
         self.metadata = torch.from_numpy(metadata.view(np.int32)).to(device=device_)
         self.columns = torch.from_numpy(cols).to(device=device_)
 
+    @classmethod
+    def from_magnitude(cls, dense, n, m, tileM):
+        """What `SrNMTensor(n, m, tileM, dense, *nm_vector_mask_sparsify(dense, n, m, tileM, exact_ties=False), dense.device)`
+        holds, for a matrix on the GPU: selected and encoded there by two kernels on torch's current stream, without a trip
+        through the host."""
+        self = cls.__new__(cls)
+        self.n, self.m, self.tileM = n, m, tileM
+        self.device = dense.device
+        self.nrows, self.ncols = dense.shape
+        geo = F.geometry(self.nrows, self.ncols, n, m, tileM)
+        self.nnz = self.nrows * geo.ksp
+        src = dense.detach()
+        if src.dtype != torch.float16:
+            src = src.to(torch.float32)
+        src = src.contiguous()
+        self.values = torch.empty(geo.n_values, dtype=torch.float16, device=self.device)
+        self.metadata = torch.empty(geo.n_metadata, dtype=torch.int32, device=self.device)
+        self.columns = torch.empty(geo.n_columns, dtype=torch.int32, device=self.device)
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.lib().spatha_vnm_convert_gpu(src.data_ptr(), src.element_size() * 8, self.nrows, self.ncols, n, m, tileM,
+                                                         self.values.data_ptr(), self.metadata.data_ptr(), self.columns.data_ptr(),
+                                                         torch.cuda.current_stream(self.device).cuda_stream), "spatha_vnm_convert_gpu")
+        return self
+
+    def _decodes_on_gpu(self, geo):
+        arrays = ((self.values, torch.float16, geo.n_values), (self.metadata, torch.int32, geo.n_metadata),
+                  (self.columns, torch.int32, geo.n_columns))
+        return all(t.is_cuda and t.device == self.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
+                   for t, dtype, count in arrays)
+
     def to_dense(self):
+        geo = F.geometry(self.nrows, self.ncols, self.n, self.m, self.tileM)
+        if self._decodes_on_gpu(geo):
+            dev = self.values.device
+            dense = torch.empty((self.nrows, self.ncols), dtype=torch.float16, device=dev)
+            bad = torch.zeros(1, dtype=torch.int32, device=dev)
+            with torch.cuda.device(dev):
+                _lib.check(_lib.lib().spatha_vnm_decode_f16_gpu(self.values.data_ptr(), self.metadata.data_ptr(),
+                                                                self.columns.data_ptr(), self.nrows, self.ncols, self.n, self.m,
+                                                                self.tileM, dense.data_ptr(), bad.data_ptr(),
+                                                                torch.cuda.current_stream(dev).cuda_stream), "spatha_vnm_decode")
+            if bad.item():
+                raise _lib.SpathaError(_lib.ERR_BAD_ARGUMENT, "spatha_vnm_decode")
+            return dense.to(device=self.device)
         dense = F.decode(self.values.float().cpu().numpy(), self.metadata.cpu().numpy().view(np.uint32),
                          self.columns.cpu().numpy().astype(np.uint32), self.nrows, self.ncols, self.n, self.m, self.tileM)
         return torch.from_numpy(dense).to(device=self.device).half()
