@@ -37,6 +37,13 @@ def nm_vector_mask_sparsify(tensor, n, m, tileM, threads=0, gpu=None, exact_ties
     return torch.from_numpy(masks), torch.from_numpy(columns)
 
 
+def _decodes_on_gpu(a, geo):
+    """Do a's three arrays have the types, sizes and place that the decoding kernel takes?"""
+    arrays = ((a.values, torch.float16, geo.n_values), (a.metadata, torch.int32, geo.n_metadata), (a.columns, torch.int32, geo.n_columns))
+    return all(t.is_cuda and t.device == a.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
+               for t, dtype, count in arrays)
+
+
 class SrNMTensor:
     """A weight matrix in V:N:M form.  values fp16 / columns int32 / metadata int32 live on
     `device`; nrows, ncols, nnz as in the reference.  `to_dense()` decodes for real (the
@@ -88,15 +95,9 @@ class SrNMTensor:
                                                          torch.cuda.current_stream(self.device).cuda_stream), "spatha_vnm_convert_gpu")
         return self
 
-    def _decodes_on_gpu(self, geo):
-        arrays = ((self.values, torch.float16, geo.n_values), (self.metadata, torch.int32, geo.n_metadata),
-                  (self.columns, torch.int32, geo.n_columns))
-        return all(t.is_cuda and t.device == self.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
-                   for t, dtype, count in arrays)
-
     def to_dense(self):
         geo = F.geometry(self.nrows, self.ncols, self.n, self.m, self.tileM)
-        if self._decodes_on_gpu(geo):
+        if _decodes_on_gpu(self, geo):
             dev = self.values.device
             dense = torch.empty((self.nrows, self.ncols), dtype=torch.float16, device=dev)
             bad = torch.zeros(1, dtype=torch.int32, device=dev)
