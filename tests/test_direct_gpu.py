@@ -1,0 +1,66 @@
+"""The kernels that read their operands without LDS staging (id 13, id 23 and the 32-row form for V = 32, 96, ...): every column
+width and wave count their launch can choose, on integer operands bit for bit against the oracle - one row tile and many, k-loops
+shorter than the waves that share them, ragged columns and k tails, both layouts, bias and fused bias."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from venom_amd import format as F
+from venom_amd import spatha
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # rows, cols, N, m, v
+    (64, 64, 8, 8, 64), (64, 300, 72, 7, 64), (256, 2048, 8, 16, 64), (128, 3300, 104, 16, 128), (1280, 5120, 304, 16, 128),
+    (1024, 4096, 512, 32, 128), (1024, 1024, 520, 16, 64), (768, 3072, 1040, 32, 64), (1024, 1024, 1040, 20, 128),
+    (1536, 640, 304, 20, 64), (4096, 512, 200, 16, 64), (4096, 1024, 512, 8, 64), (17408, 512, 16, 8, 64), (17408, 256, 32, 8, 64),
+    (35072, 512, 8, 16, 128), (35072, 512, 64, 16, 128), (1024, 16384, 64, 8, 128),
+    (32, 64, 8, 8, 32), (96, 300, 72, 7, 96), (160, 2048, 136, 16, 32), (1280, 5120, 304, 16, 32), (1024, 4096, 520, 8, 32),
+    (1024, 2048, 1040, 16, 32), (2112, 640, 264, 20, 32), (9216, 512, 8, 16, 32), (9216, 320, 32, 8, 288), (9216, 256, 64, 16, 32),
+]
+
+
+@pytest.mark.parametrize("rows,cols,N,m,v", CASES)
+@pytest.mark.parametrize("transposed", [False, True])
+def test_direct_kernels_bit_exact(gpu, rows, cols, N, m, v, transposed):
+    print("direct", rows, cols, N, m, v, transposed, flush=True)
+    vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=rows + N, integer_values=True)
+    rng = np.random.default_rng(N)
+    B = rng.integers(-4, 5, size=(cols, N)).astype(np.float16)
+    bias = rng.integers(-3, 4, size=rows).astype(np.float16)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
+    plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
+    name = plan.kernel_name(N, int(transposed), 0)
+    assert "direct_tile" in name or "skinny" in name, name
+    want = oracle.spmm(vals, meta, columns, rows, cols, 2, m, v, B, bias=bias if transposed else None, transposed_out=transposed)
+    guarded = torch.full((cols * N + 4096,), float("nan"), dtype=torch.float16, device=gpu)
+    guarded[:cols * N] = dev(B).reshape(-1)
+    dB = guarded[:cols * N].view(cols, N)
+    variants = [0] + ([23] if v % 64 == 0 else [])
+    for variant in variants:
+        got = plan.run(dB, bias=dev(bias) if transposed else None, transposed_out=transposed, variant=variant)
+        assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16)), variant
+    fused = plan.run(dB, bias=dev(bias), transposed_out=transposed, activation="none")
+    want_b = oracle.spmm(vals, meta, columns, rows, cols, 2, m, v, B, bias=bias, transposed_out=True)
+    want_b = want_b if transposed else np.ascontiguousarray(want_b.T)
+    assert np.array_equal(fused.cpu().numpy().view(np.uint16), want_b.view(np.uint16))
+
+
+def test_direct_kernel_activations(gpu):
+    """GELU in the write-out: one rounding of the exact value of the rounded, biased sum (at most one step of fp16 apart)."""
+    rows, cols, N, m, v = 256, 512, 136, 8, 64
+    vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=1, value_std=0.3)
+    rng = np.random.default_rng(2)
+    B = rng.standard_normal((cols, N)).astype(np.float16)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
+    plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
+    bias = dev(rng.standard_normal(rows).astype(np.float16))
+    for transposed in (False, True):
+        pre = plan.run(dev(B), bias=bias, transposed_out=transposed, activation="none", variant=23).double()
+        for act, approx in (("gelu", "none"), ("gelu_tanh", "tanh")):
+            got = plan.run(dev(B), bias=bias, transposed_out=transposed, activation=act, variant=23)
+            want = torch.nn.functional.gelu(pre, approximate=approx).half()
+            # one step of fp16 at the value's size (2^-10 relative, the subnormal step 2^-24 near zero)
+            assert bool(((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -10 + 2.0 ** -24).all())

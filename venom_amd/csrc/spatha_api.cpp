@@ -42,6 +42,7 @@ bool variant_has_fused_writeout(int variant) {
         case SPMM_VARIANT_T128x256_S3: case SPMM_VARIANT_DS256x128_S3_C8: case SPMM_VARIANT_DSH256x128_S3_C8:
         case SPMM_VARIANT_UP512x128_S3: case SPMM_VARIANT_DU512x128_M16: case SPMM_VARIANT_WS128x128_S3:
         case SPMM_VARIANT_WS64x256_S3: case SPMM_VARIANT_OH192x256: case SPMM_VARIANT_H64x256_S2: case SPMM_VARIANT_H64x128_S3: case SPMM_VARIANT_H64x128_S2:
+        case SPMM_VARIANT_DIRECT64: case SPMM_VARIANT_HDIRECT32:
             return true;
         default:
             return false;
@@ -61,18 +62,21 @@ bool variant_uses_buffer_descriptors(int variant) {
 
 bool variant_ok(const spatha_spmm_plan* plan, int N, int variant, bool fused = false) {
     using namespace spatha;
-    if (variant <= 0 || variant >= SPMM_VARIANT_COUNT) return false;
+    if (variant <= 0 || (variant >= SPMM_VARIANT_COUNT && variant != SPMM_VARIANT_HDIRECT32)) return false;
     if (fused && !variant_has_fused_writeout(variant)) return false;
     const int bm = spmm_variant_bm(variant);
     if (bm == 0) return false;
     const bool half_variant = variant == SPMM_VARIANT_H64x256_S2 || variant == SPMM_VARIANT_H64x128_S3 ||
-                              variant == SPMM_VARIANT_H64x128_S2 || variant == SPMM_VARIANT_DSH256x128_S3_C8;
+                              variant == SPMM_VARIANT_H64x128_S2 || variant == SPMM_VARIANT_DSH256x128_S3_C8 ||
+                              variant == SPMM_VARIANT_HDIRECT32;
     if (half_variant != (plan->half_tiles != 0)) return false;       // the packed operand order differs
     const uint64_t b_bytes = (uint64_t)plan->geo.cols * (uint64_t)N * 2u;
     if (variant == SPMM_VARIANT_DSH256x128_S3_C8) {
         if (plan->geo.m > 8 || plan->geo.rows % 256 != 0 || !plan->gtab) return false;
         return b_bytes < 0xE0000000ull && plan->apack_bytes < 0xE0000000ull;
     }
+    if (variant == SPMM_VARIANT_HDIRECT32)
+        return b_bytes < 0xE0000000ull && plan->apack_bytes < 0xE0000000ull && plan->rowtab_bytes < 0xE0000000ull;
     if (half_variant) return plan->geo.cols <= 65535 && spmm_variant_lds(variant, plan->S) <= 160 * 1024;
     const bool unified = variant == SPMM_VARIANT_UP512x128_S3 || variant == SPMM_VARIANT_DU512x128_M16;
     if (variant == SPMM_VARIANT_DS256x128_S3_C8 || variant == SPMM_VARIANT_DS256x128_S3_PP) {
@@ -164,6 +168,31 @@ struct Shape {
         const int last = N - (int)(tn - 1) * 256;
         return tn <= 4 && T * tn > grid && F * tn <= grid && last > 128;
     }
+    // Small products: kernels 23 (64 x 64 tiles) and 24 (32 x 64), straight from the L2, k-steps over a tile's waves (spmm_skinny.hip).
+    // Against the kernels chosen otherwise (ten layer shapes, 72 .. 2048 tokens, both layouts):
+    //   V % 64 == 0, at most one 64 x 64 tile per CU: 1.1x (768 x 3072 x 1040 at 128:2:32) .. 3.2x (1024 x 4096 x 128 at 64:2:16).
+    //   V % 128 == 0, up to 1.25 tiles per CU: 1.0-1.1x; beyond that 0.8-1.06x.
+    //   V % 64 == 0 only, whose staged kernels serve 64 or 256 matrix rows per tile: up to 1.6 tiles per CU 1.01-1.6x, with dense
+    //   staging (m <= 8) and up to ten k-steps at two tiles per CU still 1.22-1.25x; at 2.5 tiles per CU 0.8-0.99x.
+    // k-loops of 96 steps on V % 128 == 0 are what split runs are for (12288 x 49152 x 128 at 128:2:16: 48 us in two parts, 71 here).
+    // (Three k-steps or fewer at m <= 8 keep the dense staging that 512 x 256 x 256 at 64:2:8 is expected on.)
+    bool direct64() const {
+        const int64_t t = (int64_t)(rows / 64) * ((N + 63) / 64);
+        if (v % 128 == 0) return S < 96 && t * 4 <= cus * 5;
+        if (m <= 8 && S <= 3) return false;
+        return t * 10 <= cus * 16 || (m <= 8 && S <= 10 && t <= 2 * cus);
+    }
+    // V % 64 != 0: always up to 32 columns and, where nothing is dense-staged, up to 128 (2.1-6.2x ahead); above that against the
+    // rounds of the kernel it replaces: 64 x 256 gathered tiles take 1.2-1.6 us a k-step and round, dense-staged 256 x 128 ones
+    // 0.87, a 32 x 64 tile here 0.8-1.3 ns a k-step.  (1024 x 4096 x 1040: 13.3 against 23.5 us at 32:2:16, 21.5 against 29.9 at
+    // 32:2:8; 12288 x 12288 x 304 at 32:2:16 76 against 128; level at 1024 x 4096 x 2048, behind at 1280 x 5120 x 2048.)
+    bool direct32() const {
+        const bool staged = m <= 8 && rows % 256 == 0 && (tiles(256, 128) >= 160 || S >= 16);
+        if (N <= (staged ? 32 : 128)) return true;
+        const int64_t t = (int64_t)(rows / 32) * ((N + 63) / 64);
+        const int64_t rounds = ((staged ? tiles(256, 128) : (int64_t)((rows + 63) / 64) * ((N + 255) / 256)) + cus - 1) / cus;
+        return staged ? t <= 3 * cus * rounds : t * 2 <= (rounds == 1 ? 8 : 11) * cus * rounds;
+    }
     // 64 x 256 tiles: many tiles of few k-steps, m >= 32, row-major
     bool short_k_many() const { return m >= 32 && !transposed && tiles(64, 256) >= 2048 && S <= 8; }
 };
@@ -178,14 +207,13 @@ struct Rule {
 
 const Rule kRules[] = {
     // few columns: streaming A is all that matters, one 64-row tile per workgroup with the k-steps split over its waves, B
-    // straight from the L2 with one load per gathered row whatever N (2, 4 or 8 bytes for 16, 32 or 64 columns).  Up to 32
-    // columns: 1.3-1.5x ahead of every tiled kernel on the BERT-large matrices, 31.7 us on the GPT-3 FFN matrix (5.6 TB/s;
-    // 128-wide tiles 39-41).  33 .. 64 columns, V a multiple of 64: 5.7 us on 4096 x 1024 at 64:2:8 and 128:2:8 (tiled
-    // kernels 6.8-7.7), 31.3 us on 12288 x 12288 at 64:2:8 (49.2), 7.4 us on 1024 x 4096 at 64:2:16 (equal); on the GPT-3 FFN
-    // matrix 40.5 us, level with the 128 x 128 tiles (39.4): there the 192 registers of its four column blocks leave two
-    // workgroups per CU for three tiles per CU.
-    {V_HALF | V_128 | V_64, spatha::SPMM_VARIANT_SKINNY, [](const Shape& s) { return s.N <= 32; }},
+    // straight from the L2 with one load per gathered row whatever N (2, 4 or 8 bytes for 16, 32 or 64 columns).  1.3-3x ahead of
+    // every tiled kernel on the BERT-large matrices; GPT-3 FFN matrix 27-29 us up to 32 columns (6.3 TB/s; 128-wide tiles 39-41),
+    // 36 us at 64, level with the 128 x 128 tiles (39): there the registers of its four column blocks leave three workgroups
+    // per CU for three tiles per CU.  The same kernel with column tiles (id 23) takes fused write-outs and small products.
     {V_128 | V_64, spatha::SPMM_VARIANT_SKINNY, [](const Shape& s) { return s.N <= 64; }},
+    {V_128 | V_64, spatha::SPMM_VARIANT_DIRECT64, [](const Shape& s) { return s.N <= 64 || s.direct64(); }},
+    {V_HALF, spatha::SPMM_VARIANT_HDIRECT32, [](const Shape& s) { return s.direct32(); }},
 
     // -- V % 64 != 0 (1024 x 4096 x 4096 and 4096 x 1024 x 16384, m = 8 .. 32) --
     // m <= 8: the dense B stage is shared by eight 32-row blocks, the fill does not grow with the smaller V
@@ -329,7 +357,8 @@ const Rule kRules[] = {
 };
 
 int pick_variant(const spatha_spmm_plan* plan, int N, int variant, bool fused = false, int out_layout = SPATHA_OUT_ROW_MAJOR) {
-    if (variant != spatha::SPMM_VARIANT_AUTO) return variant_ok(plan, N, variant, fused) ? variant : -1;
+    if (variant != spatha::SPMM_VARIANT_AUTO)
+        return variant < spatha::SPMM_VARIANT_COUNT && variant_ok(plan, N, variant, fused) ? variant : -1;
     Shape s;
     s.v = plan->geo.v; s.m = plan->geo.m; s.rows = plan->geo.rows; s.N = N; s.S = plan->S;
     s.cus = plan->cus > 0 ? plan->cus : 256;

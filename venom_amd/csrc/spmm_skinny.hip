@@ -1,61 +1,87 @@
-// Kernel for few columns of B (N <= 64): streaming A is all that matters.
+// Kernels without LDS staging of the operands: few columns of B (N <= 64), and small products of any width.
 
 #include "spmm_device.h"
 
 namespace spatha {
 
 // ---------------------------------------------------------------------------
-// Skinny-N kernel (N <= 64): the product is bound by streaming A from HBM, not by the matrix units.
-// One workgroup per 64-row tile; its four waves split the k-steps (wave w takes steps w, w+4, ...),
-// so that 4 * rows/64 waves keep loads in flight, and add their fp32 partial tiles through LDS at the
-// end in a fixed order.  No LDS staging of B: a lane fetches the 16 elements of its B fragment
-// straight from global memory (B is small and stays in L2) through a buffer descriptor whose bounds
-// check returns the zeros of padding rows and of columns beyond N.  Operands of step i+1 and the row
-// table of step i+2 are requested before step i is multiplied.
+// One workgroup per 64-row tile (32 rows where V is a multiple of 32 only: half of a packed 64-row block, which is all that one
+// gathered set of B rows serves) and 16 * NB columns; its W waves split the k-steps (wave w takes steps w, w + W, ...) and add
+// their fp32 partial tiles through LDS at the end in a fixed order.  No LDS staging of B: a lane fetches the 16 elements of its
+// B fragment straight from global memory through a buffer descriptor whose bounds check returns the zeros of padding rows and
+// of columns beyond N.  Operands of a wave's next step and the row table of the one after are requested before a step is
+// multiplied.
 // NB = 1, 2 or 4 column blocks of 16.  Column block nb holds the columns NB * j + nb (j = 0 .. 15), not 16 * nb + j: lane j of
 // a block then needs NB ADJACENT columns of every gathered row, one load of 2 * NB bytes instead of NB loads of 2 bytes - 16
-// vector-memory instructions per k-step whatever N (with a load per element, 32 columns cost 39 us on the GPT-3 FFN matrix
-// where 16 cost 30).  N is a multiple of 8, so the NB columns of a lane lie all inside N or all outside.
+// vector-memory instructions per k-step whatever NB.  N is a multiple of 8, so the NB columns of a lane lie all inside N or all
+// outside.
+// What bounds it: with few tiles the trip to memory that a k-step's loads take (four waves a tile left 16 .. 192 of 256 CUs with
+// one wave per SIMD and fewer than two steps in flight: 12288 x 12288 at 64:2:8 and 8 tokens 25.1 us for 101 MB; sixteen waves:
+// 16.0); with many, the 12.8 KB of loads per 64 x 64 block and k-step through the L1 (0.8-1.2 ns a block and step over the chip).
+// It has no pipeline to fill and no stage to share, so small products end sooner than on the staged tiles: 1024 x 4096 at
+// 64:2:16 and 304 tokens 5.0 us (64 x 256 tiles 14.4), 1280 x 5120 at 32:2:16 and 304 tokens 6.2 us (staged half tiles 24.7).
 // ---------------------------------------------------------------------------
 // LEAN (four column blocks only): see the main loop.  (The lean form is compiled for three waves per SIMD - three workgroups
 // of four waves per CU - which it reaches with 158 registers.)
-template <int NB, int OUT_LAYOUT, bool LEAN = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LEAN ? 3 : 2))) void spmm_skinny_kernel(SpmmParams p) {
-    // (the partial tiles are added up two column blocks at a time: 32 KB of LDS, so that three or more workgroups share a CU)
-    constexpr int RB = NB < 2 ? NB : 2;
-    __shared__ float4_t red[4][4][RB][64];
+template <int NB, int W, bool HALF, bool LEAN>
+struct DirectCfg {
+    static constexpr int MB = HALF ? 2 : 4;                                     // instruction-row blocks per tile
+    // partial tiles are added up PB row blocks at a time, CB adjacent columns per lane
+    static constexpr int LDS_KB = LEAN ? 32 : 64;
+    static constexpr int PB = W * MB * NB <= LDS_KB ? MB : W * 2 * NB <= LDS_KB ? 2 : 1;
+    static constexpr int CB = W > 4 && NB > 2 ? 2 : NB;
+    static constexpr int UNITS = PB * (NB / CB);
+    static constexpr int WAVES_PER_EU = NB == 4 ? (LEAN || HALF ? 3 : 2) : NB == 2 ? 3 : 4;
+    static_assert(W * PB * NB <= 64, "partial tiles exceed 64 KB");
+};
+
+template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN = false>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu((DirectCfg<NB, W, HALF, LEAN>::WAVES_PER_EU))))
+void spmm_direct_kernel(SpmmParams p) {
+    using Cfg = DirectCfg<NB, W, HALF, LEAN>;
+    constexpr int MB = Cfg::MB, PB = Cfg::PB, CB = Cfg::CB;
+    static_assert(NB == 1 || NB == 2 || NB == 4, "column blocks per tile");
+    __shared__ float4_t red[W][PB][NB][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tile = blockIdx.x;
     const int S = p.S, N = p.N;
+    // an XCD owns a contiguous range of tiles, row tile after row tile: the packed A of a row tile enters one L2 only
+    const int tiles = p.tiles_m * p.tiles_n, chunk = (tiles + 7) >> 3;
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, id = xcd * chunk + local;
+    if (local >= chunk || id >= tiles) return;
+    const int tile = id / p.tiles_n, tile_n = id - tile * p.tiles_n;
+    const int half = HALF ? tile & 1 : 0;
+    const int64_t block = HALF ? tile >> 1 : tile;                              // packed 64-row block
     const int li = lane & 15, kb = lane >> 4;
-    const int64_t vb = ((int64_t)tile * 64) / p.v;
-    const char* a_tile = (const char*)p.apack + (int64_t)tile * S * APACK_BLOCK;
+    const int64_t vb = ((int64_t)tile * (16 * MB)) / p.v;
+    const char* a_tile = (const char*)p.apack + block * S * APACK_BLOCK;
     const uint32_t* rt_block = p.rowtab + vb * S * 64;
     __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, (int)p.b_bytes, 0x00020000);
     const uint32_t row_bytes = (uint32_t)N * 2u;
 
-    float4_t acc[4][NB];
+    float4_t acc[MB][NB];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int a = 0; a < MB; a++)
 #pragma unroll
         for (int b = 0; b < NB; b++) acc[a][b] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
-    auto clamp_step = [&](int st) { return st < S ? st : S - 1; };
+    struct Set {
+        half8_t a[MB];
+        uint32_t ix[MB / 2];
+    };
     auto load_rt = [&](int st, u32x4 (&rt)[4]) {
-        const uint32_t* q = rt_block + (int64_t)clamp_step(st) * 64 + 4 * kb;
+        const uint32_t* q = rt_block + (int64_t)st * 64 + 4 * kb;
 #pragma unroll
         for (int fb = 0; fb < 4; fb++) rt[fb] = *(const u32x4*)(q + 16 * fb);
     };
-    auto load_a = [&](int st, half8_t (&a)[4], uint32_t& i0, uint32_t& i1) {
-        const char* q = a_tile + (int64_t)clamp_step(st) * APACK_BLOCK;
+    auto load_a = [&](int st, Set& x) {
+        const char* q = a_tile + (int64_t)st * APACK_BLOCK;
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) a[mb] = *(const half8_t*)(q + mb * 1024 + lane * 16);
-        i0 = *(const uint32_t*)(q + 4096 + lane * 4);
-        i1 = *(const uint32_t*)(q + 4352 + lane * 4);
+        for (int mb = 0; mb < MB; mb++) x.a[mb] = *(const half8_t*)(q + (half * 2 + mb) * 1024 + lane * 16);
+#pragma unroll
+        for (int d = 0; d < MB / 2; d++) x.ix[d] = *(const uint32_t*)(q + 4096 + (half + d) * 256 + lane * 4);
     };
-    static_assert(NB == 1 || NB == 2 || NB == 4, "column blocks per tile");
-    const int col0 = NB * li;       // this lane's NB columns: col0 + nb
+    const int col0 = (tile_n * 16 + li) * NB;       // this lane's NB columns: col0 + nb
     auto load_b = [&](const u32x4 (&rt)[4], half16_t (&bf)[NB]) {
 #pragma unroll
         for (int fb = 0; fb < 4; fb++)
@@ -79,110 +105,184 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LEAN ? 3 : 
                 }
             }
     };
-
-    auto multiply = [&](const half8_t (&a)[4], uint32_t i0, uint32_t i1, const half16_t (&b)[NB]) {
+    auto multiply = [&](const Set& x, const half16_t (&b)[NB]) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            acc[0][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a[0], b[nb], acc[0][nb], (int)i0, 0, 0);
-            acc[1][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a[1], b[nb], acc[1][nb], (int)i0, 0, 1);
-            acc[2][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a[2], b[nb], acc[2][nb], (int)i1, 0, 0);
-            acc[3][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(a[3], b[nb], acc[3][nb], (int)i1, 0, 1);
-        }
-    };
-    int st = wave;
-    if constexpr (!LEAN) {
-        u32x4 rt1[4], rt2[4];
-        half8_t a0[4], a1[4];
-        uint32_t i00, i01, i10, i11;
-        half16_t b0[NB], b1[NB];
-        load_rt(st, rt1);
-        load_a(st, a0, i00, i01);
-        load_b(rt1, b0);
-        load_rt(st + 4, rt1);
-        for (; st < S; st += 4) {
-            load_rt(st + 8, rt2);
-            load_a(st + 4, a1, i10, i11);
-            load_b(rt1, b1);
-            multiply(a0, i00, i01, b0);
+        for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                a0[k] = a1[k];
-                rt1[k] = rt2[k];
+            for (int mb = 0; mb < MB; mb++) {
+                if (mb & 1) acc[mb][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(x.a[mb], b[nb], acc[mb][nb], (int)x.ix[mb >> 1], 0, 1);
+                else acc[mb][nb] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(x.a[mb], b[nb], acc[mb][nb], (int)x.ix[mb >> 1], 0, 0);
             }
-            i00 = i10;
-            i01 = i11;
+    };
+    // (every condition below is uniform over the wave: `wave` and S sit in scalar registers)
+    auto clamp_step = [&](int s) { return s < S ? s : S - 1; };
+    int st = wave;
+    if (st < S) {
+        if constexpr (!LEAN) {
+            u32x4 rt1[4], rt2[4];
+            Set x0, x1;
+            half16_t b0[NB], b1[NB];
+            load_rt(st, rt1);
+            load_a(st, x0);
+            load_b(rt1, b0);
+            load_rt(clamp_step(st + W), rt1);
+            for (; st + W < S; st += W) {
+                load_rt(clamp_step(st + 2 * W), rt2);
+                load_a(st + W, x1);
+                load_b(rt1, b1);
+                multiply(x0, b0);
+                x0 = x1;
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) b0[nb] = b1[nb];
-        }
-    } else {
-        // Four column blocks with every operand double-buffered need 192 registers: two workgroups per CU.  With more than two
-        // 64-row tiles per CU (GPT-3 FFN matrix: three) this form runs instead: only B is double-buffered, the A operands and
-        // the row table of the next step are requested behind this step's matrix instructions, into the registers those have
-        // just read; three workgroups per CU, whose loads cover one another's waits (38 against 40.5 us there; with one tile
-        // per CU or less and long k-loops it is the slower form, 33.5 against 31.2 us on 12288 x 12288 at 64:2:8; with a wave's
-        // share of the k-loop at four steps or less its shorter prologue wins again: 5.4 against 5.7 us on 4096 x 1024).
-        u32x4 rt1[4];
-        half8_t a0[4];
-        uint32_t i00, i01;
-        half16_t b0[NB], b1[NB];
-        load_rt(st, rt1);
-        load_a(st, a0, i00, i01);
-        load_b(rt1, b0);
-        load_rt(st + 4, rt1);
-        for (; st < S; st += 4) {
-            load_b(rt1, b1);
-            multiply(a0, i00, i01, b0);
-            load_a(st + 4, a0, i00, i01);
-            load_rt(st + 8, rt1);
+                for (int k = 0; k < 4; k++) rt1[k] = rt2[k];
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) b0[nb] = b1[nb];
+                for (int nb = 0; nb < NB; nb++) b0[nb] = b1[nb];
+            }
+            multiply(x0, b0);
+        } else {
+            // Four column blocks with every operand double-buffered need 192 registers: two workgroups per CU.  With more than two
+            // 64-row tiles per CU (GPT-3 FFN matrix: three) this form runs instead: only B is double-buffered, the A operands and
+            // the row table of the next step are requested behind this step's matrix instructions, into the registers those have
+            // just read; three workgroups per CU, whose loads cover one another's waits (38 against 40.5 us there; with one tile
+            // per CU or less and long k-loops it is the slower form, 33.5 against 31.2 us on 12288 x 12288 at 64:2:8; with a wave's
+            // share of the k-loop at four steps or less its shorter prologue wins again: 5.4 against 5.7 us on 4096 x 1024).
+            u32x4 rt1[4];
+            Set x;
+            half16_t b0[NB], b1[NB];
+            load_rt(st, rt1);
+            load_a(st, x);
+            load_b(rt1, b0);
+            load_rt(clamp_step(st + W), rt1);
+            for (; st + W < S; st += W) {
+                load_b(rt1, b1);
+                multiply(x, b0);
+                load_a(st + W, x);
+                load_rt(clamp_step(st + 2 * W), rt1);
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++) b0[nb] = b1[nb];
+            }
+            multiply(x, b0);
         }
     }
-    // wave w finishes instruction-row block mb = w: rows 16*ib + 4*mb + r of the tile, column NB*li + nb
-    const int out_mb = wave, ib = kb;
-    const int64_t row0 = (int64_t)tile * 64 + 16 * ib + 4 * out_mb;
+    // Unit u of a pass: row block mb = pass + u % PB (rows 16 * ib + 4 * mb + r of a 64-row tile, 8 * ib + 4 * mb + r of a 32-row
+    // one), columns col0 + (u / PB) * CB + c
+    const int ib = kb;
 #pragma unroll
-    for (int nb0 = 0; nb0 < NB; nb0 += RB) {
-        if (nb0) __syncthreads();       // the pass before has been read
+    for (int pass = 0; pass < MB; pass += PB) {
+        if (pass) __syncthreads();      // the pass before has been read
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+        for (int pb = 0; pb < PB; pb++)
 #pragma unroll
-            for (int nb = 0; nb < RB; nb++) red[wave][mb][nb][lane] = acc[mb][nb0 + nb];
+            for (int nb = 0; nb < NB; nb++) red[wave][pb][nb][lane] = acc[pass + pb][nb];
         __syncthreads();
+        for (int u = wave; u < Cfg::UNITS; u += W) {
+            const int pb = u % PB, nb0 = (u / PB) * CB, mb = pass + pb;
+            const int64_t row0 = (int64_t)tile * (16 * MB) + (HALF ? 8 : 16) * ib + 4 * mb;
+            half4_t h4[CB];
+            half4_t bias4 = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+            if (p.bias) bias4 = *(const half4_t*)(p.bias + row0);
 #pragma unroll
-        for (int nb = 0; nb < RB; nb++) {
-            float4_t sum = ((red[0][out_mb][nb][lane] + red[1][out_mb][nb][lane]) + red[2][out_mb][nb][lane]) + red[3][out_mb][nb][lane];
-            const int col = col0 + nb0 + nb;
-            half4_t h4;
+            for (int c = 0; c < CB; c++) {
+                float4_t sum = red[0][pb][nb0 + c][lane];
 #pragma unroll
-            for (int r = 0; r < 4; r++) h4[r] = (_Float16)sum[r];
+                for (int w = 1; w < W; w++) sum = sum + red[w][pb][nb0 + c][lane];
+#pragma unroll
+                for (int r = 0; r < 4; r++) h4[c][r] = (_Float16)sum[r];
+                if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED || p.fuse) h4[c] = p.bias ? h4[c] + bias4 : h4[c];
+            }
+            if (p.act == SPATHA_ACT_GELU) {
+#pragma unroll
+                for (int c = 0; c < CB; c++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) h4[c][r] = (_Float16)act_gelu_erf((float)h4[c][r]);
+            } else if (p.act == SPATHA_ACT_GELU_TANH) {
+#pragma unroll
+                for (int c = 0; c < CB; c++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) h4[c][r] = (_Float16)act_gelu_tanh((float)h4[c][r]);
+            }
+            const int col = col0 + nb0;
             if (col >= N || SPATHA_KNOB(2)) continue;
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-                if (p.bias) h4 = h4 + *(const half4_t*)(p.bias + row0);
-                *(half4_t*)(p.C + (int64_t)col * p.rows + row0) = h4;
+#pragma unroll
+                for (int c = 0; c < CB; c++) *(half4_t*)(p.C + (int64_t)(col + c) * p.rows + row0) = h4[c];
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; r++) *(_Float16*)(p.C + (row0 + r) * N + col) = h4[r];
+                for (int r = 0; r < 4; r++) {
+                    uint16_t* dst = p.C + (row0 + r) * N + col;
+                    if constexpr (CB == 4) {
+                        *(half4_t*)dst = (half4_t){h4[0][r], h4[1][r], h4[2][r], h4[3][r]};
+                    } else if constexpr (CB == 2) {
+                        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+                        *(half2_t*)dst = (half2_t){h4[0][r], h4[1][r]};
+                    } else {
+                        *(_Float16*)dst = h4[0][r];
+                    }
+                }
             }
         }
     }
 }
 
-template <int OUT_LAYOUT>
-static hipError_t launch_skinny(const SpmmParams& p, hipStream_t stream) {
-    const dim3 grid(p.rows / 64), block(256);
-    if (p.N <= 16) hipLaunchKernelGGL((spmm_skinny_kernel<1, OUT_LAYOUT>), grid, block, 0, stream, p);
-    else if (p.N <= 32) hipLaunchKernelGGL((spmm_skinny_kernel<2, OUT_LAYOUT>), grid, block, 0, stream, p);
-    else if (p.rows / 64 > 2 * p.cus || p.S <= 16) hipLaunchKernelGGL((spmm_skinny_kernel<4, OUT_LAYOUT, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((spmm_skinny_kernel<4, OUT_LAYOUT>), grid, block, 0, stream, p);
+template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN = false>
+static hipError_t launch_direct(SpmmParams p, hipStream_t stream) {
+    p.tiles_m = p.rows / (HALF ? 32 : 64);
+    p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
+    const int tiles = p.tiles_m * p.tiles_n;
+    hipLaunchKernelGGL((spmm_direct_kernel<NB, OUT_LAYOUT, W, HALF, LEAN>), dim3((tiles + 7) / 8 * 8), dim3(W * 64), 0, stream, p);
     return hipGetLastError();
 }
 
+template <int OUT_LAYOUT, bool HALF>
+static hipError_t launch_direct_family(const SpmmParams& p, hipStream_t stream) {
+    // Columns and waves per tile: the narrowest tile whose tiles still find a CU each, its k-steps over as many waves as they
+    // feed; with more tiles than CUs fewer waves, so that several workgroups share a CU.  (Every form on ten layer shapes from
+    // 768 x 3072 to 49152 x 12288, V = 32 / 64 / 128, m = 8 / 16 / 32, 8 .. 2048 tokens, both layouts: this choice is 1.1 %
+    // behind the best form on the geometric mean.  12288 x 49152 at 128:2:16 and 8 tokens, 192 tiles of 192 k-steps: 28.8 us
+    // with sixteen waves, 50.3 with four; 1024 x 4096 at 64:2:16 and 512 tokens: 5.2 us on 64 x 32 tiles of eight waves, 6.4 on
+    // 64 x 64 ones.)
+    const int64_t rows_tiles = p.rows / (HALF ? 32 : 64), cus = p.cus;
+    auto tiles = [&](int nb) { return rows_tiles * ((p.N + 16 * nb - 1) / (16 * nb)); };
+    int nb, w = 4;
+    if (tiles(1) <= cus) {
+        nb = 1;
+        w = p.S > 12 ? 16 : p.S > 4 || p.N > 16 ? 8 : 4;
+    } else if (p.N <= 16) {
+        nb = 1;
+        w = tiles(1) <= 2 * cus && p.S > 4 ? 8 : 4;
+    } else if (tiles(2) <= cus) {
+        nb = 2;
+        w = p.S > 4 ? 8 : 4;
+    } else if (p.N <= 32 || (p.S <= 4 && tiles(2) <= 3 * cus)) {
+        nb = 2;
+    } else {
+        nb = 4;
+        if (tiles(4) <= cus && (p.S >= 16 || (p.S >= 8 && tiles(4) <= (HALF ? 256 : 160)))) w = 8;
+    }
+    const bool lean = tiles(4) > cus && (p.S > 2 || tiles(4) > 2 * cus);
+    switch (nb * 100 + w) {
+        case 104: return launch_direct<1, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 108: return launch_direct<1, OUT_LAYOUT, 8, HALF>(p, stream);
+        case 116: return launch_direct<1, OUT_LAYOUT, 16, HALF>(p, stream);
+        case 204: return launch_direct<2, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 208: return launch_direct<2, OUT_LAYOUT, 8, HALF>(p, stream);
+        case 404: return lean ? launch_direct<4, OUT_LAYOUT, 4, HALF, true>(p, stream) : launch_direct<4, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 408: return launch_direct<4, OUT_LAYOUT, 8, HALF>(p, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_skinny_family(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
-    if (variant != SPMM_VARIANT_SKINNY) return hipErrorInvalidValue;
-    return out_layout == SPATHA_OUT_TRANSPOSED ? launch_skinny<SPATHA_OUT_TRANSPOSED>(p, stream)
-                                               : launch_skinny<SPATHA_OUT_ROW_MAJOR>(p, stream);
+    const bool transposed = out_layout == SPATHA_OUT_TRANSPOSED;
+    switch (variant) {
+        case SPMM_VARIANT_SKINNY:
+        case SPMM_VARIANT_DIRECT64:
+            return transposed ? launch_direct_family<SPATHA_OUT_TRANSPOSED, false>(p, stream)
+                              : launch_direct_family<SPATHA_OUT_ROW_MAJOR, false>(p, stream);
+        case SPMM_VARIANT_HDIRECT32:
+            return transposed ? launch_direct_family<SPATHA_OUT_TRANSPOSED, true>(p, stream)
+                              : launch_direct_family<SPATHA_OUT_ROW_MAJOR, true>(p, stream);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace spatha
-
