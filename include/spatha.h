@@ -278,6 +278,13 @@ int spatha_dense_gemm_f16(const uint16_t* A_dev, const uint16_t* B_dev, int rows
  * (end2end/bert_pytorch.py:85-87, called from SrnmSpmm.forward :126-136). */
 int spatha_transpose_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream);
 
+/* The same for a row count that is no multiple of 8: out_dev has cols rows of ROUND_UP(rows, 8) entries, the appended ones zero
+ * (the SpMM reads its right-hand side in 16-byte row pieces). */
+int spatha_transpose_padded_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream);
+
+/* out[rows x ROUND_UP(cols, 8)] = in[rows x cols] with zero columns appended; in_dev at any alignment. */
+int spatha_pad_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream);
+
 /* out[tokens x hidden] = LayerNorm(x + residual) over the last dimension, fp16 in and out, fp32 arithmetic
  * (the sum is rounded to fp16 first, as the separate addition would; biased variance; gamma, beta of length hidden).
  * residual_dev may be NULL (plain layer norm).  hidden % 8 == 0 and hidden <= 4096 (SPATHA_ERR_UNSUPPORTED beyond);

@@ -910,7 +910,22 @@ int spatha_transpose_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* o
     if (!in_dev || !out_dev || rows <= 0 || cols <= 0) return SPATHA_ERR_BAD_ARGUMENT;
     if (((uintptr_t)in_dev | (uintptr_t)out_dev) & 15u) return SPATHA_ERR_BAD_ARGUMENT;
     if ((rows + 63) / 64 > 65535) return SPATHA_ERR_TOO_LARGE;
-    hipError_t e = spatha::launch_transpose_f16(in_dev, rows, cols, out_dev, (hipStream_t)stream);
+    hipError_t e = spatha::launch_transpose_f16(in_dev, rows, cols, out_dev, rows, (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_transpose_padded_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream) {
+    if (!in_dev || !out_dev || rows <= 0 || cols <= 0) return SPATHA_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)in_dev | (uintptr_t)out_dev) & 15u) return SPATHA_ERR_BAD_ARGUMENT;
+    if ((rows + 63) / 64 > 65535) return SPATHA_ERR_TOO_LARGE;
+    hipError_t e = spatha::launch_transpose_f16(in_dev, rows, cols, out_dev, (rows + 7) / 8 * 8, (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_pad_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream) {
+    if (!in_dev || !out_dev || rows <= 0 || cols <= 0 || cols > INT32_MAX - 8) return SPATHA_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)in_dev & 1u) || ((uintptr_t)out_dev & 15u)) return SPATHA_ERR_BAD_ARGUMENT;
+    hipError_t e = spatha::launch_pad_columns_f16(in_dev, rows, cols, out_dev, (cols + 7) / 8 * 8, (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 

@@ -132,6 +132,16 @@ std::shared_ptr<spatha_spmm_plan> plan_for(const torch::Tensor& values, const to
     return plan;
 }
 
+// x [rows, columns], contiguous, with zero columns up to the next multiple of 8
+torch::Tensor pad_columns(const torch::Tensor& x) {
+    const int64_t columns = x.size(1);
+    torch::Tensor out = torch::empty({x.size(0), (columns + 7) / 8 * 8}, x.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
+    check(spatha_pad_columns_f16((const uint16_t*)x.data_ptr(), (int)x.size(0), (int)columns, (uint16_t*)out.data_ptr(), stream),
+          "spatha_pad_columns_f16");
+    return out;
+}
+
 torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indices, const torch::Tensor& A_values,
                   const torch::Tensor& rhs_matrix, const c10::optional<torch::Tensor>& bias, int rows, int cols, int v, int n, int m,
                   bool transposed_out, int activation, bool fused) {
@@ -153,8 +163,7 @@ torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indice
         // The library moves rows of B and C in 16-byte pieces: a token count that is no multiple of 8 runs on a copy of
         // rhs_matrix with zero columns appended, and the result is cut back (the appended columns give bias-only rows /
         // columns, which are dropped).
-        const int pad = 8 - tokens % 8;
-        torch::Tensor padded = torch::constant_pad_nd(rhs_matrix, {0, pad}, 0);
+        torch::Tensor padded = pad_columns(rhs_matrix);
         torch::Tensor full = run(A_metadata, A_indices, A_values, padded, bias, rows, cols, v, n, m, transposed_out, activation, fused);
         return transposed_out ? full.narrow(0, 0, tokens) : full.narrow(1, 0, tokens).contiguous();
     }

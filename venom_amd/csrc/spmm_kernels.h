@@ -113,7 +113,8 @@ hipError_t launch_clear_words(uint32_t* words, int count, hipStream_t stream);
 hipError_t launch_pack_gtab(const uint32_t* columns, int rows, int m, int v, int ksp, int S, int block_rows, uint16_t* gtab,
                             hipStream_t stream);
 
-hipError_t launch_transpose_f16(const uint16_t* in, int rows, int cols, uint16_t* out, hipStream_t stream);
+hipError_t launch_transpose_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
+hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
 hipError_t launch_add_layernorm_f16(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
                                     float eps, int tokens, int hidden, uint16_t* out, hipStream_t stream);
 

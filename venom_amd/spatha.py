@@ -34,6 +34,15 @@ def _check_dev(t, dtype, name):
         raise ValueError("%s must be contiguous" % name)
 
 
+def _pad_columns(x):
+    """x [rows, columns], fp16, contiguous -> a copy with zero columns appended up to the next multiple of 8."""
+    out = torch.empty((x.shape[0], (x.shape[1] + 7) // 8 * 8), dtype=torch.float16, device=x.device)
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.lib().spatha_pad_columns_f16(x.data_ptr(), x.shape[0], x.shape[1], out.data_ptr(), _stream_ptr(x.device)),
+                   "spatha_pad_columns_f16")
+    return out
+
+
 class SpmmPlan:
     """Owns the library's plan (the copies of A laid out for the sparse matrix
     instructions) for one V:N:M matrix."""
@@ -85,7 +94,7 @@ class SpmmPlan:
                 raise ValueError("bias must have %d entries" % self.rows)
         if N % 8 != 0 and N > 0:
             # the library moves rows of B and C in 16-byte pieces: run on a copy with zero columns appended, cut the result back
-            full = self.run(torch.nn.functional.pad(B, (0, 8 - N % 8)), bias, transposed_out, variant, None, activation, split,
+            full = self.run(_pad_columns(B), bias, transposed_out, variant, None, activation, split,
                             workspace)
             cut = full[:N] if transposed_out else full[:, :N]
             if out is None:
