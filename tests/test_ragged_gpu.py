@@ -19,3 +19,76 @@ def test_padded_copies(gpu, rows, cols, offset):
     t = torch.full((cols, (rows + 7) // 8 * 8), float("nan"), dtype=torch.float16, device=gpu)
     _lib.check(_lib.lib().spatha_transpose_padded_f16(x.data_ptr(), rows, cols, t.data_ptr(), spatha._stream_ptr(gpu)), "transpose")
     assert torch.equal(t, torch.nn.functional.pad(x.t(), (0, -rows % 8)))
+
+
+@pytest.mark.parametrize("shape", [(1, 128), (301, 128), (3, 5, 128), (2, 8, 128), (1, 2, 3, 128)])
+def test_layers_take_any_token_count_and_stride(gpu, shape):
+    """The layer's one-call path against the operator on a copy made by torch: token-major, feature-major, strided and sliced
+    inputs, twice each (the second call finds the transposed copy of the first), plain and feature-major results, a chain of both."""
+    from venom_amd.bert import SrnmSpmm
+
+    torch.manual_seed(0)
+    up = SrnmSpmm(torch.nn.Linear(128, 256).half().to(gpu), 2, 8, 64, magnitude=True)
+    down = SrnmSpmm(torch.nn.Linear(256, 128, bias=False).half().to(gpu), 2, 16, 32, magnitude=True)
+
+    def direct(layer, x):
+        rhs = x.reshape(-1, x.shape[-1]).T.contiguous()
+        bias = layer.bias if layer.bias is not None else torch.zeros(layer.nrows_sp, device=gpu).half()
+        out = spatha.spmm(layer.metadata, layer.columns, layer.values, rhs, bias, layer.nrows_sp, layer.ncols_sp, rhs.shape[1], layer.v,
+                          layer.n, layer.m)
+        return out.reshape(*x.shape[:-1], -1)
+
+    base = torch.randn(shape, device=gpu).half()
+    wide = torch.randn(*shape[:-1], 256, device=gpu).half()
+    tokens = base.numel() // 128
+    feature = torch.randn(128, tokens, device=gpu).half().T.reshape(shape)
+    with torch.no_grad():
+        for x in (base, wide[..., 64:192], feature, torch.nn.Parameter(base.clone())):
+            want = direct(up, x)
+            for _ in range(2):
+                got = up(x)
+                assert got.shape == want.shape and torch.equal(got, want)
+                mid = up.forward_feature_major(x, "none")
+                assert mid.shape == want.shape and torch.equal(mid, want)
+                assert torch.equal(down(mid), direct(down, mid.contiguous()))
+                # an elementwise pass between the two, and the general path on what the one-call path has kept
+                assert torch.equal(down(mid * 2), direct(down, mid.contiguous() * 2))
+            assert torch.equal(SrnmSpmm._transposed(torch.flatten(x, 0, -2)), x.detach().reshape(-1, 128).T)
+        x = base.clone()
+        first = up(x)
+        x.mul_(2)                                       # the kept copy is of the old contents
+        assert torch.equal(up(x), direct(up, x)) and not torch.equal(up(x), first)
+
+
+def test_layer_refuses_what_it_refused(gpu):
+    from venom_amd.bert import SrnmSpmm
+
+    layer = SrnmSpmm(torch.nn.Linear(128, 64).half().to(gpu), 2, 8, 64)
+    with torch.no_grad():
+        for x in (torch.randn(4, 128, device=gpu), torch.randn(4, 120, device=gpu).half(), torch.randn(4, 128).half()):
+            with pytest.raises((RuntimeError, ValueError, TypeError)):
+                layer(x)
+        with pytest.raises((RuntimeError, IndexError)):
+            layer(torch.randn(128, device=gpu).half())
+
+
+def test_plan_run_refuses_and_writes_as_before(gpu):
+    from venom_amd import format as F
+
+    vals, meta, columns = F.synthetic_vnm(64, 128, 2, 8, 64, seed=1)
+    dev = lambda a: torch.from_numpy(a).to(gpu)
+    import numpy as np
+    plan = spatha.SpmmPlan(dev(vals), dev(meta.view(np.int32)), dev(columns.view(np.int32)), 64, 128, 2, 8, 64)
+    B = torch.randn(128, 24, device=gpu).half()
+    bias = torch.randn(64, device=gpu).half()
+    out = torch.empty(64, 24, device=gpu).half()
+    version = out._version
+    assert plan.run(B, out=out) is out and out._version > version and torch.equal(out, plan.run(B))
+    with torch.inference_mode():
+        assert torch.equal(plan.run(B), out)
+    for bad, error in ((dict(B=B.float()), TypeError), (dict(B=B.cpu()), ValueError), (dict(B=B.T), ValueError),
+                       (dict(B=B, out=out.T), ValueError), (dict(B=B, out=out[:, :16].contiguous()), ValueError),
+                       (dict(B=B, bias=bias[:32], transposed_out=True), ValueError), (dict(B=B, bias=bias), RuntimeError),
+                       (dict(B=B, variant=99), RuntimeError), (dict(B=B, activation="relu6"), ValueError), (dict(B=[1]), ValueError)):
+        with pytest.raises(error):
+            plan.run(**bad)

@@ -10,6 +10,7 @@ from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # SPATHA_LIBRARY names another build of the same library (e.g. the OUT_32B ablation build)
 LIB_PATH = os.environ.get("SPATHA_LIBRARY") or os.path.join(_HERE, "lib", "libspatha.so")
+IS_DEFAULT_BUILD = not os.environ.get("SPATHA_LIBRARY")
 
 
 ERR_BAD_ARGUMENT = 1          # SPATHA_ERR_BAD_ARGUMENT

@@ -70,7 +70,7 @@ class SrnmSpmm(torch.nn.Module):
             return flat.T              # feature-major already (the output of a fused feed-forward layer): no copy
         key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
         if cls._last_rhs[0] == key:
-            return cls._last_rhs[2]
+            return cls._last_rhs[2].contiguous()       # (a copy for a ragged token count has padded rows)
         if flat.is_cuda and flat.dtype == torch.float16:
             rhs = spatha.transpose(flat.contiguous())
         else:
@@ -86,12 +86,28 @@ class SrnmSpmm(torch.nn.Module):
         key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
         cls._last_rhs = (key, flat, x_t)
 
+    @staticmethod
+    def _run_native(cls, weights, input, rows, cols, feature_major=False, activation=spatha.ACT_NONE):
+        """The layer in one call of the extension, which looks at `cls._last_rhs` itself, or None for a call it does not take."""
+        got = spatha._extension().layer_spmm(input, cls._last_rhs, weights.metadata, weights.columns, weights.values, weights.bias,
+                                             rows, cols, weights.v, weights.n, weights.m, feature_major, activation,
+                                             spatha.transpose)
+        if got is None:
+            return None
+        out, last = got
+        if last is not None:
+            cls._last_rhs = last
+        return out
+
     _group = None          # set by merge_qkv: the projections this layer is computed together with
     _group_index = 0
 
     def forward(self, input):
         if self._group is not None:
             return self._group.output(self._group_index, self.nrows_sp, input)
+        out = self._run_native(type(self), self, input, self.nrows_sp, self.ncols_sp)
+        if out is not None:
+            return out
         flat = torch.flatten(input, start_dim=0, end_dim=-2)          # [tokens, in]
         rhs = self._transposed(flat)                                  # [in, tokens], as the operator expects
         bias = self.bias if self.bias is not None else torch.zeros(self.nrows_sp, dtype=rhs.dtype, device=rhs.device)
@@ -102,6 +118,10 @@ class SrnmSpmm(torch.nn.Module):
     def forward_feature_major(self, input, activation="none"):
         """act(x W^T + b) as a [..., out] VIEW of a feature-major buffer [out, tokens]: bias and activation run in
         the kernel's write-out, and the next SrnmSpmm takes the buffer as its right-hand side without a copy."""
+        if activation in spatha._ACTIVATIONS:
+            out = self._run_native(type(self), self, input, self.nrows_sp, self.ncols_sp, True, spatha._ACTIVATIONS[activation])
+            if out is not None:
+                return out
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
         rhs = self._transposed(flat)
         out = spatha.spmm_fused(self.metadata, self.columns, self.values, rhs, self.bias, self.nrows_sp, self.ncols_sp,
@@ -134,9 +154,11 @@ class _MergedProjections:
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
         key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
         if self._last[0] != key:
-            rhs = SrnmSpmm._transposed(flat)
-            out = spatha.spmm(self.metadata, self.columns, self.values, rhs, self.bias, self.rows, self.cols, rhs.shape[1],
-                              self.v, self.n, self.m, 0, 0, 32, 4)
+            out = SrnmSpmm._run_native(SrnmSpmm, self, flat, self.rows, self.cols)
+            if out is None:
+                rhs = SrnmSpmm._transposed(flat)
+                out = spatha.spmm(self.metadata, self.columns, self.values, rhs, self.bias, self.rows, self.cols, rhs.shape[1],
+                                  self.v, self.n, self.m, 0, 0, 32, 4)
             self._last = (key, flat, out)
         start = self.starts[index]
         return self._last[2][:, start:start + nrows].reshape(*input.shape[:-1], nrows)

@@ -17,6 +17,7 @@
 
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/python_variable.h>
 
 #include <list>
 #include <map>
@@ -123,7 +124,7 @@ std::shared_ptr<spatha_spmm_plan> plan_for(const torch::Tensor& values, const to
     std::shared_ptr<spatha_spmm_plan> plan(raw, [](spatha_spmm_plan* p) { spatha_spmm_plan_destroy(p); });
     // the same three tensors at another version: the weights were rewritten in place, those plans are stale
     drop_entries([&key](const PlanEntry& e) { return same_storage(e.key, key); });
-    g_lru.push_front(PlanEntry{key, plan, values, metadata, columns});
+    g_lru.push_front(PlanEntry{key, plan, values.detach(), metadata, columns});
     g_index[key] = g_lru.begin();
     while (g_lru.size() > kMaxPlans) {
         g_index.erase(g_lru.back().key);
@@ -139,6 +140,36 @@ torch::Tensor pad_columns(const torch::Tensor& x) {
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
     check(spatha_pad_columns_f16((const uint16_t*)x.data_ptr(), (int)x.size(0), (int)columns, (uint16_t*)out.data_ptr(), stream),
           "spatha_pad_columns_f16");
+    return out;
+}
+
+// the product on a right-hand side [cols, tokens], tokens a multiple of 8, with operands that have been checked
+torch::Tensor run_full(const torch::Tensor& A_metadata, const torch::Tensor& A_indices, const torch::Tensor& A_values,
+                       const torch::Tensor& rhs, int tokens, const uint16_t* bias_ptr, int rows, int cols, int v, int n, int m,
+                       bool transposed_out, int activation, bool fused) {
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
+    // (this reference outlives the launch calls below, whatever another thread does to the cache meanwhile)
+    const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values, A_metadata, A_indices, rows, cols, n, m, v, stream);
+    torch::Tensor out = transposed_out ? torch::empty({tokens, rows}, rhs.options().requires_grad(false))
+                                       : torch::empty({rows, tokens}, rhs.options().requires_grad(false));
+    const int layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
+    // few tokens against a long k-loop: the library splits the k-loops over workgroups if it is given scratch memory
+    const bool fuses = fused && (activation != SPATHA_ACT_NONE || (!transposed_out && bias_ptr));
+    if (const size_t need = spatha_spmm_workspace_bytes(plan.get(), tokens, layout, fuses ? 1 : 0)) {
+        torch::Tensor ws = workspace_for((int)A_values.get_device(), stream, need, rhs.options());
+        check(spatha_spmm_run_ws(plan.get(), (const uint16_t*)rhs.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
+                                 fused ? activation : SPATHA_ACT_NONE, ws.data_ptr(), (size_t)ws.numel(), stream),
+              "spatha_spmm_run_ws");
+        return out;
+    }
+    if (fused)
+        check(spatha_spmm_run_fused(plan.get(), (const uint16_t*)rhs.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
+                                    activation, 0, stream),
+              "spatha_spmm_run_fused");
+    else
+        check(spatha_spmm_run(plan.get(), (const uint16_t*)rhs.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout, 0,
+                              stream),
+              "spatha_spmm_run");
     return out;
 }
 
@@ -164,33 +195,169 @@ torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indice
         // rhs_matrix with zero columns appended, and the result is cut back (the appended columns give bias-only rows /
         // columns, which are dropped).
         torch::Tensor padded = pad_columns(rhs_matrix);
-        torch::Tensor full = run(A_metadata, A_indices, A_values, padded, bias, rows, cols, v, n, m, transposed_out, activation, fused);
+        torch::Tensor full = run_full(A_metadata, A_indices, A_values, padded, (int)padded.size(1), bias_ptr, rows, cols, v, n, m,
+                                      transposed_out, activation, fused);
         return transposed_out ? full.narrow(0, 0, tokens) : full.narrow(1, 0, tokens).contiguous();
     }
-    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
-    // (this reference outlives the launch calls below, whatever another thread does to the cache meanwhile)
-    const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values.detach(), A_metadata, A_indices, rows, cols, n, m, v, stream);
-    torch::Tensor out = torch::empty(transposed_out ? std::vector<int64_t>{tokens, rows} : std::vector<int64_t>{rows, tokens},
-                                     rhs_matrix.options());
-    const int layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
-    // few tokens against a long k-loop: the library splits the k-loops over workgroups if it is given scratch memory
-    const bool fuses = fused && (activation != SPATHA_ACT_NONE || (!transposed_out && bias_ptr));
-    if (const size_t need = spatha_spmm_workspace_bytes(plan.get(), tokens, layout, fuses ? 1 : 0)) {
-        torch::Tensor ws = workspace_for((int)A_values.get_device(), stream, need, rhs_matrix.options());
-        check(spatha_spmm_run_ws(plan.get(), (const uint16_t*)rhs_matrix.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
-                                 fused ? activation : SPATHA_ACT_NONE, ws.data_ptr(), (size_t)ws.numel(), stream),
-              "spatha_spmm_run_ws");
-        return out;
-    }
-    if (fused)
-        check(spatha_spmm_run_fused(plan.get(), (const uint16_t*)rhs_matrix.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
-                                    activation, 0, stream),
-              "spatha_spmm_run_fused");
-    else
-        check(spatha_spmm_run(plan.get(), (const uint16_t*)rhs_matrix.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout, 0,
-                              stream),
-              "spatha_spmm_run");
+    return run_full(A_metadata, A_indices, A_values, rhs_matrix, tokens, bias_ptr, rows, cols, v, n, m, transposed_out, activation, fused);
+}
+
+// x [rows, columns], contiguous -> [columns, rows] in rows padded with zeros to a multiple of 8
+torch::Tensor transposed_padded(const torch::Tensor& x) {
+    torch::Tensor out = torch::empty({x.size(1), (x.size(0) + 7) / 8 * 8}, x.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
+    check(spatha_transpose_padded_f16((const uint16_t*)x.data_ptr(), (int)x.size(0), (int)x.size(1), (uint16_t*)out.data_ptr(), stream),
+          "spatha_transpose_padded_f16");
     return out;
+}
+
+// spatha.transpose for an operand in order; None where the caller's checks have to speak
+py::object transpose_f16(py::handle input) {
+    if (!THPVariable_CheckExact(input.ptr())) return py::none();
+    const torch::Tensor& x = THPVariable_Unpack(input.ptr());
+    if (!x.is_cuda() || x.layout() != torch::kStrided || x.scalar_type() != torch::kFloat16 || x.dim() != 2 || !x.is_contiguous() ||
+        x.numel() == 0 || x.size(0) % 8 != 0 || x.size(0) > 65535 * 64 || x.size(1) > INT32_MAX || ((uintptr_t)x.data_ptr() & 15))
+        return py::none();
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(x.device());
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(transposed_padded(x)));
+}
+
+bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
+    return t.defined() && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
+}
+
+// Is `key` the Python key (address, shape, strides, version, device) of `held`, and is x the same tensor at the same version?
+bool same_activation(const torch::Tensor& x, const torch::Tensor& held, const py::tuple& key) {
+    return x.data_ptr() == held.data_ptr() && x.sizes() == held.sizes() && x.strides() == held.strides() && x.device() == held.device() &&
+           key.size() == 5 && key[3].cast<int64_t>() == (int64_t)x._version();
+}
+
+// One V:N:M layer on x [..., cols], without a trip through Python per part: the right-hand side (x feature-major already, the
+// copy that `last` = (key, activation, copy) holds for this activation, or a new one with padded rows) and the product.  Returns
+// (result, new `last` or None), or None for a call this function does not take - the caller's general path decides, and refuses,
+// as ever.  feature_major: act(x W^T + b) as a [..., rows] view of a buffer [rows, tokens padded to a multiple of 8], which the
+// next layer reads as it lies; else x W^T + b as [..., rows], activation ignored.  transpose: makes the copy where no padding is
+// needed (spatha.transpose).
+py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& metadata, const torch::Tensor& columns,
+                      const torch::Tensor& values, const c10::optional<torch::Tensor>& bias, int rows, int cols, int v, int n, int m,
+                      bool feature_major, int activation, py::handle transpose) {
+    if (!THPVariable_CheckExact(input.ptr())) return py::none();
+    const torch::Tensor& x = THPVariable_Unpack(input.ptr());
+    if (!x.is_cuda() || x.layout() != torch::kStrided || x.scalar_type() != torch::kFloat16 || x.dim() < 2 || x.size(-1) != cols ||
+        x.numel() == 0 || x.is_inference())
+        return py::none();
+    const int device = (int)x.get_device();
+    if (!weight_ok(values, torch::kFloat16, device) || !weight_ok(metadata, torch::kInt32, device) ||
+        !weight_ok(columns, torch::kInt32, device) || values.is_inference())
+        return py::none();
+    const int64_t tokens = x.numel() / cols, padded = (tokens + 7) / 8 * 8;
+    if (tokens > 65535 * 64) return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(x.device());
+    torch::Tensor bias_t;
+    if (bias.has_value() && bias->defined()) {
+        if (!weight_ok(*bias, torch::kFloat16, device) || bias->numel() != rows) return py::none();
+        bias_t = *bias;
+    } else if (!feature_major) {
+        bias_t = torch::zeros({rows}, x.options().requires_grad(false));
+    }
+    const torch::Tensor flat = x.dim() == 2 ? x : x.flatten(0, -2);
+    py::object kept = py::none();
+    torch::Tensor rhs;              // its first element is that of a [cols, padded] matrix
+    auto holds_padded_rows = [&](const torch::Tensor& t, int64_t pitch) {       // [cols, tokens] with rows `pitch` apart, all in memory
+        return pitch == padded && (size_t)((t.storage_offset() + cols * padded) * 2) <= t.storage().nbytes();
+    };
+    if (flat.stride(0) == 1 && flat.stride(1) >= tokens && holds_padded_rows(flat, flat.stride(1))) {
+        rhs = flat;
+    } else {
+        torch::Tensor copy;
+        if (flat.stride(0) == 1 && flat.stride(1) == tokens) {
+            copy = flat.t();
+        } else if (last.size() == 3 && THPVariable_Check(last[1].ptr()) && THPVariable_Check(last[2].ptr()) &&
+                   same_activation(flat, THPVariable_Unpack(last[1].ptr()), last[0].cast<py::tuple>())) {
+            copy = THPVariable_Unpack(last[2].ptr());
+        } else {
+            const torch::Tensor dense = flat.contiguous();
+            if ((uintptr_t)dense.data_ptr() & 15) return py::none();
+            py::object made;
+            if (padded == tokens) {
+                made = transpose(py::reinterpret_steal<py::object>(THPVariable_Wrap(dense)));
+                if (!THPVariable_Check(made.ptr())) return py::none();
+                copy = THPVariable_Unpack(made.ptr());
+            } else {
+                copy = transposed_padded(dense).narrow(1, 0, tokens);
+                made = py::reinterpret_steal<py::object>(THPVariable_Wrap(copy));
+            }
+            const py::object held = py::reinterpret_steal<py::object>(THPVariable_Wrap(flat));
+            py::tuple shape(2), strides(2);
+            for (int d = 0; d < 2; d++) {
+                shape[d] = py::int_(flat.size(d));
+                strides[d] = py::int_(flat.stride(d));
+            }
+            kept = py::make_tuple(py::make_tuple(py::int_((uintptr_t)flat.data_ptr()), shape, strides, py::int_((int64_t)flat._version()),
+                                                 held.attr("device")),
+                                  held, made);
+        }
+        if (copy.dim() != 2 || copy.size(0) != cols || copy.size(1) != tokens || copy.scalar_type() != torch::kFloat16) return py::none();
+        rhs = copy.stride(1) == 1 && holds_padded_rows(copy, copy.stride(0)) ? copy : pad_columns(copy.contiguous());
+    }
+    const uint16_t* bias_ptr = bias_t.defined() ? (const uint16_t*)bias_t.data_ptr() : nullptr;
+    torch::Tensor out = run_full(metadata, columns, values, rhs, (int)padded, bias_ptr, rows, cols, v, n, m, !feature_major,
+                                 feature_major ? activation : SPATHA_ACT_NONE, feature_major);
+    if (padded != tokens) out = out.narrow(feature_major ? 1 : 0, 0, tokens);
+    if (feature_major) out = out.t();
+    if (x.dim() != 2) {
+        std::vector<int64_t> sizes(x.sizes().begin(), x.sizes().end());
+        sizes.back() = rows;
+        out = out.reshape(sizes);
+    }
+    return py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(out)), kept);
+}
+
+// SpmmPlan.run without a k-split, for operands in order; None where the caller's checks have to speak.  bias needs the transposed
+// layout unless `fused` (an activation, ACT_NONE among them, was named).
+py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle out, int rows, int cols, int device, bool transposed_out,
+                    bool fused, int activation, int variant) {
+    if (!THPVariable_CheckExact(rhs.ptr()) || c10::InferenceMode::is_enabled()) return py::none();
+    const torch::Tensor& B = THPVariable_Unpack(rhs.ptr());
+    if (!weight_ok(B, torch::kFloat16, device) || B.dim() != 2 || B.size(0) != cols || B.size(1) <= 0 || B.size(1) % 8 != 0 ||
+        B.size(1) > INT32_MAX)
+        return py::none();
+    const int N = (int)B.size(1);
+    const uint16_t* bias_ptr = nullptr;
+    if (!bias.is_none()) {
+        if (!THPVariable_Check(bias.ptr())) return py::none();
+        const torch::Tensor& b = THPVariable_Unpack(bias.ptr());
+        if (!weight_ok(b, torch::kFloat16, device) || b.numel() != rows) return py::none();
+        bias_ptr = (const uint16_t*)b.data_ptr();
+    }
+    torch::Tensor C;
+    if (out.is_none()) {
+        C = transposed_out ? torch::empty({N, rows}, B.options().requires_grad(false)) : torch::empty({rows, N}, B.options().requires_grad(false));
+    } else {
+        if (!THPVariable_CheckExact(out.ptr())) return py::none();
+        C = THPVariable_Unpack(out.ptr());
+        if (!weight_ok(C, torch::kFloat16, device) || C.is_inference() || C.dim() != 2 || C.size(0) != (transposed_out ? N : rows) ||
+            C.size(1) != (transposed_out ? rows : N))
+            return py::none();
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(B.device());
+    const spatha_spmm_plan* plan = (const spatha_spmm_plan*)handle;
+    const uint16_t* b_ptr = (const uint16_t*)B.data_ptr();
+    uint16_t* c_ptr = (uint16_t*)C.data_ptr();
+    const int layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+    int status;
+    {
+        const py::gil_scoped_release release;
+        status = fused ? spatha_spmm_run_fused(plan, b_ptr, N, bias_ptr, c_ptr, layout, activation, variant, stream)
+                       : spatha_spmm_run(plan, b_ptr, N, bias_ptr, c_ptr, layout, variant, stream);
+    }
+    if (status != SPATHA_OK) return py::int_(status);
+    // the kernel wrote through a raw pointer: tell torch, so that caches keyed on the tensor's version see the change
+    C.unsafeGetTensorImpl()->bump_version();
+    if (!out.is_none()) return py::reinterpret_borrow<py::object>(out);
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(C));
 }
 
 // out[B_num_cols, A_num_rows] = (A_vnm @ rhs_matrix).T + bias, fp16: the reference operator.  vec_length is V and is
@@ -248,6 +415,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
             py::arg("A_indices"), py::arg("A_values"), py::arg("rhs_matrix"), py::arg("bias"), py::arg("A_num_rows"),
             py::arg("A_num_cols"), py::arg("vec_length"), py::arg("n"), py::arg("m"), py::arg("activation") = 0,
             py::arg("transposed_out") = false);
+    mod.def("layer_spmm", &layer_spmm, "one V:N:M layer, right-hand side and product, or None");
+    mod.def("transpose", &transpose_f16, "x.T of an fp16 matrix through the library's kernel, or None");
+    mod.def("plan_run", &plan_run, "a plan's product, or None, or the status of a refusal");
     mod.def("clear_plan_cache", &clear_plan_cache, "drop every cached plan");
     mod.def("invalidate_plans", &invalidate_plans, "drop the cached plans built from this values tensor; returns how many",
             py::arg("A_values"));

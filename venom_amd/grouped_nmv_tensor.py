@@ -100,12 +100,13 @@ class SrNMTensor:
         if _decodes_on_gpu(self, geo):
             dev = self.values.device
             dense = torch.empty((self.nrows, self.ncols), dtype=torch.float16, device=dev)
-            bad = torch.zeros(1, dtype=torch.int32, device=dev)
+            bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)      # written by the kernel where an offset has no place
             with torch.cuda.device(dev):
                 _lib.check(_lib.lib().spatha_vnm_decode_f16_gpu(self.values.data_ptr(), self.metadata.data_ptr(),
                                                                 self.columns.data_ptr(), self.nrows, self.ncols, self.n, self.m,
                                                                 self.tileM, dense.data_ptr(), bad.data_ptr(),
                                                                 torch.cuda.current_stream(dev).cuda_stream), "spatha_vnm_decode")
+                torch.cuda.current_stream(dev).synchronize()
             if bad.item():
                 raise _lib.SpathaError(_lib.ERR_BAD_ARGUMENT, "spatha_vnm_decode")
             return dense.to(device=self.device)

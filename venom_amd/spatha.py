@@ -84,6 +84,17 @@ class SpmmPlan:
         split=True (automatic kernel choice only) lets the library split k-loops over workgroups where tiles alone leave CUs
         idle; the scratch memory it needs is `workspace` (a uint8 tensor on the GPU that was zero-filled once, e.g. by
         torch.zeros) or, if None, a buffer the plan keeps per stream."""
+        if not split and (activation is None or activation in _ACTIVATIONS):
+            native = _plan_run_function()
+            if native is not None:
+                # operands in order run from here in one call; anything else comes back as None and meets the checks below
+                fused = activation is not None
+                got = native(self._handle.value, B, bias, out, self.rows, self.cols, self.device.index, bool(transposed_out), fused,
+                             _ACTIVATIONS[activation], variant)
+                if type(got) is int:
+                    _lib.check(got, "spatha_spmm_run_fused" if fused else "spatha_spmm_run")
+                elif got is not None:
+                    return got
         _check_dev(B, torch.float16, "rhs")
         if B.dim() != 2 or B.shape[0] != self.cols:
             raise ValueError("rhs must be [%d, N], got %s" % (self.cols, tuple(B.shape)))
@@ -178,16 +189,28 @@ class SpmmPlan:
         return best.value, best_ms.value, auto_ms.value, {i: per[i] for i in range(n) if per[i] >= 0}
 
 
+_loaded_extension = None
+
+
 def _extension():
     """The PyTorch C++ extension that holds the operator (csrc/spatha_torch.cpp, built in place by `python -m
     venom_amd.build`): `spmm` with the reference's signature, `spmm_fused`, and the cache of plans of the matrices they
     have seen.  There is no fallback: without it the operator raises."""
-    try:
-        from . import _spatha_torch
-    except ImportError as e:
-        raise RuntimeError("the PyTorch extension venom_amd/_spatha_torch.so is not built or does not load (%s): run "
-                           "`python -m venom_amd.build`" % e)
-    return _spatha_torch
+    global _loaded_extension
+    if _loaded_extension is None:
+        try:
+            from . import _spatha_torch
+        except ImportError as e:
+            raise RuntimeError("the PyTorch extension venom_amd/_spatha_torch.so is not built or does not load (%s): run "
+                               "`python -m venom_amd.build`" % e)
+        _loaded_extension = _spatha_torch
+    return _loaded_extension
+
+
+def _plan_run_function():
+    """The extension's `plan_run`, or None where plans belong to another build of the library (SPATHA_LIBRARY) than the one
+    the extension is linked to."""
+    return _extension().plan_run if _lib.IS_DEFAULT_BUILD else None
 
 
 def clear_plan_cache():
@@ -204,6 +227,10 @@ def invalidate_plans(A_values):
 def transpose(x):
     """x[rows, cols] fp16, contiguous -> a new contiguous [cols, rows] tensor (what `x.T.contiguous()` returns),
     through the library's tiled kernel on torch's current stream."""
+    if _lib.IS_DEFAULT_BUILD:
+        out = _extension().transpose(x)
+        if out is not None:
+            return out
     _check_dev(x, torch.float16, "x")
     if x.dim() != 2:
         raise ValueError("transpose expects a matrix")

@@ -12,6 +12,8 @@ this library:
 Where it cannot, `register()` raises ImportError and `wrapper_class()` hands out the two-method stand-in the harnesses need
 (`wrapped_from_dense(...)`, `.wrapped_tensor`).  `register(sten_module)` takes the module as an argument so that the hooks can
 be exercised against any object with STEN's registration interface."""
+import sys
+
 import torch
 
 from . import spatha
@@ -31,11 +33,19 @@ class SparseTensorWrapper:
         return SparseTensorWrapper(wrapped_tensor, dense, grad_fmt)
 
 
+_searched = None            # the search path on which STEN was last not found
+
+
 def sten_module():
-    """The STEN package, or None where it is not installed."""
+    """The STEN package, or None where it is not installed.  A search that found nothing is not repeated on the same search path
+    (it walks every folder of it: 50 us, more than the conversion of a weight takes)."""
+    global _searched
+    if "sten" not in sys.modules and _searched == (sys.path, sys.meta_path):
+        return None
     try:
         import sten
     except ImportError:
+        _searched = (list(sys.path), list(sys.meta_path))
         return None
     return sten
 
