@@ -105,7 +105,7 @@ bool variant_ok(const spatha_spmm_plan* plan, int N, int variant, bool fused = f
 // MI355X (BERT-base / BERT-large / GPT-2-large / GPT-3 layer shapes, N = 2048 .. 16384, m = 4 .. 100); each rule's comment
 // says what was measured.  Later rules double as the fall-backs of earlier ones.
 struct Shape {
-    int v, m, rows, N, S;
+    int v, m, rows, cols, N, S;
     int64_t cus;
     bool fused, transposed;
     // tiles of bm x bn in the output (whole row tiles only: the kernels that take a partial row tile are never chosen by count)
@@ -182,16 +182,26 @@ struct Shape {
         if (m <= 8 && S <= 3) return false;
         return t * 10 <= cus * 16 || (m <= 8 && S <= 10 && t <= 2 * cus);
     }
-    // V % 64 != 0: always up to 32 columns and, where nothing is dense-staged, up to 128 (2.1-6.2x ahead); above that against the
-    // rounds of the kernel it replaces: 64 x 256 gathered tiles take 1.2-1.6 us a k-step and round, dense-staged 256 x 128 ones
-    // 0.87, a 32 x 64 tile here 0.8-1.3 ns a k-step.  (1024 x 4096 x 1040: 13.3 against 23.5 us at 32:2:16, 21.5 against 29.9 at
-    // 32:2:8; 12288 x 12288 x 304 at 32:2:16 76 against 128; level at 1024 x 4096 x 2048, behind at 1280 x 5120 x 2048.)
+    // V % 64 != 0: 64 x 128 gathered tiles run two workgroups a CU as long as the row table leaves room for it (75 KB of stages + 256
+    // bytes a k-step, twice: up to 28 k-steps)
+    bool half_pairs() const { return S <= 28; }
+    // V % 64 != 0: direct 32 x 64 tiles always up to 32 columns and, where nothing is dense-staged, up to 128 (2-5x ahead of the
+    // gathered tiles); above that against the rounds of the kernel they replace: a k-step of a round takes 0.9-1.4 us on gathered
+    // tiles, 0.87 us on dense-staged ones, a k-step of a tile here 0.8-1.3 ns.  At 1040 tokens: 1024 x 4096 13.5 against 17.1 us at
+    // 32:2:16, 21.9 against 30.3 (staged) at 32:2:8; 3840 x 1280 at 32:2:10 14.0 against 18.8; 12288 x 12288 x 304 at 32:2:16 76
+    // against 115; at 2048 tokens 768 x 3072 at 32:2:10 is behind (17.9 against 15.4).
     bool direct32() const {
         const bool staged = m <= 8 && rows % 256 == 0 && (tiles(256, 128) >= 160 || S >= 16);
         if (N <= (staged ? 32 : 128)) return true;
-        const int64_t t = (int64_t)(rows / 32) * ((N + 63) / 64);
-        const int64_t rounds = ((staged ? tiles(256, 128) : (int64_t)((rows + 63) / 64) * ((N + 255) / 256)) + cus - 1) / cus;
-        return staged ? t <= 3 * cus * rounds : t * 2 <= (rounds == 1 ? 8 : 11) * cus * rounds;
+        const int64_t t = (int64_t)(rows / 32) * ((N + 63) / 64), row_tiles = (rows + 63) / 64;
+        if (staged) return t <= 3 * cus * ((tiles(256, 128) + cus - 1) / cus);
+        if (half_pairs()) {
+            const int64_t rounds = (row_tiles * ((N + 127) / 128) + 2 * cus - 1) / (2 * cus);
+            // (into a second round only while B fits an XCD's L2: 1280 x 5120 x 4096 at 32:2:16 65 against 43 us)
+            return rounds == 1 ? t * 8 <= 22 * cus : rounds == 2 && t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20);
+        }
+        const int64_t rounds = (row_tiles * ((N + 255) / 256) + cus - 1) / cus;
+        return rounds <= 2 && t <= 4 * cus * rounds;
     }
     // 64 x 256 tiles: many tiles of few k-steps, m >= 32, row-major
     bool short_k_many() const { return m >= 32 && !transposed && tiles(64, 256) >= 2048 && S <= 8; }
@@ -221,9 +231,12 @@ const Rule kRules[] = {
     // half-tile kernels are 9-24 % ahead; with 32 k-steps or more dense staging leads at any tile count, 1.2-3.4x on 1024 x 4096,
     // 1280 x 5120 and 12288 x 12288)
     {V_HALF, spatha::SPMM_VARIANT_DSH256x128_S3_C8, [](const Shape& s) { return s.tiles(256, 128) >= 160 || s.S >= 16; }},
-    // the 256-wide tile is never behind the 128-wide one with two stages by more than 7 %, and up to 2x ahead
+    // 128-wide tiles in pairs of workgroups lead the 256-wide ones, one workgroup a CU, by 2-20 % at any tile count (1024 x 4096 x
+    // 4096 at 32:2:16 19.8 against 23.0 us, 12288 x 12288 x 2048 at 32:2:32 161 against 191); with longer k-loops, where only one
+    // of them fits a CU, they trail by 1.2-1.6x (12288 x 12288 x 2048 at 32:2:16, 48 k-steps: 538 against 336 us)
+    {V_HALF, spatha::SPMM_VARIANT_H64x128_S2, [](const Shape& s) { return s.half_pairs(); }},
     {V_HALF, spatha::SPMM_VARIANT_H64x256_S2, [](const Shape& s) { return s.N > 128; }},
-    // (three stages of 128 leave two waves per CU)
+    // (three stages of 128 leave one workgroup of four waves per CU)
     {V_HALF, spatha::SPMM_VARIANT_H64x128_S2, [](const Shape&) { return true; }},
     {V_HALF, spatha::SPMM_VARIANT_H64x128_S3, [](const Shape&) { return true; }},
 
@@ -360,7 +373,7 @@ int pick_variant(const spatha_spmm_plan* plan, int N, int variant, bool fused = 
     if (variant != spatha::SPMM_VARIANT_AUTO)
         return variant < spatha::SPMM_VARIANT_COUNT && variant_ok(plan, N, variant, fused) ? variant : -1;
     Shape s;
-    s.v = plan->geo.v; s.m = plan->geo.m; s.rows = plan->geo.rows; s.N = N; s.S = plan->S;
+    s.v = plan->geo.v; s.m = plan->geo.m; s.rows = plan->geo.rows; s.cols = plan->geo.cols; s.N = N; s.S = plan->S;
     s.cus = plan->cus > 0 ? plan->cus : 256;
     s.fused = fused;
     s.transposed = out_layout == SPATHA_OUT_TRANSPOSED;

@@ -391,21 +391,23 @@ static hipError_t launch_pipe(const SpmmParams& p, hipStream_t stream) {
 // A 64-row wave tile then spans two V blocks, each with its own column-loc, so a stage holds TWO
 // gathered sets of 64 B rows and the packed operands use the "half tile" row order: instruction
 // row (mb, 4*ib + r) holds tile row 32*(mb/2) + 8*ib + 4*(mb%2) + r, so that instructions 0, 1
-// multiply the first set and instructions 2, 3 the second.  A lane ends up with two runs of 8
-// consecutive matrix rows (8*ib .. +7 and 32 + 8*ib .. +7) of one output column.
+// multiply the first set and instructions 2, 3 the second.  A lane ends up with 8 consecutive
+// matrix rows (8*ib .. +7 of its wave's half) of one output column.
 // The row tables of the tile's two halves sit in LDS as 16-bit row numbers (0xffff = zero row).
-// Tile 64 x (64*WN), one wave per 64 columns; everything else as in spmm_pipe_kernel.
+// Tile 64 x (64*WN); everything else as in spmm_pipe_kernel.
+// Two waves per 64 columns, one per half of the tile's rows: each reads only the gathered set of its own half, and twice as many
+// waves issue DMA and fragment reads (one wave for both halves, the form before this one, filled at half the rate a CU's loads
+// reach: 1024 x 4096 x 4096 at 32:2:16 24.9 us on 64 x 256 tiles, now 23.0, 26.7 on 64 x 128 ones, now 19.8).
 // ---------------------------------------------------------------------------
 // Fused epilogue (t = fp16(acc) + bias[row], then the activation in fp32) for the half-tile operand order: the lane's
-// values of instruction mb are tile rows 32*(mb/2) + 8*ib + 4*(mb%2) + r.  `hi_rows` is false for the padded second half
-// of a last tile (rows % 64 == 32), whose bias entries do not exist.
+// values of instruction mb are rows row8 + 4*mb + r.  `rows_exist` is false for the padded second half of a last tile
+// (rows % 64 == 32), whose bias entries do not exist.
 template <int ACT>
-__device__ __forceinline__ void fused_bias_act_half_impl(float4_t (&acc)[4][4], const uint16_t* bias, int64_t m0, int ib,
-                                                         bool hi_rows) {
+__device__ __forceinline__ void fused_bias_act_half_impl(float4_t (&acc)[2][4], const uint16_t* bias, int64_t row8, bool rows_exist) {
 #pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
+    for (int mb = 0; mb < 2; mb++) {
         half4_t bv = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
-        if (bias && (mb < 2 || hi_rows)) bv = *(const half4_t*)(bias + m0 + 32 * (mb >> 1) + 8 * ib + 4 * (mb & 1));
+        if (bias && rows_exist) bv = *(const half4_t*)(bias + row8 + 4 * mb);
 #pragma unroll
         for (int nb = 0; nb < 4; nb++) {
             float4_t v = acc[mb][nb];
@@ -419,27 +421,28 @@ __device__ __forceinline__ void fused_bias_act_half_impl(float4_t (&acc)[4][4], 
         }
     }
 }
-__device__ __forceinline__ void fused_bias_act_half(float4_t (&acc)[4][4], const uint16_t* bias, int64_t m0, int ib, bool hi_rows,
-                                                    int act) {
-    if (act == SPATHA_ACT_GELU) fused_bias_act_half_impl<SPATHA_ACT_GELU>(acc, bias, m0, ib, hi_rows);
-    else if (act == SPATHA_ACT_GELU_TANH) fused_bias_act_half_impl<SPATHA_ACT_GELU_TANH>(acc, bias, m0, ib, hi_rows);
-    else fused_bias_act_half_impl<SPATHA_ACT_NONE>(acc, bias, m0, ib, hi_rows);
+__device__ __forceinline__ void fused_bias_act_half(float4_t (&acc)[2][4], const uint16_t* bias, int64_t row8, bool rows_exist, int act) {
+    if (act == SPATHA_ACT_GELU) fused_bias_act_half_impl<SPATHA_ACT_GELU>(acc, bias, row8, rows_exist);
+    else if (act == SPATHA_ACT_GELU_TANH) fused_bias_act_half_impl<SPATHA_ACT_GELU_TANH>(acc, bias, row8, rows_exist);
+    else fused_bias_act_half_impl<SPATHA_ACT_NONE>(acc, bias, row8, rows_exist);
 }
 
 template <int WN, int NS, int OUT_LAYOUT>
-__global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
+__global__ __launch_bounds__(WN * 128) void spmm_half_kernel(SpmmParams p) {
+    constexpr int WAVES = WN * 2, MB = 2;
     constexpr int BN = WN * 64;
     constexpr int ROW_BYTES = BN * 2;
     constexpr int B_BYTES = 64 * ROW_BYTES;          // one gathered set
     constexpr int STAGE_BYTES = 2 * B_BYTES + APACK_BLOCK;
     constexpr int CHUNKS = BN / 8;
     constexpr int RPI = 1024 / ROW_BYTES;            // rows one DMA instruction covers
-    constexpr int NB_LOADS = 128 / RPI / WN;         // B DMA instructions per wave per stage (both sets)
-    constexpr int NA_X4 = 4 / WN;
+    constexpr int NB_LOADS = 128 / RPI / WAVES;      // B DMA instructions per wave per stage (both sets)
+    constexpr int NA_X4 = WAVES < 4 ? 4 / WAVES : 1;      // (eight waves: the last four carry the index words)
     constexpr int L = NB_LOADS + NA_X4 + 1;
     constexpr int PA = NS - 1;
     constexpr int PITCH_C = 144;
     static_assert(WN == 2 || WN == 4, "A operand split");
+    static_assert(WAVES <= 4 || NS == 2, "waves with unequal shares of a stage wait for everything");
     static_assert((NS - 2) * L < 64, "vmcnt range");
 
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -455,7 +458,8 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
     const int tile_n = static_tile_column(place, xcd, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wn = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave >> 1, half = wave & 1;
     const int m0 = tile_m * 64, n0 = tile_n * BN;
     const int S = p.S, N = p.N;
     const char* a_src = (const char*)p.apack + ((int64_t)tile_m * S) * APACK_BLOCK;
@@ -466,7 +470,7 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
     const char* zero_src = (const char*)p.zeros + lane * 16;
 #pragma unroll
     for (int j = 0; j < NB_LOADS; j++) {
-        const int rho = (wn * NB_LOADS + j) * RPI + slot_row;          // 0..127; the swizzle only sees rho % 8
+        const int rho = (wave * NB_LOADS + j) * RPI + slot_row;          // 0..127; the swizzle only sees rho % 8
         const int src_chunk = slot_chunk ^ ((rho & 7) << 1);
         const int col = n0 + src_chunk * 8;
         b_col_off[j] = (col < N) ? (int64_t)col * 2 : -1;
@@ -475,10 +479,10 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
         const uint32_t stage = smem_base + (s % NS) * STAGE_BYTES;
         uint32_t rows[NB_LOADS];
 #pragma unroll
-        for (int j = 0; j < NB_LOADS; j++) rows[j] = lds_rt[s * 128 + (wn * NB_LOADS + j) * RPI + slot_row];
+        for (int j = 0; j < NB_LOADS; j++) rows[j] = lds_rt[s * 128 + (wave * NB_LOADS + j) * RPI + slot_row];
 #pragma unroll
         for (int j = 0; j < NB_LOADS; j++) {
-            const int inst = wn * NB_LOADS + j;
+            const int inst = wave * NB_LOADS + j;
             const bool ok = (rows[j] != 0xffffu) && (b_col_off[j] >= 0);
             const char* src = (const char*)p.B + (int64_t)rows[j] * N * 2 + b_col_off[j];
             src = ok ? src : zero_src;
@@ -486,18 +490,22 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
         }
         const char* ab = a_src + (int64_t)s * APACK_BLOCK;
         const uint32_t a_lds = stage + 2 * B_BYTES;
+        if (WAVES <= 4 || wave < 4) {
 #pragma unroll
-        for (int k = 0; k < NA_X4; k++) {
-            const int mb = (WN >= 4) ? wn : wn * NA_X4 + k;
-            dma_b128(ab + mb * 1024 + lane * 16, a_lds + mb * 1024);
+            for (int k = 0; k < NA_X4; k++) {
+                const int mb = wave * NA_X4 + k;
+                dma_b128(ab + mb * 1024 + lane * 16, a_lds + mb * 1024);
+            }
         }
-        const int d = wn & 1;
-        dma_b32(ab + 4096 + d * 256 + lane * 4, a_lds + 4096 + d * 256);
+        if (WAVES <= 4 || wave >= 6) {
+            const int d = wave & 1;
+            dma_b32(ab + 4096 + d * 256 + lane * 4, a_lds + 4096 + d * 256);
+        }
     };
 
-    float4_t acc[4][4];
+    float4_t acc[MB][4];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int a = 0; a < MB; a++)
 #pragma unroll
         for (int b = 0; b < 4; b++) acc[a][b] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
@@ -518,7 +526,7 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
         const uint32_t* rt0 = p.rowtab + (int64_t)(m0 / p.v) * S * 64;
         const uint32_t* rt1 = p.rowtab + (int64_t)((m0 + 32) / p.v) * S * 64;
         const bool second_half = m0 + 32 < p.rows;      // rows % 64 == 32: the last tile's second half is padding
-        for (int i = tid; i < S * 128; i += WN * 64) {
+        for (int i = tid; i < S * 128; i += WAVES * 64) {
             const int s = i >> 7, rho = i & 63;
             const uint32_t r = (i & 64) ? (second_half ? rt1[s * 64 + rho] : 0xffffffffu) : rt0[s * 64 + rho];
             lds_rt[i] = (r == 0xffffffffu) ? (uint16_t)0xffffu : (uint16_t)r;
@@ -535,74 +543,56 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
         wait_stages<L, NS - 2>(later);
         __syncthreads();
         const char* st = smem + (s % NS) * STAGE_BYTES;
-        half8_t a_cur[4];
+        const char* set = st + half * B_BYTES;
+        half8_t a_cur[2];
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) a_cur[mb] = *(const half8_t*)(st + a_off + mb * 1024);
-        const uint32_t i0 = *(const uint32_t*)(st + i_off), i1 = *(const uint32_t*)(st + i_off + 256);
-        half16_t lo0 = read_b_fragment<ROW_BYTES>(st, tr_off[0]);
-        half16_t hi0 = read_b_fragment<ROW_BYTES>(st + B_BYTES, tr_off[0]);
-        half16_t lo1 = read_b_fragment<ROW_BYTES>(st, tr_off[1]);
-        half16_t hi1 = read_b_fragment<ROW_BYTES>(st + B_BYTES, tr_off[1]);
+        for (int mb = 0; mb < 2; mb++) a_cur[mb] = *(const half8_t*)(st + a_off + (half * 2 + mb) * 1024);
+        const uint32_t i0 = *(const uint32_t*)(st + i_off + half * 256);
+        half16_t b0 = read_b_fragment<ROW_BYTES>(set, tr_off[0]);
+        half16_t b1 = read_b_fragment<ROW_BYTES>(set, tr_off[1]);
         __builtin_amdgcn_sched_barrier(0);
         if (s + PA < S) issue_stage(s + PA);
         __builtin_amdgcn_sched_barrier(0);
-        SPATHA_MMA2LO(0, lo0)
-        SPATHA_MMA2HI(0, hi0)
+        SPATHA_MMA2LO(0, b0)
         __builtin_amdgcn_sched_barrier(0);
-        lo0 = read_b_fragment<ROW_BYTES>(st, tr_off[2]);
-        hi0 = read_b_fragment<ROW_BYTES>(st + B_BYTES, tr_off[2]);
+        b0 = read_b_fragment<ROW_BYTES>(set, tr_off[2]);
         __builtin_amdgcn_sched_barrier(0);
-        SPATHA_MMA2LO(1, lo1)
-        SPATHA_MMA2HI(1, hi1)
+        SPATHA_MMA2LO(1, b1)
         __builtin_amdgcn_sched_barrier(0);
-        lo1 = read_b_fragment<ROW_BYTES>(st, tr_off[3]);
-        hi1 = read_b_fragment<ROW_BYTES>(st + B_BYTES, tr_off[3]);
+        b1 = read_b_fragment<ROW_BYTES>(set, tr_off[3]);
         __builtin_amdgcn_sched_barrier(0);
-        SPATHA_MMA2LO(2, lo0)
-        SPATHA_MMA2HI(2, hi0)
-        SPATHA_MMA2LO(3, lo1)
-        SPATHA_MMA2HI(3, hi1)
+        SPATHA_MMA2LO(2, b0)
+        SPATHA_MMA2LO(3, b1)
     }
 
     // ------------------------------------------------------------------ write-out
     const int j = lane & 15, ib = lane >> 4;
     const bool hi_rows = m0 + 32 < p.rows;
-    if (p.fuse) fused_bias_act_half(acc, p.bias, m0, ib, hi_rows, p.act);
+    if (p.fuse) fused_bias_act_half(acc, p.bias, (int64_t)m0 + 32 * half + 8 * ib, half == 0 || hi_rows, p.act);
     const uint16_t* bias = p.fuse ? nullptr : p.bias;         // the plain transposed write-out adds the bias itself
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-        // per output column the lane holds rows 8*ib .. +7 (instructions 0, 1) and 32 + 8*ib .. +7 (2, 3)
-        const int64_t row_lo = (int64_t)m0 + ib * 8, row_hi = row_lo + 32;
-        half8_t bias_lo, bias_hi = {};
-        if (bias) {
-            bias_lo = *(const half8_t*)(bias + row_lo);
-            if (hi_rows) bias_hi = *(const half8_t*)(bias + row_hi);
-        }
+        // per output column the lane holds rows 8*ib .. +7 of its half
+        const int64_t row = (int64_t)m0 + 32 * half + ib * 8;
+        if (half == 0 || hi_rows) {
+            half8_t bias8 = {};
+            if (bias) bias8 = *(const half8_t*)(bias + row);
 #pragma unroll
-        for (int nb = 0; nb < 4; nb++) {
-            const int col = n0 + wn * 64 + nb * 16 + j;
-            half8_t lo, hi;
+            for (int nb = 0; nb < 4; nb++) {
+                const int col = n0 + wn * 64 + nb * 16 + j;
+                half8_t out;
 #pragma unroll
-            for (int mb = 0; mb < 2; mb++)
+                for (int mb = 0; mb < 2; mb++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    lo[mb * 4 + r] = (_Float16)acc[mb][nb][r];
-                    hi[mb * 4 + r] = (_Float16)acc[mb + 2][nb][r];
-                }
-            if (bias) {
-                lo = lo + bias_lo;
-                hi = hi + bias_hi;
-            }
-            if (col < N) {
-                uint16_t* dst = p.C + (int64_t)col * p.rows;
-                *(half8_t*)(dst + row_lo) = lo;
-                if (hi_rows) *(half8_t*)(dst + row_hi) = hi;
+                    for (int r = 0; r < 4; r++) out[mb * 4 + r] = (_Float16)acc[mb][nb][r];
+                if (bias) out = out + bias8;
+                if (col < N) *(half8_t*)(p.C + (int64_t)col * p.rows + row) = out;
             }
         }
     } else {
         __syncthreads();                 // every wave is done reading the stages
-        char* stg = smem + wn * (64 * PITCH_C);
+        char* stg = smem + wave * (16 * MB * PITCH_C);
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+        for (int mb = 0; mb < MB; mb++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int Lr = (4 * mb + r) * 4 + ib;
@@ -613,10 +603,10 @@ __global__ __launch_bounds__(WN * 64) void spmm_half_kernel(SpmmParams p) {
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
+        for (int it = 0; it < 2 * MB; it++) {
             const int Lr = it * 8 + (lane >> 3), ch = lane & 7;
-            // slab row Lr = (4*mb + r)*4 + ib  ->  tile row 32*(mb/2) + 8*ib + 4*(mb%2) + r
-            const int row = 32 * (Lr >> 5) + 8 * (Lr & 3) + 4 * ((Lr >> 4) & 1) + ((Lr >> 2) & 3);
+            // slab row Lr = (4*mb + r)*4 + ib  ->  tile row 32*half + 8*ib + 4*mb + r
+            const int row = 32 * half + 8 * (Lr & 3) + 4 * ((Lr >> 4) & 1) + ((Lr >> 2) & 3);
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(stg + Lr * PITCH_C + ch * 16);
             if (col < N && m0 + row < p.rows) store_c16(p.C + ((int64_t)m0 + row) * N + col, v);
@@ -639,7 +629,7 @@ static hipError_t launch_half(const SpmmParams& p, hipStream_t stream) {
     }
     const int tiles = p.tiles_m * p.tiles_n;
     const int chunk = (tiles + 7) / 8;
-    hipLaunchKernelGGL(kern, dim3(chunk * 8), dim3(WN * 64), lds, stream, p);
+    hipLaunchKernelGGL(kern, dim3(chunk * 8), dim3(WN * 128), lds, stream, p);
     return hipGetLastError();
 }
 
