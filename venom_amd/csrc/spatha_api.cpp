@@ -169,39 +169,38 @@ struct Shape {
         return tn <= 4 && T * tn > grid && F * tn <= grid && last > 128;
     }
     // Small products: kernels 23 (64 x 64 tiles) and 24 (32 x 64), straight from the L2, k-steps over a tile's waves (spmm_skinny.hip).
-    // Against the kernels chosen otherwise (ten layer shapes, 72 .. 2048 tokens, both layouts):
-    //   V % 64 == 0, at most one 64 x 64 tile per CU: 1.1x (768 x 3072 x 1040 at 128:2:32) .. 3.2x (1024 x 4096 x 128 at 64:2:16).
-    //   V % 128 == 0, up to 1.25 tiles per CU: 1.0-1.1x; beyond that 0.8-1.06x.
-    //   V % 64 == 0 only, whose staged kernels serve 64 or 256 matrix rows per tile: up to 1.6 tiles per CU 1.01-1.6x, with dense
-    //   staging (m <= 8) and up to ten k-steps at two tiles per CU still 1.22-1.25x; at 2.5 tiles per CU 0.8-0.99x.
+    // Against the kernels chosen otherwise (nine layer shapes x ten formats, 104 .. 4096 tokens, both layouts; geometric means):
+    //   V % 128 == 0:      at most one tile per CU 1.3-2.2x; up to 1.25 1.03-1.08x, up to 1.6 row-major
+    //                      1.04-1.08x and transposed 0.95-1.01x (both 0.94-0.97x from 29 k-steps on); up to 2
+    //                      row-major 1.06x and transposed 0.96x up to ten k-steps, 0.95-1.0x with more; beyond 0.55-0.84x.
+    //   V % 64 == 0 only:  up to one tile per CU 1.4-3.0x, up to two 1.08-1.5x; up to 2.5, m > 8, more than ten k-steps 1.10-1.18x
+    //                      (ten or fewer 0.88x; m <= 8 0.93-1.0x); beyond 0.4-1.0x.
     // k-loops of 96 steps on V % 128 == 0 are what split runs are for (12288 x 49152 x 128 at 128:2:16: 48 us in two parts, 71 here).
     // (Three k-steps or fewer at m <= 8 keep the dense staging that 512 x 256 x 256 at 64:2:8 is expected on.)
     bool direct64() const {
         const int64_t t = (int64_t)(rows / 64) * ((N + 63) / 64);
-        if (v % 128 == 0) return S < 96 && t * 4 <= cus * 5;
+        if (v % 128 == 0)
+            return S < 96 && (t <= cus || (S <= 28 && t * 20 <= cus * (transposed ? 25 : 32)) || (S <= 10 && !transposed && t <= 2 * cus));
         if (m <= 8 && S <= 3) return false;
-        return t * 10 <= cus * 16 || (m <= 8 && S <= 10 && t <= 2 * cus);
+        return t <= 2 * cus || (m > 8 && S > 10 && t * 2 <= 5 * cus);
     }
     // V % 64 != 0: 64 x 128 gathered tiles run two workgroups a CU as long as the row table leaves room for it (75 KB of stages + 256
     // bytes a k-step, twice: up to 28 k-steps)
     bool half_pairs() const { return S <= 28; }
     // V % 64 != 0: direct 32 x 64 tiles always up to 32 columns and, where nothing is dense-staged, up to 128 (2-5x ahead of the
-    // gathered tiles); above that against the rounds of the kernel they replace: a k-step of a round takes 0.9-1.4 us on gathered
-    // tiles, 0.87 us on dense-staged ones, a k-step of a tile here 0.8-1.3 ns.  At 1040 tokens: 1024 x 4096 13.5 against 17.1 us at
-    // 32:2:16, 21.9 against 30.3 (staged) at 32:2:8; 3840 x 1280 at 32:2:10 14.0 against 18.8; 12288 x 12288 x 304 at 32:2:16 76
-    // against 115; at 2048 tokens 768 x 3072 at 32:2:10 is behind (17.9 against 15.4).
+    // gathered tiles); above that up to three tiles per CU (1.08-2.1x; at four 0.98-1.0x), with more than ten k-steps up to four
+    // (1.10-1.16x; at eight 0.8-0.93x).  Where the replaced kernel is one step into a second round, also as long as B fits an XCD's L2
+    // (4096 x 1024 x 1040 at 32:2:10 14.0 against 16.8 us; 1280 x 5120 x 4096 at 32:2:16, B 42 MB, 37 against 43 but at other
+    // shapes 10 % behind).
     bool direct32() const {
         const bool staged = m <= 8 && rows % 256 == 0 && (tiles(256, 128) >= 160 || S >= 16);
         if (N <= (staged ? 32 : 128)) return true;
         const int64_t t = (int64_t)(rows / 32) * ((N + 63) / 64), row_tiles = (rows + 63) / 64;
-        if (staged) return t <= 3 * cus * ((tiles(256, 128) + cus - 1) / cus);
-        if (half_pairs()) {
-            const int64_t rounds = (row_tiles * ((N + 127) / 128) + 2 * cus - 1) / (2 * cus);
-            // (into a second round only while B fits an XCD's L2: 1280 x 5120 x 4096 at 32:2:16 65 against 43 us)
-            return rounds == 1 ? t * 8 <= 22 * cus : rounds == 2 && t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20);
-        }
-        const int64_t rounds = (row_tiles * ((N + 255) / 256) + cus - 1) / cus;
-        return rounds <= 2 && t <= 4 * cus * rounds;
+        if (t <= (S > 10 ? 4 : 3) * cus) return true;
+        if (staged) return false;
+        const int64_t at_once = half_pairs() ? 2 * cus : cus, width = half_pairs() ? 128 : 256;
+        const int64_t rounds = (row_tiles * ((N + width - 1) / width) + at_once - 1) / at_once;
+        return rounds == 2 && (half_pairs() ? t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20) : t <= 8 * cus);
     }
     // 64 x 256 tiles: many tiles of few k-steps, m >= 32, row-major
     bool short_k_many() const { return m >= 32 && !transposed && tiles(64, 256) >= 2048 && S <= 8; }
