@@ -119,26 +119,33 @@ static bool& lds_attr_flag(const void* kern) {
 // ---------------------------------------------------------------------------
 // x * Phi(x) = max(x, 0) - a * Phi(-a), a = |x|: only the lower tail is evaluated, where Phi keeps its relative accuracy
 // (1 + erf(x / sqrt 2) would cancel), as 2^P(a) with P the degree-7 interpolant of log2 Phi(-a) on [0, 5.75] (relative
-// error of Phi below 5e-6; beyond 5.75 the term is under half the smallest fp16 subnormal).  Checked on the CPU over
-// every fp16 input: 99.4 % of the fp16 results equal the rounded exact value, none is more than one step away.
-// 14 instructions + one exponential (the erfc form with a reciprocal and an exponential needed 27 issue slots).
+// error of Phi below 5e-6).  Beyond 5.75 P falls on by itself (leading coefficient negative, P < -27.7), so the term stays under
+// half the smallest fp16 subnormal without a select.  Checked on the CPU over every fp16 input: 99.4 % of the fp16 results equal the
+// rounded exact value, none is more than one step away.  A write-out with GELU is bound by these instructions (4 clocks each per 64
+// values, 16 for an exponential): 12 + one exponential (14 with a select, 27 issue slots in the erfc form).
 __device__ __forceinline__ float act_gelu_erf(float x) {
+#pragma clang fp contract(off)
     const float a = fabsf(x);
-    const float ac = fminf(a, 5.75f);
-    float p = fmaf(ac, -1.920561127e-06f, 6.327379007e-05f);
-    p = fmaf(ac, p, -9.432987473e-04f);
-    p = fmaf(ac, p, 8.555782832e-03f);
-    p = fmaf(ac, p, -5.405129916e-02f);
-    p = fmaf(ac, p, -4.583827060e-01f);
-    p = fmaf(ac, p, -1.151278015e+00f);
-    p = fmaf(ac, p, -9.999938734e-01f);
-    const float tail = a > 5.75f ? 0.0f : a * __builtin_amdgcn_exp2f(p);
+    float p = fmaf(a, -1.920561127e-06f, 6.327379007e-05f);
+    p = fmaf(a, p, -9.432987473e-04f);
+    p = fmaf(a, p, 8.555782832e-03f);
+    p = fmaf(a, p, -5.405129916e-02f);
+    p = fmaf(a, p, -4.583827060e-01f);
+    p = fmaf(a, p, -1.151278015e+00f);
+    p = fmaf(a, p, -9.999938734e-01f);
+    const float phi = __builtin_amdgcn_exp2f(p);
+    const float tail = fminf(a, 65504.0f) * phi;           // (not a * phi: an infinite a meets phi = 0)
     return fmaxf(x, 0.0f) - tail;
 }
+// 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)): no cancellation for negative x; exp -> inf gives -0, exp -> 0 gives x.  1 / d is the
+// reciprocal instruction's result with one Newton step (where d is infinite and the step's residual NaN, -1 takes its place and
+// leaves 0): three instructions where a correctly rounded division takes ten.
+// The fp16 results are the division's bit for bit (every fp16 input); 4096 x 1024 x 16384 with this write-out, transposed: 97 -> 83 us at
+// 64:2:8, 82 -> 70 us at 128:2:16 (57 and 46 without an activation).
 __device__ __forceinline__ float act_gelu_tanh(float x) {
-    // 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)): no cancellation for negative x; exp -> inf gives -0, exp -> 0 gives x
     const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-    return x * __frcp_rn(1.0f + __expf(-2.0f * u));
+    const float d = 1.0f + __expf(-2.0f * u), r = __builtin_amdgcn_rcpf(d);
+    return x * fmaf(fmaxf(fmaf(-d, r, 1.0f), -1.0f), r, r);
 }
 template <int ACT>
 __device__ __forceinline__ void fused_bias_act_impl(float4_t (&acc)[4][4], const uint16_t* bias, int64_t row16) {
