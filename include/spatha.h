@@ -204,6 +204,13 @@ int spatha_spmm_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, 
 int spatha_spmm_run_fused(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev,
                           uint16_t* out_dev, int out_layout, int activation, int variant, void* stream);
 
+/* A few tokens as a layer holds them: out[tokens x rows] = x[tokens x cols] A^T (+ bias), fp16, any token count up to 16 - the product of
+ * spatha_spmm_run with the transposed layout, without the transposed copy of x.  x_dev, out_dev and bias_dev (may be NULL) 16-byte
+ * aligned.  SPATHA_ERR_UNSUPPORTED: more tokens, tokens * cols beyond 64 Ki entries or so (they are kept in LDS), or more row
+ * tiles than compute units; use spatha_spmm_run. */
+int spatha_spmm_run_tokens(const spatha_spmm_plan* plan, const uint16_t* x_dev, int tokens, const uint16_t* bias_dev, uint16_t* out_dev,
+                           void* stream);
+
 /* spatha_spmm_run_fused (automatic kernel choice) for callers that bring scratch memory: with a workspace the library may
  * split k-loops over several workgroups where tiles alone leave compute units idle: few tiles with long k-loops (small
  * rows x N and large K, the "split-K for small M*N" case: e.g. 1024 x 16384 x 1024 at 128:2:8 runs 128 tiles of 128

@@ -92,3 +92,36 @@ def test_plan_run_refuses_and_writes_as_before(gpu):
                        (dict(B=B, variant=99), RuntimeError), (dict(B=B, activation="relu6"), ValueError), (dict(B=[1]), ValueError)):
         with pytest.raises(error):
             plan.run(**bad)
+
+
+@pytest.mark.parametrize("rows,cols,m,v", [(64, 64, 8, 64), (128, 200, 16, 128), (256, 1024, 8, 64), (1024, 3300, 10, 128), (128, 12288, 16, 64),
+                                           (32, 64, 8, 32), (96, 300, 7, 96), (512, 2048, 16, 32)])
+@pytest.mark.parametrize("tokens", [1, 2, 5, 8, 13, 16])
+def test_a_few_tokens_as_they_lie(gpu, rows, cols, m, v, tokens):
+    """spatha_spmm_run_tokens against the oracle, bit for bit on integer operands, with and without a bias; one token more than it
+    takes, and more columns than the LDS holds, are refused."""
+    import numpy as np
+
+    import oracle
+    from venom_amd import format as F
+
+    vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=rows + tokens, integer_values=True)
+    rng = np.random.default_rng(cols)
+    x = rng.integers(-4, 5, size=(tokens, cols)).astype(np.float16)
+    bias = rng.integers(-3, 4, size=rows).astype(np.float16)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
+    plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
+    dx, dbias = dev(x), dev(bias)
+    L = _lib.lib()
+    for b in (None, dbias):
+        out = torch.full((tokens, rows), float("nan"), dtype=torch.float16, device=gpu)
+        status = L.spatha_spmm_run_tokens(plan._handle, dx.data_ptr(), tokens, None if b is None else b.data_ptr(), out.data_ptr(),
+                                          spatha._stream_ptr(gpu))
+        if tokens * cols > 63 * 1024:
+            assert status == 3
+            continue
+        assert status == 0
+        want = oracle.spmm(vals, meta, columns, rows, cols, 2, m, v, np.ascontiguousarray(x.T), bias=None if b is None else bias,
+                           transposed_out=True)
+        assert np.array_equal(out.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    assert L.spatha_spmm_run_tokens(plan._handle, dx.data_ptr(), 17, None, dx.data_ptr(), spatha._stream_ptr(gpu)) == 3

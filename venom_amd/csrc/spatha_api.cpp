@@ -817,6 +817,25 @@ int spatha_spmm_run_fused(const spatha_spmm_plan* plan, const uint16_t* B_dev, i
     return spatha::plan_run(plan, B_dev, N, bias_dev, out_dev, out_layout, activation, true, variant, stream);
 }
 
+int spatha_spmm_run_tokens(const spatha_spmm_plan* plan, const uint16_t* x_dev, int tokens, const uint16_t* bias_dev, uint16_t* out_dev,
+                           void* stream) {
+    if (!plan || !x_dev || !out_dev || tokens <= 0) return SPATHA_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)x_dev & 15) || ((uintptr_t)out_dev & 15) || ((uintptr_t)bias_dev & 15)) return SPATHA_ERR_BAD_ARGUMENT;
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev != plan->device) return SPATHA_ERR_BAD_ARGUMENT;
+    const int cus = plan->cus > 0 ? plan->cus : 256;
+    if (!spatha::token_major_fits(plan->geo.rows, plan->geo.cols, tokens, plan->half_tiles != 0, cus)) return SPATHA_ERR_UNSUPPORTED;
+    spatha::SpmmParams p = {};
+    p.apack = plan->apack; p.rowtab = plan->rowtab;
+    p.B = x_dev; p.bias = bias_dev; p.C = out_dev; p.zeros = plan->zeros;
+    p.rows = plan->geo.rows; p.cols = plan->geo.cols; p.N = tokens; p.S = plan->S; p.v = plan->geo.v; p.m = plan->geo.m;
+    p.cus = cus;
+    p.act = SPATHA_ACT_NONE;
+    p.ksplit = 1;
+    const hipError_t e = spatha::launch_token_major(p, plan->half_tiles != 0, (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
 size_t spatha_spmm_workspace_bytes(const spatha_spmm_plan* plan, int N, int out_layout, int fused) {
     if (!plan || N <= 0 || N % 8 != 0) return 0;
     const int var = pick_variant(plan, N, spatha::SPMM_VARIANT_AUTO, fused != 0, out_layout);

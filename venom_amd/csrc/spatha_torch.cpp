@@ -262,6 +262,26 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
         bias_t = torch::zeros({rows}, x.options().requires_grad(false));
     }
     const torch::Tensor flat = x.dim() == 2 ? x : x.flatten(0, -2);
+    auto result = [&](torch::Tensor out, py::object kept) -> py::object {        // out: [tokens, rows] in whatever strides
+        if (x.dim() != 2) {
+            std::vector<int64_t> sizes(x.sizes().begin(), x.sizes().end());
+            sizes.back() = rows;
+            out = out.reshape(sizes);
+        }
+        return py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(out)), kept);
+    };
+    if (!feature_major && tokens <= 16 && flat.is_contiguous() && ((uintptr_t)flat.data_ptr() & 15) == 0) {
+        // a few tokens: the kernel reads them as they lie
+        hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+        const std::shared_ptr<spatha_spmm_plan> plan = plan_for(values, metadata, columns, rows, cols, n, m, v, stream);
+        torch::Tensor out = torch::empty({tokens, rows}, x.options().requires_grad(false));
+        const int status = spatha_spmm_run_tokens(plan.get(), (const uint16_t*)flat.data_ptr(), (int)tokens,
+                                                  (const uint16_t*)bias_t.data_ptr(), (uint16_t*)out.data_ptr(), stream);
+        if (status != SPATHA_ERR_UNSUPPORTED) {
+            check(status, "spatha_spmm_run_tokens");
+            return result(out, py::none());
+        }
+    }
     py::object kept = py::none();
     torch::Tensor rhs;              // its first element is that of a [cols, padded] matrix
     auto holds_padded_rows = [&](const torch::Tensor& t, int64_t pitch) {       // [cols, tokens] with rows `pitch` apart, all in memory
@@ -305,13 +325,7 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
     torch::Tensor out = run_full(metadata, columns, values, rhs, (int)padded, bias_ptr, rows, cols, v, n, m, !feature_major,
                                  feature_major ? activation : SPATHA_ACT_NONE, feature_major);
     if (padded != tokens) out = out.narrow(feature_major ? 1 : 0, 0, tokens);
-    if (feature_major) out = out.t();
-    if (x.dim() != 2) {
-        std::vector<int64_t> sizes(x.sizes().begin(), x.sizes().end());
-        sizes.back() = rows;
-        out = out.reshape(sizes);
-    }
-    return py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(out)), kept);
+    return result(feature_major ? out.t() : out, kept);
 }
 
 // SpmmPlan.run without a k-split, for operands in order; None where the caller's checks have to speak.  bias needs the transposed

@@ -89,6 +89,10 @@ hipError_t launch_skinny_family(int variant, int out_layout, const SpmmParams& p
 hipError_t launch_pingpong(int variant, int out_layout, const SpmmParams& p, hipStream_t stream);
 hipError_t launch_onehalf(int variant, int out_layout, const SpmmParams& p, hipStream_t stream);
 
+// up to 16 tokens x [N][cols] as they lie, transposed output (spmm_skinny.hip); token_major_fits: whether the launch takes them
+bool token_major_fits(int rows, int cols, int tokens, bool half_tiles, int cus);
+hipError_t launch_token_major(const SpmmParams& p, bool half_tiles, hipStream_t stream);
+
 hipError_t launch_pack(const uint16_t* values, const uint32_t* metadata, const uint32_t* columns, int rows, int cols,
                        int m, int v, int ksp, int S, int half_tiles, uint16_t* apack, uint32_t* rowtab, hipStream_t stream);
 

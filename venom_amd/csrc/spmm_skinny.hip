@@ -23,6 +23,9 @@ namespace spatha {
 // ---------------------------------------------------------------------------
 // LEAN (four column blocks only): see the main loop.  (The lean form is compiled for three waves per SIMD - three workgroups
 // of four waves per CU - which it reaches with 158 registers.)
+// halfs between two tokens in LDS: odd in 32-bit words, so that the sixteen tokens of a fragment row sit on different banks
+__host__ __device__ constexpr int token_pitch_halfs(int cols) { return (((cols + 7) / 8 * 4) | 1) * 2; }
+
 template <int NB, int W, bool HALF, bool LEAN>
 struct DirectCfg {
     static constexpr int MB = HALF ? 2 : 4;                                     // instruction-row blocks per tile
@@ -35,13 +38,16 @@ struct DirectCfg {
     static_assert(W * PB * NB <= 64, "partial tiles exceed 64 KB");
 };
 
-template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN = false>
+template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN = false, bool TOKEN_MAJOR = false>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu((DirectCfg<NB, W, HALF, LEAN>::WAVES_PER_EU))))
 void spmm_direct_kernel(SpmmParams p) {
     using Cfg = DirectCfg<NB, W, HALF, LEAN>;
     constexpr int MB = Cfg::MB, PB = Cfg::PB, CB = Cfg::CB;
     static_assert(NB == 1 || NB == 2 || NB == 4, "column blocks per tile");
-    __shared__ float4_t red[W][PB][NB][64];
+    typedef float4_t Red[PB][NB][64];
+    __shared__ Red fixed_red[TOKEN_MAJOR ? 1 : W];
+    extern __shared__ __attribute__((aligned(16))) char dyn[];      // TOKEN_MAJOR: the tokens, then the partial tiles
+    Red* red = TOKEN_MAJOR ? (Red*)dyn : fixed_red;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int S = p.S, N = p.N;
@@ -84,12 +90,38 @@ void spmm_direct_kernel(SpmmParams p) {
         for (int d = 0; d < MB / 2; d++) x.ix[d] = *(const uint32_t*)(q + 4096 + (half + d) * 256 + lane * 4);
     };
     const int col0 = (tile_n * 16 + li) * NB;       // this lane's NB columns: col0 + nb
+    const int token_pitch = token_pitch_halfs(p.cols);
+    if constexpr (TOKEN_MAJOR) {
+        // x [N][cols] -> LDS as it lies; columns N .. 15 of the tile are never stored, they multiply token 0
+        const int pieces = (p.cols + 7) >> 3;
+        for (int i = tid; i < N * pieces; i += W * 64) {
+            const int t = i / pieces, c = (i - t * pieces) * 8;
+            const uint16_t* src = p.B + (int64_t)t * p.cols + c;
+            uint32_t* dst = (uint32_t*)((uint16_t*)dyn + t * token_pitch + c);       // 4-byte aligned: the pitch is even
+            if ((p.cols & 7) == 0) {
+                const u32x4 v = *(const u32x4*)src;
+#pragma unroll
+                for (int k = 0; k < 4; k++) dst[k] = v[k];
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    if (c + k < p.cols) ((uint16_t*)dst)[k] = src[k];
+            }
+        }
+        __syncthreads();
+    }
+    const uint16_t* token = (const uint16_t*)dyn + (li < N ? li : 0) * token_pitch;
     auto load_b = [&](const u32x4 (&rt)[4], half16_t (&bf)[NB]) {
 #pragma unroll
         for (int fb = 0; fb < 4; fb++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const uint32_t row = rt[fb][j];
+                if constexpr (TOKEN_MAJOR) {
+                    const uint16_t h = token[row != 0xFFFFFFFFu ? row : 0u];
+                    bf[0][fb * 4 + j] = __builtin_bit_cast(_Float16, (uint16_t)(row != 0xFFFFFFFFu ? h : 0));
+                    continue;
+                }
                 const uint32_t voff = (row != 0xFFFFFFFFu && col0 < N) ? row * row_bytes + (uint32_t)col0 * 2u : 0xF0000000u;
                 if constexpr (NB == 1) {
                     const uint16_t h = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc_b, (int)voff, 0, 0);
@@ -165,6 +197,7 @@ void spmm_direct_kernel(SpmmParams p) {
             multiply(x, b0);
         }
     }
+    if constexpr (TOKEN_MAJOR) __syncthreads();      // the tokens have been read: the partial tiles take their place
     // Unit u of a pass: row block mb = pass + u % PB (rows 16 * ib + 4 * mb + r of a 64-row tile, 8 * ib + 4 * mb + r of a 32-row
     // one), columns col0 + (u / PB) * CB + c
     const int ib = kb;
@@ -274,6 +307,40 @@ static hipError_t launch_direct_family(const SpmmParams& p, hipStream_t stream) 
         case 408: return launch_direct<4, OUT_LAYOUT, 8, HALF>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+// A few tokens as they lie, x [N][cols] with N <= 16 (any count), transposed output: what the transposed copy ahead of the product
+// would hold is read from LDS, where every workgroup puts the tokens first.
+// (A layer of 1024 x 1024 at 64:2:8 on 8 tokens, whole call: 7.1 us, 12.1 with a transposing kernel ahead of the product.)
+template <int W, bool HALF>
+static hipError_t launch_token_major(SpmmParams p, hipStream_t stream) {
+    using Cfg = DirectCfg<1, W, HALF, false>;
+    p.tiles_m = p.rows / (HALF ? 32 : 64);
+    p.tiles_n = 1;
+    p.walk_group = 0;
+    const size_t tokens = (size_t)p.N * token_pitch_halfs(p.cols) * 2, partial = (size_t)W * Cfg::PB * 64 * sizeof(float4_t);
+    const size_t lds = ((tokens > partial ? tokens : partial) + 15) / 16 * 16;
+    auto kern = spmm_direct_kernel<1, SPATHA_OUT_TRANSPOSED, W, HALF, false, true>;
+    if (lds > 48 * 1024) {
+        bool& attr_set = lds_attr_flag((const void*)kern);
+        if (!attr_set) {
+            hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+            if (e != hipSuccess) return e;
+            attr_set = true;
+        }
+    }
+    hipLaunchKernelGGL(kern, dim3((p.tiles_m + 7) / 8 * 8), dim3(W * 64), lds, stream, p);
+    return hipGetLastError();
+}
+
+// (one workgroup a CU where the tokens take more than half of its LDS: not with more row tiles than CUs)
+bool token_major_fits(int rows, int cols, int tokens, bool half_tiles, int cus) {
+    return tokens <= 16 && (size_t)tokens * token_pitch_halfs(cols) * 2 <= 128 * 1024 && rows / (half_tiles ? 32 : 64) <= cus;
+}
+
+hipError_t launch_token_major(const SpmmParams& p, bool half_tiles, hipStream_t stream) {
+    if (half_tiles) return p.S > 12 ? launch_token_major<16, true>(p, stream) : launch_token_major<8, true>(p, stream);
+    return p.S > 12 ? launch_token_major<16, false>(p, stream) : launch_token_major<8, false>(p, stream);
 }
 
 hipError_t launch_skinny_family(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
