@@ -55,7 +55,7 @@ enum {
     // dense-staged B (m <= 8): all 16 m dense rows of a k-step staged once for the tile's 64-row blocks
     SPMM_VARIANT_DS256x128_S3_C8 = 11,  // eight 64 x 64 consumer waves + four producers
     SPMM_VARIANT_DS256x128_S3_PP = 12,  // the eight consumers in two phase groups
-    SPMM_VARIANT_SKINNY = 13,           // N <= 64: one 64-row tile per workgroup, k split over four waves, B straight from L2
+    SPMM_VARIANT_SKINNY = 13,           // N <= 64: one 64-row tile per workgroup, k split over its waves, B straight from L2
     // V % 64 != 0: a 64-row tile spans two V blocks
     SPMM_VARIANT_H64x256_S2 = 14,       // two gathered B sets per stage
     SPMM_VARIANT_H64x128_S3 = 15,
