@@ -46,6 +46,14 @@ class NMVectorSparsifier:
             SrNMTensor(self.n, self.m, self.tileM, tensor, mask, columns, tensor.device), tensor, grad_fmt)
 
 
+def _activation_key(flat):
+    """What a kept copy of `flat` (or a result computed from it) is known by: address, shape, strides, version counter, device, and the
+    stream and graph capture that it was computed on - another stream is not ordered behind the kernel that fills the copy, and a
+    graph replays only what was recorded into it."""
+    return (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device,
+            spatha._extension().stream_key(flat.get_device()) if flat.is_cuda else None)
+
+
 class SrnmSpmm(torch.nn.Module):
     """Drop-in for nn.Linear: y = x W^T + b with W in V:N:M."""
 
@@ -60,15 +68,15 @@ class SrnmSpmm(torch.nn.Module):
         self.nrows_sp, self.ncols_sp, self.nnz = w.nrows, w.ncols, w.nnz
 
     # The query, key and value projections of a layer read the same activation: its transposed copy is
-    # kept for the next call, keyed by address, shape and version counter of the input.  The input itself
-    # is kept alive alongside, so that its address cannot be handed to another tensor while the entry exists.
+    # kept for the next call, known by `_activation_key` of the input.  The input itself is kept alive
+    # alongside, so that its address cannot be handed to another tensor while the entry exists.
     _last_rhs = (None, None, None)
 
     @classmethod
     def _transposed(cls, flat):
         if flat.stride(0) == 1 and flat.stride(1) == flat.shape[0]:
             return flat.T              # feature-major already (the output of a fused feed-forward layer): no copy
-        key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
+        key = _activation_key(flat)
         if cls._last_rhs[0] == key:
             return cls._last_rhs[2].contiguous()       # (a copy for a ragged token count has padded rows)
         if flat.is_cuda and flat.dtype == torch.float16:
@@ -83,7 +91,7 @@ class SrnmSpmm(torch.nn.Module):
         """A producer that has x[..., features] feature-major already (x_t[features, tokens]) leaves it for the layer that reads
         x next, in place of the transposed copy that layer would make."""
         flat = torch.flatten(x, start_dim=0, end_dim=-2)
-        key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
+        key = _activation_key(flat)
         cls._last_rhs = (key, flat, x_t)
 
     @staticmethod
@@ -152,7 +160,7 @@ class _MergedProjections:
 
     def output(self, index, nrows, input):
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
-        key = (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device)
+        key = _activation_key(flat)
         if self._last[0] != key:
             out = SrnmSpmm._run_native(SrnmSpmm, self, flat, self.rows, self.cols)
             if out is None:

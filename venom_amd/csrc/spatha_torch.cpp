@@ -226,10 +226,22 @@ bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
     return t.defined() && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
 }
 
-// Is `key` the Python key (address, shape, strides, version, device) of `held`, and is x the same tensor at the same version?
-bool same_activation(const torch::Tensor& x, const torch::Tensor& held, const py::tuple& key) {
+// Where work issued now on torch's current stream of `device` runs: the stream, and the capture that records it (0: none).  What one
+// call has computed may be taken by a later one only from the same place: another stream is not ordered behind it, a graph replays
+// only what was recorded into it, and what was recorded has not run.
+py::tuple stream_key(int device) {
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
+    return py::make_tuple((uintptr_t)stream, status == hipStreamCaptureStatusActive ? id : 0ull);
+}
+
+// Is `key` the Python key (address, shape, strides, version, device, stream_key) of `held`, and is x the same tensor at the same
+// version, used in the same place?
+bool same_activation(const torch::Tensor& x, const torch::Tensor& held, const py::tuple& key, const py::tuple& place) {
     return x.data_ptr() == held.data_ptr() && x.sizes() == held.sizes() && x.strides() == held.strides() && x.device() == held.device() &&
-           key.size() == 5 && key[3].cast<int64_t>() == (int64_t)x._version();
+           key.size() == 6 && key[3].cast<int64_t>() == (int64_t)x._version() && place.equal(key[5]);
 }
 
 // One V:N:M layer on x [..., cols], without a trip through Python per part: the right-hand side (x feature-major already, the
@@ -283,6 +295,7 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
         }
     }
     py::object kept = py::none();
+    const py::tuple place = stream_key(device);
     torch::Tensor rhs;              // its first element is that of a [cols, padded] matrix
     auto holds_padded_rows = [&](const torch::Tensor& t, int64_t pitch) {       // [cols, tokens] with rows `pitch` apart, all in memory
         return pitch == padded && (size_t)((t.storage_offset() + cols * padded) * 2) <= t.storage().nbytes();
@@ -294,7 +307,7 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
         if (flat.stride(0) == 1 && flat.stride(1) == tokens) {
             copy = flat.t();
         } else if (last.size() == 3 && THPVariable_Check(last[1].ptr()) && THPVariable_Check(last[2].ptr()) &&
-                   same_activation(flat, THPVariable_Unpack(last[1].ptr()), last[0].cast<py::tuple>())) {
+                   same_activation(flat, THPVariable_Unpack(last[1].ptr()), last[0].cast<py::tuple>(), place)) {
             copy = THPVariable_Unpack(last[2].ptr());
         } else {
             const torch::Tensor dense = flat.contiguous();
@@ -315,7 +328,7 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
                 strides[d] = py::int_(flat.stride(d));
             }
             kept = py::make_tuple(py::make_tuple(py::int_((uintptr_t)flat.data_ptr()), shape, strides, py::int_((int64_t)flat._version()),
-                                                 held.attr("device")),
+                                                 held.attr("device"), place),
                                   held, made);
         }
         if (copy.dim() != 2 || copy.size(0) != cols || copy.size(1) != tokens || copy.scalar_type() != torch::kFloat16) return py::none();
@@ -430,6 +443,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
             py::arg("A_num_cols"), py::arg("vec_length"), py::arg("n"), py::arg("m"), py::arg("activation") = 0,
             py::arg("transposed_out") = false);
     mod.def("layer_spmm", &layer_spmm, "one V:N:M layer, right-hand side and product, or None");
+    mod.def("stream_key", &stream_key, "(stream, capture) that work issued now on this device goes to", py::arg("device"));
     mod.def("transpose", &transpose_f16, "x.T of an fp16 matrix through the library's kernel, or None");
     mod.def("plan_run", &plan_run, "a plan's product, or None, or the status of a refusal");
     mod.def("clear_plan_cache", &clear_plan_cache, "drop every cached plan");
