@@ -60,6 +60,38 @@ def test_layers_take_any_token_count_and_stride(gpu, shape):
         assert torch.equal(up(x), direct(up, x)) and not torch.equal(up(x), first)
 
 
+def test_layers_take_feature_major_views_at_any_address(gpu):
+    """A feature-major input that starts in the middle of a buffer: a pitch that equals the padded token count does not make it a
+    right-hand side that can be read in 16-byte pieces."""
+    from venom_amd.bert import SrnmSpmm
+
+    torch.manual_seed(0)
+    up = SrnmSpmm(torch.nn.Linear(128, 256).half().to(gpu), 2, 8, 64, magnitude=True)
+    down = SrnmSpmm(torch.nn.Linear(256, 128).half().to(gpu), 2, 16, 32, magnitude=True)
+
+    def direct(layer, x):
+        return spatha.spmm(layer.metadata, layer.columns, layer.values, x.T.contiguous(), layer.bias, layer.nrows_sp, layer.ncols_sp,
+                           x.shape[0], layer.v, layer.n, layer.m)
+
+    with torch.no_grad():
+        views = [torch.randn(129, 8, device=gpu).half()[:128, 2:7].T, torch.randn(129, 24, device=gpu).half()[:128, 1:20].T,
+                 torch.randn(129, 40, device=gpu).half()[:128, 3:40].T]
+        wide = up.forward_feature_major(torch.randn(1037, 128, device=gpu).half())
+        for x in views:
+            assert x.data_ptr() % 16 != 0
+            for _ in range(2):
+                assert torch.equal(up(x), direct(up, x))
+                assert torch.equal(up.forward_feature_major(x), direct(up, x))
+        for first in (1, 3, 5, 8):
+            x = wide[first:, :128]
+            assert x.stride() == (1, 1040)
+            assert torch.equal(up(x), direct(up, x)) and torch.equal(up.forward_feature_major(x), direct(up, x))
+        assert torch.equal(down(wide[3:]), direct(down, wide[3:]))
+        refused = torch.randn(128 * 24 + 8, device=gpu).half()[1:1 + 128 * 24].view(128, 24).T      # as by the operator: no copy is due
+        with pytest.raises(RuntimeError):
+            up(refused)
+
+
 def test_layer_refuses_what_it_refused(gpu):
     from venom_amd.bert import SrnmSpmm
 

@@ -297,8 +297,10 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
     py::object kept = py::none();
     const py::tuple place = stream_key(device);
     torch::Tensor rhs;              // its first element is that of a [cols, padded] matrix
-    auto holds_padded_rows = [&](const torch::Tensor& t, int64_t pitch) {       // [cols, tokens] with rows `pitch` apart, all in memory
-        return pitch == padded && (size_t)((t.storage_offset() + cols * padded) * 2) <= t.storage().nbytes();
+    // [cols, tokens] with rows `pitch` apart, all in memory, readable in 16-byte pieces
+    auto holds_padded_rows = [&](const torch::Tensor& t, int64_t pitch) {
+        return pitch == padded && (size_t)((t.storage_offset() + cols * padded) * 2) <= t.storage().nbytes() &&
+               ((uintptr_t)t.data_ptr() & 15) == 0;
     };
     if (flat.stride(0) == 1 && flat.stride(1) >= tokens && holds_padded_rows(flat, flat.stride(1))) {
         rhs = flat;
@@ -332,7 +334,9 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
                                   held, made);
         }
         if (copy.dim() != 2 || copy.size(0) != cols || copy.size(1) != tokens || copy.scalar_type() != torch::kFloat16) return py::none();
-        rhs = copy.stride(1) == 1 && holds_padded_rows(copy, copy.stride(0)) ? copy : pad_columns(copy.contiguous());
+        if (copy.stride(1) == 1 && holds_padded_rows(copy, copy.stride(0))) rhs = copy;
+        else if (padded == tokens && ((uintptr_t)copy.data_ptr() & 15)) return py::none();       // the operator refuses the address
+        else rhs = pad_columns(copy.contiguous());
     }
     const uint16_t* bias_ptr = bias_t.defined() ? (const uint16_t*)bias_t.data_ptr() : nullptr;
     torch::Tensor out = run_full(metadata, columns, values, rhs, (int)padded, bias_ptr, rows, cols, v, n, m, !feature_major,
