@@ -85,7 +85,7 @@ class SpmmPlan:
         idle; the scratch memory it needs is `workspace` (a uint8 tensor on the GPU that was zero-filled once, e.g. by
         torch.zeros) or, if None, a buffer the plan keeps per stream."""
         if not split and (activation is None or activation in _ACTIVATIONS):
-            native = _plan_run_function()
+            native = _native("plan_run")
             if native is not None:
                 # operands in order run from here in one call; anything else comes back as None and meets the checks below
                 fused = activation is not None
@@ -207,10 +207,20 @@ def _extension():
     return _loaded_extension
 
 
-def _plan_run_function():
-    """The extension's `plan_run`, or None where plans belong to another build of the library (SPATHA_LIBRARY) than the one
-    the extension is linked to."""
-    return _extension().plan_run if _lib.IS_DEFAULT_BUILD else None
+_extension_absent = False        # an import has failed: the callers of `_native`, which do without, stop asking
+
+
+def _native(name):
+    """The extension's function of that name, or None where plans belong to another build of the library (SPATHA_LIBRARY) than the
+    one the extension is linked to, or where there is no extension: plans and the transposing kernel need libspatha.so alone."""
+    global _extension_absent
+    if _extension_absent or not _lib.IS_DEFAULT_BUILD:
+        return None
+    try:
+        return getattr(_extension(), name)
+    except RuntimeError:
+        _extension_absent = True
+        return None
 
 
 def clear_plan_cache():
@@ -227,8 +237,9 @@ def invalidate_plans(A_values):
 def transpose(x):
     """x[rows, cols] fp16, contiguous -> a new contiguous [cols, rows] tensor (what `x.T.contiguous()` returns),
     through the library's tiled kernel on torch's current stream."""
-    if _lib.IS_DEFAULT_BUILD:
-        out = _extension().transpose(x)
+    native = _native("transpose")
+    if native is not None:
+        out = native(x)
         if out is not None:
             return out
     _check_dev(x, torch.float16, "x")
