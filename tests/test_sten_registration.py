@@ -2,6 +2,10 @@
 is not installed here (its submodule is empty in the reference), so what is checked is that the hooks register what the
 reference's notebook registers (end2end/tests.ipynb cells 14 and 24) and that the registered functions compute the right
 thing; how STEN dispatches to them is STEN's business and is not covered."""
+import importlib
+import importlib.machinery
+import os
+import sys
 import types
 
 import numpy as np
@@ -44,6 +48,51 @@ def test_without_sten_the_harness_gets_the_stand_in():
     assert R.wrapper_class() is R.SparseTensorWrapper
     with pytest.raises(ImportError):
         R.register()
+
+
+def test_a_package_that_appears_later_is_found(tmp_path, monkeypatch):
+    """A search without result is not the last word: a package put into a folder of the path afterwards, one whose missing dependency
+    has been supplied, one that a finder of another kind serves."""
+    if R.sten_module() is not None:
+        pytest.skip("STEN is installed")
+    for name in ("sten", "sten_needs_this"):
+        monkeypatch.delitem(sys.modules, name, raising=False)
+    monkeypatch.syspath_prepend(str(tmp_path))
+    assert R.sten_module() is None and R.sten_module() is None
+    try:
+        (tmp_path / "sten.py").write_text("import sten_needs_this\nclass SparseTensorWrapper: pass\n")
+        importlib.invalidate_caches()
+        os.utime(tmp_path, ns=(1, 1))                        # (a second file within one tick of the clock)
+        assert R.sten_module() is None                       # there, but does not import
+        sys.modules["sten_needs_this"] = types.ModuleType("sten_needs_this")
+        assert R.sten_module() is not None and R.wrapper_class() is R.sten_module().SparseTensorWrapper
+        for name in ("sten", "sten_needs_this"):
+            del sys.modules[name]
+        (tmp_path / "sten.py").unlink()
+        importlib.invalidate_caches()
+        os.utime(tmp_path, ns=(2, 2))
+        assert R.sten_module() is None and R.sten_module() is None
+
+        class Finder:
+            there = False
+
+            def find_spec(self, name, path, target=None):
+                return importlib.machinery.ModuleSpec(name, self) if self.there and name == "sten" else None
+
+            def create_module(self, spec):
+                return None
+
+            def exec_module(self, module):
+                module.SparseTensorWrapper = R.SparseTensorWrapper
+
+        finder = Finder()
+        monkeypatch.setattr(sys, "meta_path", sys.meta_path + [finder])
+        assert R.sten_module() is None and R.sten_module() is None
+        finder.there = True
+        assert R.sten_module() is not None
+    finally:
+        for name in ("sten", "sten_needs_this"):
+            sys.modules.pop(name, None)
 
 
 def test_hooks_register_what_the_notebook_registers():

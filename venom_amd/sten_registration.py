@@ -12,7 +12,9 @@ this library:
 Where it cannot, `register()` raises ImportError and `wrapper_class()` hands out the two-method stand-in the harnesses need
 (`wrapped_from_dense(...)`, `.wrapped_tensor`).  `register(sten_module)` takes the module as an argument so that the hooks can
 be exercised against any object with STEN's registration interface."""
+import os
 import sys
+from importlib import machinery
 
 import torch
 
@@ -33,19 +35,44 @@ class SparseTensorWrapper:
         return SparseTensorWrapper(wrapped_tensor, dense, grad_fmt)
 
 
-_searched = None            # the search path on which STEN was last not found
+_absent = None              # the state of the search path in which there was no package of that name
+
+
+def _search_state():
+    """What a search for a package on the path would find is decided by: the folders, told apart and dated as the import system's
+    own listings of them are, and the finders.  None where a finder of another kind has the package, or cannot be asked."""
+    folders = []
+    for path in sys.path:
+        try:
+            st = os.stat(path or ".")
+            folders.append((path, st.st_dev, st.st_ino, st.st_mtime_ns))
+        except (OSError, ValueError, TypeError):
+            folders.append((path, None))
+    for finder in sys.meta_path:
+        if finder not in (machinery.BuiltinImporter, machinery.FrozenImporter, machinery.PathFinder):
+            try:
+                if finder.find_spec("sten", None) is not None:
+                    return None
+            except Exception:
+                return None
+    return folders, list(sys.meta_path), list(sys.path_hooks)
 
 
 def sten_module():
-    """The STEN package, or None where it is not installed.  A search that found nothing is not repeated on the same search path
-    (it walks every folder of it: 50 us, more than the conversion of a weight takes)."""
-    global _searched
-    if "sten" not in sys.modules and _searched == (sys.path, sys.meta_path):
+    """The STEN package, or None where it is not installed.  A search that found no package of that name is not repeated while
+    nothing in the folders of the path has changed (50 us, more than the conversion of a weight takes; the look at the folders:
+    10 us).  A package that is there but does not import is tried again every time."""
+    global _absent
+    state = None if "sten" in sys.modules else _search_state()
+    if state is not None and state == _absent:
         return None
     try:
         import sten
+    except ModuleNotFoundError as e:
+        if e.name == "sten":
+            _absent = state
+        return None
     except ImportError:
-        _searched = (list(sys.path), list(sys.meta_path))
         return None
     return sten
 
