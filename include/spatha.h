@@ -126,12 +126,14 @@ int spatha_vnm_select_columns_f32_gpu(const float* dense_abs, int rows, int cols
 /* Selector and encoder together on a matrix in DEVICE memory: dense_dev is row-major rows x cols, fp16 (value_bits 16) or fp32
  * (32), signed; values_dev (fp16, fp32 input rounded to nearest), metadata_dev and columns_dev hold n_values / n_metadata /
  * n_columns entries and are written whole.  The same arrays as the host path with exact_ties == 0 (the lower column among equal
- * magnitudes), without masks.  Stream ordered; nothing is allocated, copied or waited for. */
+ * magnitudes), without masks.  columns_dev on a 16-byte address, values_dev on an 8-byte one (SPATHA_ERR_BAD_ARGUMENT otherwise).
+ * Stream ordered; nothing is allocated, copied or waited for. */
 int spatha_vnm_convert_gpu(const void* dense_dev, int value_bits, int rows, int cols, int n, int m, int v, uint16_t* values_dev,
                            uint32_t* metadata_dev, uint32_t* columns_dev, void* stream);
 
 /* spatha_vnm_decode_f16 on DEVICE memory (dense_dev is overwritten).  A column offset that is not below m has no place in the
- * matrix: its entry is left out and *bad_dev, which the caller has zeroed, becomes 1.  Stream ordered. */
+ * matrix: its entry is left out and *bad_dev, which the caller has zeroed, becomes 1.  values_dev on a 4-byte address, dense_dev on
+ * a 16-byte one where cols is a multiple of 8 (SPATHA_ERR_BAD_ARGUMENT otherwise).  Stream ordered. */
 int spatha_vnm_decode_f16_gpu(const uint16_t* values_dev, const uint32_t* metadata_dev, const uint32_t* columns_dev, int rows, int cols,
                               int n, int m, int v, uint16_t* dense_dev, uint32_t* bad_dev, void* stream);
 

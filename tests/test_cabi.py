@@ -45,6 +45,35 @@ def test_spmm_entry_points_reject_bad_arguments_without_a_gpu():
     assert L.spatha_spmm_tune(None, None, 8, None, None, 0, 1, 1, None, ctypes.byref(best), ctypes.byref(ms), None, None) == 1
 
 
+def test_conversion_on_the_gpu_refuses_addresses_its_accesses_do_not_fit():
+    """The kernels read and write several entries at once; an address that does not fit is refused ahead of any device work."""
+    import pytest
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("the addresses below are made up: for a machine on which nothing can be launched")
+    L = _lib.lib()
+    base = dict(dense=4096, values=8192, metadata=12288, columns=16384, bad=20480)
+    at = lambda **moved: {k: v + moved.get(k, 0) for k, v in base.items()}
+
+    def convert(bits, p):
+        return L.spatha_vnm_convert_gpu(p["dense"], bits, 64, 64, 2, 8, 32, p["values"], p["metadata"], p["columns"], None)
+
+    def decode(cols, p):
+        return L.spatha_vnm_decode_f16_gpu(p["values"], p["metadata"], p["columns"], 64, cols, 2, 8, 32, p["dense"], p["bad"], None)
+
+    for bits, moved in ((16, dict(dense=1)), (32, dict(dense=2)), (16, dict(values=4)), (16, dict(metadata=2)), (16, dict(columns=4)),
+                        (32, dict(columns=8))):
+        assert convert(bits, at(**moved)) == 1, (bits, moved)
+    for cols, moved in ((64, dict(dense=8)), (65, dict(dense=1)), (64, dict(values=2)), (64, dict(metadata=2)), (64, dict(columns=2)),
+                        (64, dict(bad=2))):
+        assert decode(cols, at(**moved)) == 1, (cols, moved)
+    # addresses that do fit get as far as the device that is not there
+    for status in (convert(16, at(dense=2)), convert(32, at(dense=4, values=8, metadata=4, columns=16)), decode(64, at(dense=16, values=4)),
+                   decode(65, at(dense=2, columns=4, metadata=4))):
+        assert status in (4, 5), status
+
+
 def test_unified_kernels_use_no_scratch_memory(tmp_path):
     """The unified dense-staged kernels load operands into registers asynchronously (inline assembly, no wait at the
     load); a register the compiler saves to scratch memory between such a load and its wait would hold a value that has

@@ -58,3 +58,13 @@ def test_a_column_offset_beyond_the_group_is_refused(gpu):
     a.columns[5] = 8
     with pytest.raises(_lib.SpathaError):
         a.to_dense()
+
+
+def test_arrays_at_odd_addresses_are_decoded_as_before(gpu):
+    a = bert.NMVectorSparsifier(2, 8, 32, magnitude=True)(torch.randn(64, 72, device="cuda").half()).wrapped_tensor
+    want = a.to_dense()
+    for offset in (1, 2):
+        buf = torch.empty(a.values.numel() + 8, dtype=torch.float16, device="cuda")
+        buf[offset:offset + a.values.numel()] = a.values
+        a.values = buf[offset:offset + a.values.numel()]
+        same(a.to_dense(), want)

@@ -611,6 +611,10 @@ int spatha_vnm_convert_gpu(const void* dense_dev, int value_bits, int rows, int 
     int st = spatha::geometry_init(rows, cols, n, m, v, &geo);
     if (st) return st;
     if (!dense_dev || !values_dev || !metadata_dev || !columns_dev || (value_bits != 16 && value_bits != 32)) return SPATHA_ERR_BAD_ARGUMENT;
+    // (four columns, two words of values and one of metadata are written at a time)
+    if (((uintptr_t)dense_dev & (uintptr_t)(value_bits / 8 - 1)) || ((uintptr_t)values_dev & 7) || ((uintptr_t)metadata_dev & 3) ||
+        ((uintptr_t)columns_dev & 15))
+        return SPATHA_ERR_BAD_ARGUMENT;
     const int tasks = spatha::select_task_count(rows, cols, m, v, nullptr);
     if (tasks > 0 && (size_t)v * (size_t)m * sizeof(float) > 150u * 1024u) return SPATHA_ERR_TOO_LARGE;
     hipStream_t s = (hipStream_t)stream;
@@ -629,6 +633,9 @@ int spatha_vnm_decode_f16_gpu(const uint16_t* values_dev, const uint32_t* metada
     int st = spatha::geometry_init(rows, cols, n, m, v, &geo);
     if (st) return st;
     if (!values_dev || !metadata_dev || !columns_dev || !dense_dev || !bad_dev) return SPATHA_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)values_dev & 3) || ((uintptr_t)metadata_dev & 3) || ((uintptr_t)columns_dev & 3) || ((uintptr_t)bad_dev & 3) ||
+        ((uintptr_t)dense_dev & (uintptr_t)(cols % 8 == 0 ? 15 : 1)))
+        return SPATHA_ERR_BAD_ARGUMENT;
     const hipError_t e = spatha::launch_decode_f16(values_dev, metadata_dev, columns_dev, rows, cols, m, v, geo.ksp, dense_dev, bad_dev,
                                                    (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);

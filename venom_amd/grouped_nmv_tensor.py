@@ -38,10 +38,10 @@ def nm_vector_mask_sparsify(tensor, n, m, tileM, threads=0, gpu=None, exact_ties
 
 
 def _decodes_on_gpu(a, geo):
-    """Do a's three arrays have the types, sizes and place that the decoding kernel takes?"""
+    """Do a's three arrays have the types, sizes, place and addresses that the decoding kernel takes?"""
     arrays = ((a.values, torch.float16, geo.n_values), (a.metadata, torch.int32, geo.n_metadata), (a.columns, torch.int32, geo.n_columns))
     return all(t.is_cuda and t.device == a.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
-               for t, dtype, count in arrays)
+               and t.data_ptr() % 4 == 0 for t, dtype, count in arrays)
 
 
 class SrNMTensor:
