@@ -27,6 +27,8 @@
 //   F consumers : s even: fragments 0, 1 of F_(s/2)        s odd: fragments 2, 3 of F_((s-1)/2)
 //   H consumers : s odd:  fragments 0, 1 of H_((s-1)/2)    s even: fragments 2, 3 of H_(s/2 - 1)
 
+#include <type_traits>
+
 #include "spmm_device.h"
 
 namespace spatha {
@@ -96,15 +98,20 @@ struct OhRows {
         bdma_b128(v, r0, 0, smem_base + oh_slot(s) + (uint32_t)wave_ * 1024u);
     }
     // sub-stage s >= 2: the rows come from the ring slot that the row-table DMA of sub-stage s - 2 filled
-    __device__ __forceinline__ void issue_from_ring(const char* smem, int s, uint32_t smem_base) const {
+    __device__ __forceinline__ uint2 ring_rows(const char* smem, int s) const {
         const char* rr = smem + OH_RT_BASE + (s & 3) * 256;
         if (!(s & 1)) {
             const char* e = rr + ((wave_ * 2) * 2 + (lane_ >> 5)) * 4;
-            issue_f(*(const uint32_t*)e, *(const uint32_t*)(e + 8), s, smem_base);
-        } else {
-            const uint32_t row = *(const uint32_t*)(rr + (wave_ * 4 + (lane_ >> 4)) * 4);
-            issue_h(has_extra ? row : 0xffffffffu, s, smem_base);
+            return make_uint2(*(const uint32_t*)e, *(const uint32_t*)(e + 8));
         }
+        return make_uint2(*(const uint32_t*)(rr + (wave_ * 4 + (lane_ >> 4)) * 4), 0u);
+    }
+    __device__ __forceinline__ void issue_rows(uint2 rows, int s, uint32_t smem_base) const {
+        if (!(s & 1)) issue_f(rows.x, rows.y, s, smem_base);
+        else issue_h(has_extra ? rows.x : 0xffffffffu, s, smem_base);
+    }
+    __device__ __forceinline__ void issue_from_ring(const char* smem, int s, uint32_t smem_base) const {
+        issue_rows(ring_rows(smem, s), s, smem_base);
     }
     // sub-stages 0 and 1: rows through ordinary loads (vb: V block whose row table applies)
     __device__ __forceinline__ void issue_first(const SpmmParams& p, int s, uint32_t vb, uint32_t smem_base) const {
@@ -186,7 +193,7 @@ __device__ __forceinline__ void oh_producer(const SpmmParams& p, char* smem, uin
     __syncthreads();                    // the slots become write-out staging
 }
 
-template <int OUT_LAYOUT>
+template <int OUT_LAYOUT, bool FUSE>
 __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uint32_t smem_base, int wave, int lane, int full_block,
                                             int extra_block, int extra_half, int tn) {
     const int S = p.S, N = p.N;
@@ -213,74 +220,107 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
     part.issue_first(p, 0, (uint32_t)__builtin_amdgcn_readfirstlane(full_block / blocks_per_v), smem_base);
     part.issue_first(p, 1, has_extra ? (uint32_t)__builtin_amdgcn_readfirstlane(extra_block / blocks_per_v) : 0u, smem_base);
     // barrier s: wait for the wave's own share of sub-stage s (the younger share, of sub-stage s + 1, may be in flight: one
-    // instruction if that is an H sub-stage, two if F) and meet the others; the share of sub-stage s + 2 is issued behind
-    // the first LDS reads of the interval's multiply
-    auto meet = [&](int s) {
-        if (s + 1 >= 2 * S) wait_vmcnt<0>();
-        else if (s & 1) wait_vmcnt<2>();
-        else wait_vmcnt<1>();
-        __syncthreads();
-    };
-    auto issue = [&](int s) {
-        if (s + 2 < 2 * S) part.issue_from_ring(smem, s + 2, smem_base);
-    };
-    const bool works = (!on_extra || has_extra) && !SPATHA_KNOB(16);
+    // instruction if that is an H sub-stage, two if F) and meet the others.  How soon behind the barrier the share of sub-stage
+    // s + 2 is issued sets the pace: its rows are the first thing that interval s reads from LDS, the fragments' reads follow, then the
+    // loads themselves (GPT-3 FFN matrix at 256 tokens, operands from memory: 67.9 us; rows read behind the fragments 70.0, the loads
+    // behind the first four matrix instructions 72.4, behind all eight 74.8).
+    auto meet_f = [] { wait_vmcnt<1>(); __syncthreads(); };          // s even
+    auto meet_h = [] { wait_vmcnt<2>(); __syncthreads(); };          // s odd
+    auto meet_last = [] { wait_vmcnt<0>(); __syncthreads(); };       // nothing younger
     half8_t a_cur[4];
     uint32_t i0 = 0, i1 = 0;
     // (the row pitch of a B fragment read is a template argument: one instantiation per role)
     auto frag = [&](const char* st, int off) {
         return on_extra ? read_b_fragment<OH_HROW_BYTES>(st, off) : read_b_fragment<OH_ROW_BYTES>(st, off);
     };
-    // first interval of a sub-stage: operands of A (kept for the second interval) and fragments 0, 1
-    auto first_half = [&](const char* st, int s) {
-        if (works) {
+    // Two intervals of a sub-stage: operands of A (kept for the second one) and fragments 0, 1; fragments 2, 3.  Interval s issues
+    // the share of sub-stage s + 2 as long as there is one: known at compile time, the last k-steps stand behind the loops.  (As
+    // conditions inside the loops they were laid out this way or that depending on the code behind the loops: a change of the
+    // activation's instructions alone moved the plain product from 68.8 to 69.3 us.)
+    auto first_half = [&](const char* st, int s, auto issues) {
+        if (SPATHA_KNOB(16)) {
+            if constexpr (issues.value) part.issue_from_ring(smem, s + 2, smem_base);
+            return;
+        }
+        uint2 rows;
+        if constexpr (issues.value) rows = part.ring_rows(smem, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int mb = 0; mb < 4; mb++) a_cur[mb] = *(const half8_t*)(st + a_off + mb * 1024);
-            i0 = *(const uint32_t*)(st + i_off);
-            i1 = *(const uint32_t*)(st + i_off + 256);
-            half16_t bf0 = frag(st, tr0);
-            half16_t bf1 = frag(st, tr0 ^ 32);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(s);
-            __builtin_amdgcn_sched_barrier(0);
-            SPATHA_MMA4(0, bf0)
-            SPATHA_MMA4(1, bf1)
-        } else {
-            issue(s);
-        }
+        for (int mb = 0; mb < 4; mb++) a_cur[mb] = *(const half8_t*)(st + a_off + mb * 1024);
+        i0 = *(const uint32_t*)(st + i_off);
+        i1 = *(const uint32_t*)(st + i_off + 256);
+        half16_t bf0 = frag(st, tr0);
+        half16_t bf1 = frag(st, tr0 ^ 32);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (issues.value) part.issue_rows(rows, s + 2, smem_base);
+        __builtin_amdgcn_sched_barrier(0);
+        SPATHA_MMA4(0, bf0)
+        SPATHA_MMA4(1, bf1)
     };
-    auto second_half = [&](const char* st, int s) {
-        if (works) {
-            half16_t bf0 = frag(st, tr0 ^ 64);
-            half16_t bf1 = frag(st, tr0 ^ 96);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(s);
-            __builtin_amdgcn_sched_barrier(0);
-            SPATHA_MMA4(2, bf0)
-            SPATHA_MMA4(3, bf1)
-        } else {
-            issue(s);
+    auto second_half = [&](const char* st, int s, auto issues) {
+        if (SPATHA_KNOB(16)) {
+            if constexpr (issues.value) part.issue_from_ring(smem, s + 2, smem_base);
+            return;
         }
+        uint2 rows;
+        if constexpr (issues.value) rows = part.ring_rows(smem, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        half16_t bf0 = frag(st, tr0 ^ 64);
+        half16_t bf1 = frag(st, tr0 ^ 96);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (issues.value) part.issue_rows(rows, s + 2, smem_base);
+        __builtin_amdgcn_sched_barrier(0);
+        SPATHA_MMA4(2, bf0)
+        SPATHA_MMA4(3, bf1)
     };
+    constexpr std::true_type more;
+    constexpr std::false_type no_more;
     if (!on_extra) {
-        for (int k = 0; k < S; k++) {
+        for (int k = 0; k + 1 < S; k++) {
             const char* st = smem + (k & 1) * OH_PAIR;
-            meet(2 * k);
-            first_half(st, 2 * k);
-            meet(2 * k + 1);
-            second_half(st, 2 * k + 1);
+            meet_f();
+            first_half(st, 2 * k, more);
+            meet_h();
+            second_half(st, 2 * k + 1, more);
         }
+        const char* st = smem + ((S - 1) & 1) * OH_PAIR;
+        meet_f();
+        first_half(st, 2 * S - 2, no_more);
+        meet_last();
+        second_half(st, 2 * S - 1, no_more);
         __syncthreads();
-    } else {
-        meet(0);
-        issue(0);
-        for (int k = 0; k < S; k++) {
-            const char* st = smem + (k & 1) * OH_PAIR + OH_F_BYTES;
-            meet(2 * k + 1);
-            first_half(st, 2 * k + 1);
-            if (k + 1 < S) meet(2 * k + 2); else __syncthreads();
-            second_half(st, 2 * k + 2);
+    } else if (has_extra) {
+        const char* slots = smem + OH_F_BYTES;
+        meet_f();
+        if (S > 1) part.issue_from_ring(smem, 2, smem_base);
+        for (int k = 0; k + 2 < S; k++) {
+            const char* st = slots + (k & 1) * OH_PAIR;
+            meet_h();
+            first_half(st, 2 * k + 1, more);
+            meet_f();
+            second_half(st, 2 * k + 2, more);
         }
+        if (S > 1) {
+            const char* st = slots + (S & 1) * OH_PAIR;             // k-step S - 2
+            meet_h();
+            first_half(st, 2 * S - 3, more);
+            meet_f();
+            second_half(st, 2 * S - 2, no_more);
+        }
+        const char* st = slots + ((S - 1) & 1) * OH_PAIR;
+        meet_last();
+        first_half(st, 2 * S - 1, no_more);
+        __syncthreads();
+        second_half(st, 2 * S, no_more);
+    } else {
+        // no rows to multiply: the wave's share of the loads and the barriers
+        for (int s = 0; s + 2 < 2 * S; s++) {
+            if (s & 1) meet_h(); else meet_f();
+            part.issue_from_ring(smem, s + 2, smem_base);
+        }
+        meet_f();
+        meet_last();
+        __syncthreads();
     }
     __syncthreads();
     if ((on_extra && !has_extra) || SPATHA_KNOB(4)) return;
@@ -290,9 +330,9 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
     const int j16 = lane & 15, ib = lane >> 4;
     char* stg = smem + wave * (16 * OH_EPI_PITCH);
     const int col0 = tn * 256 + (on_extra ? extra_half * 128 : 0) + q * 64;
-    if (p.fuse) fused_bias_act(acc, p.bias, row0 + ib * 16, p.act);
+    if constexpr (FUSE) fused_bias_act(acc, p.bias, row0 + ib * 16, p.act);
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-        store_block_transposed_slab<true>(acc, stg, p.C, p.fuse ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
+        store_block_transposed_slab<true>(acc, stg, p.C, FUSE ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
     } else {
         // 16-row slabs through the wave's staging buffer -> 128-byte row segments
 #pragma unroll
@@ -316,7 +356,8 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
     }
 }
 
-template <int OUT_LAYOUT>
+// FUSE: bias and activation in the write-out (instances of their own: with the activations' code in it the kernel spills registers)
+template <int OUT_LAYOUT, bool FUSE>
 __global__ __launch_bounds__((OH_NC + OH_NP) * 64) void spmm_oh_kernel(SpmmParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
@@ -332,16 +373,16 @@ __global__ __launch_bounds__((OH_NC + OH_NP) * 64) void spmm_oh_kernel(SpmmParam
         else { extra_tile = F + (f >> 1); extra_half = f & 1; }
     }
     const int extra_block = extra_tile < 0 ? -1 : 2 * extra_tile;
-    if (wave < OH_NC) oh_consumer<OUT_LAYOUT>(p, smem, smem_base, wave, lane, full_block, extra_block, extra_half, tn);
+    if (wave < OH_NC) oh_consumer<OUT_LAYOUT, FUSE>(p, smem, smem_base, wave, lane, full_block, extra_block, extra_half, tn);
     else if (wave == OH_NC) oh_producer<0>(p, smem, smem_base, lane, full_block, extra_block, extra_half, tn);
     else if (wave == OH_NC + 1) oh_producer<1>(p, smem, smem_base, lane, full_block, extra_block, extra_half, tn);
     else if (wave == OH_NC + 2) oh_producer<2>(p, smem, smem_base, lane, full_block, extra_block, extra_half, tn);
     else oh_producer<3>(p, smem, smem_base, lane, full_block, extra_block, extra_half, tn);
 }
 
-template <int OUT_LAYOUT>
+template <int OUT_LAYOUT, bool FUSE>
 hipError_t launch_oh(const SpmmParams& p, hipStream_t stream) {
-    auto kern = spmm_oh_kernel<OUT_LAYOUT>;
+    auto kern = spmm_oh_kernel<OUT_LAYOUT, FUSE>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, OH_LDS);
@@ -358,8 +399,9 @@ hipError_t launch_oh(const SpmmParams& p, hipStream_t stream) {
 hipError_t launch_onehalf(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
     if (variant != SPMM_VARIANT_OH192x256) return hipErrorInvalidValue;
     if (p.v % 128 != 0 || p.rows % 128 != 0 || p.tiles_m != p.rows / 128 || p.ksplit != 1) return hipErrorInvalidValue;
-    return out_layout == SPATHA_OUT_TRANSPOSED ? launch_oh<SPATHA_OUT_TRANSPOSED>(p, stream)
-                                               : launch_oh<SPATHA_OUT_ROW_MAJOR>(p, stream);
+    if (out_layout == SPATHA_OUT_TRANSPOSED)
+        return p.fuse ? launch_oh<SPATHA_OUT_TRANSPOSED, true>(p, stream) : launch_oh<SPATHA_OUT_TRANSPOSED, false>(p, stream);
+    return p.fuse ? launch_oh<SPATHA_OUT_ROW_MAJOR, true>(p, stream) : launch_oh<SPATHA_OUT_ROW_MAJOR, false>(p, stream);
 }
 
 }  // namespace spatha
