@@ -482,11 +482,6 @@ struct TileWalkT {
     }
 };
 using TileWalk = TileWalkT<1>;
-// the same for kernels with one tile per workgroup: place in the order of columns -> tile column (tiles_n a multiple of 8: the
-// XCD's chunk is tiles_n / 8 whole columns)
-__device__ __forceinline__ int static_tile_column(int place, int xcd, int tiles_n, bool interleave) {
-    return interleave && (tiles_n & 7) == 0 ? (place - xcd * (tiles_n >> 3)) * 8 + xcd : place;
-}
 
 // ---- deferred write-out -------------------------------------------------------------------
 // A finished 64 x 64 wave tile is rounded to fp16 pairs (32 registers) and written one quarter

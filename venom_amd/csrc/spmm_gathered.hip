@@ -240,8 +240,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
     const int tile = xcd * chunk + local;
     if (local >= chunk || tile >= tiles) return;
-    const int place = tile / p.tiles_m, tile_m = tile - place * p.tiles_m;
-    const int tile_n = static_tile_column(place, xcd, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
+    const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -455,7 +454,8 @@ __global__ __launch_bounds__(WN * 128) void spmm_half_kernel(SpmmParams p) {
     const int tile = xcd * chunk + local;
     if (local >= chunk || tile >= tiles) return;
     const int place = tile / p.tiles_m, tile_m = tile - place * p.tiles_m;
-    const int tile_n = static_tile_column(place, xcd, p.tiles_n, OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR);
+    const bool interleave = OUT_LAYOUT == SPATHA_OUT_ROW_MAJOR && p.walk_group == 8;       // (launch_half)
+    const int tile_n = interleave && (p.tiles_n & 7) == 0 ? (place - xcd * (p.tiles_n >> 3)) * 8 + xcd : place;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -629,7 +629,15 @@ static hipError_t launch_half(const SpmmParams& p, hipStream_t stream) {
     }
     const int tiles = p.tiles_m * p.tiles_n;
     const int chunk = (tiles + 7) / 8;
-    hipLaunchKernelGGL(kern, dim3(chunk * 8), dim3(WN * 128), lds, stream, p);
+    // An XCD takes adjacent tile columns, or (row-major, a multiple of eight) every eighth one so that the eight write adjacent
+    // columns at a time.  Measured with one binary, operands from memory / from the memory-side cache: 64 x 128 tiles in pairs of
+    // workgroups, all resident at once 0.98 / 0.99 of the adjacent order's time (1280 x 5120 x 2048 at 32:2:16 0.97), up to two rounds
+    // 0.99, beyond 1.01 / 1.00 (1024 x 4096 x 16384 at 32:2:32 1.04); 64 x 256 tiles 1.02 / 1.03 at any count (1024 x 4096 x 4096 at
+    // 32:2:16 1.06), three stages 1.01 / 1.00.  (The tiles of spmm_pipe_kernel likewise: 128 x 128 1.00-1.02, 64 x 256 0.95-1.03 from
+    // memory and up to 1.10 from the cache: adjacent.)
+    SpmmParams q = p;
+    q.walk_group = WN == 2 && NS == 2 && p.tiles_n % 8 == 0 && tiles <= 2 * p.cus ? 8 : 1;
+    hipLaunchKernelGGL(kern, dim3(chunk * 8), dim3(WN * 128), lds, stream, q);
     return hipGetLastError();
 }
 
