@@ -294,7 +294,10 @@ static hipError_t launch_direct_family(const SpmmParams& p, hipStream_t stream) 
         nb = 2;
     } else {
         nb = 4;
-        if (tiles(4) <= cus && (p.S >= 16 || (p.S >= 8 && tiles(4) <= (HALF ? 256 : 160)))) w = 8;
+        // (eight waves against four at 130 .. 256 tiles, 1080 products, both layouts: 64-row tiles 0.90-0.98 of the speed at five to
+        // fourteen k-steps, 0.97-1.00 at sixteen, 1.03-1.06 at twenty, 1.13 at 48, whatever the number of tiles; 32-row tiles 0.95-1.03
+        // up to eight, 1.02 at ten, 1.01-1.06 at fourteen, 1.16 at 48)
+        if (tiles(4) <= cus && p.S > (HALF ? 8 : 16)) w = 8;
     }
     const bool lean = tiles(4) > cus && (p.S > 2 || tiles(4) > 2 * cus);
     switch (nb * 100 + w) {
