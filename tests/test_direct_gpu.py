@@ -18,8 +18,22 @@ CASES = [
     (1536, 640, 304, 20, 64), (4096, 512, 200, 16, 64), (4096, 1024, 512, 8, 64), (17408, 512, 16, 8, 64), (17408, 256, 32, 8, 64),
     (35072, 512, 8, 16, 128), (35072, 512, 64, 16, 128), (1024, 16384, 64, 8, 128),
     (32, 64, 8, 8, 32), (96, 300, 72, 7, 96), (160, 2048, 136, 16, 32), (1280, 5120, 304, 16, 32), (1024, 4096, 520, 8, 32),
+    (1280, 4352, 520, 16, 64), (256, 4096, 136, 16, 32), (1024, 2048, 136, 16, 32), (1024, 1536, 264, 16, 32),
     (1024, 2048, 1040, 16, 32), (2112, 640, 264, 20, 32), (9216, 512, 8, 16, 32), (9216, 320, 32, 8, 288), (9216, 256, 64, 16, 32),
 ]
+
+
+def test_the_cases_reach_every_form(gpu):
+    """Eight forms on 64-row tiles and eight on 32-row ones: columns and waves per tile as the kernel's name reports them."""
+    reached = set()
+    for rows, cols, N, m, v in CASES:
+        vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=1)
+        plan = spatha.SpmmPlan(torch.from_numpy(vals).to(gpu), torch.from_numpy(meta.view(np.int32)).to(gpu),
+                               torch.from_numpy(columns.view(np.int32)).to(gpu), rows, cols, 2, m, v)
+        reached.add(plan.kernel_name(N, 0, 0 if v % 64 else 23).split("direct_")[1])
+    columns_and_waves = ("x16_splitk4", "x16_splitk8", "x16_splitk16", "x32_splitk4", "x32_splitk8", "x64_splitk4", "x64_splitk4_lean",
+                         "x64_splitk8")
+    assert reached == {tile + form for tile in ("tile64", "tile32") for form in columns_and_waves}, sorted(reached)
 
 
 @pytest.mark.parametrize("rows,cols,N,m,v", CASES)

@@ -127,10 +127,11 @@ def test_plan_run_refuses_and_writes_as_before(gpu):
 
 
 @pytest.mark.parametrize("rows,cols,m,v", [(64, 64, 8, 64), (128, 200, 16, 128), (256, 1024, 8, 64), (1024, 3300, 10, 128), (128, 12288, 16, 64),
-                                           (32, 64, 8, 32), (96, 300, 7, 96), (512, 2048, 16, 32)])
+                                           (32, 64, 8, 32), (96, 300, 7, 96), (512, 2048, 16, 32), (512, 4096, 16, 32)])
 @pytest.mark.parametrize("tokens", [1, 2, 5, 8, 13, 16])
 def test_a_few_tokens_as_they_lie(gpu, rows, cols, m, v, tokens):
-    """spatha_spmm_run_tokens against the oracle, bit for bit on integer operands, with and without a bias; one token more than it
+    """spatha_spmm_run_tokens against the oracle, bit for bit on integer operands (eight and sixteen waves on 64-row and 32-row tiles),
+    with and without a bias; one token more than it
     takes, and more columns than the LDS holds, are refused."""
     import numpy as np
 

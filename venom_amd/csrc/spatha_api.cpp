@@ -873,6 +873,7 @@ const char* spatha_spmm_kernel_name(const spatha_spmm_plan* plan, int N, int out
     if (uneven_rest_rows(plan, N, variant, var, false))     // two launches: the rest of an uneven last round on 128 x 128 tiles
         return var == spatha::SPMM_VARIANT_T128x256_S3 ? "smfmac16x16x64_warpspec_tall_tile128x256_3stage+rest_on_tile128x128"
                                                        : "smfmac16x16x64_warpspec_tile128x256_3stage+rest_on_tile128x128";
+    if (const char* form = spatha::spmm_direct_name(var, plan->geo.rows, N, plan->S, plan->cus > 0 ? plan->cus : 256)) return form;
     return spatha::spmm_variant_name(var);
 }
 

@@ -41,9 +41,9 @@ const VariantInfo kVariants[] = {
      DsCfg<8, 3, 4, 8>::LDS_BYTES, 0, launch_densestage},
     {SPMM_VARIANT_DS256x128_S3_PP, "smfmac16x16x64_warpspec_densestage_tile256x128_3stage_pingpong", 256, 128,
      DsCfg<8, 3, 4, 8>::LDS_BYTES, 0, launch_densestage},
-    {SPMM_VARIANT_SKINNY, "smfmac16x16x64_skinny_tile64xN_splitk4", 64, 64, 64 * 1024, 0, launch_skinny_family},
-    {SPMM_VARIANT_DIRECT64, "smfmac16x16x64_direct_tile64x64_splitk", 64, 64, 64 * 1024, 0, launch_skinny_family},
-    {SPMM_VARIANT_HDIRECT32, "smfmac16x16x64_halftile_direct_tile32x64_splitk", 32, 64, 64 * 1024, 0, launch_skinny_family},
+    {SPMM_VARIANT_SKINNY, "smfmac16x16x64_skinny_tile64xN_splitk", 64, 64, 64 * 1024, 0, launch_skinny_family},
+    {SPMM_VARIANT_DIRECT64, "smfmac16x16x64_direct_tile64xN_splitk", 64, 64, 64 * 1024, 0, launch_skinny_family},
+    {SPMM_VARIANT_HDIRECT32, "smfmac16x16x64_halftile_direct_tile32xN_splitk", 32, 64, 64 * 1024, 0, launch_skinny_family},
     {SPMM_VARIANT_H64x256_S2, "smfmac16x16x64_halftile_ldsdirect_tile64x256_2stage", 64, 256, half_stage_bytes<4, 2>(), 256,
      launch_gathered},
     {SPMM_VARIANT_H64x128_S3, "smfmac16x16x64_halftile_ldsdirect_tile64x128_3stage", 64, 128, half_stage_bytes<2, 3>(), 256,

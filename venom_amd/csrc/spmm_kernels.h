@@ -90,6 +90,9 @@ hipError_t launch_skinny_family(int variant, int out_layout, const SpmmParams& p
 hipError_t launch_pingpong(int variant, int out_layout, const SpmmParams& p, hipStream_t stream);
 hipError_t launch_onehalf(int variant, int out_layout, const SpmmParams& p, hipStream_t stream);
 
+// name of the form (columns and waves per tile) that kernels 13, 23 and 24 take for a product; nullptr for the other ids
+const char* spmm_direct_name(int variant, int rows, int N, int S, int cus);
+
 // up to 16 tokens x [N][cols] as they lie, transposed output (spmm_skinny.hip); token_major_fits: whether the launch takes them
 bool token_major_fits(int rows, int cols, int tokens, bool half_tiles, int cus);
 hipError_t launch_token_major(const SpmmParams& p, bool half_tiles, hipStream_t stream);

@@ -270,47 +270,84 @@ static hipError_t launch_direct(SpmmParams p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <int OUT_LAYOUT, bool HALF>
-static hipError_t launch_direct_family(const SpmmParams& p, hipStream_t stream) {
-    // Columns and waves per tile: the narrowest tile whose tiles still find a CU each, its k-steps over as many waves as they
+// Columns (16 * nb) and waves per tile
+struct DirectForm {
+    int nb, w;
+    bool lean;
+};
+
+static DirectForm direct_form(int rows, int N, int S, bool half, int64_t cus) {
+    // The narrowest tile whose tiles still find a CU each, its k-steps over as many waves as they
     // feed; with more tiles than CUs fewer waves, so that several workgroups share a CU.  (Every form on ten layer shapes from
     // 768 x 3072 to 49152 x 12288, V = 32 / 64 / 128, m = 8 / 16 / 32, 8 .. 2048 tokens, both layouts: this choice is 1.1 %
     // behind the best form on the geometric mean.  12288 x 49152 at 128:2:16 and 8 tokens, 192 tiles of 192 k-steps: 28.8 us
     // with sixteen waves, 50.3 with four; 1024 x 4096 at 64:2:16 and 512 tokens: 5.2 us on 64 x 32 tiles of eight waves, 6.4 on
     // 64 x 64 ones.)
-    const int64_t rows_tiles = p.rows / (HALF ? 32 : 64), cus = p.cus;
-    auto tiles = [&](int nb) { return rows_tiles * ((p.N + 16 * nb - 1) / (16 * nb)); };
-    int nb, w = 4;
+    const int64_t rows_tiles = rows / (half ? 32 : 64);
+    auto tiles = [&](int nb) { return rows_tiles * ((N + 16 * nb - 1) / (16 * nb)); };
+    DirectForm f = {1, 4, false};
     if (tiles(1) <= cus) {
-        nb = 1;
-        w = p.S > 12 ? 16 : p.S > 4 || p.N > 16 ? 8 : 4;
-    } else if (p.N <= 16) {
-        nb = 1;
-        w = tiles(1) <= 2 * cus && p.S > 4 ? 8 : 4;
+        f.w = S > 12 ? 16 : S > 4 || N > 16 ? 8 : 4;
+    } else if (N <= 16) {
+        f.w = tiles(1) <= 2 * cus && S > 4 ? 8 : 4;
     } else if (tiles(2) <= cus) {
-        nb = 2;
-        w = p.S > 4 ? 8 : 4;
-    } else if (p.N <= 32 || (p.S <= 4 && tiles(2) <= 3 * cus)) {
-        nb = 2;
+        f.nb = 2;
+        f.w = S > 4 ? 8 : 4;
+    } else if (N <= 32 || (S <= 4 && tiles(2) <= 3 * cus)) {
+        f.nb = 2;
     } else {
-        nb = 4;
+        f.nb = 4;
         // (eight waves against four at 130 .. 256 tiles, 1080 products, both layouts: 64-row tiles 0.90-0.98 of the speed at five to
         // fourteen k-steps, 0.97-1.00 at sixteen, 1.03-1.06 at twenty, 1.13 at 48, whatever the number of tiles; 32-row tiles 0.95-1.03
         // up to eight, 1.02 at ten, 1.01-1.06 at fourteen, 1.16 at 48)
-        if (tiles(4) <= cus && p.S > (HALF ? 8 : 16)) w = 8;
+        if (tiles(4) <= cus && S > (half ? 8 : 16)) f.w = 8;
+        f.lean = f.w == 4 && tiles(4) > cus && (S > 2 || tiles(4) > 2 * cus);
     }
-    const bool lean = tiles(4) > cus && (p.S > 2 || tiles(4) > 2 * cus);
-    switch (nb * 100 + w) {
-        case 104: return launch_direct<1, OUT_LAYOUT, 4, HALF>(p, stream);
-        case 108: return launch_direct<1, OUT_LAYOUT, 8, HALF>(p, stream);
-        case 116: return launch_direct<1, OUT_LAYOUT, 16, HALF>(p, stream);
-        case 204: return launch_direct<2, OUT_LAYOUT, 4, HALF>(p, stream);
-        case 208: return launch_direct<2, OUT_LAYOUT, 8, HALF>(p, stream);
-        case 404: return lean ? launch_direct<4, OUT_LAYOUT, 4, HALF, true>(p, stream) : launch_direct<4, OUT_LAYOUT, 4, HALF>(p, stream);
-        case 408: return launch_direct<4, OUT_LAYOUT, 8, HALF>(p, stream);
+    return f;
+}
+
+// place of a form in the tables below, < 0: not compiled
+static int form_index(const DirectForm& f) {
+    switch (f.nb * 100 + f.w) {
+        case 104: return 0;
+        case 108: return 1;
+        case 116: return 2;
+        case 204: return 3;
+        case 208: return 4;
+        case 404: return f.lean ? 6 : 5;
+        case 408: return 7;
+        default: return -1;
+    }
+}
+
+template <int OUT_LAYOUT, bool HALF>
+static hipError_t launch_direct_family(const SpmmParams& p, hipStream_t stream) {
+    switch (form_index(direct_form(p.rows, p.N, p.S, HALF, p.cus))) {
+        case 0: return launch_direct<1, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 1: return launch_direct<1, OUT_LAYOUT, 8, HALF>(p, stream);
+        case 2: return launch_direct<1, OUT_LAYOUT, 16, HALF>(p, stream);
+        case 3: return launch_direct<2, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 4: return launch_direct<2, OUT_LAYOUT, 8, HALF>(p, stream);
+        case 5: return launch_direct<4, OUT_LAYOUT, 4, HALF>(p, stream);
+        case 6: return launch_direct<4, OUT_LAYOUT, 4, HALF, true>(p, stream);
+        case 7: return launch_direct<4, OUT_LAYOUT, 8, HALF>(p, stream);
         default: return hipErrorInvalidValue;
     }
 }
+
+#define SPATHA_DIRECT_NAMES(prefix)                                                                                                   \
+    {prefix "x16_splitk4", prefix "x16_splitk8", prefix "x16_splitk16", prefix "x32_splitk4", prefix "x32_splitk8", prefix "x64_splitk4", \
+     prefix "x64_splitk4_lean", prefix "x64_splitk8"}
+const char* spmm_direct_name(int variant, int rows, int N, int S, int cus) {
+    static const char* const names[3][8] = {SPATHA_DIRECT_NAMES("smfmac16x16x64_skinny_tile64"),
+                                            SPATHA_DIRECT_NAMES("smfmac16x16x64_direct_tile64"),
+                                            SPATHA_DIRECT_NAMES("smfmac16x16x64_halftile_direct_tile32")};
+    const int kind = variant == SPMM_VARIANT_SKINNY ? 0 : variant == SPMM_VARIANT_DIRECT64 ? 1 : variant == SPMM_VARIANT_HDIRECT32 ? 2 : -1;
+    if (kind < 0) return nullptr;
+    const int form = form_index(direct_form(rows, N, S, kind == 2, cus));
+    return form < 0 ? nullptr : names[kind][form];
+}
+#undef SPATHA_DIRECT_NAMES
 
 // A few tokens as they lie, x [N][cols] with N <= 16 (any count), transposed output: what the transposed copy ahead of the product
 // would hold is read from LDS, where every workgroup puts the tokens first.
