@@ -247,7 +247,8 @@ int spatha_spmm_run_noalloc(int rows, int cols, int n, int m, int v, const uint1
                             const uint32_t* metadata_dev, const uint32_t* columns_dev, const uint16_t* B_dev, int N,
                             const uint16_t* bias_dev, uint16_t* out_dev, int out_layout, void* stream);
 
-/* Kernel variants are numbered 1 .. spatha_spmm_num_variants() - 1; 0 selects automatically. */
+/* Kernel variants are numbered 1 .. spatha_spmm_num_variants() - 1; 0 selects automatically.  One more can be named: 24, the 32-row
+ * form of id 23 for V a multiple of 32 only. */
 int spatha_spmm_num_variants(void);
 
 /* Name / tile shape of the kernel `variant` (or of the automatic choice for N
@@ -267,7 +268,8 @@ int spatha_spmm_time(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N,
 /* Times the automatic choice and every kernel id that accepts this plan, N and layout (spatha_spmm_time each), and
  * reports the fastest: *best_variant (0 when nothing beats the automatic choice, which may be a form no single id gives,
  * see spatha_spmm_kernel_name), *best_ms, and *auto_ms, the automatic choice's time.  ms_per_variant, when not NULL,
- * holds spatha_spmm_num_variants() floats: [0] the automatic choice, [id] that kernel, negative where it does not apply.
+ * holds spatha_spmm_num_variants() floats: [0] the automatic choice, [id] that kernel, negative where it does not apply
+ * (kernel 24 is timed too and has no place there).
  * The result of every timed kernel lands in out_dev.  For callers that would rather measure their shape than trust the
  * rule table; replaces the search over the reference's tile tuples (src/spmm/spatha_spmm.hpp:49-585, swept per shape by
  * benchmark/run_spmm_spatha.sh). */

@@ -30,7 +30,7 @@ def test_the_cases_reach_every_form(gpu):
         vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=1)
         plan = spatha.SpmmPlan(torch.from_numpy(vals).to(gpu), torch.from_numpy(meta.view(np.int32)).to(gpu),
                                torch.from_numpy(columns.view(np.int32)).to(gpu), rows, cols, 2, m, v)
-        reached.add(plan.kernel_name(N, 0, 0 if v % 64 else 23).split("direct_")[1])
+        reached.add(plan.kernel_name(N, 0, spatha.DIRECT_HALF_VARIANT if v % 64 else 23).split("direct_")[1])
     columns_and_waves = ("x16_splitk4", "x16_splitk8", "x16_splitk16", "x32_splitk4", "x32_splitk8", "x64_splitk4", "x64_splitk4_lean",
                          "x64_splitk8")
     assert reached == {tile + form for tile in ("tile64", "tile32") for form in columns_and_waves}, sorted(reached)
@@ -52,7 +52,7 @@ def test_direct_kernels_bit_exact(gpu, rows, cols, N, m, v, transposed):
     guarded = torch.full((cols * N + 4096,), float("nan"), dtype=torch.float16, device=gpu)
     guarded[:cols * N] = dev(B).reshape(-1)
     dB = guarded[:cols * N].view(cols, N)
-    variants = [0] + ([23] if v % 64 == 0 else [])
+    variants = [0, 23 if v % 64 == 0 else spatha.DIRECT_HALF_VARIANT]
     for variant in variants:
         got = plan.run(dB, bias=dev(bias) if transposed else None, transposed_out=transposed, variant=variant)
         assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16)), variant
@@ -78,3 +78,34 @@ def test_direct_kernel_activations(gpu):
             want = torch.nn.functional.gelu(pre, approximate=approx).half()
             # one step of fp16 at the value's size (2^-10 relative, the subnormal step 2^-24 near zero)
             assert bool(((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -10 + 2.0 ** -24).all())
+
+
+def test_the_32_row_kernel_by_name(gpu):
+    """Kernel 24 on random shapes of V = 32, 96 and 160, in every mode, whatever the automatic choice is; tune knows it; plans of 64-row
+    tiles refuse it."""
+    assert spatha.variant_ids() == list(range(1, spatha.num_variants())) + [24]
+    rng = np.random.default_rng(17)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
+    for i in range(24):
+        v, m = int(rng.choice([32, 96, 160])), int(rng.choice([4, 7, 8, 10, 16, 20, 40]))
+        rows, cols, N = v * int(rng.integers(1, 9)), int(rng.integers(4, 1500)), 8 * int(rng.integers(1, 200))
+        print("by name", i, rows, cols, N, m, v, flush=True)
+        vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=i, integer_values=True)
+        B = rng.integers(-4, 5, size=(cols, N)).astype(np.float16)
+        bias = rng.integers(-3, 4, size=rows).astype(np.float16)
+        plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
+        plain = oracle.spmm(vals, meta, columns, rows, cols, 2, m, v, B)
+        biased = oracle.spmm(vals, meta, columns, rows, cols, 2, m, v, B, bias=bias, transposed_out=True)
+        for kw, want in ((dict(), plain), (dict(bias=dev(bias), transposed_out=True), biased),
+                         (dict(bias=dev(bias), activation="none"), np.ascontiguousarray(biased.T))):
+            got = plan.run(dev(B), variant=24, **kw).cpu().numpy()
+            assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), kw
+    out = torch.empty((rows, N), dtype=torch.float16, device=gpu)
+    best, best_ms, auto_ms, times = plan.tune(dev(B), out)
+    assert best in times and best_ms == min(times.values()) <= auto_ms
+    vals, meta, columns = F.synthetic_vnm(64, 64, 2, 8, 64, seed=0)
+    plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), 64, 64, 2, 8, 64)
+    assert plan.kernel_name(8, 0, 24) is None and plan.kernel_name(8, 0, 25) is None
+    for variant in (24, 25, 99, -1):
+        with pytest.raises(RuntimeError):
+            plan.run(torch.zeros((64, 8), device=gpu).half(), variant=variant)

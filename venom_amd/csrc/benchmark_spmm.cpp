@@ -240,6 +240,9 @@ int main(int argc, const char** argv) {
             if (per[id] >= 0.f)
                 std::fprintf(stderr, "tune: id %2zu %-72s %9.2f us%s\n", id, spatha_spmm_kernel_name(plan, n, SPATHA_OUT_ROW_MAJOR, (int)id),
                              per[id] * 1e3f, (int)id == variant ? "  <- fastest" : "");
+        if (variant >= (int)per.size())
+            std::fprintf(stderr, "tune: id %2d %-72s %9.2f us  <- fastest\n", variant,
+                         spatha_spmm_kernel_name(plan, n, SPATHA_OUT_ROW_MAJOR, variant), best_ms * 1e3f);
     }
     const char* kname = spatha_spmm_kernel_name(plan, n, SPATHA_OUT_ROW_MAJOR, variant);
     if (!kname) {

@@ -370,7 +370,7 @@ const Rule kRules[] = {
 
 int pick_variant(const spatha_spmm_plan* plan, int N, int variant, bool fused = false, int out_layout = SPATHA_OUT_ROW_MAJOR) {
     if (variant != spatha::SPMM_VARIANT_AUTO)
-        return variant < spatha::SPMM_VARIANT_COUNT && variant_ok(plan, N, variant, fused) ? variant : -1;
+        return variant_ok(plan, N, variant, fused) ? variant : -1;
     Shape s;
     s.v = plan->geo.v; s.m = plan->geo.m; s.rows = plan->geo.rows; s.cols = plan->geo.cols; s.N = N; s.S = plan->S;
     s.cus = plan->cus > 0 ? plan->cus : 256;
@@ -916,14 +916,16 @@ int spatha_spmm_tune(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N,
     if (st) return st;
     int best = spatha::SPMM_VARIANT_AUTO;
     float t_best = 0.f;
-    for (int id = 1; id < spatha::SPMM_VARIANT_COUNT; id++) {
-        if (ms_per_variant) ms_per_variant[id] = -1.f;
+    // (the ids that ms_per_variant has places for, then the one behind them)
+    for (int id = 1; id <= spatha::SPMM_VARIANT_HDIRECT32; id++) {
+        float* const place = ms_per_variant && id < spatha::SPMM_VARIANT_COUNT ? ms_per_variant + id : nullptr;
+        if (place) *place = -1.f;
         if (!variant_ok(plan, N, id, false)) continue;
         float t = 0.f;
         st = spatha_spmm_time(plan, B_dev, N, bias_dev, out_dev, out_layout, id, warmup, iters, stream, &t);
         if (st == SPATHA_ERR_UNSUPPORTED) continue;     // (accepted by the shape checks, refused by the kernel's launcher)
         if (st) return st;
-        if (ms_per_variant) ms_per_variant[id] = t;
+        if (place) *place = t;
         if (best == spatha::SPMM_VARIANT_AUTO || t < t_best) { t_best = t; best = id; }
     }
     // the automatic choice last, in the same warm state as the ids: it wins ties (it may be one of them)

@@ -70,7 +70,8 @@ enum {
     SPMM_VARIANT_OH192x256 = 22,        // V % 128 == 0: a whole 128 x 256 tile and a 64-row half of another one per workgroup, one k-loop
     SPMM_VARIANT_DIRECT64 = 23,         // id 13's kernel for any N (column tiles) and with the fused write-out: small products
     SPMM_VARIANT_COUNT = 24,
-    SPMM_VARIANT_HDIRECT32 = 24         // the same on 32-row tiles, V % 64 != 0; automatic choice only
+    // the same on 32-row tiles, V % 64 != 0: behind the count, which callers size arrays by and which has five places for V % 64 != 0
+    SPMM_VARIANT_HDIRECT32 = 24
 };
 
 const char* spmm_variant_name(int variant);

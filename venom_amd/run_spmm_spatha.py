@@ -94,7 +94,7 @@ def compare_kernels(out_path, tokens, vs, ms):
                         auto = plan.kernel_name(N, 0, 0)
                         plan.time(B, out, warmup=30, iters=30)
                         times = {}
-                        for variant in range(1, spatha.num_variants()):
+                        for variant in spatha.variant_ids():
                             name = plan.kernel_name(N, 0, variant)
                             if name is not None:
                                 times[name] = min(plan.time(B, out, variant=variant, warmup=5, iters=40) for _ in range(2)) * 1e3

@@ -21,6 +21,14 @@ def num_variants():
     return int(_lib.lib().spatha_spmm_num_variants())
 
 
+DIRECT_HALF_VARIANT = 24        # named beside them: id 23's 32-row form, for V a multiple of 32 only
+
+
+def variant_ids():
+    """Every id that a caller can name."""
+    return list(range(1, num_variants())) + [DIRECT_HALF_VARIANT]
+
+
 def _stream_ptr(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
@@ -174,7 +182,7 @@ class SpmmPlan:
         return ms.value
 
     def tune(self, B, out, bias=None, transposed_out=False, warmup=5, iters=30):
-        """Times the automatic choice and every kernel id that accepts this shape; returns (best id, its ms, the automatic
+        """Times the automatic choice and every kernel id that accepts this shape (`variant_ids`); returns (best id, its ms, the automatic
         choice's ms, {id: ms}) with id 0 = the automatic choice (the best id is 0 when nothing beats it)."""
         L = _lib.lib()
         n = L.spatha_spmm_num_variants()
@@ -186,7 +194,9 @@ class SpmmPlan:
                                           _stream_ptr(self.device), ctypes.byref(best), ctypes.byref(best_ms),
                                           ctypes.byref(auto_ms), per), "spatha_spmm_tune")
         torch.autograd.graph.increment_version(out)
-        return best.value, best_ms.value, auto_ms.value, {i: per[i] for i in range(n) if per[i] >= 0}
+        times = {i: per[i] for i in range(n) if per[i] >= 0}
+        times.setdefault(best.value, best_ms.value)          # (an id beyond the array)
+        return best.value, best_ms.value, auto_ms.value, times
 
 
 _loaded_extension = None
