@@ -176,7 +176,9 @@ struct Shape {
     //   V % 64 == 0 only:  up to one tile per CU 1.4-3.0x, up to two 1.08-1.5x; up to 2.5, m > 8, more than ten k-steps 1.10-1.18x
     //                      (ten or fewer 0.88x; m <= 8 0.93-1.0x); beyond 0.4-1.0x.
     // k-loops of 96 steps on V % 128 == 0 are what split runs are for (12288 x 49152 x 128 at 128:2:16: 48 us in two parts, 71 here).
-    // (Three k-steps or fewer at m <= 8 keep the dense staging that 512 x 256 x 256 at 64:2:8 is expected on.)
+    // Three k-steps or fewer at m <= 8 stay with dense staging although these kernels are ahead there too (up to two tiles per CU,
+    // row-major 1.2-1.9x, 512 x 256 x 256 at 64:2:8 5.9 against 3.2 us, transposed 0.97-1.5x): a caller holds the choice to that
+    // (tests/test_spmm_gpu.py asks for the dense-staged kernel at that shape).
     bool direct64() const {
         const int64_t t = (int64_t)(rows / 64) * ((N + 63) / 64);
         if (v % 128 == 0)
@@ -217,7 +219,8 @@ struct Rule {
 const Rule kRules[] = {
     // few columns: streaming A is all that matters, one 64-row tile per workgroup with the k-steps split over its waves, B
     // straight from the L2 with one load per gathered row whatever N (2, 4 or 8 bytes for 16, 32 or 64 columns).  1.3-3x ahead of
-    // every tiled kernel on the BERT-large matrices; GPT-3 FFN matrix 27-29 us up to 32 columns (6.3 TB/s; 128-wide tiles 39-41),
+    // every tiled kernel on the BERT-large matrices; GPT-3 FFN matrix, launches back to back (its 176 MB then stay in the memory-side
+    // cache; 38.7 us from memory at 16 columns), 27-29 us up to 32 columns (128-wide tiles 39-41),
     // 36 us at 64, level with the 128 x 128 tiles (39): there the registers of its four column blocks leave three workgroups
     // per CU for three tiles per CU.  The same kernel with column tiles (id 23) takes fused write-outs and small products.
     {V_128 | V_64, spatha::SPMM_VARIANT_SKINNY, [](const Shape& s) { return s.N <= 64; }},
