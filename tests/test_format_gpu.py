@@ -1,6 +1,7 @@
-"""Conversion of a matrix that lives on the GPU (search, encoding and decoding as kernels) against the host builder, which the
-oracle checks: the same arrays bit for bit - narrow and wide tails, groups without a winner, equal magnitudes, every group count
-per workgroup, strided and fp32 inputs, infinities and NaN."""
+"""Conversion of a matrix that lives on the GPU (search, encoding and decoding as kernels) against the path through the host (the
+search kernel's winners, host masks and host builder, which the oracle checks; without equal magnitudes the host's own search too): the
+same arrays bit for bit - narrow and wide tails, groups without a winner, equal magnitudes, every group count per workgroup, strided and
+fp32 inputs, infinities and NaN."""
 import numpy as np
 import pytest
 import torch
@@ -47,6 +48,10 @@ def test_conversion_equals_the_host_path(gpu, rows, cols, m, v, kind):
     want = host_matrix(w, m, v)
     for name in ("values", "metadata", "columns"):
         same(getattr(got, name), getattr(want, name))
+    if kind == "fp32":          # no two equal magnitudes or totals: the host's own search, whatever its order among equals
+        host = SrNMTensor(2, m, v, w, *nm_vector_mask_sparsify(w, 2, m, v, gpu=False), w.device)
+        for name in ("values", "metadata", "columns"):
+            same(getattr(got, name), getattr(host, name))
     assert (got.nrows, got.ncols, got.nnz, got.device) == (want.nrows, want.ncols, want.nnz, want.device)
     dense = F.decode(got.values.cpu().numpy(), got.metadata.cpu().numpy().view(np.uint32),
                      got.columns.cpu().numpy().astype(np.uint32), rows, cols, 2, m, v)

@@ -124,8 +124,9 @@ class SrnmSpmm(torch.nn.Module):
         return out.reshape(*input.shape[:-1], -1)
 
     def forward_feature_major(self, input, activation="none"):
-        """act(x W^T + b) as a [..., out] VIEW of a feature-major buffer [out, tokens]: bias and activation run in
-        the kernel's write-out, and the next SrnmSpmm takes the buffer as its right-hand side without a copy."""
+        """act(x W^T + b) as a [..., out] VIEW of a feature-major buffer [out, tokens] (its rows padded to a multiple of 8
+        tokens): bias and activation run in the kernel's write-out, and the next SrnmSpmm takes the buffer as its right-hand side
+        without a copy."""
         if activation in spatha._ACTIVATIONS:
             out = self._run_native(type(self), self, input, self.nrows_sp, self.ncols_sp, True, spatha._ACTIVATIONS[activation])
             if out is not None:
@@ -134,7 +135,7 @@ class SrnmSpmm(torch.nn.Module):
         rhs = self._transposed(flat)
         out = spatha.spmm_fused(self.metadata, self.columns, self.values, rhs, self.bias, self.nrows_sp, self.ncols_sp,
                                 self.v, self.n, self.m, activation=activation)              # [out, tokens]
-        return out.T.reshape(*input.shape[:-1], -1)     # strides (.., 1, tokens): a view, nothing moves
+        return out.T.reshape(*input.shape[:-1], -1)     # strides (.., 1, tokens): a view, nothing moves (no padding on this path)
 
 
 class _MergedProjections:
