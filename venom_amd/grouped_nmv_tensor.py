@@ -38,10 +38,14 @@ def nm_vector_mask_sparsify(tensor, n, m, tileM, threads=0, gpu=None, exact_ties
 
 
 def _decodes_on_gpu(a, geo):
-    """Do a's three arrays have the types, sizes, place and addresses that the decoding kernel takes?"""
+    """The addresses of a's three arrays where they have the types, sizes, place and alignment that the decoding kernel takes, else None."""
     arrays = ((a.values, torch.float16, geo.n_values), (a.metadata, torch.int32, geo.n_metadata), (a.columns, torch.int32, geo.n_columns))
-    return all(t.is_cuda and t.device == a.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
-               and t.data_ptr() % 4 == 0 for t, dtype, count in arrays)
+    if all(t.is_cuda and t.device == a.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
+           for t, dtype, count in arrays):
+        where = [t.data_ptr() for t, _, _ in arrays]
+        if all(address % 4 == 0 for address in where):
+            return where
+    return None
 
 
 class SrNMTensor:
@@ -97,14 +101,14 @@ class SrNMTensor:
 
     def to_dense(self):
         geo = F.geometry(self.nrows, self.ncols, self.n, self.m, self.tileM)
-        if _decodes_on_gpu(self, geo):
+        where = _decodes_on_gpu(self, geo)
+        if where is not None:
             dev = self.values.device
             dense = torch.empty((self.nrows, self.ncols), dtype=torch.float16, device=dev)
             bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)      # written by the kernel where an offset has no place
             with torch.cuda.device(dev):
-                _lib.check(_lib.lib().spatha_vnm_decode_f16_gpu(self.values.data_ptr(), self.metadata.data_ptr(),
-                                                                self.columns.data_ptr(), self.nrows, self.ncols, self.n, self.m,
-                                                                self.tileM, dense.data_ptr(), bad.data_ptr(),
+                _lib.check(_lib.lib().spatha_vnm_decode_f16_gpu(*where, self.nrows, self.ncols, self.n, self.m, self.tileM,
+                                                                dense.data_ptr(), bad.data_ptr(),
                                                                 torch.cuda.current_stream(dev).cuda_stream), "spatha_vnm_decode")
                 torch.cuda.current_stream(dev).synchronize()
             if bad.item():
