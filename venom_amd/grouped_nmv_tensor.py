@@ -39,13 +39,14 @@ def nm_vector_mask_sparsify(tensor, n, m, tileM, threads=0, gpu=None, exact_ties
 
 def _decodes_on_gpu(a, geo):
     """The addresses of a's three arrays where they have the types, sizes, place and alignment that the decoding kernel takes, else None."""
-    arrays = ((a.values, torch.float16, geo.n_values), (a.metadata, torch.int32, geo.n_metadata), (a.columns, torch.int32, geo.n_columns))
-    if all(t.is_cuda and t.device == a.values.device and t.dtype == dtype and t.numel() == count and t.is_contiguous()
-           for t, dtype, count in arrays):
-        where = [t.data_ptr() for t, _, _ in arrays]
-        if all(address % 4 == 0 for address in where):
-            return where
-    return None
+    values, metadata, columns = a.values, a.metadata, a.columns
+    if not (values.is_cuda and metadata.device == values.device and columns.device == values.device
+            and values.dtype == torch.float16 and metadata.dtype == torch.int32 and columns.dtype == torch.int32
+            and values.numel() == geo.n_values and metadata.numel() == geo.n_metadata and columns.numel() == geo.n_columns
+            and values.is_contiguous() and metadata.is_contiguous() and columns.is_contiguous()):
+        return None
+    where = values.data_ptr(), metadata.data_ptr(), columns.data_ptr()
+    return None if (where[0] | where[1] | where[2]) % 4 else where
 
 
 class SrNMTensor:
