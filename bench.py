@@ -44,7 +44,7 @@ MEASURED_TRAFFIC = {
     ("smfmac16x16x64_warpspec_storewaves_tile128x128_3stage", 1024, 4096, 4096, 8, 128):
         (61_530_000, "profiles/spmm_wsw_kernel_tile128x128_config1_128-2-8.md"),
     ("smfmac16x16x64_skinny_tile64x16_splitk4", 49152, 12288, 16, 16, 128):
-        (184_100_000, "profiles/spmm_skinny_kernel_gpt3_ffn_n16.md"),
+        (179_400_000, "profiles/spmm_direct_kernel_small_products.md"),
     ("smfmac16x16x64_warpspec_tile_and_a_half_192x256_4slots", 49152, 12288, 256, 16, 128):
         (251_500_000, "profiles/spmm_oh_kernel_gpt3_ffn_n256_128-2-16.md"),
     ("smfmac16x16x64_warpspec_tall_tile128x256_3stage", 49152, 12288, 2048, 16, 128):

@@ -2,7 +2,7 @@
 // storage map), from and to matrices that live in device memory (to_sparse_sr_nm / func2 and to_dense / func3,
 // end2end/grouped_nmv_tensor.py:345-675).  Both kernels only move data; one thread owns one metadata word (two rows, four groups)
 // or eight adjacent entries of a dense row, so that the compressed side and the dense side are each written in whole words.
-// Encoding 4096 x 1024 at 64:2:8: 7.0 us; decoding 1024 x 4096 at 128:2:16: 6.8 us (a call of to_dense 32 us, most of it the wait for
+// Encoding 4096 x 1024 at 64:2:8: 7.2 us; decoding 1024 x 4096 at 128:2:16: 6.8 us (a call of to_dense 32 us, most of it the wait for
 // the flag of the offset check; 870 us when the arrays were decoded on the host).
 
 #include <hip/hip_runtime.h>

@@ -10,8 +10,9 @@
 // subset ranks: with one group per workgroup (the form before this one) m = 8 kept 70 of 256 threads busy.  Magnitudes sit
 // in LDS column by column (pitch V + 4 words: 16-byte reads of four rows at a time, sixteen different columns on different
 // banks).
-// 4096 x 1024 at 64:2:8 (8192 groups of 70 subsets): 16.8 us; with the encoder behind it (format_gpu.hip, 7.0 us) a conversion takes
-// 41 us, 6.3 ms when magnitudes, masks and arrays went through the host.
+// 4096 x 1024 at 64:2:8 (8192 groups of 70 subsets): 28 us, 1024 x 1024 14.5; 4096 x 1024 at 64:2:16 (1820 subsets) 161.  With the
+// encoder behind it (format_gpu.hip, 7.2 us) the first conversion takes 37.5 us, 6.3 ms when magnitudes, masks and arrays went
+// through the host.
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
