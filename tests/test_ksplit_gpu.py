@@ -152,3 +152,36 @@ def test_split_gaussian_within_tolerance_and_deterministic(gpu):
     e = rel_err(runs[0], exact)
     print("k-split, Gaussian: max rel err %.3e" % e, flush=True)
     assert e <= 1e-2
+
+
+@pytest.mark.parametrize("kind", ["operator", "plan"])
+def test_a_workspace_made_in_a_capture_is_not_kept(gpu, kind):
+    """The first split run on a stream is recorded into a graph: its scratch memory is zeroed by the replays, so the eager run after the
+    capture, with no replay yet, brings its own; replays and eager runs in turn, on new operands, equal the unsplit product."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the case is sized for 256 compute units")
+    rows, cols, N, m, v = 512, 16384, 1024, 8, 128
+    vals, meta, columns, B, bias, plan = _operands(rows, cols, N, m, v, True, gpu)
+    dv, dm, dc, dB, dbias = _dev(vals, gpu), _dev(meta, gpu), _dev(columns, gpu), _dev(B, gpu), _dev(bias, gpu)
+    assert plan.workspace_bytes(N, True) > 0
+    if kind == "operator":
+        call = lambda: spatha.spmm(dm, dc, dv, dB, dbias, rows, cols, N, v, 2, m)
+    else:
+        call = lambda: plan.run(dB, bias=dbias, transposed_out=True, split=True)
+    want = lambda: plan.run(dB, bias=dbias, transposed_out=True)        # integer operands: any order of the sums
+    assert torch.equal(call(), want())                                  # on another stream: plan and kernels are ready
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream(device=gpu)
+    with torch.cuda.stream(s):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            recorded = call()
+        for seed in range(3):
+            dB.copy_(torch.from_numpy(np.random.default_rng(seed).integers(-4, 5, size=(cols, N)).astype(np.float16)))
+            expected = want()
+            assert torch.equal(call(), expected), seed
+            graph.replay()
+            s.synchronize()
+            assert torch.equal(recorded, expected) and torch.equal(call(), expected), seed
+    s.synchronize()
+    spatha.clear_plan_cache()

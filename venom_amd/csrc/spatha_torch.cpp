@@ -71,14 +71,25 @@ void check(int status, const char* what) {
                                  (status == SPATHA_ERR_HIP ? " (HIP error " + std::to_string(spatha_last_hip_error()) + ")" : ""));
 }
 
+// The capture that records what is issued to `stream` now, 0 where nothing records it.
+unsigned long long capture_of(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
+    return status == hipStreamCaptureStatusActive ? id : 0ull;
+}
+
 // Scratch memory of split runs (spatha_spmm_run_ws): one zero-initialised buffer per (device, stream), grown on demand.
 // Calls on one stream are ordered, so they can share it; the library leaves it clean after every completed call.
+// A buffer made while a graph is captured is not kept: its zeros are written by the graph's replays only.
 std::map<std::pair<int, hipStream_t>, torch::Tensor> g_workspaces;
 
 torch::Tensor workspace_for(int device, hipStream_t stream, size_t bytes, const torch::TensorOptions& like) {
     std::lock_guard<std::mutex> guard(g_lock);
-    torch::Tensor& ws = g_workspaces[{device, stream}];
-    if (!ws.defined() || (size_t)ws.numel() < bytes) ws = torch::zeros({(int64_t)bytes}, like.dtype(torch::kUInt8));
+    const auto kept = g_workspaces.find({device, stream});
+    if (kept != g_workspaces.end() && (size_t)kept->second.numel() >= bytes) return kept->second;
+    const torch::Tensor ws = torch::zeros({(int64_t)bytes}, like.dtype(torch::kUInt8));
+    if (!capture_of(stream)) g_workspaces[{device, stream}] = ws;
     return ws;
 }
 
@@ -231,10 +242,7 @@ bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
 // only what was recorded into it, and what was recorded has not run.
 py::tuple stream_key(int device) {
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    unsigned long long id = 0;
-    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
-    return py::make_tuple((uintptr_t)stream, status == hipStreamCaptureStatusActive ? id : 0ull);
+    return py::make_tuple((uintptr_t)stream, capture_of(stream));
 }
 
 // Is `key` the Python key (address, shape, strides, version, device, stream_key) of `held`, and is x the same tensor at the same

@@ -145,7 +145,9 @@ class SpmmPlan:
                 key = torch.cuda.current_stream(self.device).cuda_stream
                 workspace = self._workspaces.get(key)
                 if workspace is None or workspace.numel() < need:
-                    workspace = self._workspaces[key] = torch.zeros(need, dtype=torch.uint8, device=B.device)
+                    workspace = torch.zeros(need, dtype=torch.uint8, device=B.device)
+                    if not torch.cuda.is_current_stream_capturing():     # (its zeros would be written by the graph's replays only)
+                        self._workspaces[key] = workspace
             ws_ptr = None if workspace is None else workspace.data_ptr()
             ws_len = 0 if workspace is None else workspace.numel() * workspace.element_size()
             with torch.cuda.device(self.device):
