@@ -41,3 +41,9 @@ def test_plans_and_transpose_run_without_the_extension(gpu, without_extension):
     got = plan.run(B).float().cpu()
     assert (got - dense @ B.float().cpu()).norm() <= 1.2e-3 * got.norm()          # one rounding to fp16
     assert torch.equal(spatha.transpose(B), B.T)
+    # a norm that hands its feature-major copy on (to whatever reads it) asks for none either
+    from venom_amd.bert import SrnmSpmm
+
+    x = B.T.contiguous()
+    SrnmSpmm.offer_transposed(x, B)
+    assert SrnmSpmm._transposed(x) is B or SrnmSpmm._transposed(x).data_ptr() == B.data_ptr()

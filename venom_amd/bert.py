@@ -51,7 +51,7 @@ def _activation_key(flat):
     stream and graph capture that it was computed on - another stream is not ordered behind the kernel that fills the copy, and a
     graph replays only what was recorded into it."""
     return (flat.data_ptr(), tuple(flat.shape), tuple(flat.stride()), flat._version, flat.device,
-            spatha._extension().stream_key(flat.get_device()) if flat.is_cuda else None)
+            spatha._stream_key(flat.device) if flat.is_cuda else None)
 
 
 class SrnmSpmm(torch.nn.Module):

@@ -235,6 +235,14 @@ def _native(name):
         return None
 
 
+def _stream_key(device):
+    """(stream, capture) that work issued now on this GPU goes to; without the extension the capture counts as one."""
+    try:
+        return _extension().stream_key(device.index)
+    except RuntimeError:
+        return torch.cuda.current_stream(device).cuda_stream, torch.cuda.is_current_stream_capturing()
+
+
 def clear_plan_cache():
     _extension().clear_plan_cache()
 
