@@ -58,6 +58,31 @@ def test_conversion_equals_the_host_path(gpu, rows, cols, m, v, kind):
     same(got.to_dense(), torch.from_numpy(dense).cuda())
 
 
+@pytest.mark.parametrize("rows,cols,m,v", [(96, 300, 5, 32), (96, 1029, 7, 32), (128, 2052, 9, 64), (64, 416, 11, 64), (128, 135, 17, 128),
+                                           (512, 85, 40, 512), (960, 40, 40, 960), (960, 44, 4, 960)])
+@pytest.mark.parametrize("kind", ["gauss", "subnormal", "large", "fp32", "nan"])
+def test_search_on_packed_magnitudes_finds_the_hosts_columns(gpu, rows, cols, m, v, kind):
+    """Runs of one to five subsets per triple with every remainder, four groups to a workgroup and fewer (the encoding in a launch of its
+    own), blocks without a spare unit between columns; fp16 totals through subnormals and up to fp32's rounding of large sums, and a
+    NaN, which sends its workgroup the other way."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + 5 * cols + m)
+    w = torch.randn((rows, cols), generator=gen, device="cuda")
+    w = {"subnormal": w * 2.0 ** -21, "large": w * 9000}.get(kind, w)
+    if kind != "fp32":
+        w = w.half()
+    if kind == "nan":
+        w[rows // 2, cols // 3] = float("nan")
+    got = bert.NMVectorSparsifier(2, m, v, magnitude=True)(w).wrapped_tensor
+    # the selector's GPU search runs in fp32 and needs no tie replay for its columns; the host's own search checks it without a NaN
+    mask, columns = nm_vector_mask_sparsify(w, 2, m, v, gpu=True, exact_ties=False)
+    want = SrNMTensor(2, m, v, w, mask, columns, w.device)
+    for name in ("values", "metadata", "columns"):
+        same(getattr(got, name), getattr(want, name))
+    if kind != "nan":
+        _, host = nm_vector_mask_sparsify(w, 2, m, v, gpu=False)
+        assert torch.equal(got.columns.cpu(), host)
+
+
 def test_a_column_offset_beyond_the_group_is_refused(gpu):
     a = bert.NMVectorSparsifier(2, 8, 32, magnitude=True)(torch.randn(32, 64, device="cuda").half()).wrapped_tensor
     a.columns[5] = 8

@@ -620,13 +620,8 @@ int spatha_vnm_convert_gpu(const void* dense_dev, int value_bits, int rows, int 
         return SPATHA_ERR_BAD_ARGUMENT;
     const int tasks = spatha::select_task_count(rows, cols, m, v, nullptr);
     if (tasks > 0 && (size_t)v * (size_t)m * sizeof(float) > 150u * 1024u) return SPATHA_ERR_TOO_LARGE;
-    hipStream_t s = (hipStream_t)stream;
-    int32_t* columns = (int32_t*)columns_dev;
-    hipError_t e = value_bits == 16
-                       ? spatha::launch_select_winners_f16((const uint16_t*)dense_dev, rows, cols, m, v, device_cus(), columns, geo.ksp / 2, s)
-                       : spatha::launch_select_winners_f32((const float*)dense_dev, rows, cols, m, v, device_cus(), columns, geo.ksp / 2, s);
-    if (e == hipSuccess)
-        e = spatha::launch_encode_winners(dense_dev, value_bits, rows, cols, m, v, geo.ksp, values_dev, metadata_dev, columns, s);
+    const hipError_t e = spatha::launch_convert(dense_dev, value_bits, rows, cols, m, v, geo.ksp, device_cus(), values_dev, metadata_dev,
+                                                (int32_t*)columns_dev, (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 

@@ -106,13 +106,10 @@ hipError_t launch_pack(const uint16_t* values, const uint32_t* metadata, const u
 // (a winner's second column is at least 1).  out_pitch: entries of four per V-row block.  dense: the signed matrix or |A|.
 hipError_t launch_select_winners_f32(const float* dense_dev, int rows, int cols, int m, int v, int cus, int32_t* out_dev,
                                      int64_t out_pitch, hipStream_t stream);
-hipError_t launch_select_winners_f16(const uint16_t* dense_dev, int rows, int cols, int m, int v, int cus, int32_t* out_dev,
-                                     int64_t out_pitch, hipStream_t stream);
-
-// Encoding of the selector's choice and decoding on the GPU (format_gpu.hip); column-loc holds the search's winners on entry to
-// the encoder, which completes it (narrow tail, padding groups).  decode: *bad is set to 1 if a column offset is not below m.
-hipError_t launch_encode_winners(const void* dense_dev, int value_bits, int rows, int cols, int m, int v, int ksp, uint16_t* values,
-                                 uint32_t* metadata, int32_t* columns, hipStream_t stream);
+// Magnitude selection and encoding (select_gpu.hip), and decoding (format_gpu.hip), in device memory.  decode: *bad is set to 1 if a
+// column offset is not below m.
+hipError_t launch_convert(const void* dense_dev, int value_bits, int rows, int cols, int m, int v, int ksp, int cus, uint16_t* values,
+                          uint32_t* metadata, int32_t* columns, hipStream_t stream);
 hipError_t launch_decode_f16(const uint16_t* values, const uint32_t* metadata, const uint32_t* columns, int rows, int cols, int m,
                              int v, int ksp, uint16_t* dense, uint32_t* bad, hipStream_t stream);
 
