@@ -314,6 +314,16 @@ int spatha_add_layernorm_f16_t(const uint16_t* x_dev, const uint16_t* residual_d
                                const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
                                void* stream);
 
+/* out_t[64 * head + f][token] = the attention of every sequence and head of a batch, softmax(scale * Q K^T) V over the sequence's own
+ * tokens, no mask: q, k and v hold batch * seq rows `pitch` entries apart, head h at column 64 h (slices of one merged
+ * projection, for instance); fp16 in and out, fp32 scores, sums and output, probabilities rounded to fp16.  The result is
+ * feature-major with rows out_pitch >= batch * seq entries apart, columns up to the next multiple of 8 set to zero: the right-hand side
+ * of the output projection's spatha_spmm_run as it lies.  head_dim 64 only (SPATHA_ERR_UNSUPPORTED), scale > 0; q, k, v at
+ * 16-byte addresses, pitch % 8 == 0.  What the stock attention module of the reference's harness computes
+ * (end2end/bert_pytorch.py:170-171). */
+int spatha_attention_f16(const uint16_t* q_dev, const uint16_t* k_dev, const uint16_t* v_dev, int64_t pitch, int batch, int seq, int heads,
+                         int head_dim, float scale, uint16_t* out_t_dev, int64_t out_pitch, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

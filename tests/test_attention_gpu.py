@@ -1,0 +1,91 @@
+"""The attention kernel (attention.hip) against softmax(scale Q K^T) V in 64 bits: tiles of 128 queries and 64 keys with every kind of
+remainder, batches whose sequences start at any token, scores that make the running maximum move, one dominating key; and the
+attention module of a model that uses it against the stock one."""
+import pytest
+import torch
+
+from venom_amd import _lib, bert, spatha
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(qkv, batch, seq, heads, scale):
+    q, k, v = (t.double().reshape(batch, seq, heads, 64).transpose(1, 2).contiguous() for t in qkv.split(heads * 64, dim=1))
+    scores = scale * (q.unsqueeze(3) * k.unsqueeze(2)).sum(-1) if seq <= 64 else scale * torch.matmul(q, k.transpose(2, 3).contiguous())
+    return torch.matmul(torch.softmax(scores, -1), v).transpose(1, 2).reshape(batch, seq, heads * 64)
+
+
+@pytest.mark.parametrize("batch,seq,heads", [(1, 1, 1), (2, 5, 16), (3, 31, 3), (1, 32, 16), (5, 33, 2), (2, 64, 4), (3, 65, 5), (2, 127, 16),
+                                             (3, 127, 1), (2, 128, 3), (1, 129, 9), (2, 301, 4), (4, 512, 16), (1, 700, 2)])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_attention_matches_the_exact_result(gpu, batch, seq, heads, spread):
+    """Error bound: the probabilities and the result are rounded to fp16 (2^-11 each; the probabilities' roundings average over the
+    keys but for a dominating one), scores and sums are fp32 (a score of 600 at spread 8 is off by 600 * 64 * 2^-24 at most):
+    entries within 2^-9 of the largest |V| that they average, the whole within 6e-4."""
+    gen = torch.Generator(device=gpu).manual_seed(seq * 7 + heads)
+    qkv = torch.randn((batch * seq, 3 * heads * 64), generator=gen, device=gpu).half()
+    qkv[:, :heads * 64] *= spread
+    got = spatha._extension().attention(qkv, batch, seq, heads, 0.125)
+    assert got.shape == (batch, seq, heads * 64) and got.dtype == torch.float16
+    want = exact(qkv, batch, seq, heads, 0.125)
+    diff = got.double() - want
+    assert diff.norm().item() <= 6e-4 * want.norm().item()
+    assert diff.abs().max().item() <= 2.0 ** -9 * qkv[:, 2 * heads * 64:].abs().max().item()
+    # the buffer behind the view: padding columns are zero
+    flat = torch.as_strided(got, (heads * 64, (batch * seq + 7) // 8 * 8), ((batch * seq + 7) // 8 * 8, 1))
+    assert not flat[:, batch * seq:].any()
+
+
+def test_attention_error_is_no_larger_than_the_stock_kernels(gpu):
+    gen = torch.Generator(device=gpu).manual_seed(3)
+    for batch, seq in ((2, 512), (2, 77)):
+        qkv = torch.randn((batch * seq, 3072), generator=gen, device=gpu).half()
+        want = exact(qkv, batch, seq, 16, 0.125)
+        got = spatha._extension().attention(qkv, batch, seq, 16, 0.125)
+        q, k, v = (t.reshape(batch, seq, 16, 64).transpose(1, 2) for t in qkv.split(1024, dim=1))
+        stock = torch.nn.functional.scaled_dot_product_attention(q, k, v, scale=0.125).transpose(1, 2).reshape(batch, seq, 1024)
+        ours, theirs = ((x.double() - want).norm().item() / want.norm().item() for x in (got, stock))
+        print("relative error %.3g, the stock kernel's %.3g" % (ours, theirs))
+        assert ours <= 1.02 * theirs          # (2 %: which way the roundings fall)
+
+
+def test_attention_refuses_what_it_does_not_take(gpu):
+    x = torch.zeros((8, 3 * 64), dtype=torch.float16, device=gpu)
+    out = torch.zeros((64, 8), dtype=torch.float16, device=gpu)
+
+    def call(head_dim=64, scale=0.125, pitch=192, out_pitch=8, q=x.data_ptr()):
+        return _lib.lib().spatha_attention_f16(q, x.data_ptr(), x.data_ptr(), pitch, 1, 8, 1, head_dim, scale, out.data_ptr(), out_pitch,
+                                               torch.cuda.current_stream().cuda_stream)
+    assert call() == 0
+    assert call(head_dim=32) == 3
+    assert all(s != 0 for s in (call(scale=0.0), call(pitch=190), call(pitch=56), call(out_pitch=7), call(q=x.data_ptr() + 2), call(q=None)))
+    assert spatha._extension().attention(x.float(), 1, 8, 1, 0.125) is None
+    assert spatha._extension().attention(x, 2, 8, 1, 0.125) is None
+
+
+def test_a_models_attention_takes_the_kernel_and_falls_back(gpu):
+    """Without a mask the merged attention runs in the kernel; with one, in training mode or with a hook on a projection the stock
+    forward answers.  Two fp16 attentions: 2e-3 apart at most (each within 6e-4 of the exact result)."""
+    torch.set_grad_enabled(False)
+    model = bert.merge_qkv(bert.linear_to_spmm(bert.build_bert_large(layers=1).to(gpu).half(), 2, 8, 64))
+    stock = model.encoder.layer[0].attention.self
+    x = torch.randn((2, 40, 1024), device=gpu).half()
+    want, _ = stock(x)
+    keys = list(model.state_dict())
+    bert.fuse_add_layernorm(model, feature_major=True)
+    att = model.encoder.layer[0].attention.self
+    assert type(att) is bert.FusedSelfAttention and list(att.state_dict()) == [k[len("encoder.layer.0.attention.self."):] for k in keys
+                                                                             if k.startswith("encoder.layer.0.attention.self.")]
+    got, weights = att(x)
+    assert weights is None and got.shape == want.shape and got.stride(-1) == 80
+    assert (got.double() - want.double()).norm() <= 2e-3 * want.double().norm()
+    mask = torch.ones((2, 1, 40, 40), dtype=torch.bool, device=gpu)
+    mask[:, :, :, 30:] = False
+    masked, _ = att(x, attention_mask=mask)
+    assert masked.stride(-1) == 1 and not torch.equal(masked, got)
+    handle = att.key.register_forward_hook(lambda m, a, o: o * 0)
+    hooked, _ = att(x)
+    handle.remove()
+    v = att.value(x).float().mean(1, keepdim=True)
+    assert (hooked.float() - v).abs().max() <= 4e-3       # equal scores: every token averages V
+    assert torch.equal(att(x)[0], got)

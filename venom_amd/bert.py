@@ -159,7 +159,8 @@ class _MergedProjections:
             self.rows += l.nrows_sp
         self._last = (None, None, None)          # (key, activation held alive, [tokens, rows] result)
 
-    def output(self, index, nrows, input):
+    def merged(self, input):
+        """[tokens, rows]: all members' outputs side by side."""
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
         key = _activation_key(flat)
         if self._last[0] != key:
@@ -169,8 +170,11 @@ class _MergedProjections:
                 out = spatha.spmm(self.metadata, self.columns, self.values, rhs, self.bias, self.rows, self.cols, rhs.shape[1],
                                   self.v, self.n, self.m, 0, 0, 32, 4)
             self._last = (key, flat, out)
+        return self._last[2]
+
+    def output(self, index, nrows, input):
         start = self.starts[index]
-        return self._last[2][:, start:start + nrows].reshape(*input.shape[:-1], nrows)
+        return self.merged(input)[:, start:start + nrows].reshape(*input.shape[:-1], nrows)
 
 
 def merge_qkv(model):
@@ -185,6 +189,48 @@ def merge_qkv(model):
             for i, l in enumerate(layers):
                 l._group, l._group_index = group, i
     return model
+
+
+def _fused_self_attention():
+    """The class that `fuse_add_layernorm(feature_major=True)` gives to a BertSelfAttention whose projections are merged: the same
+    module with the library's attention kernel where that applies (`FusedSelfAttention` of this module; made on first use, so that
+    the package imports without transformers)."""
+    from transformers.models.bert.modeling_bert import BertSelfAttention
+
+    class FusedSelfAttention(BertSelfAttention):
+        """Attention over the merged projections by one kernel, which leaves its result feature-major for the output projection.
+        Without a mask, in evaluation, for fp16 and heads of 64 features; any other call takes the stock forward."""
+
+        def forward(self, hidden_states, attention_mask=None, past_key_values=None, **kwargs):
+            context = None
+            if attention_mask is None and past_key_values is None and not self.training and not self.is_causal and not self.is_decoder \
+                    and self.config._attn_implementation == "sdpa" and hidden_states.dim() == 3 \
+                    and all(v is None or k == "position_ids" for k, v in kwargs.items()):
+                context = self._attend(hidden_states)
+            if context is None:
+                return super().forward(hidden_states, attention_mask, past_key_values, **kwargs)
+            return context, None
+
+        def _attend(self, hidden_states):
+            layers = self.query, self.key, self.value
+            group = layers[0]._group
+            if group is None or self.attention_head_size != 64 or not self.scaling > 0 or len(group.starts) != 3 \
+                    or group.rows != 3 * self.all_head_size \
+                    or any(l._group is not group or l._group_index != i or l._forward_hooks or l._forward_pre_hooks
+                           for i, l in enumerate(layers)):
+                return None
+            batch, seq = hidden_states.shape[:2]
+            return spatha._extension().attention(group.merged(hidden_states), batch, seq, self.num_attention_heads, self.scaling)
+
+    FusedSelfAttention.__qualname__ = "FusedSelfAttention"
+    globals()["FusedSelfAttention"] = FusedSelfAttention
+    return FusedSelfAttention
+
+
+def __getattr__(name):
+    if name == "FusedSelfAttention":
+        return _fused_self_attention()
+    raise AttributeError("module %r has no attribute %r" % (__name__, name))
 
 
 class FusedFeedForwardIn(torch.nn.Module):
@@ -271,10 +317,14 @@ class FusedProjectionNorm(torch.nn.Module):
 
 def fuse_add_layernorm(model, feature_major=False):
     """Replaces, in place, every BertSelfOutput / BertOutput by FusedProjectionNorm (same parameters).  feature_major: for a
-    model whose projections are SrnmSpmm layers - the kernel also writes the feature-major copy the next projection reads."""
-    from transformers.models.bert.modeling_bert import BertOutput, BertSelfOutput
+    model whose projections are SrnmSpmm layers - the kernel also writes the feature-major copy the next projection reads, and where
+    `merge_qkv` has merged an attention's projections, that attention runs in the library's kernel, whose result the output
+    projection reads as it lies."""
+    from transformers.models.bert.modeling_bert import BertOutput, BertSelfAttention, BertSelfOutput
 
     for mod in model.modules():
+        if feature_major and type(mod) is BertSelfAttention and isinstance(mod.query, SrnmSpmm) and mod.query._group is not None:
+            mod.__class__ = globals().get("FusedSelfAttention") or _fused_self_attention()
         for name, child in list(mod.named_children()):
             if isinstance(child, (BertSelfOutput, BertOutput)):
                 setattr(mod, name, FusedProjectionNorm(child, feature_major))

@@ -994,4 +994,18 @@ int spatha_add_layernorm_f16_t(const uint16_t* x_dev, const uint16_t* residual_d
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 
+int spatha_attention_f16(const uint16_t* q_dev, const uint16_t* k_dev, const uint16_t* v_dev, int64_t pitch, int batch, int seq, int heads,
+                         int head_dim, float scale, uint16_t* out_t_dev, int64_t out_pitch, void* stream) {
+    if (!q_dev || !k_dev || !v_dev || !out_t_dev || batch <= 0 || seq <= 0 || heads <= 0) return SPATHA_ERR_BAD_ARGUMENT;
+    if (!(scale > 0.f) || scale > 1e30f) return SPATHA_ERR_BAD_ARGUMENT;
+    if (head_dim != 64) return SPATHA_ERR_UNSUPPORTED;
+    if ((int64_t)batch * heads > INT32_MAX / 2 || (int64_t)batch * seq > INT32_MAX / 2 || seq > (1 << 20) || heads > (1 << 20))
+        return SPATHA_ERR_TOO_LARGE;
+    if (pitch % 8 != 0 || pitch < (int64_t)heads * head_dim || out_pitch < (int64_t)batch * seq) return SPATHA_ERR_BAD_SHAPE;
+    if ((((uintptr_t)q_dev | (uintptr_t)k_dev | (uintptr_t)v_dev) & 15u) || ((uintptr_t)out_t_dev & 1u)) return SPATHA_ERR_BAD_ARGUMENT;
+    const hipError_t e = spatha::launch_attention_f16(q_dev, k_dev, v_dev, pitch, batch, seq, heads, scale, out_t_dev, out_pitch,
+                                                      (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
 }  // extern "C"

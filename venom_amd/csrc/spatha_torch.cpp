@@ -353,6 +353,28 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
     return result(feature_major ? out.t() : out, kept);
 }
 
+// The attention of `heads` heads of 64 features over qkv [batch * seq, 3 * heads * 64] (queries, keys, values side by side): [batch, seq,
+// heads * 64] as a view of a feature-major buffer, which the output projection reads as it lies.  None for an operand that the
+// kernel does not take.
+py::object attention(py::handle input, int64_t batch, int64_t seq, int64_t heads, double scale) {
+    if (!THPVariable_CheckExact(input.ptr())) return py::none();
+    const torch::Tensor& qkv = THPVariable_Unpack(input.ptr());
+    const int64_t tokens = batch * seq, hidden = heads * 64, padded = (tokens + 7) / 8 * 8;
+    if (!qkv.is_cuda() || qkv.layout() != torch::kStrided || qkv.scalar_type() != torch::kFloat16 || qkv.dim() != 2 || batch <= 0 || seq <= 0 ||
+        heads <= 0 || qkv.size(0) != tokens || qkv.size(1) != 3 * hidden || !qkv.is_contiguous() || ((uintptr_t)qkv.data_ptr() & 15) ||
+        tokens > INT32_MAX / 2 || seq > (1 << 20))
+        return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(qkv.device());
+    torch::Tensor out = torch::empty({hidden, padded}, qkv.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(qkv.get_device()).stream();
+    const uint16_t* q = (const uint16_t*)qkv.data_ptr();
+    check(spatha_attention_f16(q, q + hidden, q + 2 * hidden, 3 * hidden, (int)batch, (int)seq, (int)heads, 64, (float)scale,
+                               (uint16_t*)out.data_ptr(), padded, stream),
+          "spatha_attention_f16");
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(out.narrow(1, 0, tokens).t().view({batch, seq, hidden})));
+}
+
 // SpmmPlan.run without a k-split, for operands in order; None where the caller's checks have to speak.  bias needs the transposed
 // layout unless `fused` (an activation, ACT_NONE among them, was named).
 py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle out, int rows, int cols, int device, bool transposed_out,
@@ -455,6 +477,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
             py::arg("A_num_cols"), py::arg("vec_length"), py::arg("n"), py::arg("m"), py::arg("activation") = 0,
             py::arg("transposed_out") = false);
     mod.def("layer_spmm", &layer_spmm, "one V:N:M layer, right-hand side and product, or None");
+    mod.def("attention", &attention, "attention of merged projections, feature-major, or None");
     mod.def("stream_key", &stream_key, "(stream, capture) that work issued now on this device goes to", py::arg("device"));
     mod.def("transpose", &transpose_f16, "x.T of an fp16 matrix through the library's kernel, or None");
     mod.def("plan_run", &plan_run, "a plan's product, or None, or the status of a refusal");

@@ -127,6 +127,10 @@ hipError_t launch_add_layernorm_f16(const uint16_t* x, const uint16_t* residual,
 hipError_t launch_add_layernorm_f16_t(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
                                       float eps, int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream);
 
+// softmax(scale Q K^T) V per sequence and head of 64 features, result feature-major (attention.hip)
+hipError_t launch_attention_f16(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t pitch, int batch, int seq, int heads,
+                                float scale, uint16_t* out, int64_t out_pitch, hipStream_t stream);
+
 hipError_t launch_dense_gemm(const uint16_t* A, const uint16_t* B, int rows, int cols, int N, uint16_t* C,
                              hipStream_t stream);
 
