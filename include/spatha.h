@@ -314,6 +314,21 @@ int spatha_add_layernorm_f16_t(const uint16_t* x_dev, const uint16_t* residual_d
                                const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
                                void* stream);
 
+/* spatha_add_layernorm_f16_t for any token count: rows of out_t are ROUND_UP(tokens, 8) entries long, zeros behind the last token. */
+int spatha_add_layernorm_f16_tp(const uint16_t* x_dev, const uint16_t* residual_dev, const uint16_t* gamma_dev,
+                                const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
+                                void* stream);
+
+/* The embedding of batch x seq tokens: out[token] = LayerNorm((word[ids[token]] + type[types]) + position[positions[s]]), every sum
+ * rounded to fp16, the norm as in spatha_add_layernorm_f16; out_t (may be NULL) as in spatha_add_layernorm_f16_tp.  ids and
+ * types per token, int64 (types_stride entries from one sequence to the next, 0: one row of `seq` for all), positions per position
+ * of a sequence.  An index outside its table (words, types, positions rows) ends the kernel with a trap, as the lookups do that
+ * this replaces (the stock BertEmbeddings of the reference's harness, end2end/bert_pytorch.py:170-171). */
+int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev, int64_t types_stride, const int64_t* positions_dev, int batch,
+                               int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev, int64_t types,
+                               const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps,
+                               int hidden, uint16_t* out_dev, uint16_t* out_t_dev, void* stream);
+
 /* out_t[64 * head + f][token] = the attention of every sequence and head of a batch, softmax(scale * Q K^T) V over the sequence's own
  * tokens, no mask: q, k and v hold batch * seq rows `pitch` entries apart, head h at column 64 h (slices of one merged
  * projection, for instance); fp16 in and out, fp32 scores, sums and output, probabilities rounded to fp16.  The result is

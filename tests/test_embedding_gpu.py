@@ -1,0 +1,63 @@
+"""The embedding kernel (three table rows, two additions, LayerNorm; layernorm.hip) against the stock module's own operations, and the
+norm that pads its feature-major copy for any token count."""
+import ctypes
+
+import pytest
+import torch
+
+from venom_amd import _lib, bert
+
+pytestmark = pytest.mark.gpu
+
+
+def close(got, want):
+    """Statistics in another order: neighbouring fp16 values at most, nearly all equal (as for add_layernorm)."""
+    diff = (got.float() - want.float()).abs()
+    return (got == want).float().mean().item() >= 0.99 and bool((diff <= torch.maximum(want.float().abs() * 2.0 ** -10, torch.tensor(1e-3).to(diff))).all())
+
+
+@pytest.mark.parametrize("batch,seq", [(1, 1), (2, 5), (3, 31), (1, 33), (2, 324), (5, 77), (4, 512)])
+@pytest.mark.parametrize("types", [None, "given"])
+def test_fused_embedding_equals_the_stock_module(gpu, batch, seq, types):
+    torch.set_grad_enabled(False)
+    stock = bert.build_bert_large(layers=1).to(gpu).half()
+    fused = bert.fuse_add_layernorm(bert.merge_qkv(bert.linear_to_spmm(bert.build_bert_large(layers=1).to(gpu).half(), 2, 8, 64)), feature_major=True)
+    emb = fused.embeddings
+    assert type(emb) is bert.FusedEmbeddings and list(emb.state_dict()) == list(stock.embeddings.state_dict())
+    ids = torch.randint(0, 30522, (batch, seq), device=gpu)
+    tt = None if types is None else torch.randint(0, 2, (batch, seq), device=gpu)
+    want = stock.embeddings(input_ids=ids, token_type_ids=tt)
+    got = emb(input_ids=ids, token_type_ids=tt)
+    assert got.shape == want.shape and got.is_contiguous() and close(got, want)
+    # the copy that it hands on: padded rows, zeros behind the last token
+    copy, tokens = bert.SrnmSpmm._last_rhs[2], batch * seq
+    assert tuple(copy.shape) == (1024, tokens) and torch.equal(copy.t(), got.reshape(tokens, 1024))
+    padded = torch.as_strided(copy, (1024, copy.stride(0)), copy.stride())
+    assert copy.stride(0) == (tokens + 7) // 8 * 8 and not padded[:, tokens:].any()
+    # calls that the kernel does not take answer as the stock module does
+    position = torch.arange(seq, device=gpu).flip(0)[None]
+    assert torch.equal(emb(input_ids=ids, position_ids=position), stock.embeddings(input_ids=ids, position_ids=position))
+    x = torch.randn((batch, seq, 1024), device=gpu).half()
+    assert torch.equal(emb(inputs_embeds=x), stock.embeddings(inputs_embeds=x))
+    with torch.enable_grad():
+        assert emb(input_ids=ids).requires_grad
+
+
+@pytest.mark.parametrize("tokens,hidden", [(1, 1024), (7, 512), (33, 1024), (75, 768), (1037, 1280), (9, 4096), (130, 72)])
+def test_padded_feature_major_norm(gpu, tokens, hidden):
+    from venom_amd import spatha
+
+    gen = torch.Generator(device=gpu).manual_seed(tokens + hidden)
+    x, r = (torch.randn((tokens, hidden), generator=gen, device=gpu).half() for _ in range(2))
+    w, b = ((0.1 * torch.randn(hidden, generator=gen, device=gpu)).half() for _ in range(2))
+    want = spatha.add_layernorm(x, r, w, b, 1e-12)
+    out, copy = spatha._extension().add_layernorm(x, r, w, b, 1e-12, True)
+    pitch = (tokens + 7) // 8 * 8
+    assert torch.equal(out, want) and torch.equal(copy, want.t()) and copy.stride() == (pitch, 1)
+    guard = torch.full((hidden * pitch + 128,), 7.0, dtype=torch.float16, device=gpu)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    _lib.check(_lib.lib().spatha_add_layernorm_f16_tp(x.data_ptr(), r.data_ptr(), w.data_ptr(), b.data_ptr(), 1e-12, tokens, hidden,
+                                                      out.data_ptr(), guard[64:].data_ptr(), stream), "ln_tp")
+    padded = guard[64:-64].view(hidden, pitch)
+    assert torch.equal(padded[:, :tokens], want.t()) and not padded[:, tokens:].any()
+    assert bool((guard[:64] == 7.0).all()) and bool((guard[-64:] == 7.0).all())

@@ -227,9 +227,50 @@ def _fused_self_attention():
     return FusedSelfAttention
 
 
+def _fused_embeddings():
+    """The class that `fuse_add_layernorm` gives to a BertEmbeddings (`FusedEmbeddings` of this module; made on first use)."""
+    from transformers.models.bert.modeling_bert import BertEmbeddings
+
+    class FusedEmbeddings(BertEmbeddings):
+        """Table lookups, additions and LayerNorm by one kernel (the additions in the stock order, each rounded to fp16), with the
+        feature-major copy for the first projection if asked for.  Token ids in evaluation, without gradients, in fp16 on the GPU; any
+        other call takes the stock forward."""
+
+        feature_major = False
+
+        def forward(self, input_ids=None, token_type_ids=None, position_ids=None, inputs_embeds=None, past_key_values_length=0, **kwargs):
+            got = None
+            if input_ids is not None and position_ids is None and inputs_embeds is None and past_key_values_length == 0 and not kwargs \
+                    and not self.training:
+                got = self._embed(input_ids, token_type_ids)
+            if got is None:
+                return super().forward(input_ids, token_type_ids, position_ids, inputs_embeds, past_key_values_length, **kwargs)
+            if self.feature_major:
+                SrnmSpmm.offer_transposed(*got)
+            return got[0]
+
+        def _embed(self, input_ids, token_type_ids):
+            tables = self.word_embeddings, self.token_type_embeddings, self.position_embeddings
+            ln = self.LayerNorm
+            types = token_type_ids if token_type_ids is not None else getattr(self, "token_type_ids", None)
+            if types is None or type(input_ids) is not torch.Tensor or ln.weight is None or ln.bias is None \
+                    or getattr(self, "position_embedding_type", "absolute") != "absolute" \
+                    or any(type(t) is not torch.nn.Embedding or t.max_norm is not None or t._forward_hooks or t._forward_pre_hooks for t in tables) \
+                    or torch.is_grad_enabled() and any(t.weight.requires_grad for t in tables + (ln,)):
+                return None
+            return spatha._extension().embed_layernorm(input_ids, types, self.position_ids, *(t.weight for t in tables), ln.weight, ln.bias,
+                                                       ln.eps, self.feature_major)
+
+    FusedEmbeddings.__qualname__ = "FusedEmbeddings"
+    globals()["FusedEmbeddings"] = FusedEmbeddings
+    return FusedEmbeddings
+
+
 def __getattr__(name):
     if name == "FusedSelfAttention":
         return _fused_self_attention()
+    if name == "FusedEmbeddings":
+        return _fused_embeddings()
     raise AttributeError("module %r has no attribute %r" % (__name__, name))
 
 
@@ -307,6 +348,13 @@ class FusedProjectionNorm(torch.nn.Module):
         if self.training or not h.is_cuda or h.dtype != torch.float16 or h.shape[-1] % 8 or h.shape[-1] > 4096 \
                 or ln.weight is None or ln.bias is None:
             return ln(self.dropout(h) + input_tensor)
+        native = spatha._native("add_layernorm")
+        if native is not None:
+            got = native(h, input_tensor, ln.weight, ln.bias, ln.eps, self.feature_major)
+            if got is not None:
+                if self.feature_major:
+                    SrnmSpmm.offer_transposed(*got)
+                return got[0]
         h = h.contiguous()
         if self.feature_major and (h.numel() // h.shape[-1]) % 8 == 0:
             out, out_t = spatha.add_layernorm(h, input_tensor.contiguous(), ln.weight, ln.bias, ln.eps, feature_major=True)
@@ -316,13 +364,19 @@ class FusedProjectionNorm(torch.nn.Module):
 
 
 def fuse_add_layernorm(model, feature_major=False):
-    """Replaces, in place, every BertSelfOutput / BertOutput by FusedProjectionNorm (same parameters).  feature_major: for a
-    model whose projections are SrnmSpmm layers - the kernel also writes the feature-major copy the next projection reads, and where
+    """Replaces, in place, every BertSelfOutput / BertOutput by FusedProjectionNorm (same parameters), and has every BertEmbeddings run
+    as one kernel.  feature_major: for a
+    model whose projections are SrnmSpmm layers - the kernels also write the feature-major copy the next projection reads, and where
     `merge_qkv` has merged an attention's projections, that attention runs in the library's kernel, whose result the output
     projection reads as it lies."""
-    from transformers.models.bert.modeling_bert import BertOutput, BertSelfAttention, BertSelfOutput
+    from transformers.models.bert.modeling_bert import BertEmbeddings, BertOutput, BertSelfAttention, BertSelfOutput
 
+    # (the embedding's copy has one reader, the merged projection of the first layer)
+    merged = feature_major and any(isinstance(mod, SrnmSpmm) and mod._group is not None for mod in model.modules())
     for mod in model.modules():
+        if type(mod) is BertEmbeddings:
+            mod.__class__ = globals().get("FusedEmbeddings") or _fused_embeddings()
+            mod.feature_major = merged
         if feature_major and type(mod) is BertSelfAttention and isinstance(mod.query, SrnmSpmm) and mod.query._group is not None:
             mod.__class__ = globals().get("FusedSelfAttention") or _fused_self_attention()
         for name, child in list(mod.named_children()):

@@ -5,6 +5,8 @@
 // Numerics follow the two kernels they replace: the sum is rounded to fp16 first (packed fp16 addition = one rounding of
 // the exact sum), then mean, biased variance, 1/sqrt(var + eps) and the affine map are evaluated in fp32 and the result
 // is rounded to fp16 once.
+// The embedding of an encoder (the stock BertEmbeddings: three table rows a token, two additions, LayerNorm) is the same kernel with
+// three gathered rows in place of x and the residual; its six launches took 87 us for 16384 x 1024 (lookups 27, additions 31, norm 29).
 // One wave per token: a lane holds the token's 8-value chunks lane, lane + 64, ... in registers (two passes over
 // registers for mean and variance, no re-read), wave-wide sums through DPP-style lane exchanges.
 #include <hip/hip_runtime.h>
@@ -26,38 +28,69 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-template <int NJ>
-__global__ __launch_bounds__(256) void add_layernorm_f16_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
-                                                                const uint16_t* __restrict__ gamma,
-                                                                const uint16_t* __restrict__ beta, float eps, int tokens,
-                                                                int hidden, uint16_t* __restrict__ out) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t token = (int64_t)blockIdx.x * 4 + wave;
-    if (token >= tokens) return;
-    const int chunks = hidden >> 3;
-    const uint16_t* xr = x + token * hidden;
-    const uint16_t* rr = residual ? residual + token * hidden : nullptr;
+// What is normalised: x + residual (may be null), row by row, or (EMB) the table rows (x[ids] + residual[types]) + third[positions], each sum
+// rounded to fp16.
+struct LnArgs {
+    const uint16_t *x, *residual, *gamma, *beta;
+    float eps;
+    int tokens, hidden;
+    uint16_t *out, *out_t;
+    int out_t_pitch;             // tokens, or the next multiple of 8: the columns behind the last token are zeroed
+    const uint16_t* third;
+    const int64_t *ids, *types, *positions;      // per token; per token or (types_stride 0) per position; per position
+    int64_t types_stride;
+    int seq;
+    int64_t n_x, n_residual, n_third;            // table rows
+};
+
+// an index outside its table ends the kernel, as it does in the lookups that this replaces
+__device__ __forceinline__ int64_t table_row(int64_t index, int64_t rows) {
+    if ((uint64_t)index >= (uint64_t)rows) __builtin_trap();
+    return index;
+}
+
+template <bool EMB>
+struct LnRows {
+    const uint16_t *x, *residual, *third;
+    __device__ __forceinline__ LnRows(const LnArgs& a, int64_t token) {
+        if constexpr (EMB) {
+            const int64_t b = token / a.seq, s = token - b * a.seq;
+            x = a.x + table_row(a.ids[token], a.n_x) * a.hidden;
+            residual = a.residual + table_row(a.types[b * a.types_stride + s], a.n_residual) * a.hidden;
+            third = a.third + table_row(a.positions[s], a.n_third) * a.hidden;
+        } else {
+            x = a.x + token * a.hidden;
+            residual = a.residual ? a.residual + token * a.hidden : nullptr;
+            third = nullptr;
+        }
+    }
+};
+
+__device__ __forceinline__ ln_u32x4 add_halves(ln_u32x4 a, ln_u32x4 b) {
+    // (vector elements go through scalars: a bit cast applied to an indexed vector element reads element 0)
+    const uint32_t p[4] = {a.x, a.y, a.z, a.w}, q[4] = {b.x, b.y, b.z, b.w};
+    uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const ln_half2 t = as_half2(p[k]) + as_half2(q[k]);
+        r[k] = as_u32(t);
+    }
+    return (ln_u32x4){r[0], r[1], r[2], r[3]};
+}
+
+// One token of `hidden` features, 8-feature pieces lane, lane + 64, ... of which are in `in`: its normalised pieces through `put`(piece, words)
+template <int NJ, class Put>
+__device__ __forceinline__ void normalise(const ln_u32x4 (&in)[NJ], const LnArgs& a, int lane, Put&& put) {
+    const int chunks = a.hidden >> 3;
     float s[NJ][8];
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const int c = lane + 64 * j;
-        if (c < chunks) {
-            // (vector elements go through scalars: a bit cast applied to an indexed vector element reads element 0)
-            const ln_u32x4 av = *(const ln_u32x4*)(xr + c * 8);
-            uint32_t a[4] = {av.x, av.y, av.z, av.w};
-            if (rr) {
-                const ln_u32x4 bv = *(const ln_u32x4*)(rr + c * 8);
-                const uint32_t b[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const ln_half2 t = as_half2(a[k]) + as_half2(b[k]);
-                    a[k] = as_u32(t);
-                }
-            }
+        if (lane + 64 * j < chunks) {
+            const uint32_t w[4] = {in[j].x, in[j].y, in[j].z, in[j].w};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const ln_half2 t = as_half2(a[k]);
+                const ln_half2 t = as_half2(w[k]);
                 s[j][2 * k] = (float)t[0];
                 s[j][2 * k + 1] = (float)t[1];
                 sum += s[j][2 * k] + s[j][2 * k + 1];
@@ -67,7 +100,7 @@ __global__ __launch_bounds__(256) void add_layernorm_f16_kernel(const uint16_t* 
             for (int k = 0; k < 8; k++) s[j][k] = 0.f;
         }
     }
-    const float mean = wave_sum(sum) / (float)hidden;
+    const float mean = wave_sum(sum) / (float)a.hidden;
     float sq = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
@@ -79,13 +112,13 @@ __global__ __launch_bounds__(256) void add_layernorm_f16_kernel(const uint16_t* 
             }
         }
     }
-    const float rstd = rsqrtf(wave_sum(sq) / (float)hidden + eps);
+    const float rstd = rsqrtf(wave_sum(sq) / (float)a.hidden + a.eps);
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int c = lane + 64 * j;
         if (c < chunks) {
-            const ln_u32x4 gv = *(const ln_u32x4*)(gamma + c * 8);
-            const ln_u32x4 bv = *(const ln_u32x4*)(beta + c * 8);
+            const ln_u32x4 gv = *(const ln_u32x4*)(a.gamma + c * 8);
+            const ln_u32x4 bv = *(const ln_u32x4*)(a.beta + c * 8);
             const uint32_t g[4] = {gv.x, gv.y, gv.z, gv.w}, b[4] = {bv.x, bv.y, bv.z, bv.w};
             uint32_t ow[4];
 #pragma unroll
@@ -96,10 +129,29 @@ __global__ __launch_bounds__(256) void add_layernorm_f16_kernel(const uint16_t* 
                 y[1] = (_Float16)((s[j][2 * k + 1] - mean) * rstd * (float)g2[1] + (float)b2[1]);
                 ow[k] = as_u32(y);
             }
-            const ln_u32x4 o = {ow[0], ow[1], ow[2], ow[3]};
-            *(ln_u32x4*)(out + token * hidden + c * 8) = o;
+            put(c, (ln_u32x4){ow[0], ow[1], ow[2], ow[3]});
         }
     }
+}
+
+template <int NJ, bool EMB>
+__global__ __launch_bounds__(256) void add_layernorm_f16_kernel(LnArgs a) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t token = (int64_t)blockIdx.x * 4 + wave;
+    if (token >= a.tokens) return;
+    const int chunks = a.hidden >> 3;
+    const LnRows<EMB> rows(a, token);
+    ln_u32x4 in[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int c = lane + 64 * j;
+        if (c < chunks) {
+            in[j] = *(const ln_u32x4*)(rows.x + c * 8);
+            if (EMB || rows.residual) in[j] = add_halves(in[j], *(const ln_u32x4*)(rows.residual + c * 8));
+            if (EMB) in[j] = add_halves(in[j], *(const ln_u32x4*)(rows.third + c * 8));
+        }
+    }
+    normalise<NJ>(in, a, lane, [&](int c, ln_u32x4 o) { *(ln_u32x4*)(a.out + token * a.hidden + c * 8) = o; });
 }
 
 // The same normalisation, written twice: row-major as above and FEATURE-MAJOR, out_t[hidden][tokens] - the layout the next
@@ -108,159 +160,124 @@ __global__ __launch_bounds__(256) void add_layernorm_f16_kernel(const uint16_t* 
 // leaves the fp16 results in an LDS tile [TOK][hidden + 4] (8-byte writes; the pitch of 2 (mod 64) words keeps the column
 // reads below free of bank conflicts) and then writes the tile out by columns: a lane gathers the 8 tokens of one feature
 // and stores them as 16 bytes, four (TOK = 32) lanes side by side covering 64 contiguous bytes of a feature's row.
-template <int NJ, int TOK>
-__global__ __launch_bounds__(512) void add_layernorm_f16_t_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
-                                                                  const uint16_t* __restrict__ gamma, const uint16_t* __restrict__ beta,
-                                                                  float eps, int tokens, int hidden, uint16_t* __restrict__ out,
-                                                                  uint16_t* __restrict__ out_t) {
+template <int NJ, int TOK, bool EMB>
+__global__ __launch_bounds__(512) void add_layernorm_f16_t_kernel(LnArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t ln_tile[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int chunks = hidden >> 3;
-    const int pitch = hidden + 4;                    // halfs
+    const int chunks = a.hidden >> 3;
+    const int pitch = a.hidden + 4;                    // halfs
     const int64_t tok0 = (int64_t)blockIdx.x * TOK;
     constexpr int PER_WAVE = TOK / 8;
     // all of the wave's tokens are fetched before the first one is reduced: 2 * PER_WAVE * NJ loads of 16 bytes in flight per lane
-    ln_u32x4 xa[PER_WAVE][NJ], xb[PER_WAVE][NJ];
+    ln_u32x4 xa[PER_WAVE][NJ], xb[PER_WAVE][NJ], xc[EMB ? PER_WAVE : 1][NJ];
 #pragma unroll
     for (int t = 0; t < PER_WAVE; t++) {
         const int64_t token = tok0 + wave * PER_WAVE + t;
-        const bool live = token < tokens;
+        const bool live = token < a.tokens;
+        const LnRows<EMB> rows(a, live ? token : 0);
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             const int c = lane + 64 * j;
             const ln_u32x4 zero = {0u, 0u, 0u, 0u};
-            xa[t][j] = (live && c < chunks) ? *(const ln_u32x4*)(x + token * hidden + c * 8) : zero;
-            xb[t][j] = (live && c < chunks && residual) ? *(const ln_u32x4*)(residual + token * hidden + c * 8) : zero;
+            xa[t][j] = (live && c < chunks) ? *(const ln_u32x4*)(rows.x + c * 8) : zero;
+            xb[t][j] = (live && c < chunks && (EMB || a.residual)) ? *(const ln_u32x4*)(rows.residual + c * 8) : zero;
+            if (EMB) xc[EMB ? t : 0][j] = (live && c < chunks) ? *(const ln_u32x4*)(rows.third + c * 8) : zero;
         }
     }
 #pragma unroll
     for (int t = 0; t < PER_WAVE; t++) {
         const int local = wave * PER_WAVE + t;
         const int64_t token = tok0 + local;
-        if (token >= tokens) break;
-        float s[NJ][8];
-        float sum = 0.f;
+        if (token >= a.tokens) break;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const int c = lane + 64 * j;
-            if (c < chunks) {
-                uint32_t a[4] = {xa[t][j].x, xa[t][j].y, xa[t][j].z, xa[t][j].w};
-                if (residual) {
-                    // (x + 0 would not be the identity for -0: the addition runs only with a residual)
-                    const uint32_t b[4] = {xb[t][j].x, xb[t][j].y, xb[t][j].z, xb[t][j].w};
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const ln_half2 tt = as_half2(a[k]) + as_half2(b[k]);
-                        a[k] = as_u32(tt);
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const ln_half2 tt = as_half2(a[k]);
-                    s[j][2 * k] = (float)tt[0];
-                    s[j][2 * k + 1] = (float)tt[1];
-                    sum += s[j][2 * k] + s[j][2 * k + 1];
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < 8; k++) s[j][k] = 0.f;
-            }
+            // (x + 0 would not be the identity for -0: the addition runs only with a residual)
+            if (EMB || a.residual) xa[t][j] = add_halves(xa[t][j], xb[t][j]);
+            if (EMB) xa[t][j] = add_halves(xa[t][j], xc[EMB ? t : 0][j]);
         }
-        const float mean = wave_sum(sum) / (float)hidden;
-        float sq = 0.f;
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            if (lane + 64 * j < chunks) {
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    const float d = s[j][k] - mean;
-                    sq += d * d;
-                }
-            }
-        }
-        const float rstd = rsqrtf(wave_sum(sq) / (float)hidden + eps);
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const int c = lane + 64 * j;
-            if (c < chunks) {
-                const ln_u32x4 gv = *(const ln_u32x4*)(gamma + c * 8);
-                const ln_u32x4 bv = *(const ln_u32x4*)(beta + c * 8);
-                const uint32_t g[4] = {gv.x, gv.y, gv.z, gv.w}, b[4] = {bv.x, bv.y, bv.z, bv.w};
-                uint32_t ow[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const ln_half2 g2 = as_half2(g[k]), b2 = as_half2(b[k]);
-                    ln_half2 y;
-                    y[0] = (_Float16)((s[j][2 * k] - mean) * rstd * (float)g2[0] + (float)b2[0]);
-                    y[1] = (_Float16)((s[j][2 * k + 1] - mean) * rstd * (float)g2[1] + (float)b2[1]);
-                    ow[k] = as_u32(y);
-                }
-                const ln_u32x4 o = {ow[0], ow[1], ow[2], ow[3]};
-                *(ln_u32x4*)(out + token * hidden + c * 8) = o;
-                uint32_t* dst = (uint32_t*)(ln_tile + local * pitch + c * 8);      // 8-byte aligned: pitch % 4 == 0
-                *(uint2*)dst = make_uint2(ow[0], ow[1]);
-                *(uint2*)(dst + 2) = make_uint2(ow[2], ow[3]);
-            }
-        }
+        normalise<NJ>(xa[t], a, lane, [&](int c, ln_u32x4 o) {
+            *(ln_u32x4*)(a.out + token * a.hidden + c * 8) = o;
+            uint32_t* dst = (uint32_t*)(ln_tile + local * pitch + c * 8);      // 8-byte aligned: pitch % 4 == 0
+            *(uint2*)dst = make_uint2(o.x, o.y);
+            *(uint2*)(dst + 2) = make_uint2(o.z, o.w);
+        });
     }
     __syncthreads();
     // by columns: item = (feature f, piece p of 8 tokens)
     constexpr int PIECES = TOK / 8;
-    const int items = hidden * PIECES;
+    const int items = a.hidden * PIECES;
     for (int idx = threadIdx.x; idx < items; idx += 512) {
         const int p = idx % PIECES, f = idx / PIECES;
         const int64_t token = tok0 + p * 8;
-        if (token >= tokens) continue;                  // (tokens % 8 == 0: a piece is all there or not at all)
+        if (token >= a.tokens) continue;
         uint32_t w[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const uint32_t lo = ln_tile[(p * 8 + 2 * k) * pitch + f], hi = ln_tile[(p * 8 + 2 * k + 1) * pitch + f];
+            uint32_t lo = ln_tile[(p * 8 + 2 * k) * pitch + f], hi = ln_tile[(p * 8 + 2 * k + 1) * pitch + f];
+            if (token + 2 * k >= a.tokens) lo = 0u;              // (rows behind the last token hold nothing)
+            if (token + 2 * k + 1 >= a.tokens) hi = 0u;
             w[k] = lo | (hi << 16);
         }
         const ln_u32x4 o = {w[0], w[1], w[2], w[3]};
-        *(ln_u32x4*)(out_t + (int64_t)f * tokens + token) = o;
+        *(ln_u32x4*)(a.out_t + (int64_t)f * a.out_t_pitch + token) = o;
     }
 }
 
-template <int NJ, int TOK>
-static hipError_t launch_ln_t(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta, float eps,
-                              int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream) {
-    const int lds = TOK * (hidden + 4) * 2;
-    auto kern = add_layernorm_f16_t_kernel<NJ, TOK>;
+template <int NJ, int TOK, bool EMB>
+static hipError_t launch_ln_t(const LnArgs& a, hipStream_t stream) {
+    const int lds = TOK * (a.hidden + 4) * 2;
+    auto kern = add_layernorm_f16_t_kernel<NJ, TOK, EMB>;
     if (lds > 48 * 1024) {
         static bool raised[16] = {};
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return e;
         if (!raised[dev & 15]) {
-            e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TOK * (NJ * 512 + 4) * 2);
             if (e != hipSuccess) return e;
             raised[dev & 15] = true;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((tokens + TOK - 1) / TOK), dim3(512), lds, stream, x, residual, gamma, beta, eps, tokens, hidden, out,
-                       out_t);
+    hipLaunchKernelGGL(kern, dim3((a.tokens + TOK - 1) / TOK), dim3(512), lds, stream, a);
     return hipGetLastError();
 }
 
 // hidden <= 1024: 32 tokens per workgroup (66 KB of LDS); <= 2048: 16; <= 4096: 8
-hipError_t launch_add_layernorm_f16_t(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
-                                      float eps, int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream) {
-    if (hidden <= 512) return launch_ln_t<1, 32>(x, residual, gamma, beta, eps, tokens, hidden, out, out_t, stream);
-    if (hidden <= 1024) return launch_ln_t<2, 32>(x, residual, gamma, beta, eps, tokens, hidden, out, out_t, stream);
-    if (hidden <= 2048) return launch_ln_t<4, 16>(x, residual, gamma, beta, eps, tokens, hidden, out, out_t, stream);
-    return launch_ln_t<8, 8>(x, residual, gamma, beta, eps, tokens, hidden, out, out_t, stream);
+template <bool EMB>
+static hipError_t launch_norm(const LnArgs& a, hipStream_t stream) {
+    const int nj = (a.hidden / 8 + 63) / 64;
+    if (a.out_t) {
+        if (nj <= 1) return launch_ln_t<1, 32, EMB>(a, stream);
+        if (nj <= 2) return launch_ln_t<2, 32, EMB>(a, stream);
+        if (nj <= 4) return launch_ln_t<4, 16, EMB>(a, stream);
+        return launch_ln_t<8, 8, EMB>(a, stream);
+    }
+    const dim3 grid((a.tokens + 3) / 4), block(256);
+    if (nj <= 1) hipLaunchKernelGGL((add_layernorm_f16_kernel<1, EMB>), grid, block, 0, stream, a);
+    else if (nj <= 2) hipLaunchKernelGGL((add_layernorm_f16_kernel<2, EMB>), grid, block, 0, stream, a);
+    else if (nj <= 4) hipLaunchKernelGGL((add_layernorm_f16_kernel<4, EMB>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((add_layernorm_f16_kernel<8, EMB>), grid, block, 0, stream, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_add_layernorm_f16(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
-                                    float eps, int tokens, int hidden, uint16_t* out, hipStream_t stream) {
-    const dim3 grid((tokens + 3) / 4), block(256);
-    const int nj = (hidden / 8 + 63) / 64;
-    if (nj <= 1) hipLaunchKernelGGL(add_layernorm_f16_kernel<1>, grid, block, 0, stream, x, residual, gamma, beta, eps, tokens, hidden, out);
-    else if (nj <= 2) hipLaunchKernelGGL(add_layernorm_f16_kernel<2>, grid, block, 0, stream, x, residual, gamma, beta, eps, tokens, hidden, out);
-    else if (nj <= 4) hipLaunchKernelGGL(add_layernorm_f16_kernel<4>, grid, block, 0, stream, x, residual, gamma, beta, eps, tokens, hidden, out);
-    else hipLaunchKernelGGL(add_layernorm_f16_kernel<8>, grid, block, 0, stream, x, residual, gamma, beta, eps, tokens, hidden, out);
-    return hipGetLastError();
+                                    float eps, int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream) {
+    LnArgs a = {};
+    a.x = x; a.residual = residual; a.gamma = gamma; a.beta = beta; a.eps = eps; a.tokens = tokens; a.hidden = hidden;
+    a.out = out; a.out_t = out_t; a.out_t_pitch = (tokens + 7) / 8 * 8;
+    return launch_norm<false>(a, stream);
+}
+
+hipError_t launch_embed_layernorm_f16(const EmbeddingTables& t, const int64_t* ids, const int64_t* types, int64_t types_stride,
+                                      const int64_t* positions, int batch, int seq, const uint16_t* gamma, const uint16_t* beta, float eps,
+                                      uint16_t* out, uint16_t* out_t, hipStream_t stream) {
+    LnArgs a = {};
+    a.x = t.word; a.residual = t.type; a.third = t.position;
+    a.n_x = t.words; a.n_residual = t.types; a.n_third = t.positions;
+    a.ids = ids; a.types = types; a.types_stride = types_stride; a.positions = positions; a.seq = seq;
+    a.gamma = gamma; a.beta = beta; a.eps = eps; a.tokens = batch * seq; a.hidden = t.hidden;
+    a.out = out; a.out_t = out_t; a.out_t_pitch = (a.tokens + 7) / 8 * 8;
+    return launch_norm<true>(a, stream);
 }
 
 }  // namespace spatha

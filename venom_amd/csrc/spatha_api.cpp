@@ -968,14 +968,21 @@ int spatha_pad_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t*
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 
+namespace {
+int norm_status(uintptr_t pointers, const void* gamma_dev, const void* beta_dev, int tokens, int hidden) {
+    if (!gamma_dev || !beta_dev || tokens <= 0 || hidden <= 0) return SPATHA_ERR_BAD_ARGUMENT;
+    if (hidden % 8 != 0) return SPATHA_ERR_BAD_SHAPE;           // 16-byte pieces
+    if (hidden > 4096) return SPATHA_ERR_UNSUPPORTED;           // a lane keeps hidden / 64 values in registers
+    return ((pointers | (uintptr_t)gamma_dev | (uintptr_t)beta_dev) & 15u) ? SPATHA_ERR_BAD_ARGUMENT : SPATHA_OK;
+}
+}  // namespace
+
 int spatha_add_layernorm_f16(const uint16_t* x_dev, const uint16_t* residual_dev, const uint16_t* gamma_dev,
                              const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, void* stream) {
-    if (!x_dev || !gamma_dev || !beta_dev || !out_dev || tokens <= 0 || hidden <= 0) return SPATHA_ERR_BAD_ARGUMENT;
-    if (hidden % 8 != 0) return SPATHA_ERR_BAD_SHAPE;
-    if (hidden > 4096) return SPATHA_ERR_UNSUPPORTED;           // a lane keeps hidden / 64 values in registers
-    if (((uintptr_t)x_dev | (uintptr_t)residual_dev | (uintptr_t)gamma_dev | (uintptr_t)beta_dev | (uintptr_t)out_dev) & 15u)
-        return SPATHA_ERR_BAD_ARGUMENT;
-    hipError_t e = spatha::launch_add_layernorm_f16(x_dev, residual_dev, gamma_dev, beta_dev, eps, tokens, hidden, out_dev,
+    if (!x_dev || !out_dev) return SPATHA_ERR_BAD_ARGUMENT;
+    const int st = norm_status((uintptr_t)x_dev | (uintptr_t)residual_dev | (uintptr_t)out_dev, gamma_dev, beta_dev, tokens, hidden);
+    if (st) return st;
+    hipError_t e = spatha::launch_add_layernorm_f16(x_dev, residual_dev, gamma_dev, beta_dev, eps, tokens, hidden, out_dev, nullptr,
                                                     (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
@@ -983,14 +990,39 @@ int spatha_add_layernorm_f16(const uint16_t* x_dev, const uint16_t* residual_dev
 int spatha_add_layernorm_f16_t(const uint16_t* x_dev, const uint16_t* residual_dev, const uint16_t* gamma_dev,
                                const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
                                void* stream) {
-    if (!x_dev || !gamma_dev || !beta_dev || !out_dev || !out_t_dev || tokens <= 0 || hidden <= 0) return SPATHA_ERR_BAD_ARGUMENT;
-    if (hidden % 8 != 0 || tokens % 8 != 0) return SPATHA_ERR_BAD_SHAPE;       // 16-byte pieces of both layouts
-    if (hidden > 4096) return SPATHA_ERR_UNSUPPORTED;
-    if (((uintptr_t)x_dev | (uintptr_t)residual_dev | (uintptr_t)gamma_dev | (uintptr_t)beta_dev | (uintptr_t)out_dev |
-         (uintptr_t)out_t_dev) & 15u)
+    if (tokens > 0 && tokens % 8 != 0) return SPATHA_ERR_BAD_SHAPE;       // (spatha_add_layernorm_f16_tp pads)
+    return spatha_add_layernorm_f16_tp(x_dev, residual_dev, gamma_dev, beta_dev, eps, tokens, hidden, out_dev, out_t_dev, stream);
+}
+
+int spatha_add_layernorm_f16_tp(const uint16_t* x_dev, const uint16_t* residual_dev, const uint16_t* gamma_dev,
+                                const uint16_t* beta_dev, float eps, int tokens, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
+                                void* stream) {
+    if (!x_dev || !out_dev || !out_t_dev || tokens > INT32_MAX - 64) return SPATHA_ERR_BAD_ARGUMENT;
+    const int st = norm_status((uintptr_t)x_dev | (uintptr_t)residual_dev | (uintptr_t)out_dev | (uintptr_t)out_t_dev, gamma_dev, beta_dev,
+                               tokens, hidden);
+    if (st) return st;
+    hipError_t e = spatha::launch_add_layernorm_f16(x_dev, residual_dev, gamma_dev, beta_dev, eps, tokens, hidden, out_dev, out_t_dev,
+                                                    (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev, int64_t types_stride, const int64_t* positions_dev, int batch,
+                               int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev, int64_t types,
+                               const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps,
+                               int hidden, uint16_t* out_dev, uint16_t* out_t_dev, void* stream) {
+    if (!ids_dev || !types_dev || !positions_dev || !word_dev || !type_dev || !position_dev || !out_dev || batch <= 0 || seq <= 0 ||
+        words <= 0 || types <= 0 || positions <= 0 || (types_stride != 0 && types_stride < seq))
         return SPATHA_ERR_BAD_ARGUMENT;
-    hipError_t e = spatha::launch_add_layernorm_f16_t(x_dev, residual_dev, gamma_dev, beta_dev, eps, tokens, hidden, out_dev, out_t_dev,
-                                                      (hipStream_t)stream);
+    if ((int64_t)batch * seq > INT32_MAX - 64) return SPATHA_ERR_TOO_LARGE;
+    if (((uintptr_t)ids_dev | (uintptr_t)types_dev | (uintptr_t)positions_dev) & 7u) return SPATHA_ERR_BAD_ARGUMENT;
+    const int st = norm_status((uintptr_t)word_dev | (uintptr_t)type_dev | (uintptr_t)position_dev | (uintptr_t)out_dev | (uintptr_t)out_t_dev,
+                               gamma_dev, beta_dev, batch * seq, hidden);
+    if (st) return st;
+    spatha::EmbeddingTables tables;
+    tables.word = word_dev; tables.type = type_dev; tables.position = position_dev;
+    tables.words = words; tables.types = types; tables.positions = positions; tables.hidden = hidden;
+    hipError_t e = spatha::launch_embed_layernorm_f16(tables, ids_dev, types_dev, types_stride, positions_dev, batch, seq, gamma_dev, beta_dev,
+                                                      eps, out_dev, out_t_dev, (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 

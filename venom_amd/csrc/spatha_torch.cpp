@@ -375,6 +375,82 @@ py::object attention(py::handle input, int64_t batch, int64_t seq, int64_t heads
     return py::reinterpret_steal<py::object>(THPVariable_Wrap(out.narrow(1, 0, tokens).t().view({batch, seq, hidden})));
 }
 
+bool row_ok(const torch::Tensor& t, int device, int64_t numel) {
+    return weight_ok(t, torch::kFloat16, device) && t.numel() == numel && ((uintptr_t)t.data_ptr() & 15) == 0;
+}
+
+// x's outputs of a norm: [..., hidden] and, with feature_major, its copy [hidden, tokens] in rows padded to a multiple of 8 (else undefined)
+struct NormOut {
+    torch::Tensor out, padded;
+    int64_t tokens;
+    py::object tuple() const {
+        const py::object second = padded.defined() ? py::reinterpret_steal<py::object>(THPVariable_Wrap(padded.narrow(1, 0, tokens))) : py::none();
+        return py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(out)), second);
+    }
+};
+
+// LayerNorm(x + residual) of fp16 operands in order: (result, feature-major copy or None), or None for what the general path decides
+py::object add_layernorm(py::handle input, py::handle addend, const torch::Tensor& weight, const torch::Tensor& bias, double eps,
+                         bool feature_major) {
+    if (!THPVariable_CheckExact(input.ptr()) || !THPVariable_CheckExact(addend.ptr())) return py::none();
+    const torch::Tensor &x = THPVariable_Unpack(input.ptr()), &r = THPVariable_Unpack(addend.ptr());
+    if (!x.is_cuda() || x.layout() != torch::kStrided || x.dim() < 1 || x.numel() == 0) return py::none();
+    const int device = (int)x.get_device();
+    const int64_t hidden = x.size(-1), tokens = x.numel() / hidden;
+    if (!row_ok(x, device, x.numel()) || !row_ok(r, device, x.numel()) || r.sizes() != x.sizes() || !row_ok(weight, device, hidden) ||
+        !row_ok(bias, device, hidden) || hidden % 8 != 0 || hidden > 4096 || tokens > INT32_MAX - 64)
+        return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(x.device());
+    NormOut o;
+    o.tokens = tokens;
+    o.out = torch::empty(x.sizes(), x.options().requires_grad(false));
+    if (feature_major) o.padded = torch::empty({hidden, (tokens + 7) / 8 * 8}, x.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+    const uint16_t *xp = (const uint16_t*)x.data_ptr(), *rp = (const uint16_t*)r.data_ptr(), *g = (const uint16_t*)weight.data_ptr(),
+                   *b = (const uint16_t*)bias.data_ptr();
+    if (feature_major)
+        check(spatha_add_layernorm_f16_tp(xp, rp, g, b, (float)eps, (int)tokens, (int)hidden, (uint16_t*)o.out.data_ptr(),
+                                          (uint16_t*)o.padded.data_ptr(), stream),
+              "spatha_add_layernorm_f16_tp");
+    else
+        check(spatha_add_layernorm_f16(xp, rp, g, b, (float)eps, (int)tokens, (int)hidden, (uint16_t*)o.out.data_ptr(), stream),
+              "spatha_add_layernorm_f16");
+    return o.tuple();
+}
+
+// The embedding of ids [batch, seq]: word, type and position tables, LayerNorm; types [batch, seq] or [1, >= seq], positions [1, >= seq].  As
+// add_layernorm.
+py::object embed_layernorm(const torch::Tensor& ids, const torch::Tensor& types, const torch::Tensor& positions, const torch::Tensor& word,
+                           const torch::Tensor& type, const torch::Tensor& position, const torch::Tensor& weight, const torch::Tensor& bias,
+                           double eps, bool feature_major) {
+    if (!ids.is_cuda() || ids.layout() != torch::kStrided || ids.dim() != 2 || ids.numel() == 0) return py::none();
+    const int device = (int)ids.get_device();
+    const int64_t batch = ids.size(0), seq = ids.size(1), hidden = word.dim() == 2 ? word.size(1) : 0;
+    const bool types_shared = types.dim() == 2 && types.size(0) == 1 && types.size(1) >= seq;
+    if (!weight_ok(ids, torch::kInt64, device) || !weight_ok(types, torch::kInt64, device) || !weight_ok(positions, torch::kInt64, device) ||
+        !(types_shared || types.sizes() == ids.sizes()) || positions.dim() != 2 || positions.size(0) != 1 || positions.size(1) < seq ||
+        hidden <= 0 || hidden % 8 != 0 || hidden > 4096 || batch * seq > INT32_MAX - 64)
+        return py::none();
+    for (const torch::Tensor* t : {&word, &type, &position})
+        if (t->dim() != 2 || t->size(1) != hidden || t->size(0) <= 0 || !row_ok(*t, device, t->numel())) return py::none();
+    if (!row_ok(weight, device, hidden) || !row_ok(bias, device, hidden)) return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(ids.device());
+    NormOut o;
+    o.tokens = batch * seq;
+    o.out = torch::empty({batch, seq, hidden}, word.options().requires_grad(false));
+    if (feature_major) o.padded = torch::empty({hidden, (o.tokens + 7) / 8 * 8}, word.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+    check(spatha_embed_layernorm_f16((const int64_t*)ids.data_ptr(), (const int64_t*)types.data_ptr(), types_shared ? 0 : seq,
+                                     (const int64_t*)positions.data_ptr(), (int)batch, (int)seq, (const uint16_t*)word.data_ptr(), word.size(0),
+                                     (const uint16_t*)type.data_ptr(), type.size(0), (const uint16_t*)position.data_ptr(), position.size(0),
+                                     (const uint16_t*)weight.data_ptr(), (const uint16_t*)bias.data_ptr(), (float)eps, (int)hidden,
+                                     (uint16_t*)o.out.data_ptr(), feature_major ? (uint16_t*)o.padded.data_ptr() : nullptr, stream),
+          "spatha_embed_layernorm_f16");
+    return o.tuple();
+}
+
 // SpmmPlan.run without a k-split, for operands in order; None where the caller's checks have to speak.  bias needs the transposed
 // layout unless `fused` (an activation, ACT_NONE among them, was named).
 py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle out, int rows, int cols, int device, bool transposed_out,
@@ -478,6 +554,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
             py::arg("transposed_out") = false);
     mod.def("layer_spmm", &layer_spmm, "one V:N:M layer, right-hand side and product, or None");
     mod.def("attention", &attention, "attention of merged projections, feature-major, or None");
+    mod.def("add_layernorm", &add_layernorm, "LayerNorm(x + residual): (result, feature-major copy or None), or None");
+    mod.def("embed_layernorm", &embed_layernorm, "LayerNorm of summed table rows: (result, feature-major copy or None), or None");
     mod.def("stream_key", &stream_key, "(stream, capture) that work issued now on this device goes to", py::arg("device"));
     mod.def("transpose", &transpose_f16, "x.T of an fp16 matrix through the library's kernel, or None");
     mod.def("plan_run", &plan_run, "a plan's product, or None, or the status of a refusal");

@@ -121,11 +121,18 @@ hipError_t launch_pack_gtab(const uint32_t* columns, int rows, int m, int v, int
 
 hipError_t launch_transpose_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
 hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
+// LayerNorm(x + residual), and with out_t once more as [hidden][tokens padded to a multiple of 8]; the embedding of a token sequence
+// ahead of it in place of x and residual (layernorm.hip)
 hipError_t launch_add_layernorm_f16(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
-                                    float eps, int tokens, int hidden, uint16_t* out, hipStream_t stream);
-
-hipError_t launch_add_layernorm_f16_t(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
-                                      float eps, int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream);
+                                    float eps, int tokens, int hidden, uint16_t* out, uint16_t* out_t, hipStream_t stream);
+struct EmbeddingTables {
+    const uint16_t *word, *type, *position;      // [words][hidden], ...
+    int64_t words, types, positions;
+    int hidden;
+};
+hipError_t launch_embed_layernorm_f16(const EmbeddingTables& tables, const int64_t* ids, const int64_t* types, int64_t types_stride,
+                                      const int64_t* positions, int batch, int seq, const uint16_t* gamma, const uint16_t* beta, float eps,
+                                      uint16_t* out, uint16_t* out_t, hipStream_t stream);
 
 // softmax(scale Q K^T) V per sequence and head of 64 features, result feature-major (attention.hip)
 hipError_t launch_attention_f16(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t pitch, int batch, int seq, int heads,
