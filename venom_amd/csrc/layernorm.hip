@@ -160,13 +160,15 @@ __global__ __launch_bounds__(256) void add_layernorm_f16_kernel(LnArgs a) {
 // leaves the fp16 results in an LDS tile [TOK][hidden + 4] (8-byte writes; the pitch of 2 (mod 64) words keeps the column
 // reads below free of bank conflicts) and then writes the tile out by columns: a lane gathers the 8 tokens of one feature
 // and stores them as 16 bytes, four (TOK = 32) lanes side by side covering 64 contiguous bytes of a feature's row.
-template <int NJ, int TOK, bool EMB>
+template <int NJ, int TOK, bool EMB, bool XCD>
 __global__ __launch_bounds__(512) void add_layernorm_f16_t_kernel(LnArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t ln_tile[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int chunks = a.hidden >> 3;
     const int pitch = a.hidden + 4;                    // halfs
-    const int64_t tok0 = (int64_t)blockIdx.x * TOK;
+    // an XCD owns a contiguous range of tokens: adjacent pieces of a feature's row meet in its L2
+    const int64_t tok0 = (XCD ? (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : (int64_t)blockIdx.x) * TOK;
+    if (XCD && tok0 >= a.tokens) return;
     constexpr int PER_WAVE = TOK / 8;
     // all of the wave's tokens are fetched before the first one is reduced: 2 * PER_WAVE * NJ loads of 16 bytes in flight per lane
     ln_u32x4 xa[PER_WAVE][NJ], xb[PER_WAVE][NJ], xc[EMB ? PER_WAVE : 1][NJ];
@@ -223,10 +225,10 @@ __global__ __launch_bounds__(512) void add_layernorm_f16_t_kernel(LnArgs a) {
     }
 }
 
-template <int NJ, int TOK, bool EMB>
+template <int NJ, int TOK, bool EMB, bool XCD = false>
 static hipError_t launch_ln_t(const LnArgs& a, hipStream_t stream) {
     const int lds = TOK * (a.hidden + 4) * 2;
-    auto kern = add_layernorm_f16_t_kernel<NJ, TOK, EMB>;
+    auto kern = add_layernorm_f16_t_kernel<NJ, TOK, EMB, XCD>;
     if (lds > 48 * 1024) {
         static bool raised[16] = {};
         int dev = 0;
@@ -238,17 +240,19 @@ static hipError_t launch_ln_t(const LnArgs& a, hipStream_t stream) {
             raised[dev & 15] = true;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((a.tokens + TOK - 1) / TOK), dim3(512), lds, stream, a);
+    const int blocks = (a.tokens + TOK - 1) / TOK;
+    hipLaunchKernelGGL(kern, dim3(XCD ? (blocks + 7) / 8 * 8 : blocks), dim3(512), lds, stream, a);
     return hipGetLastError();
 }
 
-// hidden <= 1024: 32 tokens per workgroup (66 KB of LDS); <= 2048: 16; <= 4096: 8
+// hidden <= 1024: 32 tokens per workgroup (66 KB of LDS), 16 where 32 would leave half of the CUs without one (4096 x 1024 10.9 -> 8.6 us, up
+// to 1024 tokens 9.3 -> 6.5, of which 6.3 are the call; 8192 tokens level, 16384 23.2 against 25.0); <= 2048: 16; <= 4096: 8
 template <bool EMB>
 static hipError_t launch_norm(const LnArgs& a, hipStream_t stream) {
     const int nj = (a.hidden / 8 + 63) / 64;
     if (a.out_t) {
-        if (nj <= 1) return launch_ln_t<1, 32, EMB>(a, stream);
-        if (nj <= 2) return launch_ln_t<2, 32, EMB>(a, stream);
+        if (nj <= 1) return a.tokens <= 4096 ? launch_ln_t<1, 16, EMB, true>(a, stream) : launch_ln_t<1, 32, EMB>(a, stream);
+        if (nj <= 2) return a.tokens <= 4096 ? launch_ln_t<2, 16, EMB, true>(a, stream) : launch_ln_t<2, 32, EMB>(a, stream);
         if (nj <= 4) return launch_ln_t<4, 16, EMB>(a, stream);
         return launch_ln_t<8, 8, EMB>(a, stream);
     }

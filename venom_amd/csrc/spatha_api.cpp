@@ -459,6 +459,16 @@ bool split_choice(const spatha_spmm_plan* plan, int N, int requested, int chosen
     *out = c;
     return true;
 }
+
+// Does C leave by non-temporal stores, past the 256 MB memory-side cache?  From 48 MB on, unless the caller says that it is read right
+// behind this call.  With three sets of operands and results in turn (28 shapes, both layouts): results of 134 MB and more 1.14-1.7x
+// ahead (4096 x 1024 x 16384 at 64:2:8 75.3 -> 61.3 us row-major, 67 -> 57.7 transposed, at 128:2:32 54.1 -> 31.9; x 32768 at
+// 64:2:8 164.6 -> 119.9), of 50 to 67 MB 0.98-1.04x, of 33 MB level, smaller ones level or up to 4 % behind; where all buffers stay in
+// the cache level.  A chain of layers reads each result back from that cache: with such stores in all of them the two encoder layers of
+// BERT-large at 32 x 512 tokens took 695 us, 681 without.
+bool streams_out(const spatha_spmm_plan* plan, int N, bool read_next) {
+    return !read_next && (int64_t)plan->geo.rows * N * 2 >= (48ll << 20);
+}
 }  // namespace
 
 namespace spatha {
@@ -725,7 +735,7 @@ int spatha::plan_run_check(const spatha_spmm_plan* plan, const uint16_t* B_dev, 
 
 int spatha::plan_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                      int out_layout, int activation, bool fused_entry, int variant, void* stream, void* workspace,
-                     size_t workspace_bytes) {
+                     size_t workspace_bytes, bool read_next) {
     int var = -1;
     const int status = plan_run_check(plan, B_dev, N, bias_dev, out_dev, out_layout, activation, fused_entry, variant, &var);
     if (status != SPATHA_OK) return status;
@@ -743,6 +753,7 @@ int spatha::plan_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N,
     p.rowtab_bytes = (uint32_t)plan->rowtab_bytes;
     p.fuse = fuse ? 1 : 0; p.act = activation;
     p.cus = plan->cus > 0 ? plan->cus : 256;
+    p.stream_out = streams_out(plan, N, read_next) ? 1 : 0;
     p.walk_group = 1;
     if (var == spatha::SPMM_VARIANT_UP512x128_S3) {
         // Packed A larger than an XCD's L2 (plain 2:4 on a 4096-row matrix: 4.7 MB against 4 MB; it is then fetched again in
@@ -820,6 +831,12 @@ int spatha_spmm_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, 
 int spatha_spmm_run_fused(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev,
                           uint16_t* out_dev, int out_layout, int activation, int variant, void* stream) {
     return spatha::plan_run(plan, B_dev, N, bias_dev, out_dev, out_layout, activation, true, variant, stream);
+}
+
+int spatha_spmm_run_layer(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
+                          int out_layout, int activation, void* workspace_dev, size_t workspace_bytes, void* stream) {
+    return spatha::plan_run(plan, B_dev, N, bias_dev, out_dev, out_layout, activation, true, spatha::SPMM_VARIANT_AUTO, stream,
+                            workspace_dev, workspace_bytes, true);
 }
 
 int spatha_spmm_run_tokens(const spatha_spmm_plan* plan, const uint16_t* x_dev, int tokens, const uint16_t* bias_dev, uint16_t* out_dev,

@@ -42,7 +42,7 @@ int plan_run_check(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, c
 // (device memory of at least the size split_workspace_bytes names) the automatic choice may split k-loops over workgroups.
 int plan_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
              int out_layout, int activation, bool fused_entry, int variant, void* stream, void* workspace = nullptr,
-             size_t workspace_bytes = 0);
+             size_t workspace_bytes = 0, bool read_next = false);
 
 // records a HIP error for spatha_last_hip_error and returns SPATHA_ERR_HIP
 int note_hip_error(hipError_t e);

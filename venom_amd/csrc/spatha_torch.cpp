@@ -157,7 +157,7 @@ torch::Tensor pad_columns(const torch::Tensor& x) {
 // the product on a right-hand side [cols, tokens], tokens a multiple of 8, with operands that have been checked
 torch::Tensor run_full(const torch::Tensor& A_metadata, const torch::Tensor& A_indices, const torch::Tensor& A_values,
                        const torch::Tensor& rhs, int tokens, const uint16_t* bias_ptr, int rows, int cols, int v, int n, int m,
-                       bool transposed_out, int activation, bool fused) {
+                       bool transposed_out, int activation, bool fused, bool read_next = false) {
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
     // (this reference outlives the launch calls below, whatever another thread does to the cache meanwhile)
     const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values, A_metadata, A_indices, rows, cols, n, m, v, stream);
@@ -166,8 +166,17 @@ torch::Tensor run_full(const torch::Tensor& A_metadata, const torch::Tensor& A_i
     const int layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
     // few tokens against a long k-loop: the library splits the k-loops over workgroups if it is given scratch memory
     const bool fuses = fused && (activation != SPATHA_ACT_NONE || (!transposed_out && bias_ptr));
-    if (const size_t need = spatha_spmm_workspace_bytes(plan.get(), tokens, layout, fuses ? 1 : 0)) {
-        torch::Tensor ws = workspace_for((int)A_values.get_device(), stream, need, rhs.options());
+    torch::Tensor ws;
+    if (const size_t need = spatha_spmm_workspace_bytes(plan.get(), tokens, layout, fuses ? 1 : 0))
+        ws = workspace_for((int)A_values.get_device(), stream, need, rhs.options());
+    if (read_next) {
+        check(spatha_spmm_run_layer(plan.get(), (const uint16_t*)rhs.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
+                                    fused ? activation : SPATHA_ACT_NONE, ws.defined() ? ws.data_ptr() : nullptr,
+                                    ws.defined() ? (size_t)ws.numel() : 0, stream),
+              "spatha_spmm_run_layer");
+        return out;
+    }
+    if (ws.defined()) {
         check(spatha_spmm_run_ws(plan.get(), (const uint16_t*)rhs.data_ptr(), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
                                  fused ? activation : SPATHA_ACT_NONE, ws.data_ptr(), (size_t)ws.numel(), stream),
               "spatha_spmm_run_ws");
@@ -348,7 +357,7 @@ py::object layer_spmm(py::handle input, py::tuple last, const torch::Tensor& met
     }
     const uint16_t* bias_ptr = bias_t.defined() ? (const uint16_t*)bias_t.data_ptr() : nullptr;
     torch::Tensor out = run_full(metadata, columns, values, rhs, (int)padded, bias_ptr, rows, cols, v, n, m, !feature_major,
-                                 feature_major ? activation : SPATHA_ACT_NONE, feature_major);
+                                 feature_major ? activation : SPATHA_ACT_NONE, feature_major, true);
     if (padded != tokens) out = out.narrow(feature_major ? 1 : 0, 0, tokens);
     return result(feature_major ? out.t() : out, kept);
 }

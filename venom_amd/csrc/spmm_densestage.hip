@@ -226,12 +226,12 @@ __device__ __forceinline__ void ds_consumer(const SpmmParams& p, const TileWalk&
             if (pre) fused_bias_act(acc[0], p.bias, (int64_t)cm0 + ib * 16, p.act);
             if (!SPATHA_KNOB(4)) {
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                    store_block_transposed_slab4(acc[0], stg, p.C, p.fuse ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
+                    store_block_transposed_slab4(acc[0], stg, OutC(p), p.fuse ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
                                                  lane, !SPATHA_KNOB(2));
                 else if (p.fuse && !pre && p.bias)
-                    store_block_row_major_tr4<true>(acc[0], stg, p.C, (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), p.bias);
+                    store_block_row_major_tr4<true>(acc[0], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), p.bias);
                 else
-                    store_block_row_major_tr4<false>(acc[0], stg, p.C, (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
+                    store_block_row_major_tr4<false>(acc[0], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
             }
         } else
 #pragma unroll
@@ -241,16 +241,16 @@ __device__ __forceinline__ void ds_consumer(const SpmmParams& p, const TileWalk&
             if (pre) fused_bias_act(acc[h], p.bias, (int64_t)cm0 + h * 64 + ib * 16, p.act);
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                 if (!SPATHA_KNOB(4))
-                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C, p.fuse ? nullptr : p.bias,
+                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), p.fuse ? nullptr : p.bias,
                                                 (int64_t)cm0 + h * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
             } else if (!SPATHA_KNOB(4)) {
                 // two copies, so that the plain path carries nothing of the bias path
                 if (p.fuse && !pre && p.bias)
-                    store_block_row_major_tr<Cfg::NC == 8, Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C,
+                    store_block_row_major_tr<Cfg::NC == 8, Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p),
                                                                          (int64_t)cm0 + h * 64, cn0 + wn * 64, N, lane,
                                                                          !SPATHA_KNOB(2), p.bias);
                 else
-                    store_block_row_major_tr<Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C,
+                    store_block_row_major_tr<Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p),
                                                            (int64_t)cm0 + h * 64, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
             }
         }
@@ -387,10 +387,10 @@ __device__ __forceinline__ void ds_consumer_half(const SpmmParams& p, const Tile
         const bool pre = p.fuse && (p.act != SPATHA_ACT_NONE || OUT_LAYOUT == SPATHA_OUT_TRANSPOSED);
         if (pre) fused_bias_act(acc, p.bias, (int64_t)cm0 + ib * 16, p.act);
         if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C, p.fuse ? nullptr : p.bias,
+            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), p.fuse ? nullptr : p.bias,
                                         (int64_t)cm0, cn0 + wn * 64, p.rows, N, lane, true);
         else
-            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C, (int64_t)cm0, cn0 + wn * 64, N,
+            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), (int64_t)cm0, cn0 + wn * 64, N,
                                            lane, true, (p.fuse && !pre) ? p.bias : nullptr);
         walk.next(c_tm, c_tn);
     }
@@ -493,7 +493,7 @@ __device__ __forceinline__ void ds_consumer_pp(const SpmmParams& p, const TileWa
                 }
             }
         } else if (!SPATHA_KNOB(4)) {
-            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, p.C, (int64_t)cm0,
+            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), (int64_t)cm0,
                                            cn0 + wn * 64, N, lane, !SPATHA_KNOB(2));
         }
         SPATHA_PROF_MARK(2)

@@ -71,8 +71,10 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Row-major stores of C: 16 bytes per lane.  Built with -DSPATHA_OUT_32B (the counterpart of the reference's OUT_32B
 // ablation switch, CMakeLists.txt:25-33) the same bytes leave as four 4-byte stores, to measure what the wide
 // stores are worth; assembly, so that the compiler cannot merge them again.
+// stream: a result that outgrows what the memory-side cache takes in beside the operands (SpmmParams::stream_out): non-temporal stores
+// pass that cache by, where ordinary and written-through ones first push older results out of it.
 template <bool WRITE_THROUGH = false>
-__device__ __forceinline__ void store_c16(uint16_t* dst, u32x4 v) {
+__device__ __forceinline__ void store_c16(uint16_t* dst, u32x4 v, bool stream) {
 #ifdef SPATHA_OUT_32B
     asm volatile(
         "global_store_dword %0, %1, off\n\t"
@@ -85,13 +87,21 @@ __device__ __forceinline__ void store_c16(uint16_t* dst, u32x4 v) {
     // out the operand panels the other workgroups of the XCD are re-reading.  Pays in the dense-staged kernels
     // (4096 x 1024 x 16384 at 64:2:8: 63.7 -> 62.2 us row-major, 66.3 -> 60.7 us transposed + bias) and in the tall
     // kernel's transposed write-out (1024 x 4096 x 16384 at 128:2:16: 33 -> 30.4 us), not in the 128 x 128 tiles
-    // (37.7 -> 39.3 us at 128:2:32); the non-temporal hint costs 3 us everywhere.
+    // (37.7 -> 39.3 us at 128:2:32); where the buffers stay in the memory-side cache the non-temporal hint costs up to 3 us.
     // The s_nop covers the two wait states that the hardware needs between a store of more than 64 bits and a VALU
     // write of its data registers: the compiler inserts them for its own stores, not after an asm statement.
-    if (WRITE_THROUGH) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
+    if (stream) asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
+    else if (WRITE_THROUGH) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
     else *(u32x4*)dst = v;
 #endif
 }
+
+// where a write-out goes and how
+struct OutC {
+    uint16_t* at;
+    bool stream;
+    __device__ __forceinline__ explicit OutC(const SpmmParams& p) : at(p.C), stream(p.stream_out != 0) {}
+};
 
 // "Dynamic LDS limit raised" flags, one per (kernel, device): the attribute is a per-device property of a kernel.
 static bool& lds_attr_flag(const void* kern) {
@@ -266,7 +276,7 @@ constexpr int TT_SLAB_BYTES = 8 * TT_PITCH;        // per wave
 // Transposed write-out (C^T[N][rows], + bias) of one wave's 64 x 64 block through an LDS slab of 8 columns x 64 rows,
 // so that every store instruction covers whole 128-byte lines (defined further down).
 template <bool WRITE_THROUGH = false>
-__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, uint16_t* C,
+__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC C,
                                                             const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                             int lane, bool stores_on);
 
@@ -496,7 +506,7 @@ __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
 
 // rows 4*MB..4*MB+3 (+16*ib) of the pending wave tile -> row-major C through the wave's LDS slab
 template <int MB, int EPI_PITCH>
-__device__ __forceinline__ void store_slab_row_major(const uint32_t (&pend)[4][4][2], char* stg, uint16_t* C, int64_t row_base,
+__device__ __forceinline__ void store_slab_row_major(const uint32_t (&pend)[4][4][2], char* stg, OutC C, int64_t row_base,
                                                      int col_base, int N, int lane, bool enable) {
     const int j16 = lane & 15, ib = lane >> 4;
 #pragma unroll
@@ -515,7 +525,7 @@ __device__ __forceinline__ void store_slab_row_major(const uint32_t (&pend)[4][4
         const int row = 16 * (Lr & 3) + 4 * MB + (Lr >> 2);
         const int col = col_base + ch * 8;
         u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-        if (col < N && enable) store_c16(C + (row_base + row) * N + col, v);
+        if (col < N && enable) store_c16(C.at + (row_base + row) * N + col, v, C.stream);
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -537,7 +547,7 @@ __device__ __forceinline__ void store_block_transposed(const uint32_t (&pend)[4]
 // Straight from the accumulators a lane could only store 16-byte pieces 32 bytes apart; through the slab every
 // store instruction writes 8 output rows (columns of C) x 128 contiguous bytes.
 template <bool WRITE_THROUGH>
-__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, uint16_t* C,
+__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC C,
                                                             const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                             int lane, bool stores_on) {
     const int j16 = lane & 15, ib = lane >> 4;     // as accumulator lane: column j16 of a 16-column block, rows 16*ib + 4*mb + r
@@ -566,7 +576,7 @@ __device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc
             const u32x4 v = *(const u32x4*)(stg + rn * TT_PITCH + rc * 16);
             __builtin_amdgcn_wave_barrier();
             const int col = col0 + nb * 16 + hf * 8 + rn;
-            if (col < N && stores_on) store_c16<WRITE_THROUGH>(C + (int64_t)col * rows_total + row0 + rc * 8, v);
+            if (col < N && stores_on) store_c16<WRITE_THROUGH>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v, C.stream);
         }
     }
 }
@@ -612,7 +622,7 @@ constexpr int TR8_SLAB_BYTES = 64 * TR8_PITCH;     // per wave, 8 slab rows at a
 // the first store, and the phases read them from LDS; a bias load inside a phase would make that phase wait on the
 // vector-memory counter, i.e. for every store issued so far.
 template <bool ROWS8, bool BIAS_VIA_SLAB = false, bool WRITE_THROUGH = true>
-__device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4][4], char* stg, uint16_t* C, int64_t row0,
+__device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4][4], char* stg, OutC C, int64_t row0,
                                                          int col0, int N, int lane, bool stores_on,
                                                          const uint16_t* bias = nullptr) {
     static_assert(!BIAS_VIA_SLAB || ROWS8, "the spare bytes sit behind the 8-row slab");
@@ -664,7 +674,7 @@ __device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4
         short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, stg + roff));
         short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4_t, stg + roff + 4 * PITCH));
         __builtin_amdgcn_wave_barrier();
-        if (ph > 0 && live) store_c16<WRITE_THROUGH>(C + (row0 + held_row) * N + out_col, held);
+        if (ph > 0 && live) store_c16<WRITE_THROUGH>(C.at + (row0 + held_row) * N + out_col, held, C.stream);
         held.x = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
         held.y = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
         held.z = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
@@ -672,7 +682,7 @@ __device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4
         const int q = 8 * sidx + q_lo;
         held_row = 16 * (q >> 2) + 4 * mb + (q & 3);
     }
-    if (live) store_c16<WRITE_THROUGH>(C + (row0 + held_row) * N + out_col, held);
+    if (live) store_c16<WRITE_THROUGH>(C.at + (row0 + held_row) * N + out_col, held, C.stream);
     __builtin_amdgcn_wave_barrier();
 }
 
@@ -680,7 +690,7 @@ __device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4
 // phases' LDS writes and transposing / row reads are in flight before the first store waits for its data, so a 64 x 64
 // block costs two LDS round trips instead of eight.
 template <bool WITH_BIAS>
-__device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[4][4], char* stg, uint16_t* C, int64_t row0,
+__device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[4][4], char* stg, OutC C, int64_t row0,
                                                           int col0, int N, int lane, bool stores_on, const uint16_t* bias) {
     constexpr int PITCH = TR8_PITCH, SLAB = TR8_SLAB_BYTES;
     const int j16 = lane & 15, ib = lane >> 4;
@@ -732,13 +742,13 @@ __device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[
             v.y = (uint32_t)(uint16_t)lo[k][2] | ((uint32_t)(uint16_t)lo[k][3] << 16);
             v.z = (uint32_t)(uint16_t)hi[k][0] | ((uint32_t)(uint16_t)hi[k][1] << 16);
             v.w = (uint32_t)(uint16_t)hi[k][2] | ((uint32_t)(uint16_t)hi[k][3] << 16);
-            if (live) store_c16<true>(C + (row0 + row) * N + out_col, v);
+            if (live) store_c16<true>(C.at + (row0 + row) * N + out_col, v, C.stream);
         }
     }
     __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&acc)[4][4], char* stg, uint16_t* C,
+__device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&acc)[4][4], char* stg, OutC C,
                                                              const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                              int lane, bool stores_on) {
     const int j16 = lane & 15, ib = lane >> 4;     // as accumulator lane: column j16 of a 16-column block, rows 16*ib + 4*mb + r
@@ -772,7 +782,7 @@ __device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&ac
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int col = col0 + (grp * 2 + (k >> 1)) * 16 + (k & 1) * 8 + rn;
-            if (col < N && stores_on) store_c16<true>(C + (int64_t)col * rows_total + row0 + rc * 8, v[k]);
+            if (col < N && stores_on) store_c16<true>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v[k], C.stream);
         }
     }
     __builtin_amdgcn_wave_barrier();

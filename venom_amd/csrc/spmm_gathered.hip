@@ -184,7 +184,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_kernel(SpmmParams p) {
             const int row = 16 * (L & 3) + (L >> 2);
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(st + L * PITCH_C + ch * 16);
-            if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v);
+            if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
         }
     }
 }
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
     const uint16_t* bias = p.fuse ? nullptr : p.bias;
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
         __syncthreads();                 // every wave is done reading the stages: their memory becomes the slabs
-        store_block_transposed_slab<true>(acc, smem + wave * TT_SLAB_BYTES, p.C, bias, (int64_t)m0 + wm * 64, n0 + wn * 64,
+        store_block_transposed_slab<true>(acc, smem + wave * TT_SLAB_BYTES, OutC(p), bias, (int64_t)m0 + wm * 64, n0 + wn * 64,
                                           p.rows, N, lane, true);
     } else if (!SPATHA_KNOB(4)) {
         __syncthreads();                 // every wave is done reading the stages
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(stg + Lr * PITCH_C + ch * 16);
             // (256-wide tiles: written through, 0-13 % faster on the BERT-large / GPT-2-large layer shapes; the 128-wide ones lose)
-            if (col < N && !SPATHA_KNOB(2)) store_c16<(WN >= 4)>(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v);
+            if (col < N && !SPATHA_KNOB(2)) store_c16<(WN >= 4)>(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
         }
     }
 }
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(WN * 128) void spmm_half_kernel(SpmmParams p) {
             const int row = 32 * half + 8 * (Lr & 3) + 4 * ((Lr >> 4) & 1) + ((Lr >> 2) & 3);
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(stg + Lr * PITCH_C + ch * 16);
-            if (col < N && m0 + row < p.rows) store_c16(p.C + ((int64_t)m0 + row) * N + col, v);
+            if (col < N && m0 + row < p.rows) store_c16(p.C + ((int64_t)m0 + row) * N + col, v, p.stream_out != 0);
         }
     }
 }
@@ -887,7 +887,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
                     const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                     const int col = cn0 + wn * 64 + ch * 8;
                     u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v);
+                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
                 }
                 __builtin_amdgcn_wave_barrier();
             }

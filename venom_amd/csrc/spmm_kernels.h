@@ -37,6 +37,7 @@ struct SpmmParams {
     long long* prof;          // development cycle-accounting buffer (SPATHA_DEV_PROFILE builds), else null
     int fuse;                 // 1: bias and activation are applied ahead of the write-out (fused_bias_act)
     int act;                  // SPATHA_ACT_*
+    int stream_out;           // 1: C leaves by non-temporal stores (the staged kernels; streams_out in spatha_api.cpp)
     int debug;                // development knobs (0 in production): 1 = skip B loads, 2 = skip C stores
 };
 

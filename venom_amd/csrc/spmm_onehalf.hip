@@ -335,7 +335,7 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
     const int col0 = tn * 256 + (on_extra ? extra_half * 128 : 0) + q * 64;
     if constexpr (FUSE) fused_bias_act(acc, p.bias, row0 + ib * 16, p.act);
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-        store_block_transposed_slab<true>(acc, stg, p.C, FUSE ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
+        store_block_transposed_slab<true>(acc, stg, OutC(p), FUSE ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
     } else {
         // 16-row slabs through the wave's staging buffer -> 128-byte row segments
 #pragma unroll
@@ -352,7 +352,7 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
                 const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                 const int col = col0 + ch * 8;
                 u32x4 v = *(const u32x4*)(stg + Lr * OH_EPI_PITCH + ch * 16);
-                if (col < N) store_c16(p.C + (row0 + row) * N + col, v);
+                if (col < N) store_c16(p.C + (row0 + row) * N + col, v, p.stream_out != 0);
             }
             __builtin_amdgcn_wave_barrier();
         }

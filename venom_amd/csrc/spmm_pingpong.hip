@@ -289,10 +289,10 @@ __device__ __forceinline__ void up_wave(const SpmmParams& p, const Walk& walk, c
                     // one on all 64 accumulator registers of the block); the write-out itself is then the plain one
                     if constexpr (FUSE) fused_bias_act_narrow(acc[wn], p.bias, (int64_t)cm0 + (lane >> 4) * 16, p.act);
                     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                        store_block_transposed_slab4(acc[wn], stg, p.C, FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
+                        store_block_transposed_slab4(acc[wn], stg, OutC(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
                                                      lane, !(UP_KNOBS & 32));
                     else
-                        store_block_row_major_tr4<false>(acc[wn], stg, p.C, (int64_t)cm0, cn0 + wn * 64, N, lane, !(UP_KNOBS & 32), nullptr);
+                        store_block_row_major_tr4<false>(acc[wn], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !(UP_KNOBS & 32), nullptr);
                 }
             }
             zero_acc();

@@ -255,10 +255,10 @@ __global__ __launch_bounds__(512) void spmm_du_kernel(SpmmParams p) {
                 // on all 64 accumulator registers of the block); the write-out itself is then the plain one
                 if constexpr (FUSE) fused_bias_act_narrow(acc[wn], p.bias, (int64_t)cm0 + ib * 16, p.act);
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                    store_block_transposed_slab<true>(acc[wn], stg, p.C, FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows,
+                    store_block_transposed_slab<true>(acc[wn], stg, OutC(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows,
                                                       N, lane, true);
                 else
-                    store_block_row_major_tr<true>(acc[wn], stg, p.C, (int64_t)cm0, cn0 + wn * 64, N, lane, true);
+                    store_block_row_major_tr<true>(acc[wn], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, true);
             }
             zero_acc();
             walk.next(c_tm, c_tn);

@@ -240,7 +240,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& wal
         if (p.fuse) fused_bias_act(acc, p.bias, (int64_t)cm0 + wm * 64 + ib * 16, p.act);
         const uint16_t* bias = p.fuse ? nullptr : p.bias;
         if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), p.C, bias,
+            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), OutC(p), bias,
                                               (int64_t)cm0 + wm * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
         } else if (!SPATHA_KNOB(4)) {
             // 16-row slabs through a wave-private LDS buffer -> 128-byte row segments
@@ -259,7 +259,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& wal
                     const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                     const int col = cn0 + wn * 64 + ch * 8;
                     u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v);
+                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
                 }
                 __builtin_amdgcn_wave_barrier();
             }
@@ -306,10 +306,10 @@ __device__ __forceinline__ void ws_consumer_deferred(const SpmmParams& p, const 
         } else {
             const int64_t rb = (int64_t)pm0 + wm * 64;
             const int cb = pn0 + wn * 64;
-            if (part == 0) store_slab_row_major<0, EPI_PITCH>(pend, stg, p.C, rb, cb, N, lane, stores_on);
-            else if (part == 1) store_slab_row_major<1, EPI_PITCH>(pend, stg, p.C, rb, cb, N, lane, stores_on);
-            else if (part == 2) store_slab_row_major<2, EPI_PITCH>(pend, stg, p.C, rb, cb, N, lane, stores_on);
-            else store_slab_row_major<3, EPI_PITCH>(pend, stg, p.C, rb, cb, N, lane, stores_on);
+            if (part == 0) store_slab_row_major<0, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
+            else if (part == 1) store_slab_row_major<1, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
+            else if (part == 2) store_slab_row_major<2, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
+            else store_slab_row_major<3, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
         }
     };
     for (int c_tile = 0; c_tile < walk.my_tiles; c_tile++) {
@@ -441,7 +441,7 @@ __device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const Tile
             if (p.fuse) fused_bias_act(acc[h], p.bias, (int64_t)cm0 + h * 64 + ib * 16, p.act);
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                 if (!SPATHA_KNOB(4))
-                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), p.C, p.fuse ? nullptr : p.bias,
+                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), OutC(p), p.fuse ? nullptr : p.bias,
                                                 (int64_t)cm0 + h * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
             } else if (!SPATHA_KNOB(4)) {
                 char* stg = smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH);
@@ -459,7 +459,7 @@ __device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const Tile
                         const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                         const int col = cn0 + wn * 64 + ch * 8;
                         u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                        if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + h * 64 + row) * N + col, v);
+                        if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + h * 64 + row) * N + col, v, p.stream_out != 0);
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
@@ -713,12 +713,12 @@ __device__ __forceinline__ void wsw_storer(const SpmmParams& p, const TileWalk& 
             if (i >= next_piece && i < next_piece + count) {
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                     const int col = h_tn * BN + srow + RPP * i;         // staging row = tile column
-                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i]);
+                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i], p.stream_out != 0);
                 } else {
                     const int q = 8 * (i & 1) + q_lo;                  // piece i: slab of mb = i / 2, lane groups 2*(i & 1), + 1
                     const int row = blk_row0 + 16 * (q >> 2) + 4 * (i >> 1) + (q & 3);
                     const int col = h_tn * BN + blk_col;
-                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i]);
+                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i], p.stream_out != 0);
                 }
             }
         }
