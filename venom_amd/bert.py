@@ -32,7 +32,9 @@ class NMVectorSparsifier:
         nrows, ncols = tensor.shape
         if self.magnitude and tensor.is_cuda:
             # model conversion of a weight that lives on the GPU: selected and encoded there
-            return wrapper_class().wrapped_from_dense(SrNMTensor.from_magnitude(tensor, self.n, self.m, self.tileM), tensor, grad_fmt)
+            # (the kernels first: they run while the wrapper's class is looked up)
+            converted = SrNMTensor.from_magnitude(tensor, self.n, self.m, self.tileM)
+            return wrapper_class().wrapped_from_dense(converted, tensor, grad_fmt)
         if self.magnitude:
             # model conversion: equal magnitudes (frequent in fp16 weights) go to the lower column, no history replay
             mask, columns = nm_vector_mask_sparsify(tensor, self.n, self.m, self.tileM, exact_ties=not tensor.is_cuda)

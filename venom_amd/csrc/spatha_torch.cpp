@@ -144,6 +144,68 @@ std::shared_ptr<spatha_spmm_plan> plan_for(const torch::Tensor& values, const to
     return plan;
 }
 
+bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
+    return t.defined() && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
+}
+
+// The V:N:M arrays of a matrix in order on the GPU, magnitude selection and encoding: (values, metadata, columns), or None for what the
+// general path decides, and refuses.
+py::object convert(py::handle input, int n, int m, int v) {
+    if (!THPVariable_CheckExact(input.ptr())) return py::none();
+    const torch::Tensor& x = THPVariable_Unpack(input.ptr());
+    if (!x.is_cuda() || x.layout() != torch::kStrided || x.dim() != 2 || x.numel() == 0 || !x.is_contiguous() || x.size(0) > INT32_MAX ||
+        x.size(1) > INT32_MAX || (x.scalar_type() != torch::kFloat16 && x.scalar_type() != torch::kFloat32))
+        return py::none();
+    spatha_vnm_geometry geo;
+    const int rows = (int)x.size(0), cols = (int)x.size(1);
+    if (spatha_vnm_geometry_init(rows, cols, n, m, v, &geo) != SPATHA_OK) return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(x.device());
+    const torch::TensorOptions on = torch::TensorOptions().device(x.device());
+    torch::Tensor values = torch::empty({geo.n_values}, on.dtype(torch::kFloat16)), metadata = torch::empty({geo.n_metadata}, on.dtype(torch::kInt32)),
+                  columns = torch::empty({geo.n_columns}, on.dtype(torch::kInt32));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
+    if (spatha_vnm_convert_gpu(x.data_ptr(), x.scalar_type() == torch::kFloat16 ? 16 : 32, rows, cols, n, m, v, (uint16_t*)values.data_ptr(),
+                               (uint32_t*)metadata.data_ptr(), (uint32_t*)columns.data_ptr(), stream) != SPATHA_OK)
+        return py::none();
+    auto wrap = [](const torch::Tensor& t) { return py::reinterpret_steal<py::object>(THPVariable_Wrap(t)); };
+    return py::make_tuple(wrap(values), wrap(metadata), wrap(columns));
+}
+
+// The dense fp16 matrix [rows, cols] of arrays in order on the GPU, complete on return; None for arrays that the kernel does not take, a
+// status where a column offset has no place in its group.
+py::object to_dense(py::handle values_h, py::handle metadata_h, py::handle columns_h, int rows, int cols, int n, int m, int v) {
+    if (!THPVariable_CheckExact(values_h.ptr()) || !THPVariable_CheckExact(metadata_h.ptr()) || !THPVariable_CheckExact(columns_h.ptr()))
+        return py::none();
+    const torch::Tensor &values = THPVariable_Unpack(values_h.ptr()), &metadata = THPVariable_Unpack(metadata_h.ptr()),
+                        &columns = THPVariable_Unpack(columns_h.ptr());
+    if (!values.is_cuda()) return py::none();
+    const int device = (int)values.get_device();
+    spatha_vnm_geometry geo;
+    if (spatha_vnm_geometry_init(rows, cols, n, m, v, &geo) != SPATHA_OK || !weight_ok(values, torch::kFloat16, device) ||
+        !weight_ok(metadata, torch::kInt32, device) || !weight_ok(columns, torch::kInt32, device) || values.numel() != geo.n_values ||
+        metadata.numel() != geo.n_metadata || columns.numel() != geo.n_columns ||
+        (((uintptr_t)values.data_ptr() | (uintptr_t)metadata.data_ptr() | (uintptr_t)columns.data_ptr()) & 3u))
+        return py::none();
+    const torch::NoGradGuard no_grad;
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(values.device());
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+    torch::Tensor dense = torch::empty({rows, cols}, torch::TensorOptions().device(values.device()).dtype(torch::kFloat16));
+    torch::Tensor flag = torch::empty({1}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
+    volatile int* bad = flag.data_ptr<int>();
+    *bad = 0;
+    check(spatha_vnm_decode_f16_gpu((const uint16_t*)values.data_ptr(), (const uint32_t*)metadata.data_ptr(), (const uint32_t*)columns.data_ptr(),
+                                    rows, cols, n, m, v, (uint16_t*)dense.data_ptr(), (uint32_t*)flag.data_ptr(), stream),
+          "spatha_vnm_decode");
+    {
+        const py::gil_scoped_release release;
+        const hipError_t e = hipStreamSynchronize(stream);
+        if (e != hipSuccess) throw std::runtime_error(std::string("spatha_vnm_decode: ") + hipGetErrorString(e));
+    }
+    if (*bad) return py::int_((int)SPATHA_ERR_BAD_ARGUMENT);
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(dense));
+}
+
 // x [rows, columns], contiguous, with zero columns up to the next multiple of 8
 torch::Tensor pad_columns(const torch::Tensor& x) {
     const int64_t columns = x.size(1);
@@ -240,10 +302,6 @@ py::object transpose_f16(py::handle input) {
         return py::none();
     const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(x.device());
     return py::reinterpret_steal<py::object>(THPVariable_Wrap(transposed_padded(x)));
-}
-
-bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
-    return t.defined() && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
 }
 
 // Where work issued now on torch's current stream of `device` runs: the stream, and the capture that records it (0: none).  What one
@@ -565,6 +623,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
     mod.def("attention", &attention, "attention of merged projections, feature-major, or None");
     mod.def("add_layernorm", &add_layernorm, "LayerNorm(x + residual): (result, feature-major copy or None), or None");
     mod.def("embed_layernorm", &embed_layernorm, "LayerNorm of summed table rows: (result, feature-major copy or None), or None");
+    mod.def("convert", &convert, "the V:N:M arrays of a matrix on the GPU, or None");
+    mod.def("to_dense", &to_dense, "the matrix of V:N:M arrays on the GPU, or None, or the status of a refusal");
     mod.def("stream_key", &stream_key, "(stream, capture) that work issued now on this device goes to", py::arg("device"));
     mod.def("transpose", &transpose_f16, "x.T of an fp16 matrix through the library's kernel, or None");
     mod.def("plan_run", &plan_run, "a plan's product, or None, or the status of a refusal");

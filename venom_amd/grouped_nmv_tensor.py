@@ -7,7 +7,7 @@ time: all work is done by libspatha.so through the C ABI."""
 import numpy as np
 import torch
 
-from . import _lib
+from . import _lib, spatha
 from . import format as F
 
 
@@ -85,6 +85,12 @@ class SrNMTensor:
         self.n, self.m, self.tileM = n, m, tileM
         self.device = dense.device
         self.nrows, self.ncols = dense.shape
+        native = spatha._native("convert")
+        got = native(dense, n, m, tileM) if native is not None else None
+        if got is not None:
+            self.values, self.metadata, self.columns = got
+            self.nnz = self.values.numel()              # nrows * ksp
+            return self
         geo = F.geometry(self.nrows, self.ncols, n, m, tileM)
         self.nnz = self.nrows * geo.ksp
         src = dense.detach()
@@ -101,6 +107,13 @@ class SrNMTensor:
         return self
 
     def to_dense(self):
+        native = spatha._native("to_dense")
+        if native is not None:
+            got = native(self.values, self.metadata, self.columns, self.nrows, self.ncols, self.n, self.m, self.tileM)
+            if type(got) is int:
+                raise _lib.SpathaError(got, "spatha_vnm_decode")
+            if got is not None:
+                return got.to(device=self.device)
         geo = F.geometry(self.nrows, self.ncols, self.n, self.m, self.tileM)
         where = _decodes_on_gpu(self, geo)
         if where is not None:
