@@ -231,6 +231,14 @@ int spatha_spmm_workspace_init(void* workspace_dev, size_t workspace_bytes, void
 int spatha_spmm_run_ws(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                        int out_layout, int activation, void* workspace_dev, size_t workspace_bytes, void* stream);
 
+/* A product for any N, C in rows of N entries (or transposed), B in rows b_pitch >= N entries apart, where the kernel that would be chosen for
+ * the next multiple of 8 is one that needs no 16-byte row pieces (few columns, small products).  SPATHA_ERR_UNSUPPORTED where it is
+ * not - pad B and cut C then (spatha_pad_columns_f16, spatha_cut_columns_f16) - and, with b_pitch no multiple of 8, where a padded
+ * B is faster (b_pitch = ROUND_UP(N, 8); nothing is to be cut).  fused: as in spatha_spmm_run_fused (a bias with row-major
+ * output), else the contract of spatha_spmm_run.  The same numbers as the padded product's. */
+int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, int b_pitch, int N, const uint16_t* bias_dev, uint16_t* out_dev,
+                           int out_layout, int activation, int fused, void* stream);
+
 /* spatha_spmm_run_ws (workspace NULL, 0 where none is wanted) for a result that the caller's next operation reads: it is written so that
  * it stays in the memory-side cache.  The other entry points let results of 48 MB and more pass that cache by, which is faster
  * where other data goes through it before the result is read. */
@@ -301,6 +309,9 @@ int spatha_transpose_padded_f16(const uint16_t* in_dev, int rows, int cols, uint
 
 /* out[rows x ROUND_UP(cols, 8)] = in[rows x cols] with zero columns appended; in_dev at any alignment. */
 int spatha_pad_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream);
+
+/* out[rows x cols] = the first cols columns of in, whose rows are ROUND_UP(cols, 8) entries apart; out_dev at any alignment. */
+int spatha_cut_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream);
 
 /* out[tokens x hidden] = LayerNorm(x + residual) over the last dimension, fp16 in and out, fp32 arithmetic
  * (the sum is rounded to fp16 first, as the separate addition would; biased variance; gamma, beta of length hidden).

@@ -21,6 +21,65 @@ def test_padded_copies(gpu, rows, cols, offset):
     assert torch.equal(t, torch.nn.functional.pad(x.t(), (0, -rows % 8)))
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (64, 8), (65, 9), (130, 301), (1280, 1037), (63, 4097)])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_cut_results(gpu, rows, cols, offset):
+    full = torch.randn(rows, (cols + 7) // 8 * 8, device=gpu).half()
+    buf = torch.full((rows * cols + 64,), 7.0, dtype=torch.float16, device=gpu)
+    out = buf[8 + offset:8 + offset + rows * cols]
+    _lib.check(_lib.lib().spatha_cut_columns_f16(full.data_ptr(), rows, cols, out.data_ptr(), spatha._stream_ptr(gpu)), "cut")
+    assert torch.equal(out.view(rows, cols), full[:, :cols])
+    assert bool((buf[:8 + offset] == 7.0).all()) and bool((buf[8 + offset + rows * cols:] == 7.0).all())
+
+
+@pytest.mark.parametrize("rows,cols,v,m", [(64, 96, 64, 8), (128, 70, 128, 16), (1024, 1024, 64, 8), (96, 200, 32, 10), (2048, 512, 32, 16),
+                                           (5120, 1280, 128, 16), (5120, 1280, 64, 10), (33024, 256, 64, 4)])
+@pytest.mark.parametrize("tokens", [1, 2, 7, 15, 17, 18, 31, 33, 35, 47, 63, 65, 70, 129, 301, 1037])
+def test_ragged_products_equal_the_padded_ones(gpu, rows, cols, v, m, tokens):
+    """B and C as they lie (where a kernel without 16-byte pieces is chosen) or a padded copy and a cut: bit for bit the padded product,
+    nothing written around C, and a NaN or infinity next to a lane's last columns stays where it belongs."""
+    from venom_amd import format as F
+
+    vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=tokens)
+    plan = spatha.SpmmPlan(torch.from_numpy(vals).to(gpu), torch.from_numpy(meta.view("int32")).to(gpu),
+                           torch.from_numpy(columns.view("int32")).to(gpu), rows, cols, 2, m, v)
+    gen = torch.Generator(device=gpu).manual_seed(rows + tokens)
+    B = torch.randn((cols, tokens), generator=gen, device=gpu).half()
+    if tokens > 2:
+        B[cols // 2, 0] = float("nan")
+        B[cols // 3, tokens // 2] = float("inf")
+    bias = torch.randn(rows, generator=gen, device=gpu).half()
+    padded = spatha._pad_columns(B)
+    act = {} if v == 32 else {"activation": "gelu"}
+    for kwargs in ({}, {"transposed_out": True}, {"transposed_out": True, "bias": bias}, {"bias": bias, "activation": "none"}, {"bias": bias, **act},
+                   {"bias": bias, "transposed_out": True, **act}):
+        if "bias" in kwargs and not kwargs.get("transposed_out") and "activation" not in kwargs:
+            continue
+        full = plan.run(padded, **kwargs)
+        want = full[:tokens] if kwargs.get("transposed_out") else full[:, :tokens]
+        got = plan.run(B, **kwargs)
+        assert got.is_contiguous() and got.shape == want.shape
+        assert torch.equal(got.view(torch.int16), want.contiguous().view(torch.int16)), kwargs
+    out = torch.full((rows * tokens + 64,), 7.0, dtype=torch.float16, device=gpu)
+    for layout in (0, 1):
+        name = plan.kernel_name((tokens + 7) // 8 * 8, out_layout=layout)
+        direct = "_direct_tile" in name or "skinny" in name
+        large = tokens > 16 and tokens % (2 if tokens <= 32 else 4) and rows // 64 * -(-(-(-cols // m) * 2) // 32) * -(-tokens // 64) > 8000
+        for src, pitch, takes in ((B, tokens, direct and not large), (padded, padded.shape[1], direct)):
+            if pitch % 8 == 0 and src is B:
+                continue
+            status = _lib.lib().spatha_spmm_run_ragged(plan._handle, src.data_ptr(), pitch, tokens, None, out[32:].data_ptr(), layout, 0, 0,
+                                                       spatha._stream_ptr(gpu))
+            assert status == (0 if takes else 3), (name, pitch)
+            assert bool((out[:32] == 7.0).all()) and bool((out[32 + rows * tokens:] == 7.0).all())
+            if takes:
+                want = plan.run(padded, transposed_out=bool(layout))
+                want = want[:tokens] if layout else want[:, :tokens].contiguous()
+                assert torch.equal(out[32:32 + rows * tokens].view(torch.int16), want.reshape(-1).view(torch.int16))
+    with pytest.raises(Exception):
+        plan.run(B, bias=bias)              # a bias needs the transposed layout or an activation, ragged or not
+
+
 @pytest.mark.parametrize("shape", [(1, 128), (301, 128), (3, 5, 128), (2, 8, 128), (1, 2, 3, 128)])
 def test_layers_take_any_token_count_and_stride(gpu, shape):
     """The layer's one-call path against the operator on a copy made by torch: token-major, feature-major, strided and sliced

@@ -60,6 +60,7 @@ SIGNATURES = {
     "spatha_spmm_run_tokens": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
     "spatha_spmm_run_ws": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, ctypes.c_size_t, c_void_p]),
     "spatha_spmm_run_layer": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, ctypes.c_size_t, c_void_p]),
+    "spatha_spmm_run_ragged": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "spatha_spmm_num_variants": (c_int, []),
     "spatha_spmm_kernel_name": (c_char_p, [c_void_p, c_int, c_int, c_int]),
     "spatha_spmm_time": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, POINTER(c_float)]),
@@ -76,6 +77,7 @@ SIGNATURES = {
     "spatha_embed_layernorm_f16": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                            c_int64, c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p]),
     "spatha_attention_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_void_p]),
+    "spatha_cut_columns_f16": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p]),
     "spatha_add_layernorm_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_void_p]),
     "spatha_add_layernorm_f16_t": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p]),
 }

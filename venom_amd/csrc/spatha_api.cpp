@@ -744,7 +744,7 @@ int spatha::plan_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N,
     p.apack = plan->apack; p.rowtab = plan->rowtab;
     p.B = B_dev; p.bias = bias_dev; p.C = out_dev; p.zeros = plan->zeros; p.gtab = plan->gtab;
     p.gtab_bytes = (uint32_t)plan->gtab_bytes;
-    p.rows = plan->geo.rows; p.cols = plan->geo.cols; p.N = N; p.S = plan->S; p.v = plan->geo.v; p.m = plan->geo.m;
+    p.rows = plan->geo.rows; p.cols = plan->geo.cols; p.N = N; p.b_pitch = N; p.S = plan->S; p.v = plan->geo.v; p.m = plan->geo.m;
     const int bm = spatha::spmm_variant_bm(var), bn = spatha::spmm_variant_bn(var);
     p.tiles_m = (plan->geo.rows + bm - 1) / bm;     // (only the half-tile kernels see rows % 64 != 0: a padded last tile)
     p.tiles_n = (N + bn - 1) / bn;
@@ -837,6 +837,38 @@ int spatha_spmm_run_layer(const spatha_spmm_plan* plan, const uint16_t* B_dev, i
                           int out_layout, int activation, void* workspace_dev, size_t workspace_bytes, void* stream) {
     return spatha::plan_run(plan, B_dev, N, bias_dev, out_dev, out_layout, activation, true, spatha::SPMM_VARIANT_AUTO, stream,
                             workspace_dev, workspace_bytes, true);
+}
+
+int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, int b_pitch, int N, const uint16_t* bias_dev, uint16_t* out_dev,
+                           int out_layout, int activation, int fused, void* stream) {
+    if (N <= 0 || N > INT32_MAX - 8 || b_pitch < N || b_pitch > INT32_MAX - 8) return SPATHA_ERR_BAD_ARGUMENT;
+    // the checks and the choice of the padded product: what it refuses is refused, and the sums run in its order
+    const int padded = (N + 7) / 8 * 8;
+    int var = -1;
+    const int status = spatha::plan_run_check(plan, B_dev, padded, bias_dev, out_dev, out_layout, activation, fused != 0,
+                                              spatha::SPMM_VARIANT_AUTO, &var);
+    if (status != SPATHA_OK) return status;
+    if (var != spatha::SPMM_VARIANT_SKINNY && var != spatha::SPMM_VARIANT_DIRECT64 && var != spatha::SPMM_VARIANT_HDIRECT32)
+        return SPATHA_ERR_UNSUPPORTED;
+    // Loads of two or four columns at odd addresses take the L1 a third longer: 0.3 ns per 64 x 64 block and k-step over the chip
+    // (12288 x 12288 at 128:2:16 and 17 tokens, 9216 of them, 11.5 -> 14.4 us; 49152 x 12288 at 64:2:4, 147456 of them, 132 -> 170;
+    // 16 tokens and fewer, and even counts in their place, level), the padded copy 2.6 us.
+    if (N > 16 && b_pitch % (N <= 32 ? 2 : 4) != 0 && (int64_t)(plan->geo.rows / 64) * plan->S * ((N + 63) / 64) > 8000)
+        return SPATHA_ERR_UNSUPPORTED;
+    if ((uint64_t)plan->geo.cols * (uint64_t)b_pitch * 2u >= 0xE0000000ull) return SPATHA_ERR_UNSUPPORTED;
+    spatha::SpmmParams p = {};
+    p.apack = plan->apack; p.rowtab = plan->rowtab;
+    p.B = B_dev; p.bias = bias_dev; p.C = out_dev; p.zeros = plan->zeros;
+    p.rows = plan->geo.rows; p.cols = plan->geo.cols; p.N = N; p.b_pitch = b_pitch; p.S = plan->S; p.v = plan->geo.v; p.m = plan->geo.m;
+    p.b_bytes = (uint32_t)((uint64_t)plan->geo.cols * (uint64_t)b_pitch * 2u);
+    p.apack_bytes = (uint32_t)plan->apack_bytes;
+    p.rowtab_bytes = (uint32_t)plan->rowtab_bytes;
+    p.fuse = activation != SPATHA_ACT_NONE || (out_layout == SPATHA_OUT_ROW_MAJOR && bias_dev) ? 1 : 0;
+    p.act = activation;
+    p.cus = plan->cus > 0 ? plan->cus : 256;
+    p.ksplit = 1;
+    const hipError_t e = spatha::launch_spmm(var, out_layout, p, (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 
 int spatha_spmm_run_tokens(const spatha_spmm_plan* plan, const uint16_t* x_dev, int tokens, const uint16_t* bias_dev, uint16_t* out_dev,
@@ -982,6 +1014,13 @@ int spatha_pad_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t*
     if (!in_dev || !out_dev || rows <= 0 || cols <= 0 || cols > INT32_MAX - 8) return SPATHA_ERR_BAD_ARGUMENT;
     if (((uintptr_t)in_dev & 1u) || ((uintptr_t)out_dev & 15u)) return SPATHA_ERR_BAD_ARGUMENT;
     hipError_t e = spatha::launch_pad_columns_f16(in_dev, rows, cols, out_dev, (cols + 7) / 8 * 8, (hipStream_t)stream);
+    return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_cut_columns_f16(const uint16_t* in_dev, int rows, int cols, uint16_t* out_dev, void* stream) {
+    if (!in_dev || !out_dev || rows <= 0 || cols <= 0 || cols > INT32_MAX - 8) return SPATHA_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)in_dev & 15u) || ((uintptr_t)out_dev & 1u)) return SPATHA_ERR_BAD_ARGUMENT;
+    hipError_t e = spatha::launch_cut_columns_f16(in_dev, rows, cols, (cols + 7) / 8 * 8, out_dev, (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 

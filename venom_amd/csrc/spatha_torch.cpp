@@ -216,6 +216,31 @@ torch::Tensor pad_columns(const torch::Tensor& x) {
     return out;
 }
 
+// full [rows, columns padded to a multiple of 8] -> [rows, columns], contiguous
+torch::Tensor cut_columns(const torch::Tensor& full, int64_t columns) {
+    torch::Tensor out = torch::empty({full.size(0), columns}, full.options().requires_grad(false));
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(full.get_device()).stream();
+    check(spatha_cut_columns_f16((const uint16_t*)full.data_ptr(), (int)full.size(0), (int)columns, (uint16_t*)out.data_ptr(), stream),
+          "spatha_cut_columns_f16");
+    return out;
+}
+
+// The product on `tokens` columns of a right-hand side, which may have more (padding), or an undefined tensor where it takes another
+// kernel or a padded right-hand side
+torch::Tensor run_ragged(const spatha_spmm_plan* plan, const torch::Tensor& rhs, int tokens, const uint16_t* bias_ptr, int rows,
+                         bool transposed_out, int activation, bool fused) {
+    if ((uintptr_t)rhs.data_ptr() & 15) return torch::Tensor();
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(rhs.get_device()).stream();
+    torch::Tensor out = transposed_out ? torch::empty({tokens, rows}, rhs.options().requires_grad(false))
+                                       : torch::empty({rows, tokens}, rhs.options().requires_grad(false));
+    const int status = spatha_spmm_run_ragged(plan, (const uint16_t*)rhs.data_ptr(), (int)rhs.size(1), tokens, bias_ptr,
+                                              (uint16_t*)out.data_ptr(), transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR,
+                                              activation, fused ? 1 : 0, stream);
+    if (status == SPATHA_ERR_UNSUPPORTED) return torch::Tensor();
+    check(status, "spatha_spmm_run_ragged");
+    return out;
+}
+
 // the product on a right-hand side [cols, tokens], tokens a multiple of 8, with operands that have been checked
 torch::Tensor run_full(const torch::Tensor& A_metadata, const torch::Tensor& A_indices, const torch::Tensor& A_values,
                        const torch::Tensor& rhs, int tokens, const uint16_t* bias_ptr, int rows, int cols, int v, int n, int m,
@@ -273,13 +298,20 @@ torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indice
     const int tokens = (int)rhs_matrix.size(1);
     const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(A_values.device());
     if (tokens % 8 != 0 && tokens > 0) {
-        // The library moves rows of B and C in 16-byte pieces: a token count that is no multiple of 8 runs on a copy of
-        // rhs_matrix with zero columns appended, and the result is cut back (the appended columns give bias-only rows /
-        // columns, which are dropped).
+        // Most kernels move rows of B and C in 16-byte pieces: where one of those is chosen, a token count that is no multiple of 8
+        // runs on a copy of rhs_matrix with zero columns appended, and the result is cut back (the appended columns give
+        // bias-only rows / columns, which are dropped).
+        hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
+        const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values, A_metadata, A_indices, rows, cols, n, m, v, stream);
+        const int act = fused ? activation : SPATHA_ACT_NONE;
+        torch::Tensor out = run_ragged(plan.get(), rhs_matrix, tokens, bias_ptr, rows, transposed_out, act, fused);
+        if (out.defined()) return out;
         torch::Tensor padded = pad_columns(rhs_matrix);
+        out = run_ragged(plan.get(), padded, tokens, bias_ptr, rows, transposed_out, act, fused);
+        if (out.defined()) return out;
         torch::Tensor full = run_full(A_metadata, A_indices, A_values, padded, (int)padded.size(1), bias_ptr, rows, cols, v, n, m,
-                                      transposed_out, activation, fused);
-        return transposed_out ? full.narrow(0, 0, tokens) : full.narrow(1, 0, tokens).contiguous();
+                                      transposed_out, activation, fused, !transposed_out);
+        return transposed_out ? full.narrow(0, 0, tokens) : cut_columns(full, tokens);
     }
     return run_full(A_metadata, A_indices, A_values, rhs_matrix, tokens, bias_ptr, rows, cols, v, n, m, transposed_out, activation, fused);
 }
@@ -524,9 +556,10 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
                     bool fused, int activation, int variant) {
     if (!THPVariable_CheckExact(rhs.ptr()) || c10::InferenceMode::is_enabled()) return py::none();
     const torch::Tensor& B = THPVariable_Unpack(rhs.ptr());
-    if (!weight_ok(B, torch::kFloat16, device) || B.dim() != 2 || B.size(0) != cols || B.size(1) <= 0 || B.size(1) % 8 != 0 ||
-        B.size(1) > INT32_MAX)
+    if (!weight_ok(B, torch::kFloat16, device) || B.dim() != 2 || B.size(0) != cols || B.size(1) <= 0 || B.size(1) > INT32_MAX - 8)
         return py::none();
+    const bool ragged = B.size(1) % 8 != 0;
+    if (ragged && (variant != 0 || !out.is_none())) return py::none();
     const int N = (int)B.size(1);
     const uint16_t* bias_ptr = nullptr;
     if (!bias.is_none()) {
@@ -534,6 +567,34 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
         const torch::Tensor& b = THPVariable_Unpack(bias.ptr());
         if (!weight_ok(b, torch::kFloat16, device) || b.numel() != rows) return py::none();
         bias_ptr = (const uint16_t*)b.data_ptr();
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(B.device());
+    const spatha_spmm_plan* plan = (const spatha_spmm_plan*)handle;
+    if (ragged) {
+        if (!fused && !transposed_out && bias_ptr) return py::none();          // (refused)
+        const torch::NoGradGuard no_grad;
+        torch::Tensor got = run_ragged(plan, B, N, bias_ptr, rows, transposed_out, activation, fused), padded;
+        if (!got.defined()) {
+            padded = pad_columns(B);
+            got = run_ragged(plan, padded, N, bias_ptr, rows, transposed_out, activation, fused);
+        }
+        if (!got.defined()) {
+            const int64_t n_padded = padded.size(1);
+            got = transposed_out ? torch::empty({n_padded, rows}, B.options().requires_grad(false))
+                                 : torch::empty({rows, n_padded}, B.options().requires_grad(false));
+            hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
+            const uint16_t* b_ptr = (const uint16_t*)padded.data_ptr();
+            uint16_t* c_ptr = (uint16_t*)got.data_ptr();
+            // (a row-major result is read at once, by the cut)
+            const int status = !transposed_out ? spatha_spmm_run_layer(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_ROW_MAJOR,
+                                                                       activation, nullptr, 0, stream)
+                               : fused ? spatha_spmm_run_fused(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, activation,
+                                                               0, stream)
+                                       : spatha_spmm_run(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, 0, stream);
+            if (status != SPATHA_OK) return py::int_(status);
+            got = transposed_out ? got.narrow(0, 0, N) : cut_columns(got, N);
+        }
+        return py::reinterpret_steal<py::object>(THPVariable_Wrap(got));
     }
     torch::Tensor C;
     if (out.is_none()) {
@@ -545,8 +606,6 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
             C.size(1) != (transposed_out ? rows : N))
             return py::none();
     }
-    const c10::hip::HIPGuardMasqueradingAsCUDA device_guard(B.device());
-    const spatha_spmm_plan* plan = (const spatha_spmm_plan*)handle;
     const uint16_t* b_ptr = (const uint16_t*)B.data_ptr();
     uint16_t* c_ptr = (uint16_t*)C.data_ptr();
     const int layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;

@@ -21,6 +21,7 @@ struct SpmmParams {
     uint16_t* C;              // rows x N, or N x rows when transposed
     int rows, cols, N, S, v;
     int m;                    // dense columns per group (dense-staged kernels)
+    int b_pitch;              // columns from one row of B to the next (the direct kernels; N everywhere else)
     uint32_t b_bytes, apack_bytes, rowtab_bytes;   // sizes for buffer descriptors (persistent kernels)
     int tiles_m, tiles_n;
     int cus;                  // compute units of the device the launch goes to (grid size of the persistent kernels)
@@ -121,6 +122,7 @@ hipError_t launch_pack_gtab(const uint32_t* columns, int rows, int m, int v, int
                             hipStream_t stream);
 
 hipError_t launch_transpose_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
+hipError_t launch_cut_columns_f16(const uint16_t* in, int rows, int cols, int pitch, uint16_t* out, hipStream_t stream);
 hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream);
 // LayerNorm(x + residual), and with out_t once more as [hidden][tokens padded to a multiple of 8]; the embedding of a token sequence
 // ahead of it in place of x and residual (layernorm.hip)

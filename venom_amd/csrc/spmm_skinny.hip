@@ -13,8 +13,9 @@ namespace spatha {
 // multiplied.
 // NB = 1, 2 or 4 column blocks of 16.  Column block nb holds the columns NB * j + nb (j = 0 .. 15), not 16 * nb + j: lane j of
 // a block then needs NB ADJACENT columns of every gathered row, one load of 2 * NB bytes instead of NB loads of 2 bytes - 16
-// vector-memory instructions per k-step whatever NB.  N is a multiple of 8, so the NB columns of a lane lie all inside N or all
-// outside.
+// vector-memory instructions per k-step whatever NB.  B (rows b_pitch apart) and C are addressed at whatever alignment their rows
+// have, so that a ragged token count needs no padded copies (spatha_spmm_run_ragged: 4096 x 1024 at 64:2:8 and 301 tokens with GELU,
+// row-major, 9.5 us, 23.0 with a launch for each copy).
 // What bounds it: with few tiles the trip to memory that a k-step's loads take (four waves a tile left 16 .. 192 of 256 CUs with
 // one wave per SIMD and fewer than two steps in flight: 12288 x 12288 at 64:2:8 and 8 tokens 25.1 us for 101 MB; sixteen waves:
 // 16.0); with many, the 12.8 KB of loads per 64 x 64 block and k-step through the L1 (0.8-1.2 ns a block and step over the chip).
@@ -25,6 +26,10 @@ namespace spatha {
 // of four waves per CU - which it reaches with 158 registers.)
 // halfs between two tokens in LDS: odd in 32-bit words, so that the sixteen tokens of a fragment row sit on different banks
 __host__ __device__ constexpr int token_pitch_halfs(int cols) { return (((cols + 7) / 8 * 4) | 1) * 2; }
+
+// adjacent columns of C at whatever alignment
+struct __attribute__((packed, aligned(2))) Piece4 { half4_t v; };
+struct __attribute__((packed, aligned(2))) Piece2 { half2_t v; };
 
 template <int NB, int W, bool HALF, bool LEAN>
 struct DirectCfg {
@@ -65,7 +70,7 @@ void spmm_direct_kernel(SpmmParams p) {
     const char* a_tile = (const char*)p.apack + block * S * APACK_BLOCK;
     const uint32_t* rt_block = p.rowtab + vb * S * 64;
     __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, (int)p.b_bytes, 0x00020000);
-    const uint32_t row_bytes = (uint32_t)N * 2u;
+    const uint32_t row_bytes = (uint32_t)p.b_pitch * 2u;
 
     float4_t acc[MB][NB];
 #pragma unroll
@@ -89,7 +94,13 @@ void spmm_direct_kernel(SpmmParams p) {
 #pragma unroll
         for (int d = 0; d < MB / 2; d++) x.ix[d] = *(const uint32_t*)(q + 4096 + (half + d) * 256 + lane * 4);
     };
-    const int col0 = (tile_n * 16 + li) * NB;       // this lane's NB columns: col0 + nb
+    // This lane's NB columns, col0 + nb.  Where rows of B have no padding that the last lane's could reach into, that lane moves down.
+    const int lane_col = (tile_n * 16 + li) * NB;
+    const int col0 = p.b_pitch % NB != 0 && lane_col > N - NB ? N - NB : lane_col;
+    // (lanes beyond N fetch nothing in groups of four; single ones fetch what the last lane does: four lanes of which some are out of the
+    // descriptor's range take the load a third longer - 49152 x 12288 at 64:2:4 and 18 tokens 170 against 132 us)
+    const bool fetches = lane_col < (N + 4 * NB - 1) / (4 * NB) * (4 * NB), stores = lane_col < N;
+    const uint32_t fetch_col = (uint32_t)(lane_col < N ? col0 : p.b_pitch % NB != 0 ? N - NB : (N - 1) / NB * NB);
     const int token_pitch = token_pitch_halfs(p.cols);
     if constexpr (TOKEN_MAJOR) {
         // x [N][cols] -> LDS as it lies; columns N .. 15 of the tile are never stored, they multiply token 0
@@ -122,7 +133,7 @@ void spmm_direct_kernel(SpmmParams p) {
                     bf[0][fb * 4 + j] = __builtin_bit_cast(_Float16, (uint16_t)(row != 0xFFFFFFFFu ? h : 0));
                     continue;
                 }
-                const uint32_t voff = (row != 0xFFFFFFFFu && col0 < N) ? row * row_bytes + (uint32_t)col0 * 2u : 0xF0000000u;
+                const uint32_t voff = (row != 0xFFFFFFFFu && fetches) ? row * row_bytes + fetch_col * 2u : 0xF0000000u;
                 if constexpr (NB == 1) {
                     const uint16_t h = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc_b, (int)voff, 0, 0);
                     bf[0][fb * 4 + j] = __builtin_bit_cast(_Float16, h);
@@ -236,22 +247,29 @@ void spmm_direct_kernel(SpmmParams p) {
                     for (int r = 0; r < 4; r++) h4[c][r] = (_Float16)act_gelu_tanh((float)h4[c][r]);
             }
             const int col = col0 + nb0;
-            if (col >= N || SPATHA_KNOB(2)) continue;
+            if (!stores || SPATHA_KNOB(2)) continue;
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
 #pragma unroll
-                for (int c = 0; c < CB; c++) *(half4_t*)(p.C + (int64_t)(col + c) * p.rows + row0) = h4[c];
+                for (int c = 0; c < CB; c++)
+                    if (CB == 1 || col + c < N) *(half4_t*)(p.C + (int64_t)(col + c) * p.rows + row0) = h4[c];
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     uint16_t* dst = p.C + (row0 + r) * N + col;
                     if constexpr (CB == 4) {
-                        *(half4_t*)dst = (half4_t){h4[0][r], h4[1][r], h4[2][r], h4[3][r]};
+                        if (col + 4 <= N) {
+                            ((Piece4*)dst)->v = (half4_t){h4[0][r], h4[1][r], h4[2][r], h4[3][r]};
+                            continue;
+                        }
                     } else if constexpr (CB == 2) {
-                        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-                        *(half2_t*)dst = (half2_t){h4[0][r], h4[1][r]};
-                    } else {
-                        *(_Float16*)dst = h4[0][r];
+                        if (col + 2 <= N) {
+                            ((Piece2*)dst)->v = (half2_t){h4[0][r], h4[1][r]};
+                            continue;
+                        }
                     }
+#pragma unroll
+                    for (int c = 0; c < CB; c++)
+                        if (CB == 1 || col + c < N) *((_Float16*)dst + c) = h4[c][r];
                 }
             }
         }

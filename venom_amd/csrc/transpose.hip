@@ -68,40 +68,64 @@ hipError_t launch_transpose_f16(const uint16_t* in, int rows, int cols, uint16_t
     return hipGetLastError();
 }
 
-// out[r][c] = in[r][c], zeros from cols to pitch (a multiple of 8): the padded copy of a right-hand side whose column count is no
-// multiple of 8.  One thread per 16 bytes of the copy; a piece is read by one load at whatever alignment its row has.  Bound by
-// launch and latency at the sizes it is used for: a product of 5120 x 1280 at 64:2:10 with 1037 columns takes 16.2 us with it,
-// 19.0 with a fill and a strided copy in its place.
-__global__ __launch_bounds__(256) void pad_columns_f16_kernel(const uint16_t* __restrict__ in, int rows, int cols,
-                                                              uint16_t* __restrict__ out, int pitch) {
-    struct __attribute__((packed, aligned(2))) Piece {
-        tr_u32x4 v;
-    };
-    const int pieces = pitch >> 3;
-    const int64_t total = (int64_t)rows * pieces;
-    for (int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x; id < total; id += (int64_t)gridDim.x * 256) {
-        const int64_t r = id / pieces;
+namespace {
+struct __attribute__((packed, aligned(2))) Unaligned16 {
+    tr_u32x4 v;
+};
+}  // namespace
+
+// out[r][c] = in[r][c] for c < cols, rows in_pitch and out_pitch apart.  PAD: zeros from cols to out_pitch, a multiple of 8 (the padded copy of
+// a right-hand side whose column count is no multiple of 8); else in_pitch is one, and the ragged rows of a result are cut out.  A
+// thread takes one 16-byte piece, and the ragged side goes by one access at whatever alignment its row has.  Bound by launch and
+// latency at most sizes: 1280 x 1037 2.85 us padded, 3.1 with two rows a thread, of which an empty launch is 2.4; cutting 3072 x 2785
+// 7.5 us, 9.6 as a strided copy.
+template <bool PAD>
+__global__ __launch_bounds__(256) void repitch_f16_kernel(const uint16_t* __restrict__ in, int rows, int cols, int in_pitch,
+                                                          uint16_t* __restrict__ out, int out_pitch) {
+    const uint32_t pieces = (uint32_t)(cols + 7) >> 3;
+    const uint64_t total = (uint64_t)rows * pieces;
+    for (uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x; id < total; id += (uint64_t)gridDim.x * 256) {
+        const uint64_t r = total >> 32 ? id / pieces : (uint32_t)id / pieces;
         const int c = (int)(id - r * pieces) * 8;
-        const uint16_t* src = in + r * cols + c;
+        const uint16_t* src = in + r * in_pitch + c;
+        uint16_t* dst = out + r * out_pitch + c;
         tr_u32x4 v;
-        if (c + 8 <= cols) {
-            v = ((const Piece*)src)->v;
+        if (!PAD) {
+            v = *(const tr_u32x4*)src;
+        } else if (c + 8 <= cols) {
+            v = ((const Unaligned16*)src)->v;
         } else {
             uint16_t e[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) e[k] = c + k < cols ? src[k] : (uint16_t)0;
+            for (int i = 0; i < 8; i++) e[i] = c + i < cols ? src[i] : (uint16_t)0;
             v = (tr_u32x4){e[0] | ((uint32_t)e[1] << 16), e[2] | ((uint32_t)e[3] << 16), e[4] | ((uint32_t)e[5] << 16),
                            e[6] | ((uint32_t)e[7] << 16)};
         }
-        *(tr_u32x4*)(out + r * pitch + c) = v;
+        if (PAD) {
+            *(tr_u32x4*)dst = v;
+        } else if (c + 8 <= cols) {
+            ((Unaligned16*)dst)->v = v;
+        } else {
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (c + i < cols) dst[i] = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
+        }
     }
 }
 
-hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream) {
-    const int64_t blocks = ((int64_t)rows * (pitch / 8) + 255) / 256;
-    hipLaunchKernelGGL(pad_columns_f16_kernel, dim3((unsigned)(blocks < 65535 * 8 ? blocks : 65535 * 8)), dim3(256), 0, stream, in, rows,
-                       cols, out, pitch);
+template <bool PAD>
+static hipError_t launch_repitch(const uint16_t* in, int rows, int cols, int in_pitch, uint16_t* out, int out_pitch, hipStream_t stream) {
+    const int64_t blocks = ((int64_t)rows * ((cols + 7) / 8) + 255) / 256;
+    hipLaunchKernelGGL(repitch_f16_kernel<PAD>, dim3((unsigned)(blocks < 65535 * 8 ? blocks : 65535 * 8)), dim3(256), 0, stream, in, rows,
+                       cols, in_pitch, out, out_pitch);
     return hipGetLastError();
+}
+hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream) {
+    return launch_repitch<true>(in, rows, cols, cols, out, pitch, stream);
+}
+hipError_t launch_cut_columns_f16(const uint16_t* in, int rows, int cols, int pitch, uint16_t* out, hipStream_t stream) {
+    return launch_repitch<false>(in, rows, cols, pitch, out, cols, stream);
 }
 
 }  // namespace spatha
