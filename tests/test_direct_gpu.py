@@ -62,6 +62,33 @@ def test_direct_kernels_bit_exact(gpu, rows, cols, N, m, v, transposed):
     assert np.array_equal(fused.cpu().numpy().view(np.uint16), want_b.view(np.uint16))
 
 
+# V = 32 beyond four tiles per CU: 17 and 18, 29 and 30, 93 and 94 k-steps at both ends of the column counts that go to 32-row tiles
+LONG_CASES = [(12288, 2720, 136, 10, 32, 24), (12288, 2560, 136, 10, 32, 16), (12288, 2880, 192, 10, 32, 24), (12288, 2880, 200, 10, 32, 16),
+              (12288, 4640, 264, 10, 32, 24), (12288, 4800, 384, 10, 32, 24), (12288, 4800, 256, 10, 32, 14), (12288, 4800, 392, 10, 32, 14),
+              (12288, 14880, 256, 10, 32, 24), (12288, 14880, 392, 10, 32, 15)]
+
+
+@pytest.mark.parametrize("rows,cols,N,m,v,kernel", LONG_CASES)
+def test_many_tiles_with_long_k_loops(gpu, rows, cols, N, m, v, kernel):
+    """The automatic choice is the kernel named last, and its result is the oracle's on rows of the first, a middle and the last V block."""
+    print("long", rows, cols, N, m, v, flush=True)
+    vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=N, integer_values=True)
+    B = np.random.default_rng(N).integers(-2, 3, size=(cols, N)).astype(np.float16)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
+    plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
+    for transposed in (False, True):
+        assert plan.kernel_name(N, int(transposed), 0) == plan.kernel_name(N, int(transposed), kernel)
+    got = plan.run(dev(B)).cpu().numpy()
+    turned = plan.run(dev(B), transposed_out=True).cpu().numpy()
+    assert np.array_equal(turned.T.view(np.uint16), got.view(np.uint16))
+    # whole matrices of one V block each: their part of the storage arrays
+    blocks, groups = rows // v, len(columns) // (rows // v)
+    for block in (0, blocks // 2 + 1, blocks - 1):
+        part = lambda a: np.ascontiguousarray(a.reshape(blocks, -1)[block])
+        want = oracle.spmm(part(vals), part(meta), part(columns), v, cols, 2, m, v, B)
+        assert np.array_equal(got[block * v:(block + 1) * v].view(np.uint16), want.view(np.uint16)), block
+
+
 def test_direct_kernel_activations(gpu):
     """GELU in the write-out: one rounding of the exact value of the rounded, biased sum (at most one step of fp16 apart)."""
     rows, cols, N, m, v = 256, 512, 136, 8, 64

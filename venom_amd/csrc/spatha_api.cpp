@@ -200,10 +200,19 @@ struct Shape {
         const int64_t t = (int64_t)(rows / 32) * ((N + 63) / 64), row_tiles = (rows + 63) / 64;
         if (t <= (S > 10 ? 4 : 3) * cus) return true;
         if (staged) return false;
+        if (S > 16 && direct32_long()) return true;
         const int64_t at_once = half_pairs() ? 2 * cus : cus, width = half_pairs() ? 128 : 256;
         const int64_t rounds = (row_tiles * ((N + width - 1) / width) + at_once - 1) / at_once;
         return rounds == 2 && (half_pairs() ? t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20) : t <= 8 * cus);
     }
+    // The same kernel at any number of tiles, by the columns of 64 that its tiles pay for against the 128 or 256 of the gathered ones
+    // (12288 .. 49152 x 12288 and 12288 x 49152, m = 10 .. 40, both layouts): up to 192 columns 0.97-1.09x on 49152 rows, 1.13-1.34x on the
+    // others; 257 .. 384 from 29 k-steps on, where two 256-wide tiles stand against it, 0.98-1.39x (fewer k-steps, pairs of 128-wide tiles:
+    // 0.7-1.3x); 193 .. 256 only where no 256-wide tile fits any more (half_wide; 1.39-1.85x, below that 0.8-1.06x).  More columns
+    // 0.5-1.1x and as often behind as ahead.
+    bool direct32_long() const { return N <= 192 || (!half_pairs() && N > 256 && N <= 384) || (!half_wide() && N <= 256); }
+    // V % 64 != 0: two stages of a 64 x 256 gathered tile (137 KB) and the row table fit the LDS of a CU up to 92 k-steps
+    bool half_wide() const { return S <= 92; }
     // 64 x 256 tiles: many tiles of few k-steps, m >= 32, row-major
     bool short_k_many() const { return m >= 32 && !transposed && tiles(64, 256) >= 2048 && S <= 8; }
 };
@@ -238,9 +247,10 @@ const Rule kRules[] = {
     // of them fits a CU, they trail by 1.2-1.6x (12288 x 12288 x 2048 at 32:2:16, 48 k-steps: 538 against 336 us)
     {V_HALF, spatha::SPMM_VARIANT_H64x128_S2, [](const Shape& s) { return s.half_pairs(); }},
     {V_HALF, spatha::SPMM_VARIANT_H64x256_S2, [](const Shape& s) { return s.N > 128; }},
-    // (three stages of 128 leave one workgroup of four waves per CU)
+    // one workgroup a CU in any case: three stages of 128 lead two by 1.1-1.4x (12288 x 49152 x 1040 at 32:2:16, 192 k-steps: 1189
+    // against 1634 us; 512 columns 471 against 538) as long as the row table leaves room for them
+    {V_HALF, spatha::SPMM_VARIANT_H64x128_S3, [](const Shape& s) { return !s.half_wide(); }},
     {V_HALF, spatha::SPMM_VARIANT_H64x128_S2, [](const Shape&) { return true; }},
-    {V_HALF, spatha::SPMM_VARIANT_H64x128_S3, [](const Shape&) { return true; }},
 
     // -- unified 512 x 128 tiles --
     // m <= 8, two phase groups: 3-13 % ahead of the dense-staged 256 x 128 tiles when its tiles fill whole rounds of the CUs
