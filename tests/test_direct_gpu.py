@@ -62,10 +62,17 @@ def test_direct_kernels_bit_exact(gpu, rows, cols, N, m, v, transposed):
     assert np.array_equal(fused.cpu().numpy().view(np.uint16), want_b.view(np.uint16))
 
 
-# V = 32 beyond four tiles per CU: 17 and 18, 29 and 30, 93 and 94 k-steps at both ends of the column counts that go to 32-row tiles
+# (the kernel named last is the automatic choice)  V = 32 beyond four tiles per CU: 16 and 17, 29, 30 and 93 k-steps at both ends of the column counts that go to 32-row tiles
 LONG_CASES = [(12288, 2720, 136, 10, 32, 24), (12288, 2560, 136, 10, 32, 16), (12288, 2880, 192, 10, 32, 24), (12288, 2880, 200, 10, 32, 16),
               (12288, 4640, 264, 10, 32, 24), (12288, 4800, 384, 10, 32, 24), (12288, 4800, 256, 10, 32, 14), (12288, 4800, 392, 10, 32, 14),
-              (12288, 14880, 256, 10, 32, 24), (12288, 14880, 392, 10, 32, 15)]
+              (12288, 14880, 256, 10, 32, 24), (12288, 14880, 392, 10, 32, 15),
+              # one step into a second round of 64 x 128 tiles, B beyond 4 MB: 8 3/4 tiles per CU and more; four k-steps
+              (1280, 4096, 3528, 16, 32, 24), (1280, 4096, 3592, 16, 32, 16), (1280, 2048, 3528, 32, 32, 16),
+              # V = 64: 16 k-steps and 15, 32
+              (36864, 4096, 72, 16, 64, 23), (36864, 3840, 72, 16, 64, 4), (36864, 8192, 72, 16, 64, 23),
+              # V = 128: 32, 24 and 23, 96, 48 and 26 k-steps (kernel 20 goes with row-major output, 6 with transposed)
+              (12288, 8192, 640, 16, 128, 20), (24576, 6144, 264, 16, 128, 22), (24576, 5888, 264, 16, 128, 20),
+              (12288, 12288, 640, 8, 128, 12), (36864, 4096, 1024, 10, 128, 22)]
 
 
 @pytest.mark.parametrize("rows,cols,N,m,v,kernel", LONG_CASES)
@@ -77,7 +84,8 @@ def test_many_tiles_with_long_k_loops(gpu, rows, cols, N, m, v, kernel):
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).to(gpu)
     plan = spatha.SpmmPlan(dev(vals), dev(meta), dev(columns), rows, cols, 2, m, v)
     for transposed in (False, True):
-        assert plan.kernel_name(N, int(transposed), 0) == plan.kernel_name(N, int(transposed), kernel)
+        named = 6 if kernel == 20 and transposed else kernel
+        assert plan.kernel_name(N, int(transposed), 0) == plan.kernel_name(N, int(transposed), named)
     got = plan.run(dev(B)).cpu().numpy()
     turned = plan.run(dev(B), transposed_out=True).cpu().numpy()
     assert np.array_equal(turned.T.view(np.uint16), got.view(np.uint16))

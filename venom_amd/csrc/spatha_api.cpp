@@ -191,9 +191,10 @@ struct Shape {
     bool half_pairs() const { return S <= 28; }
     // V % 64 != 0: direct 32 x 64 tiles always up to 32 columns and, where nothing is dense-staged, up to 128 (2-5x ahead of the
     // gathered tiles); above that up to three tiles per CU (1.08-2.1x; at four 0.98-1.0x), with more than ten k-steps up to four
-    // (1.10-1.16x; at eight 0.8-0.93x).  Where the replaced kernel is one step into a second round, also as long as B fits an XCD's L2
-    // (4096 x 1024 x 1040 at 32:2:10 14.0 against 16.8 us; 1280 x 5120 x 4096 at 32:2:16, B 42 MB, 37 against 43 but at other
-    // shapes 10 % behind).
+    // (1.10-1.16x; at eight 0.8-0.93x).  Where the replaced kernel is one step into a second round (1280 .. 12288 x 1024 .. 12288,
+    // m = 10, 16, 32, both layouts, 990 products): up to 8 3/4 tiles per CU from five k-steps on (1.2x in the mean, none of 176
+    // products more than 3 % behind; 4096 x 4096 x 1040 at 32:2:16 31.1 against 35.9 us), up to eleven as long as B fits an XCD's L2
+    // (1.08-1.14x; with a larger B 0.84-1.1x); fewer k-steps 0.98-1.09x.
     bool direct32() const {
         const bool staged = m <= 8 && rows % 256 == 0 && (tiles(256, 128) >= 160 || S >= 16);
         if (N <= (staged ? 32 : 128)) return true;
@@ -203,7 +204,9 @@ struct Shape {
         if (S > 16 && direct32_long()) return true;
         const int64_t at_once = half_pairs() ? 2 * cus : cus, width = half_pairs() ? 128 : 256;
         const int64_t rounds = (row_tiles * ((N + width - 1) / width) + at_once - 1) / at_once;
-        return rounds == 2 && (half_pairs() ? t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20) : t <= 8 * cus);
+        if (rounds != 2) return false;
+        if (!half_pairs()) return t <= 8 * cus;
+        return (S > 4 && t * 4 <= 35 * cus) || (t <= 11 * cus && (int64_t)cols * N * 2 <= (4 << 20));
     }
     // The same kernel at any number of tiles, by the columns of 64 that its tiles pay for against the 128 or 256 of the gathered ones
     // (12288 .. 49152 x 12288 and 12288 x 49152, m = 10 .. 40, both layouts): up to 192 columns 0.97-1.09x on 49152 rows, 1.13-1.34x on the
@@ -213,6 +216,15 @@ struct Shape {
     bool direct32_long() const { return N <= 192 || (!half_pairs() && N > 256 && N <= 384) || (!half_wide() && N <= 256); }
     // V % 64 != 0: two stages of a 64 x 256 gathered tile (137 KB) and the row table fit the LDS of a CU up to 92 k-steps
     bool half_wide() const { return S <= 92; }
+    // dense-staged 256 x 128 tiles: the form in two phase groups leads the eight-consumer form row-major by 2-5 % up to 768 tiles of 32
+    // k-steps or fewer; with more of them by 5-12 % at m = 7 and 8 whatever the count (12288 x 12288 x 640 at 128:2:8 70 against 84 us) and
+    // by 1-7 % at m = 4, transposed by 3-11 % at m = 7 and 8 (level in one round of 33 .. 64 k-steps; m = 4: level, up to 14 % behind).
+    // It has no fused write-out.
+    bool two_phases() const {
+        if (fused) return false;
+        if (S <= 32) return !transposed && tiles(256, 128) <= 768;
+        return !transposed || (m > 5 && (S > 64 || tiles(256, 128) > cus));
+    }
     // 64 x 256 tiles: many tiles of few k-steps, m >= 32, row-major
     bool short_k_many() const { return m >= 32 && !transposed && tiles(64, 256) >= 2048 && S <= 8; }
 };
@@ -283,16 +295,15 @@ const Rule kRules[] = {
     // k-steps, 45 against 65 us on 128 x 128 tiles; 12288 x 12288 x 512 at 2:4 115 against 127 us on 128 x 256 tiles)
     // (from 160 tiles on, as row-major: with fewer - 1024 x 4096 x 2048 / 4096, 1280 x 5120 x 2048: 64 .. 128 tiles - the
     // gathered 128 x 128 tiles are 13-35 % ahead)
+    {V_128, spatha::SPMM_VARIANT_DS256x128_S3_PP,
+     [](const Shape& s) { return s.transposed && s.two_phases() && s.m <= 8 && s.S <= 40 && s.tiles(256, 128) >= 160; }},
     {V_128, spatha::SPMM_VARIANT_DS256x128_S3_C8,
      [](const Shape& s) { return s.transposed && s.m <= 8 && (s.S <= 40 || s.m <= 5) && s.tiles(256, 128) >= 160; }},
     // row-major, m <= 8: dense staging leads the gathered tiles by 5-35 % as soon as its 256 x 128 tiles fill three quarters
-    // of the CUs (BERT layer shapes, N = 2048 .. 16384; from 160 tiles on the GPT-2-large ones).  Up to 768 tiles the form in
-    // two phase groups leads the eight-consumer form by 2-5 %; it has no fused write-out, and falls behind on long k-loops
-    // (12288 x 12288 x 2048 at 64:2:8, 96 k-steps: 255 us against 239 us)
+    // of the CUs (BERT layer shapes, N = 2048 .. 16384; from 160 tiles on the GPT-2-large ones)
     {V_128, spatha::SPMM_VARIANT_DS256x128_S3_PP,
      [](const Shape& s) {
-         const int64_t t = s.tiles(256, 128);
-         return !s.transposed && !s.fused && s.m <= 8 && s.rows % 256 == 0 && t >= 160 && t <= 768 && s.S <= 32;
+         return !s.transposed && s.two_phases() && s.m <= 8 && s.rows % 256 == 0 && s.tiles(256, 128) >= 160 && (s.S <= 64 || s.m <= 5);
      }},
     {V_128, spatha::SPMM_VARIANT_DS256x128_S3_C8,
      [](const Shape& s) {
@@ -345,8 +356,7 @@ const Rule kRules[] = {
 
     // -- V a multiple of 64 only --
     // m <= 8: staging the dense B rows once for four 64-row blocks halves the L2 -> LDS traffic; the two forms as above
-    {V_64, spatha::SPMM_VARIANT_DS256x128_S3_PP,
-     [](const Shape& s) { return !s.transposed && !s.fused && s.tiles(256, 128) <= 768 && s.S <= 32; }},
+    {V_64, spatha::SPMM_VARIANT_DS256x128_S3_PP, [](const Shape& s) { return s.two_phases(); }},
     {V_64, spatha::SPMM_VARIANT_DS256x128_S3_C8, [](const Shape&) { return true; }},
     // m > 8, row-major, two or three k-steps per tile and six rounds or more of 64 x 256 tiles: the producer/consumer kernel
     // with store waves, 9-10 % ahead of the plain one and of the per-tile pipeline (4096 x 1024 x 16384 at 64:2:32, 3072 x
@@ -381,6 +391,83 @@ const Rule kRules[] = {
     {V_64, spatha::SPMM_VARIANT_64x256, [](const Shape&) { return true; }},
 };
 
+// Long k-loops: what a launch takes is rounds of its tiles over the CUs times what a k-step of one such round takes, whatever the
+// matrix.  us a k-step, medians over 12288 .. 49152 x 12288, 12288 x 49152, 4096 x 16384, 8192 x 8192, 16384 x 4096, 20480 x 5120 and
+// 24576 x 8192, m = 4 .. 40, 72 .. 4096 columns, both layouts (the middle 80 % of products within 10 %, the direct tiles' 20):
+//   V % 128 == 0: 128 x 128 tiles 0.45, 128 x 256 0.69, a tile and a half 0.92 (0.975 where its last column tile has nothing for the
+//     second half; 1.02 in several rounds: 0.91 in short bursts, but its sixteen waves draw the most power and hold the clock lowest
+//     when launches follow each other for long), dense-staged 256 x 128 0.65 .. 0.78 and 512 x 128 0.96 .. 1.1 with m;
+//   V % 64 == 0 only, m > 8: 64 x 256 tiles 0.68 (0.64 from 64 k-steps on), in pairs of workgroups 0.61; direct 64 x 64 tiles, several on
+//     a CU, 0.27 for as many as CUs without rounding up.
+// 0: not priced.
+float round_price(const Shape& s, int variant) {
+    using namespace spatha;
+    const int64_t grid = (s.cus / 8) * 8;
+    auto rounds = [&](int64_t tiles) { return (float)((tiles + grid - 1) / grid); };
+    switch (variant) {
+        case SPMM_VARIANT_W128x128_S3: case SPMM_VARIANT_WS128x128_S3: return 0.45f * rounds(s.tiles(128, 128));
+        case SPMM_VARIANT_W128x256_S3: case SPMM_VARIANT_T128x256_S3: return 0.69f * rounds(s.tiles(128, 256));
+        case SPMM_VARIANT_OH192x256: {
+            const int64_t per_column = (2 * (int64_t)(s.rows / 128) + 2) / 3, tn = (s.N + 255) / 256;
+            const bool whole = s.N - (tn - 1) * 256 > 128;
+            const float n = rounds(per_column * tn);
+            return (n > 1.f ? 1.02f : whole ? 0.92f : 0.975f) * n;
+        }
+        case SPMM_VARIANT_DS256x128_S3_PP: case SPMM_VARIANT_DS256x128_S3_C8:
+            return (s.m <= 5 ? 0.65f : s.m <= 7 ? 0.72f : 0.78f) * rounds(s.tiles(256, 128));
+        case SPMM_VARIANT_UP512x128_S3: return (s.m <= 5 ? 0.96f : s.m <= 7 ? 1.06f : 1.1f) * rounds(s.tiles(512, 128));
+        case SPMM_VARIANT_P64x256_S2: return (s.S <= 28 ? 0.61f : 0.89f) * rounds(s.tiles(64, 256));
+        case SPMM_VARIANT_R64x256_S3: return (s.S < 64 ? 0.68f : 0.64f) * rounds(s.tiles(64, 256));
+        case SPMM_VARIANT_DIRECT64: return 0.27f * (float)s.tiles(64, 64) / (float)grid;
+        default: return 0.f;
+    }
+}
+
+int uneven_rest_rows(const spatha_spmm_plan* plan, int N, int requested, int chosen, bool fused);
+
+// The kernel the rules chose, or one whose rounds promise clearly less.  (Three sets of operands in turn, launches following each other for
+// 40 ms a side: in shorter runs the clock is higher and flatters the kernels that draw the most power.)
+//   V % 128 == 0, 24 k-steps or more, 10 %: 289 of 2436 products of the sizes above change, 1.18x faster in the mean, none of 146 timed
+//     more than 2 % behind (12288 x 12288 x 640: at 128:2:16 two rounds of 128 x 256 tiles 65 us, of 128 x 128 44; at 128:2:8 120 us,
+//     one round of dense-staged tiles 70).  Not where the launch is half a round or less: runs that bring a workspace split those
+//     k-loops.
+//   V % 64 == 0 only, m > 8, 16 k-steps or more: direct tiles, 102 of 1722 change, 1.27x faster in the mean, two of 83 timed 3-4 % behind
+//     (36864 x 12288 x 72 at 64:2:16 90 -> 52 us, 12288 x 12288 x 264 68 -> 48).  20 % where pairs of workgroups share a CU, 8 %
+//     elsewhere.  m <= 8: no price tells the dense-staged kernels apart from the gathered ones there, half of what would change is slower.
+// With fewer k-steps a tile's start and write-out weigh in and the rules above are as good.
+int by_rounds(const spatha_spmm_plan* plan, const Shape& s, int chosen) {
+    using namespace spatha;
+    const int64_t grid = (s.cus / 8) * 8;
+    if (s.cus < 8 || plan->half_tiles) return chosen;
+    float best = round_price(s, chosen);
+    if (best == 0.f) return chosen;
+    auto offer = [&](int variant) {
+        const float price = round_price(s, variant);
+        if (price < best && variant_ok(plan, s.N, variant, s.fused)) {
+            best = price;
+            chosen = variant;
+        }
+    };
+    // (dense-staged and unified tiles go by m alone, and to rows their tiles divide, which variant_ok holds them to)
+    if (s.v % 128 == 0) {
+        if (s.S < 24 || s.tiles(128, chosen == SPMM_VARIANT_T128x256_S3 ? 256 : 128) * 2 <= grid) return chosen;
+        if (uneven_rest_rows(plan, s.N, SPMM_VARIANT_AUTO, chosen, s.fused))
+            best = 0.69f * (float)(s.tiles(128, 256) / grid) + 0.5f;      // whole rounds and one of 128 x 128 tiles behind them
+        best *= 0.9f;
+        offer(s.transposed ? SPMM_VARIANT_W128x128_S3 : SPMM_VARIANT_WS128x128_S3);
+        offer(SPMM_VARIANT_T128x256_S3);
+        offer(SPMM_VARIANT_OH192x256);
+        if (s.m <= 8) {
+            offer(s.two_phases() ? SPMM_VARIANT_DS256x128_S3_PP : SPMM_VARIANT_DS256x128_S3_C8);
+            offer(SPMM_VARIANT_UP512x128_S3);
+        }
+    } else if (s.m > 8 && s.S >= 16 && (chosen == SPMM_VARIANT_P64x256_S2 || chosen == SPMM_VARIANT_R64x256_S3)) {
+        best *= chosen == SPMM_VARIANT_P64x256_S2 ? 0.8f : 0.92f;
+        offer(SPMM_VARIANT_DIRECT64);
+    }
+    return chosen;
+}
+
 int pick_variant(const spatha_spmm_plan* plan, int N, int variant, bool fused = false, int out_layout = SPATHA_OUT_ROW_MAJOR) {
     if (variant != spatha::SPMM_VARIANT_AUTO)
         return variant_ok(plan, N, variant, fused) ? variant : -1;
@@ -391,7 +478,7 @@ int pick_variant(const spatha_spmm_plan* plan, int N, int variant, bool fused = 
     s.transposed = out_layout == SPATHA_OUT_TRANSPOSED;
     const unsigned v_class = plan->half_tiles ? V_HALF : s.v % 128 == 0 ? V_128 : s.v % 64 == 0 ? V_64 : 0u;
     for (const Rule& r : kRules)
-        if ((r.v_classes & v_class) && r.when(s) && variant_ok(plan, N, r.variant, fused)) return r.variant;
+        if ((r.v_classes & v_class) && r.when(s) && variant_ok(plan, N, r.variant, fused)) return by_rounds(plan, s, r.variant);
     return -1;
 }
 
