@@ -96,6 +96,14 @@ __device__ __forceinline__ void store_c16(uint16_t* dst, u32x4 v, bool stream) {
 #endif
 }
 
+// Whether C leaves by non-temporal stores, read where the kernel starts: left to the compiler it is loaded in front of the first store,
+// and every tile's write-out begins with that load's latency.
+__device__ __forceinline__ bool streams(const SpmmParams& p) {
+    int s = p.stream_out;
+    asm volatile("" : "+s"(s));
+    return s != 0;
+}
+
 // where a write-out goes and how
 struct OutC {
     uint16_t* at;
