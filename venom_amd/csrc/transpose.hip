@@ -79,16 +79,17 @@ struct __attribute__((packed, aligned(2))) Unaligned16 {
 // thread takes one 16-byte piece, and the ragged side goes by one access at whatever alignment its row has.  Bound by launch and
 // latency at most sizes: 1280 x 1037 2.85 us padded, 3.1 with two rows a thread, of which an empty launch is 2.4; cutting 3072 x 2785
 // 7.5 us, 9.6 as a strided copy.
-template <bool PAD>
+// Index counts pieces: 32 bits wherever they suffice, a 64-bit division by a variable is a subroutine.
+template <bool PAD, typename Index>
 __global__ __launch_bounds__(256) void repitch_f16_kernel(const uint16_t* __restrict__ in, int rows, int cols, int in_pitch,
                                                           uint16_t* __restrict__ out, int out_pitch) {
     const uint32_t pieces = (uint32_t)(cols + 7) >> 3;
-    const uint64_t total = (uint64_t)rows * pieces;
-    for (uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x; id < total; id += (uint64_t)gridDim.x * 256) {
-        const uint64_t r = total >> 32 ? id / pieces : (uint32_t)id / pieces;
-        const int c = (int)(id - r * pieces) * 8;
-        const uint16_t* src = in + r * in_pitch + c;
-        uint16_t* dst = out + r * out_pitch + c;
+    const Index total = (Index)rows * pieces;
+    for (Index id = (Index)blockIdx.x * 256 + threadIdx.x; id < total; id += (Index)gridDim.x * 256) {
+        const uint32_t r = (uint32_t)(id / pieces);
+        const int c = (int)(id - (Index)r * pieces) * 8;
+        const uint16_t* src = in + (int64_t)r * in_pitch + c;
+        uint16_t* dst = out + (int64_t)r * out_pitch + c;
         tr_u32x4 v;
         if (!PAD) {
             v = *(const tr_u32x4*)src;
@@ -116,9 +117,11 @@ __global__ __launch_bounds__(256) void repitch_f16_kernel(const uint16_t* __rest
 
 template <bool PAD>
 static hipError_t launch_repitch(const uint16_t* in, int rows, int cols, int in_pitch, uint16_t* out, int out_pitch, hipStream_t stream) {
-    const int64_t blocks = ((int64_t)rows * ((cols + 7) / 8) + 255) / 256;
-    hipLaunchKernelGGL(repitch_f16_kernel<PAD>, dim3((unsigned)(blocks < 65535 * 8 ? blocks : 65535 * 8)), dim3(256), 0, stream, in, rows,
-                       cols, in_pitch, out, out_pitch);
+    const int64_t pieces = (int64_t)rows * ((cols + 7) / 8), blocks = (pieces + 255) / 256;
+    const unsigned grid = (unsigned)(blocks < 65535 * 8 ? blocks : 65535 * 8);
+    // (a thread's next piece must not wrap either: a stride of 2^27 pieces at most below 2^31)
+    auto kern = pieces < (1ll << 31) ? repitch_f16_kernel<PAD, uint32_t> : repitch_f16_kernel<PAD, uint64_t>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, in, rows, cols, in_pitch, out, out_pitch);
     return hipGetLastError();
 }
 hipError_t launch_pad_columns_f16(const uint16_t* in, int rows, int cols, uint16_t* out, int pitch, hipStream_t stream) {
