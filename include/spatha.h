@@ -240,7 +240,7 @@ int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, 
                            int out_layout, int activation, int fused, void* stream);
 
 /* spatha_spmm_run_ws (workspace NULL, 0 where none is wanted) for a result that the caller's next operation reads: it is written so that
- * it stays in the memory-side cache.  The other entry points let results of 48 MB and more pass that cache by, which is faster
+ * it stays in the memory-side cache.  The other entry points let results of 96 MB and more pass that cache by, which is faster
  * where other data goes through it before the result is read. */
 int spatha_spmm_run_layer(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                           int out_layout, int activation, void* workspace_dev, size_t workspace_bytes, void* stream);

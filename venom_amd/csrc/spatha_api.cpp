@@ -557,14 +557,14 @@ bool split_choice(const spatha_spmm_plan* plan, int N, int requested, int chosen
     return true;
 }
 
-// Does C leave by non-temporal stores, past the 256 MB memory-side cache?  From 48 MB on, unless the caller says that it is read right
+// Does C leave by non-temporal stores, past the 256 MB memory-side cache?  From 96 MB on, unless the caller says that it is read right
 // behind this call.  With three sets of operands and results in turn (28 shapes, both layouts): results of 134 MB and more 1.14-1.7x
-// ahead (4096 x 1024 x 16384 at 64:2:8 75.3 -> 61.3 us row-major, 67 -> 57.7 transposed, at 128:2:32 54.1 -> 31.9; x 32768 at
-// 64:2:8 164.6 -> 119.9), of 50 to 67 MB 0.98-1.04x, of 33 MB level, smaller ones level or up to 4 % behind; where all buffers stay in
-// the cache level.  A chain of layers reads each result back from that cache: with such stores in all of them the two encoder layers of
-// BERT-large at 32 x 512 tokens took 695 us, 681 without.
+// ahead (4096 x 1024 x 16384 at 64:2:8 73.3 -> 56.7 us row-major, 69.9 -> 55.5 transposed, at 128:2:32 53.3 -> 31.5), of 50 to 67 MB
+// 0.98-1.04x, smaller ones level or up to 4 % behind.  On one set that stays in the cache, launches following each other for long: 134 MB
+// 56.8 -> 56.2 and 55.6 -> 55.2 us (OutC::streams), 67 MB 28.4 -> 29.3.  A chain of layers reads each result back from that cache: with
+// such stores in all of them the two encoder layers of BERT-large at 32 x 512 tokens took 695 us, 681 without.
 bool streams_out(const spatha_spmm_plan* plan, int N, bool read_next) {
-    return !read_next && (int64_t)plan->geo.rows * N * 2 >= (48ll << 20);
+    return !read_next && (int64_t)plan->geo.rows * N * 2 >= (96ll << 20);
 }
 }  // namespace
 

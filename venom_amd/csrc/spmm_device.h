@@ -109,6 +109,11 @@ struct OutC {
     uint16_t* at;
     bool stream;
     __device__ __forceinline__ explicit OutC(const SpmmParams& p) : at(p.C), stream(p.stream_out != 0) {}
+    // Three of four stores of a block, where a write-out knows its store's number i: the quarter left to the memory-side cache finds room
+    // there, and writing it to memory is spared where the next launch overwrites it.  4096 x 1024 x 16384 at 64:2:8, launches following
+    // each other for long, one set of operands / three in turn: 57.0 / 57.3 us; all of them non-temporal 59.6 / 59.8 (at the power limit
+    // writes to memory cost clock), every second 57.1 / 72.7, none 57.0 / 73.3.
+    __device__ __forceinline__ bool streams(int i) const { return stream && (i & 3) != 0; }
 };
 
 // "Dynamic LDS limit raised" flags, one per (kernel, device): the attribute is a per-device property of a kernel.
@@ -750,7 +755,7 @@ __device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[
             v.y = (uint32_t)(uint16_t)lo[k][2] | ((uint32_t)(uint16_t)lo[k][3] << 16);
             v.z = (uint32_t)(uint16_t)hi[k][0] | ((uint32_t)(uint16_t)hi[k][1] << 16);
             v.w = (uint32_t)(uint16_t)hi[k][2] | ((uint32_t)(uint16_t)hi[k][3] << 16);
-            if (live) store_c16<true>(C.at + (row0 + row) * N + out_col, v, C.stream);
+            if (live) store_c16<true>(C.at + (row0 + row) * N + out_col, v, C.streams(k));
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -790,7 +795,7 @@ __device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&ac
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int col = col0 + (grp * 2 + (k >> 1)) * 16 + (k & 1) * 8 + rn;
-            if (col < N && stores_on) store_c16<true>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v[k], C.stream);
+            if (col < N && stores_on) store_c16<true>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v[k], C.streams(k));
         }
     }
     __builtin_amdgcn_wave_barrier();
