@@ -1,0 +1,109 @@
+"""Which calls the fused embedding and attention modules take, and which they leave to the stock modules: hooks, replaced and
+subclassed parts, operands of other shapes and places.  Runs on the CPU with a stand-in for the library's kernels; what the kernels
+compute is in test_embedding_gpu.py and test_attention_gpu.py."""
+import types
+
+import pytest
+import torch
+
+from venom_amd import bert, spatha
+
+TAKEN = 7.0          # what the stand-in answers
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The calls that reach the library."""
+    calls = []
+
+    def embed_layernorm(ids, *args):
+        calls.append(args)
+        return torch.full((*ids.shape, 64), TAKEN), None
+
+    have = {"embed_layernorm": embed_layernorm}
+    monkeypatch.setattr(spatha, "_extension", lambda: types.SimpleNamespace(**have))
+    monkeypatch.setattr(spatha, "_native", have.get)
+    return calls
+
+
+def make_embeddings():
+    from transformers.models.bert.modeling_bert import BertConfig, BertEmbeddings
+
+    torch.manual_seed(0)
+    return BertEmbeddings(BertConfig(hidden_size=64, num_hidden_layers=1, num_attention_heads=1, intermediate_size=64, vocab_size=50)).eval()
+
+
+def fused_embeddings():
+    holder = torch.nn.ModuleDict({"embeddings": make_embeddings()})
+    return bert.fuse_add_layernorm(holder)["embeddings"]
+
+
+class DoubledNorm(torch.nn.LayerNorm):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+class ScaledNorm(torch.nn.Module):
+    """Another norm with a LayerNorm's attributes."""
+
+    def __init__(self, like):
+        super().__init__()
+        self.weight, self.bias, self.eps = like.weight, like.bias, like.eps
+
+    def forward(self, x):
+        return x * self.weight
+
+
+def doubled(module, args, out):
+    return 2 * out
+
+
+def change_nothing(e):
+    pass
+
+
+def own_forward(e):
+    e.LayerNorm.forward = lambda x: 3 * x
+
+
+def subclassed(e):
+    norm = DoubledNorm(64)
+    norm.load_state_dict(e.LayerNorm.state_dict())
+    e.LayerNorm = norm
+
+
+def live_dropout(e):
+    torch.manual_seed(5)
+    e.dropout.train()
+
+
+CHANGES = [lambda e: e.LayerNorm.register_forward_hook(doubled), lambda e: e.LayerNorm.register_forward_pre_hook(lambda m, a: (2 * a[0] + 1,)),
+           lambda e: e.dropout.register_forward_hook(doubled), lambda e: e.dropout.register_forward_pre_hook(lambda m, a: (2 * a[0],)),
+           lambda e: e.word_embeddings.register_forward_hook(doubled), own_forward, subclassed,
+           lambda e: setattr(e, "LayerNorm", ScaledNorm(e.LayerNorm)), lambda e: setattr(e, "dropout", torch.nn.Tanh()), live_dropout]
+
+
+@pytest.mark.parametrize("change", [change_nothing] + CHANGES)
+def test_embedding_parts_that_do_more_than_the_kernel_run(kernels, change):
+    stock, fused = make_embeddings(), fused_embeddings()
+    ids = torch.arange(12).reshape(2, 6)
+    with torch.no_grad():
+        change(stock)
+        want = stock(input_ids=ids)
+        change(fused)
+        got = fused(input_ids=ids)
+    if change is change_nothing:
+        assert len(kernels) == 1 and bool((got == TAKEN).all())
+    else:
+        assert not kernels and torch.equal(got, want)
+
+
+def test_a_hook_on_every_module_sees_the_embeddings_norm(kernels):
+    fused, seen = fused_embeddings(), []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, o: seen.append(type(m)))
+    try:
+        with torch.no_grad():
+            fused(input_ids=torch.arange(6)[None])
+    finally:
+        handle.remove()
+    assert not kernels and torch.nn.LayerNorm in seen

@@ -193,6 +193,11 @@ def merge_qkv(model):
     return model
 
 
+def _runs_as(module, cls):
+    """Does a call of `module` run the forward of `cls` and nothing else: no subclass, no hook, no forward of its own?"""
+    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+
+
 def _fused_self_attention():
     """The class that `fuse_add_layernorm(feature_major=True)` gives to a BertSelfAttention whose projections are merged: the same
     module with the library's attention kernel where that applies (`FusedSelfAttention` of this module; made on first use, so that
@@ -255,9 +260,12 @@ def _fused_embeddings():
             tables = self.word_embeddings, self.token_type_embeddings, self.position_embeddings
             ln = self.LayerNorm
             types = token_type_ids if token_type_ids is not None else getattr(self, "token_type_ids", None)
-            if types is None or type(input_ids) is not torch.Tensor or ln.weight is None or ln.bias is None \
+            if types is None or type(input_ids) is not torch.Tensor \
                     or getattr(self, "position_embedding_type", "absolute") != "absolute" \
-                    or any(type(t) is not torch.nn.Embedding or t.max_norm is not None or t._forward_hooks or t._forward_pre_hooks for t in tables) \
+                    or not _runs_as(ln, torch.nn.LayerNorm) or ln.weight is None or ln.bias is None or ln.weight.dim() != 1 \
+                    or not _runs_as(self.dropout, torch.nn.Dropout) or self.dropout.training \
+                    or any(not _runs_as(t, torch.nn.Embedding) or t.max_norm is not None for t in tables) \
+                    or torch.nn.modules.module._has_any_global_hook() \
                     or torch.is_grad_enabled() and any(t.weight.requires_grad for t in tables + (ln,)):
                 return None
             return spatha._extension().embed_layernorm(input_ids, types, self.position_ids, *(t.weight for t in tables), ln.weight, ln.bias,
