@@ -260,7 +260,9 @@ def _fused_embeddings():
             tables = self.word_embeddings, self.token_type_embeddings, self.position_embeddings
             ln = self.LayerNorm
             types = token_type_ids if token_type_ids is not None else getattr(self, "token_type_ids", None)
+            # (the model's own row of token types covers its longest sequence and is cut; a caller's has the ids' length)
             if types is None or type(input_ids) is not torch.Tensor \
+                    or token_type_ids is not None and token_type_ids.shape[-1:] != input_ids.shape[-1:] \
                     or getattr(self, "position_embedding_type", "absolute") != "absolute" \
                     or not _runs_as(ln, torch.nn.LayerNorm) or ln.weight is None or ln.bias is None or ln.weight.dim() != 1 \
                     or not _runs_as(self.dropout, torch.nn.Dropout) or self.dropout.training \
