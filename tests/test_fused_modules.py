@@ -129,3 +129,30 @@ def test_token_types_of_a_caller_have_the_ids_length(kernels, batch, seq, types,
     assert bool(kernels) == taken
     if not taken:
         assert got == want if isinstance(want, str) else torch.equal(got, want)
+
+
+def test_the_embedding_needs_no_extension(monkeypatch):
+    """A dense model, on the CPU here, asks for none: the stock forward answers where there is no extension and where there is one."""
+    import sys
+
+    import venom_amd
+
+    ids = torch.arange(12).reshape(2, 6)
+    with torch.no_grad():
+        want = make_embeddings()(input_ids=ids)
+        assert torch.equal(fused_embeddings()(input_ids=ids), want)
+        monkeypatch.setitem(sys.modules, "venom_amd._spatha_torch", None)       # importing it raises ImportError
+        monkeypatch.delattr(venom_amd, "_spatha_torch", raising=False)
+        monkeypatch.setattr(spatha, "_loaded_extension", None)
+        monkeypatch.setattr(spatha, "_extension_absent", False)
+        assert torch.equal(fused_embeddings()(input_ids=ids), want)
+
+
+def test_the_embedding_goes_with_the_default_build_only(monkeypatch):
+    """Where SPATHA_LIBRARY names another build, the extension, which is linked to the default one, is not asked."""
+    from venom_amd import _lib
+
+    monkeypatch.setattr(_lib, "IS_DEFAULT_BUILD", False)
+    monkeypatch.setattr(spatha, "_extension", lambda: pytest.fail("the extension was asked"))
+    with torch.no_grad():
+        fused_embeddings()(input_ids=torch.arange(6)[None])

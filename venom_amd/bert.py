@@ -270,8 +270,9 @@ def _fused_embeddings():
                     or torch.nn.modules.module._has_any_global_hook() \
                     or torch.is_grad_enabled() and any(t.weight.requires_grad for t in tables + (ln,)):
                 return None
-            return spatha._extension().embed_layernorm(input_ids, types, self.position_ids, *(t.weight for t in tables), ln.weight, ln.bias,
-                                                       ln.eps, self.feature_major)
+            native = spatha._native("embed_layernorm")
+            return native and native(input_ids, types, self.position_ids, *(t.weight for t in tables), ln.weight, ln.bias, ln.eps,
+                                     self.feature_major)
 
     FusedEmbeddings.__qualname__ = "FusedEmbeddings"
     globals()["FusedEmbeddings"] = FusedEmbeddings
