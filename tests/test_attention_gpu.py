@@ -89,3 +89,31 @@ def test_a_models_attention_takes_the_kernel_and_falls_back(gpu):
     v = att.value(x).float().mean(1, keepdim=True)
     assert (hooked.float() - v).abs().max() <= 4e-3       # equal scores: every token averages V
     assert torch.equal(att(x)[0], got)
+
+
+def softmax_average(qkv, batch, seq, heads, scale):
+    """`exact` with every product spelled out: an infinity or NaN meets the operands of its own query, key and feature only, and a
+    probability of exactly zero takes no part."""
+    q, k, v = (t.double().cpu().reshape(batch, seq, heads, 64).transpose(1, 2) for t in qkv.split(heads * 64, dim=1))
+    p = torch.softmax(scale * (q.unsqueeze(3) * k.unsqueeze(2)).sum(-1), -1).unsqueeze(-1)          # [batch, heads, query, key, 1]
+    terms = torch.where(p == 0, torch.zeros((), dtype=torch.float64), p * v.unsqueeze(2))
+    return terms.sum(3).transpose(1, 2).reshape(batch, seq, heads * 64)
+
+
+def same_kinds(got, want):
+    """The same infinities and NaN in the same places, and the finite entries as near as in the tests above."""
+    got, finite = got.double().cpu(), torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
+    assert (got - want)[finite].norm() <= 6e-4 * want[finite].norm()
+
+
+@pytest.mark.parametrize("seq", [1, 5, 40, 64, 65, 127, 130])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_an_infinity_in_the_last_value_reaches_its_feature_alone(gpu, seq, value):
+    """Keys behind a sequence's end have probability zero, and zero times infinity would be NaN: their values have to be zeros."""
+    gen = torch.Generator(device=gpu).manual_seed(seq)
+    qkv = torch.randn((2 * seq, 3 * 2 * 64), generator=gen, device=gpu).half()
+    qkv[seq - 1, 2 * 128 + 64 + 5] = value          # first sequence, second head, feature 5 of V
+    got = spatha._extension().attention(qkv, 2, seq, 2, 0.125)
+    same_kinds(got, softmax_average(qkv, 2, seq, 2, 0.125))

@@ -29,6 +29,9 @@ constexpr int kRowBytes = kHead * 2, kTileBytes = kKeys * kRowBytes;
 constexpr int kOutPitch = kQueries + 8;          // halfs between two features of the finished tile in LDS
 
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
+
+// values of the keys behind a sequence's end (they have probability zero, and zero times an infinity is NaN)
+__device__ const uint4 kNoValues = {0u, 0u, 0u, 0u};
 }  // namespace
 
 struct AttentionParams {
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
             const int row = wave * 16 + i * 8, key = t * kKeys + row + dma_row;
             const int64_t at = (int64_t)(key < seq ? key : seq - 1) * p.pitch + dma_piece * 8;
             dma_b128(k_base + at, dst + row * kRowBytes);
-            dma_b128(v_base + at, dst + kTileBytes + row * kRowBytes);
+            dma_b128(key < seq ? (const void*)(v_base + at) : (const void*)&kNoValues, dst + kTileBytes + row * kRowBytes);
         }
     };
     load_tile(0);
