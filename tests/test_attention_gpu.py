@@ -117,3 +117,17 @@ def test_an_infinity_in_the_last_value_reaches_its_feature_alone(gpu, seq, value
     qkv[seq - 1, 2 * 128 + 64 + 5] = value          # first sequence, second head, feature 5 of V
     got = spatha._extension().attention(qkv, 2, seq, 2, 0.125)
     same_kinds(got, softmax_average(qkv, 2, seq, 2, 0.125))
+
+
+@pytest.mark.parametrize("seq,barred", [(65, 64), (130, 64), (130, 128), (200, 70), (96, 95)])
+def test_keys_of_score_minus_infinity_take_no_part(gpu, seq, barred):
+    """Whole tiles of them ahead of the first finite score leave nothing behind; a query with nothing else is NaN, as in torch's softmax."""
+    gen = torch.Generator(device=gpu).manual_seed(seq + barred)
+    qkv = torch.randn((2 * seq, 3 * 64), generator=gen, device=gpu).half()
+    qkv[:, 3] = qkv[:, 3].abs() + 0.5             # feature 3 of every query is positive
+    qkv[:barred, 64 + 3] = float("-inf")          # the first sequence's first keys
+    qkv[seq:, 64 + 3] = float("-inf")             # every key of the second one
+    got = spatha._extension().attention(qkv, 2, seq, 1, 0.125)
+    want = softmax_average(qkv, 2, seq, 1, 0.125)
+    assert torch.isfinite(want[0]).all() and torch.isnan(want[1]).all()
+    same_kinds(got, want)

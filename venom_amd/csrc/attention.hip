@@ -95,7 +95,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
     for (int mb = 0; mb < 2; mb++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[mb][i] = 0.f;
-    float peak = -__builtin_inff(), sum = 0.f;        // of the scaled scores (in powers of two); this lane's share of the sum
+    // of the scaled scores (in powers of two; finite from the start, so that a first tile of scores -inf adds exp2(-inf) = 0); this lane's
+    // share of the sum
+    float peak = -__FLT_MAX__, sum = 0.f;
     const float c = p.scale_log2;
 
     for (int t = 0; t < tiles; t++) {
