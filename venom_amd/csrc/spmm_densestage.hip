@@ -109,8 +109,8 @@ __device__ __forceinline__ void ds_producer(const SpmmParams& p, const TileWalk&
     }
 }
 
-template <class Cfg, int OUT_LAYOUT>
-__device__ __forceinline__ void ds_consumer(const SpmmParams& p, const TileWalk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int OUT_LAYOUT, class Params>
+__device__ __forceinline__ void ds_consumer(const Params& p, const TileWalk& walk, char* smem, int wave, int lane) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
     const int S = p.S, N = p.N;
@@ -226,12 +226,12 @@ __device__ __forceinline__ void ds_consumer(const SpmmParams& p, const TileWalk&
             if (pre) fused_bias_act(acc[0], p.bias, (int64_t)cm0 + ib * 16, p.act);
             if (!SPATHA_KNOB(4)) {
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                    store_block_transposed_slab4(acc[0], stg, OutC(p), p.fuse ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
+                    store_block_transposed_slab4(acc[0], stg, out_of(p), p.fuse ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
                                                  lane, !SPATHA_KNOB(2));
                 else if (p.fuse && !pre && p.bias)
-                    store_block_row_major_tr4<true>(acc[0], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), p.bias);
+                    store_block_row_major_tr4<true>(acc[0], stg, out_of(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), p.bias);
                 else
-                    store_block_row_major_tr4<false>(acc[0], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
+                    store_block_row_major_tr4<false>(acc[0], stg, out_of(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
             }
         } else
 #pragma unroll
@@ -241,16 +241,16 @@ __device__ __forceinline__ void ds_consumer(const SpmmParams& p, const TileWalk&
             if (pre) fused_bias_act(acc[h], p.bias, (int64_t)cm0 + h * 64 + ib * 16, p.act);
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                 if (!SPATHA_KNOB(4))
-                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), p.fuse ? nullptr : p.bias,
+                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p), p.fuse ? nullptr : p.bias,
                                                 (int64_t)cm0 + h * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
             } else if (!SPATHA_KNOB(4)) {
                 // two copies, so that the plain path carries nothing of the bias path
                 if (p.fuse && !pre && p.bias)
-                    store_block_row_major_tr<Cfg::NC == 8, Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p),
+                    store_block_row_major_tr<Cfg::NC == 8, Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p),
                                                                          (int64_t)cm0 + h * 64, cn0 + wn * 64, N, lane,
                                                                          !SPATHA_KNOB(2), p.bias);
                 else
-                    store_block_row_major_tr<Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p),
+                    store_block_row_major_tr<Cfg::NC == 8>(acc[h], smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p),
                                                            (int64_t)cm0 + h * 64, cn0 + wn * 64, N, lane, !SPATHA_KNOB(2), nullptr);
             }
         }
@@ -292,8 +292,8 @@ __device__ __forceinline__ void half_to_standard_order(float4_t (&acc)[4][4], in
 // multiply a fragment gathered with the first half's table entry, instructions 2, 3 one gathered with the second's
 // (gtab then has one entry per 32-row block).  The dense B stage is the same, so the fill traffic does not grow with
 // the smaller V; only the consumers read twice as many fragments.
-template <class Cfg, int OUT_LAYOUT>
-__device__ __forceinline__ void ds_consumer_half(const SpmmParams& p, const TileWalk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int OUT_LAYOUT, class Params>
+__device__ __forceinline__ void ds_consumer_half(const Params& p, const TileWalk& walk, char* smem, int wave, int lane) {
     static_assert(Cfg::NC == 8, "one 64-row block per consumer wave");
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
@@ -387,10 +387,10 @@ __device__ __forceinline__ void ds_consumer_half(const SpmmParams& p, const Tile
         const bool pre = p.fuse && (p.act != SPATHA_ACT_NONE || OUT_LAYOUT == SPATHA_OUT_TRANSPOSED);
         if (pre) fused_bias_act(acc, p.bias, (int64_t)cm0 + ib * 16, p.act);
         if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), p.fuse ? nullptr : p.bias,
+            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p), p.fuse ? nullptr : p.bias,
                                         (int64_t)cm0, cn0 + wn * 64, p.rows, N, lane, true);
         else
-            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), (int64_t)cm0, cn0 + wn * 64, N,
+            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p), (int64_t)cm0, cn0 + wn * 64, N,
                                            lane, true, (p.fuse && !pre) ? p.bias : nullptr);
         walk.next(c_tm, c_tn);
     }
@@ -403,8 +403,8 @@ __device__ __forceinline__ void ds_consumer_half(const SpmmParams& p, const Tile
 // registers from stage s as soon as the instructions that read it are issued, and reach the
 // next barrier once stage s sits in registers.  On every SIMD one wave's LDS latency is thus
 // covered by the other wave's matrix work, with a single register set per wave.
-template <class Cfg, int OUT_LAYOUT, bool LATE>
-__device__ __forceinline__ void ds_consumer_pp(const SpmmParams& p, const TileWalk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int OUT_LAYOUT, bool LATE, class Params>
+__device__ __forceinline__ void ds_consumer_pp(const Params& p, const TileWalk& walk, char* smem, int wave, int lane) {
     static_assert(Cfg::NC == 8, "ping-pong needs two consumer waves per SIMD");
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
@@ -493,7 +493,7 @@ __device__ __forceinline__ void ds_consumer_pp(const SpmmParams& p, const TileWa
                 }
             }
         } else if (!SPATHA_KNOB(4)) {
-            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, OutC(p), (int64_t)cm0,
+            store_block_row_major_tr<true>(acc, smem + Cfg::EPI_BASE + wave * Cfg::SLAB_BYTES, out_of(p), (int64_t)cm0,
                                            cn0 + wn * 64, N, lane, !SPATHA_KNOB(2));
         }
         SPATHA_PROF_MARK(2)
@@ -589,8 +589,8 @@ __device__ __forceinline__ void ds_consumer_pp(const SpmmParams& p, const TileWa
     SPATHA_PROF_FLUSH
 }
 
-template <int M, int NS, int NP, int OUT_LAYOUT>
-__global__ __launch_bounds__((8 + NP) * 64) void spmm_dspp_kernel(SpmmParams p) {
+template <int M, int NS, int NP, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__((8 + NP) * 64) void spmm_dspp_kernel(Params p) {
     using Cfg = DsCfg<M, NS, NP, 8>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
@@ -612,8 +612,8 @@ __global__ __launch_bounds__((8 + NP) * 64) void spmm_dspp_kernel(SpmmParams p) 
     }
 }
 
-template <int M, int NS, int NP, int NC, int OUT_LAYOUT, bool HALF = false>
-__global__ __launch_bounds__((NC + NP) * 64) void spmm_ds_kernel(SpmmParams p) {
+template <int M, int NS, int NP, int NC, int OUT_LAYOUT, bool HALF, class Params>
+__global__ __launch_bounds__((NC + NP) * 64) void spmm_ds_kernel(Params p) {
     using Cfg = DsCfg<M, NS, NP, NC, (NC == 8 && !HALF)>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
@@ -639,16 +639,16 @@ __global__ __launch_bounds__((NC + NP) * 64) void spmm_ds_kernel(SpmmParams p) {
     }
 }
 
-template <int M, int NS, int NP, int NC, int OUT_LAYOUT, bool PINGPONG = false, bool HALF = false>
-static hipError_t launch_ds(const SpmmParams& p, hipStream_t stream) {
+template <int M, int NS, int NP, int NC, int OUT_LAYOUT, bool PINGPONG = false, bool HALF = false, class Params>
+static hipError_t launch_ds(const Params& p, hipStream_t stream) {
     using Cfg = DsCfg<M, NS, NP, NC>;
     constexpr int lds = Cfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     static_assert(!PINGPONG || NC == 8, "ping-pong needs eight consumer waves");
     const int cus = p.cus;        // compute units of the plan's device
-    void (*kern)(SpmmParams);
-    if constexpr (PINGPONG) kern = spmm_dspp_kernel<M, NS, NP, OUT_LAYOUT>;
-    else kern = spmm_ds_kernel<M, NS, NP, NC, OUT_LAYOUT, HALF>;
+    void (*kern)(Params);
+    if constexpr (PINGPONG) kern = spmm_dspp_kernel<M, NS, NP, OUT_LAYOUT, Params>;
+    else kern = spmm_ds_kernel<M, NS, NP, NC, OUT_LAYOUT, HALF, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -664,7 +664,8 @@ static hipError_t launch_ds(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_densestage(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+template <class Params>
+static hipError_t launch_densestage_form(int variant, int out_layout, const Params& p, hipStream_t stream) {
     const bool t = out_layout == SPATHA_OUT_TRANSPOSED;
     switch (variant) {
         case SPMM_VARIANT_DS256x128_S3_C8:
@@ -677,6 +678,10 @@ hipError_t launch_densestage(int variant, int out_layout, const SpmmParams& p, h
                      : launch_ds<8, 3, 4, 8, SPATHA_OUT_ROW_MAJOR, false, true>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_densestage(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+    return in_form_of(p, [&](const auto& q) { return launch_densestage_form(variant, out_layout, q, stream); });
 }
 
 }  // namespace spatha

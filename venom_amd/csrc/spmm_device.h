@@ -38,6 +38,7 @@
 
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -96,25 +97,36 @@ __device__ __forceinline__ void store_c16(uint16_t* dst, u32x4 v, bool stream) {
 #endif
 }
 
-// Whether C leaves by non-temporal stores, read where the kernel starts: left to the compiler it is loaded in front of the first store,
-// and every tile's write-out begins with that load's latency.
-__device__ __forceinline__ bool streams(const SpmmParams& p) {
-    int s = p.stream_out;
-    asm volatile("" : "+s"(s));
-    return s != 0;
+// Parameters of a launch whose result leaves by non-temporal stores (SpmmParams::stream_out).  A type of its own, so that the staged
+// kernels are compiled for each of the two kinds of result and neither carries a branch of the other's: with one in front of the
+// stores products of 8 to 70 MB took 1-2 % longer (1024 x 4096 x 4096 at 128:2:8 17.6 us against 17.3, 5120 x 1280 x 4096 at
+// 64:2:10 31.6 against 31.2).
+struct StreamedParams : SpmmParams {};
+template <class Params>
+constexpr bool kStreams = std::is_same<Params, StreamedParams>::value;
+
+template <class Launch>
+hipError_t in_form_of(const SpmmParams& p, Launch&& launch) {
+    if (!p.stream_out) return launch(p);
+    StreamedParams s;
+    static_cast<SpmmParams&>(s) = p;
+    return launch(s);
 }
 
 // where a write-out goes and how
+template <bool STREAM>
 struct OutC {
     uint16_t* at;
-    bool stream;
-    __device__ __forceinline__ explicit OutC(const SpmmParams& p) : at(p.C), stream(p.stream_out != 0) {}
-    // Three of four stores of a block, where a write-out knows its store's number i: the quarter left to the memory-side cache finds room
-    // there, and writing it to memory is spared where the next launch overwrites it.  4096 x 1024 x 16384 at 64:2:8, launches following
-    // each other for long, one set of operands / three in turn: 57.0 / 57.3 us; all of them non-temporal 59.6 / 59.8 (at the power limit
-    // writes to memory cost clock), every second 57.1 / 72.7, none 57.0 / 73.3.
-    __device__ __forceinline__ bool streams(int i) const { return stream && (i & 3) != 0; }
+    static constexpr bool stream = STREAM;
+    // Three of four stores of a block in the write-outs of the kernels that run at the power limit, where writes to memory cost clock, and
+    // of the store waves (store number i): the quarter left to the memory-side cache stays there where the same result is written
+    // again soon.  4096 x 1024 x 16384 at 64:2:8, launches following each other for long, one set of operands and results / three / six
+    // in turn: 55.2-57.8 / 57-72 (as the sets happen to lie) / 75 us; all of them non-temporal 57.7-61 / 58-61 / 58-61, none
+    // 54.1-55.1 / 72 / 72.
+    __device__ __forceinline__ static constexpr bool streams(int i) { return STREAM && (i & 3) != 0; }
 };
+template <class Params>
+__device__ __forceinline__ OutC<kStreams<Params>> out_of(const Params& p) { return {p.C}; }
 
 // "Dynamic LDS limit raised" flags, one per (kernel, device): the attribute is a per-device property of a kernel.
 static bool& lds_attr_flag(const void* kern) {
@@ -288,8 +300,8 @@ constexpr int TT_PITCH = 144;                      // 64 rows x 2 B + 16 B pad (
 constexpr int TT_SLAB_BYTES = 8 * TT_PITCH;        // per wave
 // Transposed write-out (C^T[N][rows], + bias) of one wave's 64 x 64 block through an LDS slab of 8 columns x 64 rows,
 // so that every store instruction covers whole 128-byte lines (defined further down).
-template <bool WRITE_THROUGH = false>
-__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC C,
+template <bool WRITE_THROUGH = false, bool STREAM>
+__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC<STREAM> C,
                                                             const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                             int lane, bool stores_on);
 
@@ -518,8 +530,8 @@ __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
 }
 
 // rows 4*MB..4*MB+3 (+16*ib) of the pending wave tile -> row-major C through the wave's LDS slab
-template <int MB, int EPI_PITCH>
-__device__ __forceinline__ void store_slab_row_major(const uint32_t (&pend)[4][4][2], char* stg, OutC C, int64_t row_base,
+template <int MB, int EPI_PITCH, bool STREAM>
+__device__ __forceinline__ void store_slab_row_major(const uint32_t (&pend)[4][4][2], char* stg, OutC<STREAM> C, int64_t row_base,
                                                      int col_base, int N, int lane, bool enable) {
     const int j16 = lane & 15, ib = lane >> 4;
 #pragma unroll
@@ -559,8 +571,8 @@ __device__ __forceinline__ void store_block_transposed(const uint32_t (&pend)[4]
 // Transposed write-out (C^T[N][rows], + bias) of one wave's 64 x 64 block through an LDS slab of 8 columns x 64 rows.
 // Straight from the accumulators a lane could only store 16-byte pieces 32 bytes apart; through the slab every
 // store instruction writes 8 output rows (columns of C) x 128 contiguous bytes.
-template <bool WRITE_THROUGH>
-__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC C,
+template <bool WRITE_THROUGH, bool STREAM>
+__device__ __forceinline__ void store_block_transposed_slab(const float4_t (&acc)[4][4], char* stg, OutC<STREAM> C,
                                                             const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                             int lane, bool stores_on) {
     const int j16 = lane & 15, ib = lane >> 4;     // as accumulator lane: column j16 of a 16-column block, rows 16*ib + 4*mb + r
@@ -634,8 +646,8 @@ constexpr int TR8_SLAB_BYTES = 64 * TR8_PITCH;     // per wave, 8 slab rows at a
 // BIAS_VIA_SLAB (needs ROWS8 and 128 spare bytes behind the slab): the block's 64 bias values are fetched once, ahead of
 // the first store, and the phases read them from LDS; a bias load inside a phase would make that phase wait on the
 // vector-memory counter, i.e. for every store issued so far.
-template <bool ROWS8, bool BIAS_VIA_SLAB = false, bool WRITE_THROUGH = true>
-__device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4][4], char* stg, OutC C, int64_t row0,
+template <bool ROWS8, bool BIAS_VIA_SLAB = false, bool WRITE_THROUGH = true, bool STREAM>
+__device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4][4], char* stg, OutC<STREAM> C, int64_t row0,
                                                          int col0, int N, int lane, bool stores_on,
                                                          const uint16_t* bias = nullptr) {
     static_assert(!BIAS_VIA_SLAB || ROWS8, "the spare bytes sit behind the 8-row slab");
@@ -702,8 +714,8 @@ __device__ __forceinline__ void store_block_row_major_tr(const float4_t (&acc)[4
 // The same two write-outs with four slabs per wave (stg: 4 slabs, then 128 bytes for the block's bias values): four
 // phases' LDS writes and transposing / row reads are in flight before the first store waits for its data, so a 64 x 64
 // block costs two LDS round trips instead of eight.
-template <bool WITH_BIAS>
-__device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[4][4], char* stg, OutC C, int64_t row0,
+template <bool WITH_BIAS, bool STREAM>
+__device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[4][4], char* stg, OutC<STREAM> C, int64_t row0,
                                                           int col0, int N, int lane, bool stores_on, const uint16_t* bias) {
     constexpr int PITCH = TR8_PITCH, SLAB = TR8_SLAB_BYTES;
     const int j16 = lane & 15, ib = lane >> 4;
@@ -761,7 +773,8 @@ __device__ __forceinline__ void store_block_row_major_tr4(const float4_t (&acc)[
     __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&acc)[4][4], char* stg, OutC C,
+template <bool STREAM>
+__device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&acc)[4][4], char* stg, OutC<STREAM> C,
                                                              const uint16_t* bias, int64_t row0, int col0, int rows_total, int N,
                                                              int lane, bool stores_on) {
     const int j16 = lane & 15, ib = lane >> 4;     // as accumulator lane: column j16 of a 16-column block, rows 16*ib + 4*mb + r

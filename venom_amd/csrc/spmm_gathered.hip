@@ -8,8 +8,8 @@ namespace spatha {
 // ---------------------------------------------------------------------------
 // Main SpMM kernel.  Workgroup = WM x WN waves, each owning a 64 x 64 tile of C.
 // ---------------------------------------------------------------------------
-template <int WM, int WN, int OUT_LAYOUT>
-__global__ __launch_bounds__(WM* WN * 64) void spmm_kernel(SpmmParams p) {
+template <int WM, int WN, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__(WM* WN * 64) void spmm_kernel(Params p) {
     constexpr int NT = WM * WN * 64;
     constexpr int BM = WM * 64, BN = WN * 64;
     constexpr int PITCH_B = BN * 2 + 32;             // bytes per gathered-B row in LDS
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_kernel(SpmmParams p) {
             const int row = 16 * (L & 3) + (L >> 2);
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(st + L * PITCH_C + ch * 16);
-            if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
+            if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, kStreams<Params>);
         }
     }
 }
@@ -213,8 +213,8 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_kernel(SpmmParams p) {
 //   [.., + WM*APACK_BLOCK)      per 64-row wave tile: 4 KiB A operands + 512 B index words
 // ---------------------------------------------------------------------------
 
-template <int WM, int WN, int NS, int OUT_LAYOUT>
-__global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
+template <int WM, int WN, int NS, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(Params p) {
     constexpr int NW = WM * WN;
     constexpr int BM = WM * 64, BN = WN * 64;
     constexpr int ROW_BYTES = BN * 2;
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
     const uint16_t* bias = p.fuse ? nullptr : p.bias;
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
         __syncthreads();                 // every wave is done reading the stages: their memory becomes the slabs
-        store_block_transposed_slab<true>(acc, smem + wave * TT_SLAB_BYTES, OutC(p), bias, (int64_t)m0 + wm * 64, n0 + wn * 64,
+        store_block_transposed_slab<true>(acc, smem + wave * TT_SLAB_BYTES, out_of(p), bias, (int64_t)m0 + wm * 64, n0 + wn * 64,
                                           p.rows, N, lane, true);
     } else if (!SPATHA_KNOB(4)) {
         __syncthreads();                 // every wave is done reading the stages
@@ -359,19 +359,19 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_pipe_kernel(SpmmParams p) {
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(stg + Lr * PITCH_C + ch * 16);
             // (256-wide tiles: written through, 0-13 % faster on the BERT-large / GPT-2-large layer shapes; the 128-wide ones lose)
-            if (col < N && !SPATHA_KNOB(2)) store_c16<(WN >= 4)>(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
+            if (col < N && !SPATHA_KNOB(2)) store_c16<(WN >= 4)>(p.C + ((int64_t)m0 + wm * 64 + row) * N + col, v, kStreams<Params>);
         }
     }
 }
 
-template <int WM, int WN, int NS, int OUT_LAYOUT>
-static hipError_t launch_pipe(const SpmmParams& p, hipStream_t stream) {
+template <int WM, int WN, int NS, int OUT_LAYOUT, class Params>
+static hipError_t launch_pipe(const Params& p, hipStream_t stream) {
     constexpr int BN = WN * 64;
     constexpr int stage_bytes = NS * (64 * BN * 2 + WM * APACK_BLOCK);
     static_assert(stage_bytes >= WM * WN * 64 * 144, "the epilogue staging reuses the stage buffers");
     const int lds = stage_bytes + p.S * 256;
     if (lds > 160 * 1024) return hipErrorInvalidValue;     // callers check with spmm_variant_fits first
-    auto kern = spmm_pipe_kernel<WM, WN, NS, OUT_LAYOUT>;
+    auto kern = spmm_pipe_kernel<WM, WN, NS, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -426,8 +426,8 @@ __device__ __forceinline__ void fused_bias_act_half(float4_t (&acc)[2][4], const
     else fused_bias_act_half_impl<SPATHA_ACT_NONE>(acc, bias, row8, rows_exist);
 }
 
-template <int WN, int NS, int OUT_LAYOUT>
-__global__ __launch_bounds__(WN * 128) void spmm_half_kernel(SpmmParams p) {
+template <int WN, int NS, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__(WN * 128) void spmm_half_kernel(Params p) {
     constexpr int WAVES = WN * 2, MB = 2;
     constexpr int BN = WN * 64;
     constexpr int ROW_BYTES = BN * 2;
@@ -609,18 +609,18 @@ __global__ __launch_bounds__(WN * 128) void spmm_half_kernel(SpmmParams p) {
             const int row = 32 * half + 8 * (Lr & 3) + 4 * ((Lr >> 4) & 1) + ((Lr >> 2) & 3);
             const int col = n0 + wn * 64 + ch * 8;
             u32x4 v = *(const u32x4*)(stg + Lr * PITCH_C + ch * 16);
-            if (col < N && m0 + row < p.rows) store_c16(p.C + ((int64_t)m0 + row) * N + col, v, p.stream_out != 0);
+            if (col < N && m0 + row < p.rows) store_c16(p.C + ((int64_t)m0 + row) * N + col, v, kStreams<Params>);
         }
     }
 }
 
-template <int WN, int NS, int OUT_LAYOUT>
-static hipError_t launch_half(const SpmmParams& p, hipStream_t stream) {
+template <int WN, int NS, int OUT_LAYOUT, class Params>
+static hipError_t launch_half(const Params& p, hipStream_t stream) {
     constexpr int stage_bytes = half_stage_bytes<WN, NS>();
     static_assert(stage_bytes >= WN * 64 * 144, "the write-out staging reuses the stage buffers");
     const int lds = stage_bytes + p.S * 256;
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    auto kern = spmm_half_kernel<WN, NS, OUT_LAYOUT>;
+    auto kern = spmm_half_kernel<WN, NS, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -635,7 +635,7 @@ static hipError_t launch_half(const SpmmParams& p, hipStream_t stream) {
     // 0.99, beyond 1.01 / 1.00 (1024 x 4096 x 16384 at 32:2:32 1.04); 64 x 256 tiles 1.02 / 1.03 at any count (1024 x 4096 x 4096 at
     // 32:2:16 1.06), three stages 1.01 / 1.00.  (The tiles of spmm_pipe_kernel likewise: 128 x 128 1.00-1.02, 64 x 256 0.95-1.03 from
     // memory and up to 1.10 from the cache: adjacent.)
-    SpmmParams q = p;
+    Params q = p;
     q.walk_group = WN == 2 && NS == 2 && p.tiles_n % 8 == 0 && tiles <= 2 * p.cus ? 8 : 1;
     hipLaunchKernelGGL(kern, dim3(chunk * 8), dim3(WN * 128), lds, stream, q);
     return hipGetLastError();
@@ -662,8 +662,8 @@ static hipError_t launch_half(const SpmmParams& p, hipStream_t stream) {
 // and waits with s_waitcnt vmcnt(k * LOADS) for the batch issued NS-1 steps earlier.
 // ---------------------------------------------------------------------------
 
-template <int WM, int WN, int NS, int OUT_LAYOUT>
-__global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p) {
+template <int WM, int WN, int NS, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(Params p) {
     using Cfg = PersistCfg<WM, WN, NS>;
     constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
@@ -887,7 +887,7 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
                     const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                     const int col = cn0 + wn * 64 + ch * 8;
                     u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
+                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, kStreams<Params>);
                 }
                 __builtin_amdgcn_wave_barrier();
             }
@@ -896,13 +896,13 @@ __global__ __launch_bounds__(WM* WN * 64) void spmm_persist_kernel(SpmmParams p)
     }
 }
 
-template <int WM, int WN, int NS, int OUT_LAYOUT>
-static hipError_t launch_persist(const SpmmParams& p, hipStream_t stream) {
+template <int WM, int WN, int NS, int OUT_LAYOUT, class Params>
+static hipError_t launch_persist(const Params& p, hipStream_t stream) {
     using Cfg = PersistCfg<WM, WN, NS>;
     constexpr int lds = Cfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     const int cus = p.cus;        // compute units of the plan's device
-    auto kern = spmm_persist_kernel<WM, WN, NS, OUT_LAYOUT>;
+    auto kern = spmm_persist_kernel<WM, WN, NS, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -923,13 +923,13 @@ static hipError_t launch_persist(const SpmmParams& p, hipStream_t stream) {
 // ---------------------------------------------------------------------------
 // Host-side launchers
 // ---------------------------------------------------------------------------
-template <int WM, int WN, int OUT_LAYOUT>
-static hipError_t launch_variant(const SpmmParams& p, hipStream_t stream) {
+template <int WM, int WN, int OUT_LAYOUT, class Params>
+static hipError_t launch_variant(const Params& p, hipStream_t stream) {
     constexpr int BN = WN * 64;
     constexpr int stage_bytes = 2 * 64 * (BN * 2 + 32);
     constexpr int epi_bytes = WM * WN * 64 * 144;
     constexpr int lds = stage_bytes > epi_bytes ? stage_bytes : epi_bytes;
-    auto kern = spmm_kernel<WM, WN, OUT_LAYOUT>;
+    auto kern = spmm_kernel<WM, WN, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set && lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -942,7 +942,8 @@ static hipError_t launch_variant(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_gathered(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+template <class Params>
+static hipError_t launch_gathered_form(int variant, int out_layout, const Params& p, hipStream_t stream) {
     const bool t = out_layout == SPATHA_OUT_TRANSPOSED;
     switch (variant) {
         case SPMM_VARIANT_128x128:
@@ -963,6 +964,10 @@ hipError_t launch_gathered(int variant, int out_layout, const SpmmParams& p, hip
             return t ? launch_half<2, 2, SPATHA_OUT_TRANSPOSED>(p, stream) : launch_half<2, 2, SPATHA_OUT_ROW_MAJOR>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_gathered(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+    return in_form_of(p, [&](const auto& q) { return launch_gathered_form(variant, out_layout, q, stream); });
 }
 
 }  // namespace spatha

@@ -21,7 +21,6 @@ struct SpmmParams {
     uint16_t* C;              // rows x N, or N x rows when transposed
     int rows, cols, N, S, v;
     int m;                    // dense columns per group (dense-staged kernels)
-    int b_pitch;              // columns from one row of B to the next (the direct kernels; N everywhere else)
     uint32_t b_bytes, apack_bytes, rowtab_bytes;   // sizes for buffer descriptors (persistent kernels)
     int tiles_m, tiles_n;
     int cus;                  // compute units of the device the launch goes to (grid size of the persistent kernels)
@@ -38,8 +37,9 @@ struct SpmmParams {
     long long* prof;          // development cycle-accounting buffer (SPATHA_DEV_PROFILE builds), else null
     int fuse;                 // 1: bias and activation are applied ahead of the write-out (fused_bias_act)
     int act;                  // SPATHA_ACT_*
-    int stream_out;           // 1: C leaves by non-temporal stores (the staged kernels; streams_out in spatha_api.cpp)
     int debug;                // development knobs (0 in production): 1 = skip B loads, 2 = skip C stores
+    int b_pitch;              // columns from one row of B to the next (the direct kernels; N everywhere else)
+    int stream_out;           // 1: C leaves by non-temporal stores (read on the host: StreamedParams)
 };
 
 enum {

@@ -196,8 +196,8 @@ __device__ __forceinline__ void oh_producer(const SpmmParams& p, char* smem, uin
     __syncthreads();                    // the slots become write-out staging
 }
 
-template <int OUT_LAYOUT, bool FUSE>
-__device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uint32_t smem_base, int wave, int lane, int full_block,
+template <int OUT_LAYOUT, bool FUSE, class Params>
+__device__ __forceinline__ void oh_consumer(const Params& p, char* smem, uint32_t smem_base, int wave, int lane, int full_block,
                                             int extra_block, int extra_half, int tn) {
     const int S = p.S, N = p.N;
     const bool on_extra = wave >= 8;
@@ -335,7 +335,7 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
     const int col0 = tn * 256 + (on_extra ? extra_half * 128 : 0) + q * 64;
     if constexpr (FUSE) fused_bias_act(acc, p.bias, row0 + ib * 16, p.act);
     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-        store_block_transposed_slab<true>(acc, stg, OutC(p), FUSE ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
+        store_block_transposed_slab<true>(acc, stg, out_of(p), FUSE ? nullptr : p.bias, row0, col0, p.rows, N, lane, true);
     } else {
         // 16-row slabs through the wave's staging buffer -> 128-byte row segments
 #pragma unroll
@@ -352,7 +352,7 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
                 const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                 const int col = col0 + ch * 8;
                 u32x4 v = *(const u32x4*)(stg + Lr * OH_EPI_PITCH + ch * 16);
-                if (col < N) store_c16(p.C + (row0 + row) * N + col, v, p.stream_out != 0);
+                if (col < N) store_c16(p.C + (row0 + row) * N + col, v, kStreams<Params>);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -360,8 +360,8 @@ __device__ __forceinline__ void oh_consumer(const SpmmParams& p, char* smem, uin
 }
 
 // FUSE: bias and activation in the write-out (instances of their own: with the activations' code in it the kernel spills registers)
-template <int OUT_LAYOUT, bool FUSE>
-__global__ __launch_bounds__((OH_NC + OH_NP) * 64) void spmm_oh_kernel(SpmmParams p) {
+template <int OUT_LAYOUT, bool FUSE, class Params>
+__global__ __launch_bounds__((OH_NC + OH_NP) * 64) void spmm_oh_kernel(Params p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -383,9 +383,9 @@ __global__ __launch_bounds__((OH_NC + OH_NP) * 64) void spmm_oh_kernel(SpmmParam
     else oh_producer<3>(p, smem, smem_base, lane, full_block, extra_block, extra_half, tn);
 }
 
-template <int OUT_LAYOUT, bool FUSE>
-hipError_t launch_oh(const SpmmParams& p, hipStream_t stream) {
-    auto kern = spmm_oh_kernel<OUT_LAYOUT, FUSE>;
+template <int OUT_LAYOUT, bool FUSE, class Params>
+hipError_t launch_oh(const Params& p, hipStream_t stream) {
+    auto kern = spmm_oh_kernel<OUT_LAYOUT, FUSE, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, OH_LDS);
@@ -402,9 +402,11 @@ hipError_t launch_oh(const SpmmParams& p, hipStream_t stream) {
 hipError_t launch_onehalf(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
     if (variant != SPMM_VARIANT_OH192x256) return hipErrorInvalidValue;
     if (p.v % 128 != 0 || p.rows % 128 != 0 || p.tiles_m != p.rows / 128 || p.ksplit != 1) return hipErrorInvalidValue;
-    if (out_layout == SPATHA_OUT_TRANSPOSED)
-        return p.fuse ? launch_oh<SPATHA_OUT_TRANSPOSED, true>(p, stream) : launch_oh<SPATHA_OUT_TRANSPOSED, false>(p, stream);
-    return p.fuse ? launch_oh<SPATHA_OUT_ROW_MAJOR, true>(p, stream) : launch_oh<SPATHA_OUT_ROW_MAJOR, false>(p, stream);
+    return in_form_of(p, [&](const auto& q) {
+        if (out_layout == SPATHA_OUT_TRANSPOSED)
+            return q.fuse ? launch_oh<SPATHA_OUT_TRANSPOSED, true>(q, stream) : launch_oh<SPATHA_OUT_TRANSPOSED, false>(q, stream);
+        return q.fuse ? launch_oh<SPATHA_OUT_ROW_MAJOR, true>(q, stream) : launch_oh<SPATHA_OUT_ROW_MAJOR, false>(q, stream);
+    });
 }
 
 }  // namespace spatha

@@ -74,8 +74,8 @@ __device__ __forceinline__ void pload_b64(u32x2& r, uint32_t voff, i32x4 rsrc, u
 // The whole life of one wave.  LATE is the wave's phase group (false: X, true: Y), a template argument so that each group
 // runs straight-line code of its own: an operand set that is in flight must never meet, at a join of two paths, a
 // version of itself that is not (the register copy the compiler may place there would copy a value that has not arrived).
-template <int OUT_LAYOUT, bool FUSE, bool GROUPED, bool LATE, class Walk>
-__device__ __forceinline__ void up_wave(const SpmmParams& p, const Walk& walk, char* smem, uint32_t smem_base, int wave,
+template <int OUT_LAYOUT, bool FUSE, bool GROUPED, bool LATE, class Params, class Walk>
+__device__ __forceinline__ void up_wave(const Params& p, const Walk& walk, char* smem, uint32_t smem_base, int wave,
                                         int lane) {
     using Cfg = UpCfg;
     constexpr int NB = Cfg::NB;
@@ -289,10 +289,10 @@ __device__ __forceinline__ void up_wave(const SpmmParams& p, const Walk& walk, c
                     // one on all 64 accumulator registers of the block); the write-out itself is then the plain one
                     if constexpr (FUSE) fused_bias_act_narrow(acc[wn], p.bias, (int64_t)cm0 + (lane >> 4) * 16, p.act);
                     if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                        store_block_transposed_slab4(acc[wn], stg, OutC(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
+                        store_block_transposed_slab4(acc[wn], stg, out_of(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows, N,
                                                      lane, !(UP_KNOBS & 32));
                     else
-                        store_block_row_major_tr4<false>(acc[wn], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !(UP_KNOBS & 32), nullptr);
+                        store_block_row_major_tr4<false>(acc[wn], stg, out_of(p), (int64_t)cm0, cn0 + wn * 64, N, lane, !(UP_KNOBS & 32), nullptr);
                 }
             }
             zero_acc();
@@ -308,8 +308,8 @@ __device__ __forceinline__ void up_wave(const SpmmParams& p, const Walk& walk, c
 #undef SPATHA_UP_WAIT_ALL
 }
 
-template <int OUT_LAYOUT, bool FUSE, bool GROUPED, int WALK>
-__global__ __launch_bounds__(512) void spmm_up_kernel(SpmmParams p) {
+template <int OUT_LAYOUT, bool FUSE, bool GROUPED, int WALK, class Params>
+__global__ __launch_bounds__(512) void spmm_up_kernel(Params p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -327,12 +327,12 @@ __global__ __launch_bounds__(512) void spmm_up_kernel(SpmmParams p) {
     else up_wave<OUT_LAYOUT, FUSE, GROUPED, false>(p, walk, smem, smem_base, wave, lane);
 }
 
-template <int OUT_LAYOUT, bool FUSE, bool GROUPED, int WALK>
-static hipError_t launch_up_walk(const SpmmParams& p, hipStream_t stream) {
+template <int OUT_LAYOUT, bool FUSE, bool GROUPED, int WALK, class Params>
+static hipError_t launch_up_walk(const Params& p, hipStream_t stream) {
     constexpr int lds = UpCfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     const int cus = p.cus;        // compute units of the plan's device
-    void (*kern)(SpmmParams) = spmm_up_kernel<OUT_LAYOUT, FUSE, GROUPED, WALK>;
+    void (*kern)(Params) = spmm_up_kernel<OUT_LAYOUT, FUSE, GROUPED, WALK, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         // the kernel's register loads complete asynchronously into named variables: an instantiation that keeps
@@ -354,8 +354,8 @@ static hipError_t launch_up_walk(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <int OUT_LAYOUT, bool FUSE, bool GROUPED>
-static hipError_t launch_up(const SpmmParams& p, hipStream_t stream) {
+template <int OUT_LAYOUT, bool FUSE, bool GROUPED, class Params>
+static hipError_t launch_up(const Params& p, hipStream_t stream) {
     if (p.walk_group == UP_WALK_ROWS && p.tiles_m % 4 == 0) return launch_up_walk<OUT_LAYOUT, FUSE, GROUPED, UP_WALK_ROWS>(p, stream);
     return launch_up_walk<OUT_LAYOUT, FUSE, GROUPED, 1>(p, stream);
 }
@@ -365,7 +365,8 @@ static hipError_t launch_up(const SpmmParams& p, hipStream_t stream) {
 #define SPATHA_UP_GROUPED_MAX_M 5
 #endif
 
-hipError_t launch_pingpong(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+template <class Params>
+static hipError_t launch_up_form(int variant, int out_layout, const Params& p, hipStream_t stream) {
     if (variant != SPMM_VARIANT_UP512x128_S3) return hipErrorInvalidValue;
     // (the plain instantiations carry nothing of the fused write-out; the form of the matrix phase follows m, see there)
     const bool t = out_layout == SPATHA_OUT_TRANSPOSED, grouped = p.m <= SPATHA_UP_GROUPED_MAX_M;
@@ -375,6 +376,10 @@ hipError_t launch_pingpong(int variant, int out_layout, const SpmmParams& p, hip
     }
     if (grouped) return t ? launch_up<SPATHA_OUT_TRANSPOSED, false, true>(p, stream) : launch_up<SPATHA_OUT_ROW_MAJOR, false, true>(p, stream);
     return t ? launch_up<SPATHA_OUT_TRANSPOSED, false, false>(p, stream) : launch_up<SPATHA_OUT_ROW_MAJOR, false, false>(p, stream);
+}
+
+hipError_t launch_pingpong(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+    return in_form_of(p, [&](const auto& q) { return launch_up_form(variant, out_layout, q, stream); });
 }
 
 }  // namespace spatha

@@ -32,8 +32,8 @@ __device__ __forceinline__ void bload_b64(u32x2& r, uint32_t voff, i32x4 rsrc, u
 
 // FUSE: the instantiation that can apply bias / activation ahead of the write-out (kept apart: its temporaries would
 // otherwise push the plain kernel over the register budget)
-template <int OUT_LAYOUT, bool FUSE, int M_>
-__global__ __launch_bounds__(512) void spmm_du_kernel(SpmmParams p) {
+template <int OUT_LAYOUT, bool FUSE, int M_, class Params>
+__global__ __launch_bounds__(512) void spmm_du_kernel(Params p) {
     using Cfg = DuCfg<M_>;
     constexpr int NB = Cfg::NB;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::NS, PA = Cfg::PA, STAGE_BYTES = Cfg::STAGE_BYTES;
@@ -255,10 +255,10 @@ __global__ __launch_bounds__(512) void spmm_du_kernel(SpmmParams p) {
                 // on all 64 accumulator registers of the block); the write-out itself is then the plain one
                 if constexpr (FUSE) fused_bias_act_narrow(acc[wn], p.bias, (int64_t)cm0 + ib * 16, p.act);
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED)
-                    store_block_transposed_slab<true>(acc[wn], stg, OutC(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows,
+                    store_block_transposed_slab<true>(acc[wn], stg, out_of(p), FUSE ? nullptr : p.bias, (int64_t)cm0, cn0 + wn * 64, p.rows,
                                                       N, lane, true);
                 else
-                    store_block_row_major_tr<true>(acc[wn], stg, OutC(p), (int64_t)cm0, cn0 + wn * 64, N, lane, true);
+                    store_block_row_major_tr<true>(acc[wn], stg, out_of(p), (int64_t)cm0, cn0 + wn * 64, N, lane, true);
             }
             zero_acc();
             walk.next(c_tm, c_tn);
@@ -271,12 +271,12 @@ __global__ __launch_bounds__(512) void spmm_du_kernel(SpmmParams p) {
 #undef SPATHA_DU_WAIT
 }
 
-template <int OUT_LAYOUT, bool FUSE, int M_ = 8>
-static hipError_t launch_du(const SpmmParams& p, hipStream_t stream) {
+template <int OUT_LAYOUT, bool FUSE, int M_, class Params>
+static hipError_t launch_du(const Params& p, hipStream_t stream) {
     constexpr int lds = DuCfg<M_>::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     const int cus = p.cus;        // compute units of the plan's device
-    void (*kern)(SpmmParams) = spmm_du_kernel<OUT_LAYOUT, FUSE, M_>;
+    void (*kern)(Params) = spmm_du_kernel<OUT_LAYOUT, FUSE, M_, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         // The kernel's register loads complete asynchronously into named variables; a compiler-made copy of such a
@@ -299,7 +299,8 @@ static hipError_t launch_du(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_unified(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+template <class Params>
+static hipError_t launch_unified_form(int variant, int out_layout, const Params& p, hipStream_t stream) {
     const bool t = out_layout == SPATHA_OUT_TRANSPOSED;
     switch (variant) {
         case SPMM_VARIANT_DU512x128_M16:
@@ -308,6 +309,10 @@ hipError_t launch_unified(int variant, int out_layout, const SpmmParams& p, hipS
             return t ? launch_du<SPATHA_OUT_TRANSPOSED, false, 16>(p, stream) : launch_du<SPATHA_OUT_ROW_MAJOR, false, 16>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_unified(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+    return in_form_of(p, [&](const auto& q) { return launch_unified_form(variant, out_layout, q, stream); });
 }
 
 }  // namespace spatha

@@ -1,8 +1,6 @@
 // Producer / consumer kernels on gathered B stages: consumer waves only read LDS and issue matrix instructions,
 // producer waves only compute addresses and issue the global -> LDS DMA.
 
-#include <type_traits>
-
 #include "spmm_device.h"
 
 namespace spatha {
@@ -201,8 +199,8 @@ __device__ __forceinline__ bool ksplit_exchange(float4_t (&acc)[4][4], const Spm
     return true;
 }
 
-template <class Cfg, int WN, int OUT_LAYOUT, class Walk = TileWalk>
-__device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int WN, int OUT_LAYOUT, class Params, class Walk>
+__device__ __forceinline__ void ws_consumer(const Params& p, const Walk& walk, char* smem, int wave, int lane) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
     constexpr int EPI_PITCH = Cfg::EPI_PITCH;
@@ -242,7 +240,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& wal
         if (p.fuse) fused_bias_act(acc, p.bias, (int64_t)cm0 + wm * 64 + ib * 16, p.act);
         const uint16_t* bias = p.fuse ? nullptr : p.bias;
         if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
-            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), OutC(p), bias,
+            store_block_transposed_slab<true>(acc, smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), out_of(p), bias,
                                               (int64_t)cm0 + wm * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
         } else if (!SPATHA_KNOB(4)) {
             // 16-row slabs through a wave-private LDS buffer -> 128-byte row segments
@@ -261,7 +259,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& wal
                     const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                     const int col = cn0 + wn * 64 + ch * 8;
                     u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, p.stream_out != 0);
+                    if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + wm * 64 + row) * N + col, v, kStreams<Params>);
                 }
                 __builtin_amdgcn_wave_barrier();
             }
@@ -269,8 +267,8 @@ __device__ __forceinline__ void ws_consumer(const SpmmParams& p, const Walk& wal
     }
 }
 
-template <class Cfg, int WN, int OUT_LAYOUT>
-__device__ __forceinline__ void ws_consumer_deferred(const SpmmParams& p, const TileWalk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int WN, int OUT_LAYOUT, class Params>
+__device__ __forceinline__ void ws_consumer_deferred(const Params& p, const TileWalk& walk, char* smem, int wave, int lane) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
     constexpr int EPI_PITCH = Cfg::EPI_PITCH;
@@ -308,10 +306,10 @@ __device__ __forceinline__ void ws_consumer_deferred(const SpmmParams& p, const 
         } else {
             const int64_t rb = (int64_t)pm0 + wm * 64;
             const int cb = pn0 + wn * 64;
-            if (part == 0) store_slab_row_major<0, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
-            else if (part == 1) store_slab_row_major<1, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
-            else if (part == 2) store_slab_row_major<2, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
-            else store_slab_row_major<3, EPI_PITCH>(pend, stg, OutC(p), rb, cb, N, lane, stores_on);
+            if (part == 0) store_slab_row_major<0, EPI_PITCH>(pend, stg, out_of(p), rb, cb, N, lane, stores_on);
+            else if (part == 1) store_slab_row_major<1, EPI_PITCH>(pend, stg, out_of(p), rb, cb, N, lane, stores_on);
+            else if (part == 2) store_slab_row_major<2, EPI_PITCH>(pend, stg, out_of(p), rb, cb, N, lane, stores_on);
+            else store_slab_row_major<3, EPI_PITCH>(pend, stg, out_of(p), rb, cb, N, lane, stores_on);
         }
     };
     for (int c_tile = 0; c_tile < walk.my_tiles; c_tile++) {
@@ -397,8 +395,8 @@ __device__ __forceinline__ void mma_stage_tall(const char* st, int a_off, int i_
     SPATHA_MMA8(3, bf1)
 }
 
-template <class Cfg, int WN, int OUT_LAYOUT>
-__device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const TileWalk& walk, char* smem, int wave, int lane) {
+template <class Cfg, int WN, int OUT_LAYOUT, class Params>
+__device__ __forceinline__ void ws_consumer_tall(const Params& p, const TileWalk& walk, char* smem, int wave, int lane) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, NS = Cfg::PA + 1;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, B_BYTES = Cfg::B_BYTES, STAGE_BYTES = Cfg::STAGE_BYTES;
     constexpr int EPI_PITCH = Cfg::EPI_PITCH;
@@ -443,7 +441,7 @@ __device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const Tile
             if (p.fuse) fused_bias_act(acc[h], p.bias, (int64_t)cm0 + h * 64 + ib * 16, p.act);
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                 if (!SPATHA_KNOB(4))
-                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), OutC(p), p.fuse ? nullptr : p.bias,
+                    store_block_transposed_slab<true>(acc[h], smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH), out_of(p), p.fuse ? nullptr : p.bias,
                                                 (int64_t)cm0 + h * 64, cn0 + wn * 64, p.rows, N, lane, !SPATHA_KNOB(2));
             } else if (!SPATHA_KNOB(4)) {
                 char* stg = smem + Cfg::EPI_BASE + wave * (16 * EPI_PITCH);
@@ -461,7 +459,7 @@ __device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const Tile
                         const int row = 16 * (Lr & 3) + 4 * mb + (Lr >> 2);
                         const int col = cn0 + wn * 64 + ch * 8;
                         u32x4 v = *(const u32x4*)(stg + Lr * EPI_PITCH + ch * 16);
-                        if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + h * 64 + row) * N + col, v, p.stream_out != 0);
+                        if (col < N && !SPATHA_KNOB(2)) store_c16(p.C + ((int64_t)cm0 + h * 64 + row) * N + col, v, kStreams<Params>);
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
@@ -472,8 +470,8 @@ __device__ __forceinline__ void ws_consumer_tall(const SpmmParams& p, const Tile
 }
 
 // Tile 128 x (64 * WN): WN tall consumers + NP producers.
-template <int WN, int NS, int NP, int OUT_LAYOUT>
-__global__ __launch_bounds__((WN + NP) * 64) void spmm_wst_kernel(SpmmParams p) {
+template <int WN, int NS, int NP, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__((WN + NP) * 64) void spmm_wst_kernel(Params p) {
     using Cfg = WsCfg<2, WN, NS, NP>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t smem_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
@@ -497,13 +495,13 @@ __global__ __launch_bounds__((WN + NP) * 64) void spmm_wst_kernel(SpmmParams p) 
     }
 }
 
-template <int WN, int NS, int NP, int OUT_LAYOUT>
-static hipError_t launch_wst(const SpmmParams& p, hipStream_t stream) {
+template <int WN, int NS, int NP, int OUT_LAYOUT, class Params>
+static hipError_t launch_wst(const Params& p, hipStream_t stream) {
     using Cfg = WsCfg<2, WN, NS, NP>;
     constexpr int lds = Cfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     const int cus = p.cus;        // compute units of the plan's device
-    auto kern = spmm_wst_kernel<WN, NS, NP, OUT_LAYOUT>;
+    auto kern = spmm_wst_kernel<WN, NS, NP, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -520,8 +518,8 @@ static hipError_t launch_wst(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, bool DEFER = false, int WALK_GROUP = 1>
-__global__ __launch_bounds__((WM * WN + NP) * 64) void spmm_ws_kernel(SpmmParams p) {
+template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, bool DEFER, int WALK_GROUP, class Params>
+__global__ __launch_bounds__((WM * WN + NP) * 64) void spmm_ws_kernel(Params p) {
     using Cfg = WsCfg<WM, WN, NS, NP>;
     static_assert(NP == 2 || NP == 4, "producer count");
     static_assert(!(DEFER && WALK_GROUP != 1), "the deferred write-out walks column-first only");
@@ -552,13 +550,13 @@ __global__ __launch_bounds__((WM * WN + NP) * 64) void spmm_ws_kernel(SpmmParams
     }
 }
 
-template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, bool DEFER = false, int WALK_GROUP = 1>
-static hipError_t launch_ws(const SpmmParams& p, hipStream_t stream) {
+template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, bool DEFER = false, int WALK_GROUP = 1, class Params>
+static hipError_t launch_ws(const Params& p, hipStream_t stream) {
     using Cfg = WsCfg<WM, WN, NS, NP>;
     constexpr int lds = Cfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     const int cus = p.cus;        // compute units of the plan's device
-    auto kern = spmm_ws_kernel<WM, WN, NS, NP, OUT_LAYOUT, DEFER, WALK_GROUP>;
+    auto kern = spmm_ws_kernel<WM, WN, NS, NP, OUT_LAYOUT, DEFER, WALK_GROUP, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -661,11 +659,10 @@ __device__ __forceinline__ void wsw_consumer(const SpmmParams& p, const TileWalk
     __syncthreads();        // the last tile's hand-over
 }
 
-template <class Cfg, int OUT_LAYOUT>
-__device__ __forceinline__ void wsw_storer(const SpmmParams& p, const TileWalk& walk, char* smem, int sw, int lane) {
+template <class Cfg, int OUT_LAYOUT, class Params>
+__device__ __forceinline__ void wsw_storer(const Params& p, const TileWalk& walk, char* smem, int sw, int lane) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, PITCH = Cfg::STG_PITCH;
     const int S = p.S, N = p.N;
-    const bool stream = streams(p);
     const char* stg = smem + Cfg::EPI_BASE;
     // this wave's quarter of the staged tile, 8 pieces of 1 KB (16 bytes per lane).  Transposed output: BN / 4 staging rows
     // (tile columns of BM rows), a piece = RPP of them.  Row-major output: the block of consumer wave `sw`, a piece = one
@@ -710,27 +707,22 @@ __device__ __forceinline__ void wsw_storer(const SpmmParams& p, const TileWalk& 
         h_tn = tn;
         next_piece = 0;
     };
-    // (one branch for all pieces of a step: taken in front of every store it costs 0.1 us of 17 at 1024 x 4096 x 4096, 128:2:8)
-    auto store_some = [&](int count, auto nt) {
+    auto store_pieces = [&](int count) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             if (i >= next_piece && i < next_piece + count) {
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                     const int col = h_tn * BN + srow + RPP * i;         // staging row = tile column
-                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i], nt && (i & 3) != 0);
+                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i], kStreams<Params> && (i & 3) != 0);
                 } else {
                     const int q = 8 * (i & 1) + q_lo;                  // piece i: slab of mb = i / 2, lane groups 2*(i & 1), + 1
                     const int row = blk_row0 + 16 * (q >> 2) + 4 * (i >> 1) + (q & 3);
                     const int col = h_tn * BN + blk_col;
-                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i], nt && (i & 3) != 0);
+                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i], kStreams<Params> && (i & 3) != 0);
                 }
             }
         }
         next_piece += count;
-    };
-    auto store_pieces = [&](int count) {
-        if (stream) store_some(count, std::true_type());
-        else store_some(count, std::false_type());
     };
     int c_tm = walk.tm0, c_tn = walk.tn0;
     for (int c_tile = 0; c_tile < walk.my_tiles; c_tile++) {
@@ -750,8 +742,8 @@ __device__ __forceinline__ void wsw_storer(const SpmmParams& p, const TileWalk& 
     store_pieces(8);
 }
 
-template <int WM, int WN, int NS, int NP, int OUT_LAYOUT>
-__global__ __launch_bounds__((8 + NP) * 64) void spmm_wsw_kernel(SpmmParams p) {
+template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, class Params>
+__global__ __launch_bounds__((8 + NP) * 64) void spmm_wsw_kernel(Params p) {
     using Cfg = WswCfg<WM, WN, NS, NP>;
     static_assert((NP == 2 || NP == 4) && Cfg::THREADS == (8 + NP) * 64, "wave counts");
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -774,14 +766,14 @@ __global__ __launch_bounds__((8 + NP) * 64) void spmm_wsw_kernel(SpmmParams p) {
     }
 }
 
-template <int WM, int WN, int NS, int NP, int OUT_LAYOUT>
-static hipError_t launch_wsw(const SpmmParams& p, hipStream_t stream) {
+template <int WM, int WN, int NS, int NP, int OUT_LAYOUT, class Params>
+static hipError_t launch_wsw(const Params& p, hipStream_t stream) {
     using Cfg = WswCfg<WM, WN, NS, NP>;
     constexpr int lds = Cfg::LDS_BYTES;
     static_assert(lds <= 160 * 1024, "LDS budget");
     if (p.S < 2) return hipErrorInvalidValue;
     const int cus = p.cus;        // compute units of the plan's device
-    auto kern = spmm_wsw_kernel<WM, WN, NS, NP, OUT_LAYOUT>;
+    auto kern = spmm_wsw_kernel<WM, WN, NS, NP, OUT_LAYOUT, Params>;
     bool& attr_set = lds_attr_flag((const void*)kern);
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -797,7 +789,8 @@ static hipError_t launch_wsw(const SpmmParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_warpspec(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+template <class Params>
+static hipError_t launch_warpspec_form(int variant, int out_layout, const Params& p, hipStream_t stream) {
     const bool t = out_layout == SPATHA_OUT_TRANSPOSED;
     switch (variant) {
         case SPMM_VARIANT_W128x128_S3:
@@ -820,6 +813,10 @@ hipError_t launch_warpspec(int variant, int out_layout, const SpmmParams& p, hip
             return t ? launch_wsw<1, 4, 3, 2, SPATHA_OUT_TRANSPOSED>(p, stream) : launch_wsw<1, 4, 3, 2, SPATHA_OUT_ROW_MAJOR>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_warpspec(int variant, int out_layout, const SpmmParams& p, hipStream_t stream) {
+    return in_form_of(p, [&](const auto& q) { return launch_warpspec_form(variant, out_layout, q, stream); });
 }
 
 }  // namespace spatha
