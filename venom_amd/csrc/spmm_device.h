@@ -118,11 +118,13 @@ template <bool STREAM>
 struct OutC {
     uint16_t* at;
     static constexpr bool stream = STREAM;
-    // Three of four stores of a block in the write-outs of the kernels that run at the power limit, where writes to memory cost clock, and
-    // of the store waves (store number i): the quarter left to the memory-side cache stays there where the same result is written
-    // again soon.  4096 x 1024 x 16384 at 64:2:8, launches following each other for long, one set of operands and results / three / six
-    // in turn: 55.2-57.8 / 57-72 (as the sets happen to lie) / 75 us; all of them non-temporal 57.7-61 / 58-61 / 58-61, none
-    // 54.1-55.1 / 72 / 72.
+    // Three of four stores (number i) in the row-major write-out through four slabs alone: its kernels run at the power limit, where
+    // writes to memory cost clock, and the quarter left to the memory-side cache stays there where the same result is written again
+    // soon.  4096 x 1024 x 16384 at 64:2:8, launches following each other for long, on three cards, one set of operands and results /
+    // three / six in turn: 55.2-57.8 / 57-72 (as the sets happen to lie) / 75-76 us; all of them non-temporal 57.7-61 / 58-61 / 58-61,
+    // none 54.1-55.1 / 71-72 / 72.  Elsewhere all of them: the quarter costs the rotating sets as much and spares nothing (transposed
+    // 56.2-57.1 / 56.3-57.9 / 67.4, all 56.0-57.8 / 56.2-57.7 / 56.4-57.9; store waves, 4096 x 1024 x 16384 at 128:2:32 row-major 31.5
+    // / 31.6-50 / 55.8, all 31.4 / 31.5 / 31.6).
     __device__ __forceinline__ static constexpr bool streams(int i) { return STREAM && (i & 3) != 0; }
 };
 template <class Params>
@@ -808,7 +810,7 @@ __device__ __forceinline__ void store_block_transposed_slab4(const float4_t (&ac
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int col = col0 + (grp * 2 + (k >> 1)) * 16 + (k & 1) * 8 + rn;
-            if (col < N && stores_on) store_c16<true>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v[k], C.streams(k));
+            if (col < N && stores_on) store_c16<true>(C.at + (int64_t)col * rows_total + row0 + rc * 8, v[k], C.stream);
         }
     }
     __builtin_amdgcn_wave_barrier();

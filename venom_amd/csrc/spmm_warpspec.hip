@@ -713,12 +713,12 @@ __device__ __forceinline__ void wsw_storer(const Params& p, const TileWalk& walk
             if (i >= next_piece && i < next_piece + count) {
                 if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
                     const int col = h_tn * BN + srow + RPP * i;         // staging row = tile column
-                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i], kStreams<Params> && (i & 3) != 0);
+                    if (col < N) store_c16<true>(p.C + (int64_t)col * p.rows + h_tm * BM + chunk * 8, held[i], kStreams<Params>);
                 } else {
                     const int q = 8 * (i & 1) + q_lo;                  // piece i: slab of mb = i / 2, lane groups 2*(i & 1), + 1
                     const int row = blk_row0 + 16 * (q >> 2) + 4 * (i >> 1) + (q & 3);
                     const int col = h_tn * BN + blk_col;
-                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i], kStreams<Params> && (i & 3) != 0);
+                    if (col < N) store_c16<true>(p.C + ((int64_t)h_tm * BM + row) * N + col, held[i], kStreams<Params>);
                 }
             }
         }
