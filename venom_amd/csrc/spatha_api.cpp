@@ -558,13 +558,19 @@ bool split_choice(const spatha_spmm_plan* plan, int N, int requested, int chosen
 }
 
 // Does C leave by non-temporal stores, past the 256 MB memory-side cache?  From 96 MB on, unless the caller says that it is read right
-// behind this call.  With three sets of operands and results in turn (28 shapes, both layouts): results of 134 MB and more 1.14-1.7x
-// ahead (4096 x 1024 x 16384 at 64:2:8 73.3 -> 56.7 us row-major, 69.9 -> 55.5 transposed, at 128:2:32 53.3 -> 31.5), of 50 to 67 MB
-// 0.98-1.04x, smaller ones level or up to 4 % behind.  On one set that stays in the cache, launches following each other for long: 134 MB
-// 56.8 -> 56.2 and 55.6 -> 55.2 us (OutC::streams), 67 MB 28.4 -> 29.3.  A chain of layers reads each result back from that cache: with
-// such stores in all of them the two encoder layers of BERT-large at 32 x 512 tokens took 695 us, 681 without.
-bool streams_out(const spatha_spmm_plan* plan, int N, bool read_next) {
-    return !read_next && (int64_t)plan->geo.rows * N * 2 >= (96ll << 20);
+// behind this call, and where the rows of C are whole 64-byte pieces.
+// 4096 x 1024 x 16384 (134 MB), V = 32 .. 128, m = 4 .. 32, both layouts, launches following each other for long: three and six sets of
+// operands and results in turn 1.05-1.7x ahead (64:2:8 73 -> 57-61 us row-major, 66 -> 56 transposed, 128:2:32 53.6 -> 31.6); one set,
+// which stays in the cache, 0.92-1.05x (64:2:16 row-major 44.8 -> 47.6, transposed 44.3 -> 46.3; 128:2:32 30.3 -> 31.6 and 33.4 -> 31.7;
+// 49152 x 12288 x 2048 at 128:2:16, 201 MB, 458 -> 440).  12288 x 12288 x 4096 at 128:2:10, 100 MB behind 77 k-steps, is 1-2 % behind
+// on rotating sets.  Results of 50 to 67 MB 0.98-1.04x, smaller ones level or up to 4 % behind.  A chain of layers reads each result
+// back from that cache: with such stores in all of them the two encoder layers of BERT-large at 32 x 512 tokens took 695 us, 681 without.
+// Rows of another length end in parts of 64-byte pieces, which the cache would put together and memory has to read first: the
+// same products on 16368 and 16376 columns 0.48-0.98x on one set and 0.94-1.5x on several (128:2:32 38.5 -> 80.6 and 85 -> 81 us),
+// 12288 x 2048 .. 8192 x 4104 at 128:2:20 0.82-0.95x and 0.89-1.01x.
+bool streams_out(const spatha_spmm_plan* plan, int N, int out_layout, bool read_next) {
+    if (read_next || (out_layout == SPATHA_OUT_ROW_MAJOR && N % 32 != 0)) return false;
+    return (int64_t)plan->geo.rows * N * 2 >= (96ll << 20);
 }
 }  // namespace
 
@@ -850,7 +856,7 @@ int spatha::plan_run(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N,
     p.rowtab_bytes = (uint32_t)plan->rowtab_bytes;
     p.fuse = fuse ? 1 : 0; p.act = activation;
     p.cus = plan->cus > 0 ? plan->cus : 256;
-    p.stream_out = streams_out(plan, N, read_next) ? 1 : 0;
+    p.stream_out = streams_out(plan, N, out_layout, read_next) ? 1 : 0;
     p.walk_group = 1;
     if (var == spatha::SPMM_VARIANT_UP512x128_S3) {
         // Packed A larger than an XCD's L2 (plain 2:4 on a 4096-row matrix: 4.7 MB against 4 MB; it is then fetched again in
