@@ -131,3 +131,23 @@ def test_keys_of_score_minus_infinity_take_no_part(gpu, seq, barred):
     want = softmax_average(qkv, 2, seq, 1, 0.125)
     assert torch.isfinite(want[0]).all() and torch.isnan(want[1]).all()
     same_kinds(got, want)
+
+
+def fused_attention(gpu, layers=1):
+    model = bert.merge_qkv(bert.linear_to_spmm(bert.build_bert_large(layers=layers).to(gpu).half(), 2, 8, 64))
+    return bert.fuse_add_layernorm(model, feature_major=True).encoder.layer[0].attention.self
+
+
+@torch.no_grad()
+def test_the_fused_attention_keeps_no_product(gpu, monkeypatch):
+    """Its projections have one reader: every forward computes them, and none outlives it (the three separate projections share theirs)."""
+    att = fused_attention(gpu)
+    group, x = att.query._group, torch.randn((2, 40, 1024), device=gpu).half()
+    computed = []
+    run = bert.SrnmSpmm._run_native
+    monkeypatch.setattr(bert.SrnmSpmm, "_run_native", staticmethod(lambda *a, **k: computed.append(1) or run(*a, **k)))
+    first = att(x)[0]
+    assert len(computed) == 1 and group._last == (None, None, None)
+    assert torch.equal(att(x)[0], first) and len(computed) == 2 and group._last == (None, None, None)
+    q, k, v = att.query(x), att.key(x), att.value(x)
+    assert len(computed) == 3 and torch.equal(group._last[2], torch.cat([q, k, v], -1).reshape(80, 3072))

@@ -161,22 +161,22 @@ class _MergedProjections:
             self.rows += l.nrows_sp
         self._last = (None, None, None)          # (key, activation held alive, [tokens, rows] result)
 
-    def merged(self, input):
-        """[tokens, rows]: all members' outputs side by side."""
+    def product(self, flat):
+        """flat [tokens, cols] -> [tokens, rows]: all members' outputs side by side."""
+        out = SrnmSpmm._run_native(SrnmSpmm, self, flat, self.rows, self.cols)
+        if out is None:
+            rhs = SrnmSpmm._transposed(flat)
+            out = spatha.spmm(self.metadata, self.columns, self.values, rhs, self.bias, self.rows, self.cols, rhs.shape[1],
+                              self.v, self.n, self.m, 0, 0, 32, 4)
+        return out
+
+    def output(self, index, nrows, input):
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
         key = _activation_key(flat)
         if self._last[0] != key:
-            out = SrnmSpmm._run_native(SrnmSpmm, self, flat, self.rows, self.cols)
-            if out is None:
-                rhs = SrnmSpmm._transposed(flat)
-                out = spatha.spmm(self.metadata, self.columns, self.values, rhs, self.bias, self.rows, self.cols, rhs.shape[1],
-                                  self.v, self.n, self.m, 0, 0, 32, 4)
-            self._last = (key, flat, out)
-        return self._last[2]
-
-    def output(self, index, nrows, input):
+            self._last = (key, flat, self.product(flat))
         start = self.starts[index]
-        return self.merged(input)[:, start:start + nrows].reshape(*input.shape[:-1], nrows)
+        return self._last[2][:, start:start + nrows].reshape(*input.shape[:-1], nrows)
 
 
 def merge_qkv(model):
@@ -224,10 +224,12 @@ def _fused_self_attention():
             if group is None or self.attention_head_size != 64 or not self.scaling > 0 or len(group.starts) != 3 \
                     or group.rows != 3 * self.all_head_size \
                     or any(l._group is not group or l._group_index != i or l._forward_hooks or l._forward_pre_hooks
-                           for i, l in enumerate(layers)):
+                           for i, l in enumerate(layers)) \
+                    or not hidden_states.is_cuda or hidden_states.dtype != torch.float16 or hidden_states.numel() == 0:
                 return None
             batch, seq = hidden_states.shape[:2]
-            return spatha._extension().attention(group.merged(hidden_states), batch, seq, self.num_attention_heads, self.scaling)
+            return spatha._extension().attention(group.product(torch.flatten(hidden_states, 0, 1)), batch, seq, self.num_attention_heads,
+                                                 self.scaling)
 
     FusedSelfAttention.__qualname__ = "FusedSelfAttention"
     globals()["FusedSelfAttention"] = FusedSelfAttention
