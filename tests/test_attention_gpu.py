@@ -151,3 +151,45 @@ def test_the_fused_attention_keeps_no_product(gpu, monkeypatch):
     assert torch.equal(att(x)[0], first) and len(computed) == 2 and group._last == (None, None, None)
     q, k, v = att.query(x), att.key(x), att.value(x)
     assert len(computed) == 3 and torch.equal(group._last[2], torch.cat([q, k, v], -1).reshape(80, 3072))
+
+
+def replaced(att):
+    linear = torch.nn.Linear(1024, 1024, device=att.key.values.device, dtype=torch.float16)
+    att.query = linear
+
+
+class Doubling(bert.SrnmSpmm):
+    def forward(self, input):
+        return 2 * super().forward(input)
+
+
+def subclassed(att):
+    att.value.__class__ = Doubling
+
+
+def own_forward(att):
+    forward = att.value.forward
+    att.value.forward = lambda x: 3 * forward(x)
+
+
+@pytest.mark.parametrize("change", [replaced, subclassed, own_forward])
+@torch.no_grad()
+def test_projections_that_do_more_than_the_product_run(gpu, change):
+    from transformers.models.bert.modeling_bert import BertSelfAttention
+
+    att, x = fused_attention(gpu), torch.randn((2, 24, 1024), device=gpu).half()
+    plain = att(x)[0]
+    change(att)
+    got = att(x)[0]
+    assert torch.equal(got, BertSelfAttention.forward(att, x)[0]) and not torch.allclose(got, plain, atol=1e-2)
+
+
+@torch.no_grad()
+def test_a_hook_on_every_module_sees_the_projections(gpu):
+    att, x, seen = fused_attention(gpu), torch.randn((2, 24, 1024), device=gpu).half(), []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, o: seen.append(m))
+    try:
+        att(x)
+    finally:
+        handle.remove()
+    assert all(any(m is p for m in seen) for p in (att.query, att.key, att.value))

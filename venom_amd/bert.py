@@ -220,16 +220,18 @@ def _fused_self_attention():
 
         def _attend(self, hidden_states):
             layers = self.query, self.key, self.value
+            if not all(_runs_as(l, SrnmSpmm) for l in layers) or torch.nn.modules.module._has_any_global_hook():
+                return None
             group = layers[0]._group
             if group is None or self.attention_head_size != 64 or not self.scaling > 0 or len(group.starts) != 3 \
-                    or group.rows != 3 * self.all_head_size \
-                    or any(l._group is not group or l._group_index != i or l._forward_hooks or l._forward_pre_hooks
-                           for i, l in enumerate(layers)) \
+                    or group.rows != 3 * self.all_head_size or any(l._group is not group or l._group_index != i for i, l in enumerate(layers)) \
                     or not hidden_states.is_cuda or hidden_states.dtype != torch.float16 or hidden_states.numel() == 0:
                 return None
+            native = spatha._native("attention")
+            if native is None:
+                return None
             batch, seq = hidden_states.shape[:2]
-            return spatha._extension().attention(group.product(torch.flatten(hidden_states, 0, 1)), batch, seq, self.num_attention_heads,
-                                                 self.scaling)
+            return native(group.product(torch.flatten(hidden_states, 0, 1)), batch, seq, self.num_attention_heads, self.scaling)
 
     FusedSelfAttention.__qualname__ = "FusedSelfAttention"
     globals()["FusedSelfAttention"] = FusedSelfAttention
