@@ -193,3 +193,15 @@ def test_a_hook_on_every_module_sees_the_projections(gpu):
     finally:
         handle.remove()
     assert all(any(m is p for m in seen) for p in (att.query, att.key, att.value))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@torch.no_grad()
+def test_autocast_decides_the_type_of_the_context(gpu, dtype):
+    from transformers.models.bert.modeling_bert import BertSelfAttention
+
+    att, x = fused_attention(gpu), torch.randn((2, 24, 1024), device=gpu).half()
+    with torch.autocast("cuda", dtype=dtype):
+        got, want = att(x)[0], BertSelfAttention.forward(att, x)[0]
+    assert got.dtype == want.dtype == dtype
+    assert (got.double() - want.double()).norm() <= 2e-3 * want.double().norm()          # (two fp16 attentions, or the same bits)

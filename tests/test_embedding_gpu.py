@@ -61,3 +61,18 @@ def test_padded_feature_major_norm(gpu, tokens, hidden):
     padded = guard[64:-64].view(hidden, pitch)
     assert torch.equal(padded[:, :tokens], want.t()) and not padded[:, tokens:].any()
     assert bool((guard[:64] == 7.0).all()) and bool((guard[-64:] == 7.0).all())
+
+
+def one_embedding(gpu):
+    return bert.fuse_add_layernorm(bert.build_bert_large(layers=1).to(gpu).half()).embeddings
+
+
+@torch.no_grad()
+def test_autocast_decides_the_type_of_the_embedding(gpu):
+    """Under autocast LayerNorm runs, and answers, in fp32."""
+    from transformers.models.bert.modeling_bert import BertEmbeddings
+
+    emb, ids = one_embedding(gpu), torch.randint(0, 30522, (2, 24), device=gpu)
+    with torch.autocast("cuda", dtype=torch.float16):
+        got, want = emb(input_ids=ids), BertEmbeddings.forward(emb, ids)
+    assert want.dtype == torch.float32 and got.dtype == torch.float32 and torch.equal(got, want)

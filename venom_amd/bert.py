@@ -225,7 +225,8 @@ def _fused_self_attention():
             group = layers[0]._group
             if group is None or self.attention_head_size != 64 or not self.scaling > 0 or len(group.starts) != 3 \
                     or group.rows != 3 * self.all_head_size or any(l._group is not group or l._group_index != i for i, l in enumerate(layers)) \
-                    or not hidden_states.is_cuda or hidden_states.dtype != torch.float16 or hidden_states.numel() == 0:
+                    or not hidden_states.is_cuda or hidden_states.dtype != torch.float16 or hidden_states.numel() == 0 \
+                    or torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
                 return None
             native = spatha._native("attention")
             if native is None:
@@ -272,6 +273,7 @@ def _fused_embeddings():
                     or not _runs_as(self.dropout, torch.nn.Dropout) or self.dropout.training \
                     or any(not _runs_as(t, torch.nn.Embedding) or t.max_norm is not None for t in tables) \
                     or torch.nn.modules.module._has_any_global_hook() \
+                    or torch.is_autocast_enabled("cuda") \
                     or torch.is_grad_enabled() and any(t.weight.requires_grad for t in tables + (ln,)):
                 return None
             native = spatha._native("embed_layernorm")
