@@ -76,3 +76,13 @@ def test_autocast_decides_the_type_of_the_embedding(gpu):
     with torch.autocast("cuda", dtype=torch.float16):
         got, want = emb(input_ids=ids), BertEmbeddings.forward(emb, ids)
     assert want.dtype == torch.float32 and got.dtype == torch.float32 and torch.equal(got, want)
+
+
+@torch.no_grad()
+def test_a_trace_of_the_embedding_follows_its_ids(gpu):
+    from transformers.models.bert.modeling_bert import BertEmbeddings
+
+    emb = one_embedding(gpu)
+    first, second = (torch.randint(0, 30522, (2, 24), device=gpu) for _ in range(2))
+    traced = torch.jit.trace(emb, (first,), check_trace=False)
+    assert torch.equal(traced(second), BertEmbeddings.forward(emb, second))

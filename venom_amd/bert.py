@@ -273,7 +273,7 @@ def _fused_embeddings():
                     or not _runs_as(self.dropout, torch.nn.Dropout) or self.dropout.training \
                     or any(not _runs_as(t, torch.nn.Embedding) or t.max_norm is not None for t in tables) \
                     or torch.nn.modules.module._has_any_global_hook() \
-                    or torch.is_autocast_enabled("cuda") \
+                    or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() \
                     or torch.is_grad_enabled() and any(t.weight.requires_grad for t in tables + (ln,)):
                 return None
             native = spatha._native("embed_layernorm")
