@@ -86,3 +86,16 @@ def test_a_trace_of_the_embedding_follows_its_ids(gpu):
     first, second = (torch.randint(0, 30522, (2, 24), device=gpu) for _ in range(2))
     traced = torch.jit.trace(emb, (first,), check_trace=False)
     assert torch.equal(traced(second), BertEmbeddings.forward(emb, second))
+
+
+@torch.no_grad()
+def test_transformed_weights_take_the_stock_embedding(gpu):
+    """Tables in batches (vmap) and tables with tangents (forward-mode differentiation)."""
+    emb, ids = one_embedding(gpu), torch.randint(0, 30522, (2, 24), device=gpu)
+    table = emb.word_embeddings.weight
+    tables = torch.stack([table, 2 * table])
+    call = lambda w: torch.func.functional_call(emb, {"word_embeddings.weight": w}, (ids,))
+    got = torch.vmap(call)(tables)
+    assert got.shape == (2, 2, 24, 1024) and all(close(g, call(w)) for g, w in zip(got, tables))
+    _, tangent = torch.func.jvp(call, (table,), (table,))
+    assert float(tangent.abs().max()) > 0

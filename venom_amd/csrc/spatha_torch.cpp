@@ -144,8 +144,15 @@ std::shared_ptr<spatha_spmm_plan> plan_for(const torch::Tensor& values, const to
     return plan;
 }
 
+// memory of its own: no subclass that dispatches to Python and none of functorch's wrappers
+bool plain(const torch::Tensor& t) {
+    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                           c10::DispatchKey::Functionalize});
+    return !t.key_set().has_any(wrapped);
+}
+
 bool weight_ok(const torch::Tensor& t, c10::ScalarType type, int device) {
-    return t.defined() && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
+    return t.defined() && plain(t) && t.is_cuda() && t.get_device() == device && t.scalar_type() == type && t.is_contiguous();
 }
 
 // The V:N:M arrays of a matrix in order on the GPU, magnitude selection and encoding: (values, metadata, columns), or None for what the
@@ -523,7 +530,10 @@ py::object add_layernorm(py::handle input, py::handle addend, const torch::Tenso
 py::object embed_layernorm(const torch::Tensor& ids, const torch::Tensor& types, const torch::Tensor& positions, const torch::Tensor& word,
                            const torch::Tensor& type, const torch::Tensor& position, const torch::Tensor& weight, const torch::Tensor& bias,
                            double eps, bool feature_major) {
-    if (!ids.is_cuda() || ids.layout() != torch::kStrided || ids.dim() != 2 || ids.numel() == 0) return py::none();
+    if (!plain(ids) || !ids.is_cuda() || ids.layout() != torch::kStrided || ids.dim() != 2 || ids.numel() == 0) return py::none();
+    // (a tangent of forward-mode differentiation is the stock operations' to carry on)
+    for (const torch::Tensor* t : {&word, &type, &position, &weight, &bias})
+        if (!plain(*t) || t->_fw_grad(0).defined()) return py::none();
     const int device = (int)ids.get_device();
     const int64_t batch = ids.size(0), seq = ids.size(1), hidden = word.dim() == 2 ? word.size(1) : 0;
     const bool types_shared = types.dim() == 2 && types.size(0) == 1 && types.size(1) >= seq;
