@@ -99,3 +99,14 @@ def test_transformed_weights_take_the_stock_embedding(gpu):
     assert got.shape == (2, 2, 24, 1024) and all(close(g, call(w)) for g, w in zip(got, tables))
     _, tangent = torch.func.jvp(call, (table,), (table,))
     assert float(tangent.abs().max()) > 0
+
+
+@pytest.mark.parametrize("tokens", [7, 8])
+def test_norms_run_in_inference_mode(gpu, tokens):
+    """Its tensors have no version to know a handed-on copy by: none is offered."""
+    norm = bert.fuse_add_layernorm(bert.build_bert_large(layers=1).to(gpu).half(), feature_major=True).encoder.layer[0].attention.output
+    x, r = (torch.randn((1, tokens, 1024), device=gpu).half() for _ in range(2))
+    with torch.no_grad():
+        want = norm(x, r)
+    with torch.inference_mode():
+        assert torch.equal(norm(x, r), want)

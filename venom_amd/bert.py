@@ -91,7 +91,9 @@ class SrnmSpmm(torch.nn.Module):
     @classmethod
     def offer_transposed(cls, x, x_t):
         """A producer that has x[..., features] feature-major already (x_t[features, tokens]) leaves it for the layer that reads
-        x next, in place of the transposed copy that layer would make."""
+        x next, in place of the transposed copy that layer would make.  (An inference tensor has no version to know it by.)"""
+        if x.is_inference():
+            return
         flat = torch.flatten(x, start_dim=0, end_dim=-2)
         key = _activation_key(flat)
         cls._last_rhs = (key, flat, x_t)
