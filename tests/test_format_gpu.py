@@ -98,3 +98,20 @@ def test_arrays_at_odd_addresses_are_decoded_as_before(gpu):
         buf[offset:offset + a.values.numel()] = a.values
         a.values = buf[offset:offset + a.values.numel()]
         same(a.to_dense(), want)
+
+
+def test_decoding_up_to_the_last_row_that_31_bits_count(gpu):
+    """The last rows lie within one stride of 2^31: a row counter of 32 bits would pass it and start again below zero."""
+    rows, cols, m, v = 2 ** 31 - 32, 4, 4, 32
+    if torch.cuda.mem_get_info()[0] < 160 << 30:
+        pytest.skip("needs 107 GB of GPU memory, and as much again to be a good neighbour")
+    a = SrNMTensor.__new__(SrNMTensor)
+    a.n, a.m, a.tileM, a.nrows, a.ncols, a.device = 2, m, v, rows, cols, torch.device("cuda:0")
+    a.values = torch.ones(rows * 16, dtype=torch.float16, device="cuda")
+    a.metadata = torch.full((rows // 2 * 2,), 0x44444444, dtype=torch.int32, device="cuda")             # the first two columns of every group
+    a.columns = torch.arange(4, dtype=torch.int32, device="cuda").repeat(rows // v * 8)
+    dense = a.to_dense()
+    one = 0x3c00
+    assert dense.shape == (rows, cols) and bool((dense.view(torch.int64).view(-1) == one | one << 16).all())
+    del a, dense
+    torch.cuda.empty_cache()

@@ -20,10 +20,12 @@ __global__ __launch_bounds__(256) void decode_kernel(const uint16_t* __restrict_
     const int64_t n_columns = (int64_t)(rows / v) * ngroups * 4, threads = (int64_t)gridDim.x * gridDim.y * 256;
     for (int64_t i = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < n_columns; i += threads)
         if (columns[i] >= (uint32_t)m) *bad = 1u;
-    const int c0 = ((int)blockIdx.x * 64 + (threadIdx.x & 63)) * 8;
-    if (c0 >= cols) return;
-    const int stop = c0 + 8 < cols ? c0 + 8 : cols, g0 = c0 / m;
-    for (int r = (int)blockIdx.y * 4 + (int)(threadIdx.x >> 6); r < rows; r += (int)gridDim.y * 4) {
+    // (rows and columns go up to 2^31 - 1: the counters beyond the last ones need a bit more)
+    const uint32_t first = (blockIdx.x * 64u + (threadIdx.x & 63u)) * 8u;
+    if (first >= (uint32_t)cols) return;
+    const int c0 = (int)first, stop = cols - c0 > 8 ? c0 + 8 : cols, g0 = c0 / m;
+    for (int64_t row = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6); row < rows; row += (int64_t)gridDim.y * 4) {
+        const int r = (int)row;
         const uint16_t* vrow = values + (int64_t)(r >> 4) * 16 * ksp + ((r >> 2) & 3) * 32 + ((r >> 1) & 1) * 4 + (r & 1) * 2;
         const uint32_t* mrow = metadata + (int64_t)(r >> 5) * (ksp >> 3) * 16 + ((r & 31) >> 1);
         const uint32_t* crow = columns + (int64_t)(r / v) * ngroups * 4;
@@ -47,14 +49,14 @@ __global__ __launch_bounds__(256) void decode_kernel(const uint16_t* __restrict_
         } else {
 #pragma unroll
             for (int k = 0; k < 8; k++)
-                if (c0 + k < cols) dst[k] = (uint16_t)out[k];
+                if (k < cols - c0) dst[k] = (uint16_t)out[k];
         }
     }
 }
 
 hipError_t launch_decode_f16(const uint16_t* values, const uint32_t* metadata, const uint32_t* columns, int rows, int cols, int m,
                              int v, int ksp, uint16_t* dense, uint32_t* bad, hipStream_t stream) {
-    const int across = (cols + 511) / 512;
+    const int across = (int)(((int64_t)cols + 511) / 512);
     const dim3 grid((unsigned)across, (unsigned)((rows + 3) / 4 < 65535 ? (rows + 3) / 4 : 65535)), block(256);
     hipLaunchKernelGGL(decode_kernel, grid, block, 0, stream, values, metadata, columns, rows, cols, m, v, ksp, dense, bad);
     return hipGetLastError();
