@@ -239,6 +239,10 @@ int spatha_spmm_run_ws(const spatha_spmm_plan* plan, const uint16_t* B_dev, int 
 int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, int b_pitch, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                            int out_layout, int activation, int fused, void* stream);
 
+/* How spatha_spmm_run_ragged takes N columns, asked before anything is allocated for them: 2 = from B in rows of N entries, 1 = from a
+ * padded B (b_pitch = ROUND_UP(N, 8)) only, 0 = not at all.  fuse: an activation, or a bias with row-major output, is applied. */
+int spatha_spmm_ragged_route(const spatha_spmm_plan* plan, int N, int out_layout, int fuse);
+
 /* spatha_spmm_run_ws (workspace NULL, 0 where none is wanted) for a result that the caller's next operation reads: it is written so that
  * it stays in the memory-side cache.  The other entry points let results of 96 MB and more pass that cache by, which is faster
  * where other data goes through it before the result is read. */

@@ -217,3 +217,26 @@ def test_a_few_tokens_as_they_lie(gpu, rows, cols, m, v, tokens):
                            transposed_out=True)
         assert np.array_equal(out.cpu().numpy().view(np.uint16), want.view(np.uint16))
     assert L.spatha_spmm_run_tokens(plan._handle, dx.data_ptr(), 17, None, dx.data_ptr(), spatha._stream_ptr(gpu)) == 3
+
+
+def test_a_ragged_product_allocates_for_the_route_it_takes(gpu):
+    """A result, and for the staged kernels the padded right-hand side and, row-major, the cut copy: nothing for the routes not taken."""
+    from venom_amd import format as F
+
+    def allocations(call):
+        call()
+        before = torch.cuda.memory_stats(gpu)["allocation.all.allocated"]
+        call()
+        return torch.cuda.memory_stats(gpu)["allocation.all.allocated"] - before
+
+    for rows, cols, v, m, tokens, staged in [(5120, 1280, 64, 10, 1037, True), (1024, 1024, 64, 8, 187, False), (49152, 256, 64, 4, 1037, True)]:
+        vals, meta, columns = F.synthetic_vnm(rows, cols, 2, m, v, seed=tokens)
+        arrays = [torch.from_numpy(a.view("int32") if a.dtype != "float16" else a).to(gpu) for a in (vals, meta, columns)]
+        plan = spatha.SpmmPlan(*arrays, rows, cols, 2, m, v)
+        B, bias = torch.randn((cols, tokens), device=gpu).half(), torch.randn(rows, device=gpu).half()
+        name = plan.kernel_name((tokens + 7) // 8 * 8)
+        assert staged == ("_direct_tile" not in name and "skinny" not in name), name
+        assert allocations(lambda: plan.run(B)) == (3 if staged else 1)
+        assert allocations(lambda: plan.run(B, transposed_out=True)) == (2 if staged else 1)
+        assert allocations(lambda: spatha.spmm(arrays[1], arrays[2], arrays[0], B, bias, rows, cols, tokens, v, 2, m)) == (2 if staged else 1)
+        assert [_lib.lib().spatha_spmm_ragged_route(plan._handle, tokens, layout, 0) for layout in (0, 1)] == ([0, 0] if staged else [2, 2])

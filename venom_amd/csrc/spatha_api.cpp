@@ -942,6 +942,25 @@ int spatha_spmm_run_layer(const spatha_spmm_plan* plan, const uint16_t* B_dev, i
                             workspace_dev, workspace_bytes, true);
 }
 
+namespace {
+// Is `var`, chosen for the next multiple of 8, a kernel that takes N columns of B in rows b_pitch apart, and faster from them than from a
+// padded copy?
+bool ragged_kernel_takes(const spatha_spmm_plan* plan, int var, int b_pitch, int N) {
+    if (var != spatha::SPMM_VARIANT_SKINNY && var != spatha::SPMM_VARIANT_DIRECT64 && var != spatha::SPMM_VARIANT_HDIRECT32) return false;
+    // Loads of two or four columns at odd addresses take the L1 a third longer: 0.3 ns per 64 x 64 block and k-step over the chip
+    // (12288 x 12288 at 128:2:16 and 17 tokens, 9216 of them, 11.5 -> 14.4 us; 49152 x 12288 at 64:2:4, 147456 of them, 132 -> 170;
+    // 16 tokens and fewer, and even counts in their place, level), the padded copy 2.6 us.
+    if (N > 16 && b_pitch % (N <= 32 ? 2 : 4) != 0 && (int64_t)(plan->geo.rows / 64) * plan->S * ((N + 63) / 64) > 8000) return false;
+    return (uint64_t)plan->geo.cols * (uint64_t)b_pitch * 2u < 0xE0000000ull;
+}
+}  // namespace
+
+int spatha_spmm_ragged_route(const spatha_spmm_plan* plan, int N, int out_layout, int fuse) {
+    if (!plan || N <= 0 || N > INT32_MAX - 8) return 0;
+    const int padded = (N + 7) / 8 * 8, var = pick_variant(plan, padded, spatha::SPMM_VARIANT_AUTO, fuse != 0, out_layout);
+    return var < 0 ? 0 : ragged_kernel_takes(plan, var, N, N) ? 2 : ragged_kernel_takes(plan, var, padded, N) ? 1 : 0;
+}
+
 int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, int b_pitch, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                            int out_layout, int activation, int fused, void* stream) {
     if (N <= 0 || N > INT32_MAX - 8 || b_pitch < N || b_pitch > INT32_MAX - 8) return SPATHA_ERR_BAD_ARGUMENT;
@@ -951,14 +970,7 @@ int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, 
     const int status = spatha::plan_run_check(plan, B_dev, padded, bias_dev, out_dev, out_layout, activation, fused != 0,
                                               spatha::SPMM_VARIANT_AUTO, &var);
     if (status != SPATHA_OK) return status;
-    if (var != spatha::SPMM_VARIANT_SKINNY && var != spatha::SPMM_VARIANT_DIRECT64 && var != spatha::SPMM_VARIANT_HDIRECT32)
-        return SPATHA_ERR_UNSUPPORTED;
-    // Loads of two or four columns at odd addresses take the L1 a third longer: 0.3 ns per 64 x 64 block and k-step over the chip
-    // (12288 x 12288 at 128:2:16 and 17 tokens, 9216 of them, 11.5 -> 14.4 us; 49152 x 12288 at 64:2:4, 147456 of them, 132 -> 170;
-    // 16 tokens and fewer, and even counts in their place, level), the padded copy 2.6 us.
-    if (N > 16 && b_pitch % (N <= 32 ? 2 : 4) != 0 && (int64_t)(plan->geo.rows / 64) * plan->S * ((N + 63) / 64) > 8000)
-        return SPATHA_ERR_UNSUPPORTED;
-    if ((uint64_t)plan->geo.cols * (uint64_t)b_pitch * 2u >= 0xE0000000ull) return SPATHA_ERR_UNSUPPORTED;
+    if (!ragged_kernel_takes(plan, var, b_pitch, N)) return SPATHA_ERR_UNSUPPORTED;
     spatha::SpmmParams p = {};
     p.apack = plan->apack; p.rowtab = plan->rowtab;
     p.B = B_dev; p.bias = bias_dev; p.C = out_dev; p.zeros = plan->zeros;

@@ -232,19 +232,22 @@ torch::Tensor cut_columns(const torch::Tensor& full, int64_t columns) {
     return out;
 }
 
-// The product on `tokens` columns of a right-hand side, which may have more (padding), or an undefined tensor where it takes another
-// kernel or a padded right-hand side
-torch::Tensor run_ragged(const spatha_spmm_plan* plan, const torch::Tensor& rhs, int tokens, const uint16_t* bias_ptr, int rows,
-                         bool transposed_out, int activation, bool fused) {
-    if ((uintptr_t)rhs.data_ptr() & 15) return torch::Tensor();
+// The product on a right-hand side of any number of columns where a kernel is chosen that takes it, from rhs as it lies or a padded copy;
+// else an undefined tensor, and `padded` holds the copy for the caller's product.
+torch::Tensor run_ragged(const spatha_spmm_plan* plan, const torch::Tensor& rhs, const uint16_t* bias_ptr, int rows, bool transposed_out,
+                         int activation, bool fused, torch::Tensor& padded) {
+    const int tokens = (int)rhs.size(1), layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
+    const int route = spatha_spmm_ragged_route(plan, tokens, layout, activation != SPATHA_ACT_NONE || (!transposed_out && bias_ptr) ? 1 : 0);
+    const bool as_it_lies = route == 2 && ((uintptr_t)rhs.data_ptr() & 15) == 0;
+    if (!as_it_lies) padded = pad_columns(rhs);
+    if (route == 0) return torch::Tensor();
+    const torch::Tensor& B = as_it_lies ? rhs : padded;
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(rhs.get_device()).stream();
     torch::Tensor out = transposed_out ? torch::empty({tokens, rows}, rhs.options().requires_grad(false))
                                        : torch::empty({rows, tokens}, rhs.options().requires_grad(false));
-    const int status = spatha_spmm_run_ragged(plan, (const uint16_t*)rhs.data_ptr(), (int)rhs.size(1), tokens, bias_ptr,
-                                              (uint16_t*)out.data_ptr(), transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR,
-                                              activation, fused ? 1 : 0, stream);
-    if (status == SPATHA_ERR_UNSUPPORTED) return torch::Tensor();
-    check(status, "spatha_spmm_run_ragged");
+    check(spatha_spmm_run_ragged(plan, (const uint16_t*)B.data_ptr(), (int)B.size(1), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
+                                 activation, fused ? 1 : 0, stream),
+          "spatha_spmm_run_ragged");
     return out;
 }
 
@@ -310,11 +313,8 @@ torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indice
         // bias-only rows / columns, which are dropped).
         hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
         const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values, A_metadata, A_indices, rows, cols, n, m, v, stream);
-        const int act = fused ? activation : SPATHA_ACT_NONE;
-        torch::Tensor out = run_ragged(plan.get(), rhs_matrix, tokens, bias_ptr, rows, transposed_out, act, fused);
-        if (out.defined()) return out;
-        torch::Tensor padded = pad_columns(rhs_matrix);
-        out = run_ragged(plan.get(), padded, tokens, bias_ptr, rows, transposed_out, act, fused);
+        torch::Tensor padded, out = run_ragged(plan.get(), rhs_matrix, bias_ptr, rows, transposed_out, fused ? activation : SPATHA_ACT_NONE,
+                                               fused, padded);
         if (out.defined()) return out;
         torch::Tensor full = run_full(A_metadata, A_indices, A_values, padded, (int)padded.size(1), bias_ptr, rows, cols, v, n, m,
                                       transposed_out, activation, fused, !transposed_out);
@@ -583,11 +583,7 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
     if (ragged) {
         if (!fused && !transposed_out && bias_ptr) return py::none();          // (refused)
         const torch::NoGradGuard no_grad;
-        torch::Tensor got = run_ragged(plan, B, N, bias_ptr, rows, transposed_out, activation, fused), padded;
-        if (!got.defined()) {
-            padded = pad_columns(B);
-            got = run_ragged(plan, padded, N, bias_ptr, rows, transposed_out, activation, fused);
-        }
+        torch::Tensor padded, got = run_ragged(plan, B, bias_ptr, rows, transposed_out, activation, fused, padded);
         if (!got.defined()) {
             const int64_t n_padded = padded.size(1);
             got = transposed_out ? torch::empty({n_padded, rows}, B.options().requires_grad(false))
