@@ -63,10 +63,10 @@ def test_attention_refuses_what_it_does_not_take(gpu):
     assert spatha._extension().attention(x, 2, 8, 1, 0.125) is None
 
 
+@torch.no_grad()
 def test_a_models_attention_takes_the_kernel_and_falls_back(gpu):
     """Without a mask the merged attention runs in the kernel; with one, in training mode or with a hook on a projection the stock
     forward answers.  Two fp16 attentions: 2e-3 apart at most (each within 6e-4 of the exact result)."""
-    torch.set_grad_enabled(False)
     model = bert.merge_qkv(bert.linear_to_spmm(bert.build_bert_large(layers=1).to(gpu).half(), 2, 8, 64))
     stock = model.encoder.layer[0].attention.self
     x = torch.randn((2, 40, 1024), device=gpu).half()

@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from venom_amd import _lib, bert
+from venom_amd import _lib, bert, spatha
 
 pytestmark = pytest.mark.gpu
 
@@ -18,8 +18,8 @@ def close(got, want):
 
 @pytest.mark.parametrize("batch,seq", [(1, 1), (2, 5), (3, 31), (1, 33), (2, 324), (5, 77), (4, 512)])
 @pytest.mark.parametrize("types", [None, "given"])
+@torch.no_grad()
 def test_fused_embedding_equals_the_stock_module(gpu, batch, seq, types):
-    torch.set_grad_enabled(False)
     stock = bert.build_bert_large(layers=1).to(gpu).half()
     fused = bert.fuse_add_layernorm(bert.merge_qkv(bert.linear_to_spmm(bert.build_bert_large(layers=1).to(gpu).half(), 2, 8, 64)), feature_major=True)
     emb = fused.embeddings
@@ -45,8 +45,6 @@ def test_fused_embedding_equals_the_stock_module(gpu, batch, seq, types):
 
 @pytest.mark.parametrize("tokens,hidden", [(1, 1024), (7, 512), (33, 1024), (75, 768), (1037, 1280), (9, 4096), (130, 72)])
 def test_padded_feature_major_norm(gpu, tokens, hidden):
-    from venom_amd import spatha
-
     gen = torch.Generator(device=gpu).manual_seed(tokens + hidden)
     x, r = (torch.randn((tokens, hidden), generator=gen, device=gpu).half() for _ in range(2))
     w, b = ((0.1 * torch.randn(hidden, generator=gen, device=gpu)).half() for _ in range(2))
@@ -110,3 +108,38 @@ def test_norms_run_in_inference_mode(gpu, tokens):
         want = norm(x, r)
     with torch.inference_mode():
         assert torch.equal(norm(x, r), want)
+
+
+@pytest.mark.parametrize("batch,seq", [(3, 37), (2, 64)])
+@torch.no_grad()
+def test_the_whole_fused_encoder_tracks_the_unfused_one(gpu, monkeypatch, batch, seq):
+    """Every fusion at once, two layers: the kernels run, every right-hand side is handed on (no layer makes a transposed copy of its own),
+    and the last hidden state is the unfused layers'.  Each is off by 7e-4 (norm) from the same encoder in fp32: twice that apart."""
+    def build():
+        torch.manual_seed(11)
+        return bert.linear_to_spmm(bert.build_bert_large(layers=2).to(gpu).half(), 2, 8, 64, magnitude=True)
+
+    plain = build()
+    fused = bert.fuse_add_layernorm(bert.merge_qkv(bert.fuse_feed_forward(build(), activation_in_kernel=True)), feature_major=True)
+    ext, calls, copies = spatha._extension(), [], []
+
+    def counted(name):
+        native = getattr(ext, name)
+
+        def call(*args):
+            calls.append(name)
+            got = native(*args)
+            assert got is not None
+            if name == "layer_spmm" and got[1] is not None:
+                copies.append(args[0].shape)
+            return got
+        monkeypatch.setattr(ext, name, call)
+
+    ids = torch.randint(0, 30522, (batch, seq), device=gpu)
+    want = plain(ids).last_hidden_state
+    for name in ("embed_layernorm", "layer_spmm", "attention", "add_layernorm"):
+        counted(name)
+    got = fused(ids).last_hidden_state
+    one = ["layer_spmm", "attention", "layer_spmm", "add_layernorm", "layer_spmm", "layer_spmm", "add_layernorm"]
+    assert calls == ["embed_layernorm"] + 2 * one and not copies
+    assert (got.double() - want.double()).norm() <= 1.4e-3 * want.double().norm()
