@@ -244,8 +244,9 @@ int spatha_spmm_run_ragged(const spatha_spmm_plan* plan, const uint16_t* B_dev, 
 int spatha_spmm_ragged_route(const spatha_spmm_plan* plan, int N, int out_layout, int fuse);
 
 /* spatha_spmm_run_ws (workspace NULL, 0 where none is wanted) for a result that the caller's next operation reads: it is written so that
- * it stays in the memory-side cache.  The other entry points let results of 96 MB and more pass that cache by, which is faster
- * where other data goes through it before the result is read. */
+ * it stays in the memory-side cache.  The other entry points let results of 96 MB and more pass that cache by (where the chosen kernel writes
+ * whole 16-byte pieces of rows, and row-major with N % 32 == 0), which is faster where other data goes through it before the result
+ * is read or written again, and up to 8 % slower where nothing does. */
 int spatha_spmm_run_layer(const spatha_spmm_plan* plan, const uint16_t* B_dev, int N, const uint16_t* bias_dev, uint16_t* out_dev,
                           int out_layout, int activation, void* workspace_dev, size_t workspace_bytes, void* stream);
 

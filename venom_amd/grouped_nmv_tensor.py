@@ -79,7 +79,7 @@ class SrNMTensor:
     @classmethod
     def from_magnitude(cls, dense, n, m, tileM):
         """What `SrNMTensor(n, m, tileM, dense, *nm_vector_mask_sparsify(dense, n, m, tileM, exact_ties=False), dense.device)`
-        holds, for a matrix on the GPU: selected and encoded there by two kernels on torch's current stream, without a trip
+        holds, for a matrix on the GPU: selected and encoded there, in one launch or two, on torch's current stream, without a trip
         through the host."""
         self = cls.__new__(cls)
         self.n, self.m, self.tileM = n, m, tileM
