@@ -15,6 +15,7 @@ struct SpmmParams {
     const uint32_t* rowtab;   // gathered B row per LDS row
     const uint16_t* gtab;     // dense-staged kernels: LDS offset per (64-row block, step, lane class, fragment), or null
     uint32_t gtab_bytes;      // size of gtab (buffer descriptor of the unified dense-staged kernel)
+    int b_pitch;              // columns from one row of B to the next (the direct kernels; N everywhere else)
     const uint16_t* B;        // cols x N, row-major
     const uint16_t* bias;     // rows, or null
     const void* zeros;        // >= 1 KiB of zero bytes (source of zero-filled B rows)
@@ -38,7 +39,6 @@ struct SpmmParams {
     int fuse;                 // 1: bias and activation are applied ahead of the write-out (fused_bias_act)
     int act;                  // SPATHA_ACT_*
     int debug;                // development knobs (0 in production): 1 = skip B loads, 2 = skip C stores
-    int b_pitch;              // columns from one row of B to the next (the direct kernels; N everywhere else)
     int stream_out;           // 1: C leaves by non-temporal stores (read on the host: StreamedParams)
 };
 

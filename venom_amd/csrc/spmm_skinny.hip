@@ -13,9 +13,11 @@ namespace spatha {
 // multiplied.
 // NB = 1, 2 or 4 column blocks of 16.  Column block nb holds the columns NB * j + nb (j = 0 .. 15), not 16 * nb + j: lane j of
 // a block then needs NB ADJACENT columns of every gathered row, one load of 2 * NB bytes instead of NB loads of 2 bytes - 16
-// vector-memory instructions per k-step whatever NB.  B (rows b_pitch apart) and C are addressed at whatever alignment their rows
-// have, so that a ragged token count needs no padded copies (spatha_spmm_run_ragged: 4096 x 1024 at 64:2:8 and 301 tokens with GELU,
-// row-major, 9.5 us, 23.0 with a launch for each copy).
+// vector-memory instructions per k-step whatever NB.  N is a multiple of 8, so the NB columns of a lane lie all inside N or all
+// outside; RAGGED: any N, B (rows b_pitch apart) and C addressed at whatever alignment their rows have, so that a ragged token count
+// needs no padded copies (spatha_spmm_run_ragged: 4096 x 1024 at 64:2:8 and 301 tokens with GELU, row-major, 9.5 us, 23.0 with a
+// launch for each copy).  Instances of their own: one for all counts took 2-5 % longer at multiples of 8 (768 x 3072 x 760 at 128:2:8
+// 8.7 -> 8.9 us, 768 x 768 x 48 at 64:2:40 3.1 -> 3.3).
 // What bounds it: with few tiles the trip to memory that a k-step's loads take (four waves a tile left 16 .. 192 of 256 CUs with
 // one wave per SIMD and fewer than two steps in flight: 12288 x 12288 at 64:2:8 and 8 tokens 25.1 us for 101 MB; sixteen waves:
 // 16.0); with many, the 12.8 KB of loads per 64 x 64 block and k-step through the L1 (0.8-1.2 ns a block and step over the chip).
@@ -27,9 +29,13 @@ namespace spatha {
 // halfs between two tokens in LDS: odd in 32-bit words, so that the sixteen tokens of a fragment row sit on different banks
 __host__ __device__ constexpr int token_pitch_halfs(int cols) { return (((cols + 7) / 8 * 4) | 1) * 2; }
 
-// adjacent columns of C at whatever alignment
-struct __attribute__((packed, aligned(2))) Piece4 { half4_t v; };
-struct __attribute__((packed, aligned(2))) Piece2 { half2_t v; };
+// adjacent columns of C; ANYWHERE: at whatever alignment
+template <bool ANYWHERE, class Columns>
+__device__ __forceinline__ void store_columns(uint16_t* dst, Columns v) {
+    struct __attribute__((packed, aligned(2))) Piece { Columns v; };
+    if (ANYWHERE) ((Piece*)dst)->v = v;
+    else *(Columns*)dst = v;
+}
 
 template <int NB, int W, bool HALF, bool LEAN>
 struct DirectCfg {
@@ -43,7 +49,7 @@ struct DirectCfg {
     static_assert(W * PB * NB <= 64, "partial tiles exceed 64 KB");
 };
 
-template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN = false, bool TOKEN_MAJOR = false>
+template <int NB, int OUT_LAYOUT, int W, bool HALF, bool LEAN, bool TOKEN_MAJOR, bool RAGGED>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu((DirectCfg<NB, W, HALF, LEAN>::WAVES_PER_EU))))
 void spmm_direct_kernel(SpmmParams p) {
     using Cfg = DirectCfg<NB, W, HALF, LEAN>;
@@ -56,6 +62,10 @@ void spmm_direct_kernel(SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int S = p.S, N = p.N;
+    int b_pitch = RAGGED ? p.b_pitch : N;
+    uint32_t b_bytes = p.b_bytes;
+    // (read at the start: left to the compiler, the first load of B waits for them, 0.1 us)
+    if constexpr (RAGGED) asm volatile("" : "+s"(b_pitch), "+s"(b_bytes));
     // an XCD owns a contiguous range of tiles, row tile after row tile (the packed A of a row tile enters one L2 only) or, with
     // walk_group 1, column tile after column tile (the same for a column of B)
     const int tiles = p.tiles_m * p.tiles_n, chunk = (tiles + 7) >> 3;
@@ -69,8 +79,8 @@ void spmm_direct_kernel(SpmmParams p) {
     const int64_t vb = ((int64_t)tile * (16 * MB)) / p.v;
     const char* a_tile = (const char*)p.apack + block * S * APACK_BLOCK;
     const uint32_t* rt_block = p.rowtab + vb * S * 64;
-    __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, (int)p.b_bytes, 0x00020000);
-    const uint32_t row_bytes = (uint32_t)p.b_pitch * 2u;
+    __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, (int)b_bytes, 0x00020000);
+    const uint32_t row_bytes = (uint32_t)b_pitch * 2u;
 
     float4_t acc[MB][NB];
 #pragma unroll
@@ -94,13 +104,13 @@ void spmm_direct_kernel(SpmmParams p) {
 #pragma unroll
         for (int d = 0; d < MB / 2; d++) x.ix[d] = *(const uint32_t*)(q + 4096 + (half + d) * 256 + lane * 4);
     };
-    // This lane's NB columns, col0 + nb.  Where rows of B have no padding that the last lane's could reach into, that lane moves down.
+    // This lane's NB columns, col0 + nb.  Where ragged rows of B have no padding that the last lane's could reach into, that lane moves down.
     const int lane_col = (tile_n * 16 + li) * NB;
-    const int col0 = p.b_pitch % NB != 0 && lane_col > N - NB ? N - NB : lane_col;
-    // (lanes beyond N fetch nothing in groups of four; single ones fetch what the last lane does: four lanes of which some are out of the
-    // descriptor's range take the load a third longer - 49152 x 12288 at 64:2:4 and 18 tokens 170 against 132 us)
+    const int col0 = RAGGED && b_pitch % NB != 0 && lane_col > N - NB ? N - NB : lane_col;
+    // (lanes beyond a ragged N fetch nothing in groups of four; single ones fetch what the last lane does: four lanes of which some are out
+    // of the descriptor's range take the load a third longer - 49152 x 12288 at 64:2:4 and 18 tokens 170 against 132 us)
     const bool fetches = lane_col < (N + 4 * NB - 1) / (4 * NB) * (4 * NB), stores = lane_col < N;
-    const uint32_t fetch_col = (uint32_t)(lane_col < N ? col0 : p.b_pitch % NB != 0 ? N - NB : (N - 1) / NB * NB);
+    const uint32_t fetch_col = (uint32_t)(!RAGGED || lane_col < N ? col0 : b_pitch % NB != 0 ? N - NB : (N - 1) / NB * NB);
     const int token_pitch = token_pitch_halfs(p.cols);
     if constexpr (TOKEN_MAJOR) {
         // x [N][cols] -> LDS as it lies; columns N .. 15 of the tile are never stored, they multiply token 0
@@ -133,7 +143,7 @@ void spmm_direct_kernel(SpmmParams p) {
                     bf[0][fb * 4 + j] = __builtin_bit_cast(_Float16, (uint16_t)(row != 0xFFFFFFFFu ? h : 0));
                     continue;
                 }
-                const uint32_t voff = (row != 0xFFFFFFFFu && fetches) ? row * row_bytes + fetch_col * 2u : 0xF0000000u;
+                const uint32_t voff = (row != 0xFFFFFFFFu && (RAGGED ? fetches : col0 < N)) ? row * row_bytes + fetch_col * 2u : 0xF0000000u;
                 if constexpr (NB == 1) {
                     const uint16_t h = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc_b, (int)voff, 0, 0);
                     bf[0][fb * 4 + j] = __builtin_bit_cast(_Float16, h);
@@ -247,29 +257,25 @@ void spmm_direct_kernel(SpmmParams p) {
                     for (int r = 0; r < 4; r++) h4[c][r] = (_Float16)act_gelu_tanh((float)h4[c][r]);
             }
             const int col = col0 + nb0;
-            if (!stores || SPATHA_KNOB(2)) continue;
+            if ((RAGGED ? !stores : col >= N) || SPATHA_KNOB(2)) continue;
             if (OUT_LAYOUT == SPATHA_OUT_TRANSPOSED) {
 #pragma unroll
                 for (int c = 0; c < CB; c++)
-                    if (CB == 1 || col + c < N) *(half4_t*)(p.C + (int64_t)(col + c) * p.rows + row0) = h4[c];
+                    if (!RAGGED || CB == 1 || col + c < N) *(half4_t*)(p.C + (int64_t)(col + c) * p.rows + row0) = h4[c];
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     uint16_t* dst = p.C + (row0 + r) * N + col;
-                    if constexpr (CB == 4) {
-                        if (col + 4 <= N) {
-                            ((Piece4*)dst)->v = (half4_t){h4[0][r], h4[1][r], h4[2][r], h4[3][r]};
-                            continue;
-                        }
-                    } else if constexpr (CB == 2) {
-                        if (col + 2 <= N) {
-                            ((Piece2*)dst)->v = (half2_t){h4[0][r], h4[1][r]};
-                            continue;
-                        }
-                    }
+                    if constexpr (CB == 1) {
+                        *(_Float16*)dst = h4[0][r];
+                    } else if (!RAGGED || col + CB <= N) {
+                        if constexpr (CB == 4) store_columns<RAGGED>(dst, (half4_t){h4[0][r], h4[1][r], h4[2][r], h4[3][r]});
+                        else store_columns<RAGGED>(dst, (half2_t){h4[0][r], h4[1][r]});
+                    } else {
 #pragma unroll
-                    for (int c = 0; c < CB; c++)
-                        if (CB == 1 || col + c < N) *((_Float16*)dst + c) = h4[c][r];
+                        for (int c = 0; c < CB; c++)
+                            if (col + c < N) *((_Float16*)dst + c) = h4[c][r];
+                    }
                 }
             }
         }
@@ -284,7 +290,9 @@ static hipError_t launch_direct(SpmmParams p, hipStream_t stream) {
     // B 17 MB: 13.4 us column after column, 20.7 row after row; 1280 x 5120 x 104 at 64:2:8, A 3.7, B 1.1 MB: 8.9 against 7.2.)
     p.walk_group = p.b_bytes > p.apack_bytes ? 1 : 0;
     const int tiles = p.tiles_m * p.tiles_n;
-    hipLaunchKernelGGL((spmm_direct_kernel<NB, OUT_LAYOUT, W, HALF, LEAN>), dim3((tiles + 7) / 8 * 8), dim3(W * 64), 0, stream, p);
+    auto kern = p.N % 8 == 0 && p.b_pitch == p.N ? spmm_direct_kernel<NB, OUT_LAYOUT, W, HALF, LEAN, false, false>
+                                                 : spmm_direct_kernel<NB, OUT_LAYOUT, W, HALF, LEAN, false, true>;
+    hipLaunchKernelGGL(kern, dim3((tiles + 7) / 8 * 8), dim3(W * 64), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -378,7 +386,7 @@ static hipError_t launch_token_major(SpmmParams p, hipStream_t stream) {
     p.walk_group = 0;
     const size_t tokens = (size_t)p.N * token_pitch_halfs(p.cols) * 2, partial = (size_t)W * Cfg::PB * 64 * sizeof(float4_t);
     const size_t lds = ((tokens > partial ? tokens : partial) + 15) / 16 * 16;
-    auto kern = spmm_direct_kernel<1, SPATHA_OUT_TRANSPOSED, W, HALF, false, true>;
+    auto kern = spmm_direct_kernel<1, SPATHA_OUT_TRANSPOSED, W, HALF, false, true, false>;
     if (lds > 48 * 1024) {
         bool& attr_set = lds_attr_flag((const void*)kern);
         if (!attr_set) {
