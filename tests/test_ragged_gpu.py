@@ -240,3 +240,17 @@ def test_a_ragged_product_allocates_for_the_route_it_takes(gpu):
         assert allocations(lambda: plan.run(B, transposed_out=True)) == (2 if staged else 1)
         assert allocations(lambda: spatha.spmm(arrays[1], arrays[2], arrays[0], B, bias, rows, cols, tokens, v, 2, m)) == (2 if staged else 1)
         assert [_lib.lib().spatha_spmm_ragged_route(plan._handle, tokens, layout, 0) for layout in (0, 1)] == ([0, 0] if staged else [2, 2])
+
+
+@pytest.mark.parametrize("v,tokens", [(64, 17), (64, 24), (32, 17)])
+def test_refusals_carry_their_status(gpu, v, tokens):
+    """A bias at an address that the kernels do not read: the same error for ragged counts as for others."""
+    from venom_amd import format as F
+
+    vals, meta, columns = F.synthetic_vnm(128, 128, 2, 8, v, seed=1)
+    plan = spatha.SpmmPlan(torch.from_numpy(vals).to(gpu), torch.from_numpy(meta.view("int32")).to(gpu),
+                           torch.from_numpy(columns.view("int32")).to(gpu), 128, 128, 2, 8, v)
+    bias = torch.zeros(136, dtype=torch.float16, device=gpu)[1:129]
+    with pytest.raises(_lib.SpathaError) as refused:
+        plan.run(torch.zeros((128, tokens), dtype=torch.float16, device=gpu), bias, transposed_out=True)
+    assert refused.value.status == _lib.ERR_BAD_ARGUMENT

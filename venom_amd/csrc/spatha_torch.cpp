@@ -233,9 +233,10 @@ torch::Tensor cut_columns(const torch::Tensor& full, int64_t columns) {
 }
 
 // The product on a right-hand side of any number of columns where a kernel is chosen that takes it, from rhs as it lies or a padded copy;
-// else an undefined tensor, and `padded` holds the copy for the caller's product.
+// else an undefined tensor, and `padded` holds the copy for the caller's product.  status: of that kernel's run, which may be a refusal.
 torch::Tensor run_ragged(const spatha_spmm_plan* plan, const torch::Tensor& rhs, const uint16_t* bias_ptr, int rows, bool transposed_out,
-                         int activation, bool fused, torch::Tensor& padded) {
+                         int activation, bool fused, torch::Tensor& padded, int& status) {
+    status = SPATHA_OK;
     const int tokens = (int)rhs.size(1), layout = transposed_out ? SPATHA_OUT_TRANSPOSED : SPATHA_OUT_ROW_MAJOR;
     const int route = spatha_spmm_ragged_route(plan, tokens, layout, activation != SPATHA_ACT_NONE || (!transposed_out && bias_ptr) ? 1 : 0);
     const bool as_it_lies = route == 2 && ((uintptr_t)rhs.data_ptr() & 15) == 0;
@@ -245,9 +246,8 @@ torch::Tensor run_ragged(const spatha_spmm_plan* plan, const torch::Tensor& rhs,
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(rhs.get_device()).stream();
     torch::Tensor out = transposed_out ? torch::empty({tokens, rows}, rhs.options().requires_grad(false))
                                        : torch::empty({rows, tokens}, rhs.options().requires_grad(false));
-    check(spatha_spmm_run_ragged(plan, (const uint16_t*)B.data_ptr(), (int)B.size(1), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
-                                 activation, fused ? 1 : 0, stream),
-          "spatha_spmm_run_ragged");
+    status = spatha_spmm_run_ragged(plan, (const uint16_t*)B.data_ptr(), (int)B.size(1), tokens, bias_ptr, (uint16_t*)out.data_ptr(), layout,
+                                    activation, fused ? 1 : 0, stream);
     return out;
 }
 
@@ -313,8 +313,10 @@ torch::Tensor run(const torch::Tensor& A_metadata, const torch::Tensor& A_indice
         // bias-only rows / columns, which are dropped).
         hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(A_values.get_device()).stream();
         const std::shared_ptr<spatha_spmm_plan> plan = plan_for(A_values, A_metadata, A_indices, rows, cols, n, m, v, stream);
+        int status;
         torch::Tensor padded, out = run_ragged(plan.get(), rhs_matrix, bias_ptr, rows, transposed_out, fused ? activation : SPATHA_ACT_NONE,
-                                               fused, padded);
+                                               fused, padded, status);
+        check(status, "spatha_spmm_run_ragged");
         if (out.defined()) return out;
         torch::Tensor full = run_full(A_metadata, A_indices, A_values, padded, (int)padded.size(1), bias_ptr, rows, cols, v, n, m,
                                       transposed_out, activation, fused, !transposed_out);
@@ -583,7 +585,9 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
     if (ragged) {
         if (!fused && !transposed_out && bias_ptr) return py::none();          // (refused)
         const torch::NoGradGuard no_grad;
-        torch::Tensor padded, got = run_ragged(plan, B, bias_ptr, rows, transposed_out, activation, fused, padded);
+        int status;
+        torch::Tensor padded, got = run_ragged(plan, B, bias_ptr, rows, transposed_out, activation, fused, padded, status);
+        if (status != SPATHA_OK) return py::int_(status);
         if (!got.defined()) {
             const int64_t n_padded = padded.size(1);
             got = transposed_out ? torch::empty({n_padded, rows}, B.options().requires_grad(false))
@@ -592,11 +596,10 @@ py::object plan_run(size_t handle, py::handle rhs, py::handle bias, py::handle o
             const uint16_t* b_ptr = (const uint16_t*)padded.data_ptr();
             uint16_t* c_ptr = (uint16_t*)got.data_ptr();
             // (a row-major result is read at once, by the cut)
-            const int status = !transposed_out ? spatha_spmm_run_layer(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_ROW_MAJOR,
-                                                                       activation, nullptr, 0, stream)
-                               : fused ? spatha_spmm_run_fused(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, activation,
-                                                               0, stream)
-                                       : spatha_spmm_run(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, 0, stream);
+            status = !transposed_out ? spatha_spmm_run_layer(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_ROW_MAJOR, activation,
+                                                             nullptr, 0, stream)
+                     : fused ? spatha_spmm_run_fused(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, activation, 0, stream)
+                             : spatha_spmm_run(plan, b_ptr, (int)n_padded, bias_ptr, c_ptr, SPATHA_OUT_TRANSPOSED, 0, stream);
             if (status != SPATHA_OK) return py::int_(status);
             got = transposed_out ? got.narrow(0, 0, N) : cut_columns(got, N);
         }
