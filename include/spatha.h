@@ -351,6 +351,14 @@ int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev,
                                const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps,
                                int hidden, uint16_t* out_dev, uint16_t* out_t_dev, void* stream);
 
+/* The same with types looked up at the position ids, as the stock module does with the row of token types that it keeps:
+ * type[types_row_dev[positions[s]]].  A position outside that row (types_row entries) ends the kernel with a trap too. */
+int spatha_embed_layernorm_own_types_f16(const int64_t* ids_dev, const int64_t* types_row_dev, int64_t types_row, const int64_t* positions_dev,
+                                         int batch, int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev,
+                                         int64_t types, const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev,
+                                         const uint16_t* beta_dev, float eps, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
+                                         void* stream);
+
 /* out_t[64 * head + f][token] = the attention of every sequence and head of a batch, softmax(scale * Q K^T) V over the sequence's own
  * tokens, no mask: q, k and v hold batch * seq rows `pitch` entries apart, head h at column 64 h (slices of one merged
  * projection, for instance); fp16 in and out, fp32 scores, sums and output, probabilities rounded to fp16.  The result is

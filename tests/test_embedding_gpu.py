@@ -99,6 +99,22 @@ def test_transformed_weights_take_the_stock_embedding(gpu):
     assert float(tangent.abs().max()) > 0
 
 
+@pytest.mark.parametrize("feature_major", [False, True])
+@pytest.mark.parametrize("batch,seq", [(1, 1), (2, 31), (3, 512)])
+@torch.no_grad()
+def test_the_models_own_types_go_by_position(gpu, feature_major, batch, seq):
+    """The stock module looks its row of token types up at the position ids, and takes a caller's as they lie."""
+    from transformers.models.bert.modeling_bert import BertEmbeddings
+
+    emb = one_embedding(gpu)
+    emb.feature_major = feature_major
+    emb.token_type_ids = (torch.arange(512, device=gpu) * 7 // 5 % 2)[None]
+    emb.position_ids = (torch.arange(512, device=gpu) * 5 + 3).remainder(512)[None]
+    ids = torch.randint(0, 30522, (batch, seq), device=gpu)
+    for types in (None, emb.token_type_ids[:, :seq], emb.token_type_ids[:, :seq].expand(batch, seq).contiguous()):
+        assert close(emb(input_ids=ids, token_type_ids=types), BertEmbeddings.forward(emb, ids, types))
+
+
 @pytest.mark.parametrize("tokens", [7, 8])
 def test_norms_run_in_inference_mode(gpu, tokens):
     """Its tensors have no version to know a handed-on copy by: none is offered."""

@@ -113,7 +113,7 @@ def test_a_hook_on_every_module_sees_the_embeddings_norm(kernels):
                                                    (2, 6, (1, 9), False), (1, 6, (1, 512), False), (1, 1, (1, 9), False), (2, 1, (1, 2), False),
                                                    (2, 6, (1, 1), False), (2, 6, (2, 1), False)])
 def test_token_types_of_a_caller_have_the_ids_length(kernels, batch, seq, types, taken):
-    """The model's own row of token types is longer than the sequence and cut; a caller's is not."""
+    """The model's own row of token types is longer than the sequence; a caller's is not."""
     stock, fused = make_embeddings(), fused_embeddings()
     ids = torch.arange(batch * seq).reshape(batch, seq)
     tt = None if types is None else torch.ones(types, dtype=torch.int64)

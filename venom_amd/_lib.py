@@ -77,6 +77,8 @@ SIGNATURES = {
     "spatha_add_layernorm_f16_tp": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "spatha_embed_layernorm_f16": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                            c_int64, c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p]),
+    "spatha_embed_layernorm_own_types_f16": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p, c_int64, c_void_p, c_int64,
+                                                     c_void_p, c_int64, c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p]),
     "spatha_attention_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_void_p]),
     "spatha_cut_columns_f16": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p]),
     "spatha_add_layernorm_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_void_p]),

@@ -267,7 +267,8 @@ def _fused_embeddings():
             tables = self.word_embeddings, self.token_type_embeddings, self.position_embeddings
             ln = self.LayerNorm
             types = token_type_ids if token_type_ids is not None else getattr(self, "token_type_ids", None)
-            # (the model's own row of token types covers its longest sequence and is cut; a caller's has the ids' length)
+            # (the model's own row of token types covers its longest sequence and is looked up at the position ids; a caller's has the ids'
+            # length)
             if types is None or type(input_ids) is not torch.Tensor \
                     or token_type_ids is not None and token_type_ids.shape[-1:] != input_ids.shape[-1:] \
                     or getattr(self, "position_embedding_type", "absolute") != "absolute" \
@@ -280,7 +281,7 @@ def _fused_embeddings():
                 return None
             native = spatha._native("embed_layernorm")
             return native and native(input_ids, types, self.position_ids, *(t.weight for t in tables), ln.weight, ln.bias, ln.eps,
-                                     self.feature_major)
+                                     self.feature_major, token_type_ids is None)
 
     FusedEmbeddings.__qualname__ = "FusedEmbeddings"
     globals()["FusedEmbeddings"] = FusedEmbeddings

@@ -40,8 +40,8 @@ struct LnArgs {
 };
 struct EmbeddingArgs : LnArgs {
     const uint16_t* third;
-    const int64_t *ids, *types, *positions;      // per token; per token or (types_stride 0) per position; per position
-    int64_t types_stride;
+    const int64_t *ids, *types, *positions;      // per token; per token, (types_stride 0) per position or (types_row) per position id; per position
+    int64_t types_stride, types_row;             // types_row: entries of `types` where that is looked up at the position ids, else 0
     int seq;
     int64_t n_x, n_residual, n_third;            // table rows
 };
@@ -60,9 +60,10 @@ struct LnRows {
     __device__ __forceinline__ LnRows(const Args<EMB>& a, const uint16_t* x0, const uint16_t* residual0, int64_t token) {
         if constexpr (EMB) {
             const int64_t b = token / a.seq, s = token - b * a.seq;
+            const int64_t position = a.positions[s], at = a.types_row ? table_row(position, a.types_row) : b * a.types_stride + s;
             x = x0 + table_row(a.ids[token], a.n_x) * a.hidden;
-            residual = residual0 + table_row(a.types[b * a.types_stride + s], a.n_residual) * a.hidden;
-            third = a.third + table_row(a.positions[s], a.n_third) * a.hidden;
+            residual = residual0 + table_row(a.types[at], a.n_residual) * a.hidden;
+            third = a.third + table_row(position, a.n_third) * a.hidden;
         } else {
             x = x0 + token * a.hidden;
             residual = residual0 + token * a.hidden;         // (read only where there is one)
@@ -289,13 +290,13 @@ hipError_t launch_add_layernorm_f16(const uint16_t* x, const uint16_t* residual,
 }
 
 hipError_t launch_embed_layernorm_f16(const EmbeddingTables& t, const int64_t* ids, const int64_t* types, int64_t types_stride,
-                                      const int64_t* positions, int batch, int seq, const uint16_t* gamma, const uint16_t* beta, float eps,
-                                      uint16_t* out, uint16_t* out_t, hipStream_t stream) {
+                                      int64_t types_row, const int64_t* positions, int batch, int seq, const uint16_t* gamma,
+                                      const uint16_t* beta, float eps, uint16_t* out, uint16_t* out_t, hipStream_t stream) {
     EmbeddingArgs a = {};
     a.eps = eps; a.tokens = batch * seq; a.hidden = t.hidden; a.out_t_pitch = (a.tokens + 7) / 8 * 8;
     a.third = t.position;
     a.n_x = t.words; a.n_residual = t.types; a.n_third = t.positions;
-    a.ids = ids; a.types = types; a.types_stride = types_stride; a.positions = positions; a.seq = seq;
+    a.ids = ids; a.types = types; a.types_stride = types_stride; a.types_row = types_row; a.positions = positions; a.seq = seq;
     return launch_norm<true>(a, {t.word, t.type, gamma, beta, out, out_t}, stream);
 }
 

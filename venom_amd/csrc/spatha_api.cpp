@@ -1177,10 +1177,11 @@ int spatha_add_layernorm_f16_tp(const uint16_t* x_dev, const uint16_t* residual_
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
 }
 
-int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev, int64_t types_stride, const int64_t* positions_dev, int batch,
-                               int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev, int64_t types,
-                               const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps,
-                               int hidden, uint16_t* out_dev, uint16_t* out_t_dev, void* stream) {
+static int embed_layernorm(const int64_t* ids_dev, const int64_t* types_dev, int64_t types_stride, int64_t types_row,
+                           const int64_t* positions_dev, int batch, int seq, const uint16_t* word_dev, int64_t words,
+                           const uint16_t* type_dev, int64_t types, const uint16_t* position_dev, int64_t positions,
+                           const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps, int hidden, uint16_t* out_dev,
+                           uint16_t* out_t_dev, void* stream) {
     if (!ids_dev || !types_dev || !positions_dev || !word_dev || !type_dev || !position_dev || !out_dev || batch <= 0 || seq <= 0 ||
         words <= 0 || types <= 0 || positions <= 0 || (types_stride != 0 && types_stride < seq))
         return SPATHA_ERR_BAD_ARGUMENT;
@@ -1192,9 +1193,27 @@ int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev,
     spatha::EmbeddingTables tables;
     tables.word = word_dev; tables.type = type_dev; tables.position = position_dev;
     tables.words = words; tables.types = types; tables.positions = positions; tables.hidden = hidden;
-    hipError_t e = spatha::launch_embed_layernorm_f16(tables, ids_dev, types_dev, types_stride, positions_dev, batch, seq, gamma_dev, beta_dev,
-                                                      eps, out_dev, out_t_dev, (hipStream_t)stream);
+    hipError_t e = spatha::launch_embed_layernorm_f16(tables, ids_dev, types_dev, types_stride, types_row, positions_dev, batch, seq,
+                                                      gamma_dev, beta_dev, eps, out_dev, out_t_dev, (hipStream_t)stream);
     return e == hipSuccess ? SPATHA_OK : hip_fail(e);
+}
+
+int spatha_embed_layernorm_f16(const int64_t* ids_dev, const int64_t* types_dev, int64_t types_stride, const int64_t* positions_dev, int batch,
+                               int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev, int64_t types,
+                               const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev, const uint16_t* beta_dev, float eps,
+                               int hidden, uint16_t* out_dev, uint16_t* out_t_dev, void* stream) {
+    return embed_layernorm(ids_dev, types_dev, types_stride, 0, positions_dev, batch, seq, word_dev, words, type_dev, types, position_dev,
+                           positions, gamma_dev, beta_dev, eps, hidden, out_dev, out_t_dev, stream);
+}
+
+int spatha_embed_layernorm_own_types_f16(const int64_t* ids_dev, const int64_t* types_row_dev, int64_t types_row, const int64_t* positions_dev,
+                                         int batch, int seq, const uint16_t* word_dev, int64_t words, const uint16_t* type_dev,
+                                         int64_t types, const uint16_t* position_dev, int64_t positions, const uint16_t* gamma_dev,
+                                         const uint16_t* beta_dev, float eps, int hidden, uint16_t* out_dev, uint16_t* out_t_dev,
+                                         void* stream) {
+    if (types_row <= 0) return SPATHA_ERR_BAD_ARGUMENT;
+    return embed_layernorm(ids_dev, types_row_dev, 0, types_row, positions_dev, batch, seq, word_dev, words, type_dev, types, position_dev,
+                           positions, gamma_dev, beta_dev, eps, hidden, out_dev, out_t_dev, stream);
 }
 
 int spatha_attention_f16(const uint16_t* q_dev, const uint16_t* k_dev, const uint16_t* v_dev, int64_t pitch, int batch, int seq, int heads,

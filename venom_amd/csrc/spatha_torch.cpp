@@ -527,11 +527,11 @@ py::object add_layernorm(py::handle input, py::handle addend, const torch::Tenso
     return o.tuple();
 }
 
-// The embedding of ids [batch, seq]: word, type and position tables, LayerNorm; types [batch, seq] or [1, >= seq], positions [1, >= seq].  As
-// add_layernorm.
+// The embedding of ids [batch, seq]: word, type and position tables, LayerNorm; types [batch, seq] or [1, >= seq] (own_types: the
+// model's row of them, looked up at the position ids), positions [1, >= seq].  As add_layernorm.
 py::object embed_layernorm(const torch::Tensor& ids, const torch::Tensor& types, const torch::Tensor& positions, const torch::Tensor& word,
                            const torch::Tensor& type, const torch::Tensor& position, const torch::Tensor& weight, const torch::Tensor& bias,
-                           double eps, bool feature_major) {
+                           double eps, bool feature_major, bool own_types) {
     if (!plain(ids) || !ids.is_cuda() || ids.layout() != torch::kStrided || ids.dim() != 2 || ids.numel() == 0) return py::none();
     // (a tangent of forward-mode differentiation is the stock operations' to carry on)
     for (const torch::Tensor* t : {&word, &type, &position, &weight, &bias})
@@ -540,7 +540,7 @@ py::object embed_layernorm(const torch::Tensor& ids, const torch::Tensor& types,
     const int64_t batch = ids.size(0), seq = ids.size(1), hidden = word.dim() == 2 ? word.size(1) : 0;
     const bool types_shared = types.dim() == 2 && types.size(0) == 1 && types.size(1) >= seq;
     if (!weight_ok(ids, torch::kInt64, device) || !weight_ok(types, torch::kInt64, device) || !weight_ok(positions, torch::kInt64, device) ||
-        !(types_shared || types.sizes() == ids.sizes()) || positions.dim() != 2 || positions.size(0) != 1 || positions.size(1) < seq ||
+        !(types_shared || (!own_types && types.sizes() == ids.sizes())) || positions.dim() != 2 || positions.size(0) != 1 || positions.size(1) < seq ||
         hidden <= 0 || hidden % 8 != 0 || hidden > 4096 || batch * seq > INT32_MAX - 64)
         return py::none();
     for (const torch::Tensor* t : {&word, &type, &position})
@@ -553,11 +553,12 @@ py::object embed_layernorm(const torch::Tensor& ids, const torch::Tensor& types,
     o.out = torch::empty({batch, seq, hidden}, word.options().requires_grad(false));
     if (feature_major) o.padded = torch::empty({hidden, (o.tokens + 7) / 8 * 8}, word.options().requires_grad(false));
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream();
-    check(spatha_embed_layernorm_f16((const int64_t*)ids.data_ptr(), (const int64_t*)types.data_ptr(), types_shared ? 0 : seq,
-                                     (const int64_t*)positions.data_ptr(), (int)batch, (int)seq, (const uint16_t*)word.data_ptr(), word.size(0),
-                                     (const uint16_t*)type.data_ptr(), type.size(0), (const uint16_t*)position.data_ptr(), position.size(0),
-                                     (const uint16_t*)weight.data_ptr(), (const uint16_t*)bias.data_ptr(), (float)eps, (int)hidden,
-                                     (uint16_t*)o.out.data_ptr(), feature_major ? (uint16_t*)o.padded.data_ptr() : nullptr, stream),
+    auto* embed = own_types ? &spatha_embed_layernorm_own_types_f16 : &spatha_embed_layernorm_f16;
+    check(embed((const int64_t*)ids.data_ptr(), (const int64_t*)types.data_ptr(), own_types ? types.size(1) : types_shared ? 0 : seq,
+                (const int64_t*)positions.data_ptr(), (int)batch, (int)seq, (const uint16_t*)word.data_ptr(), word.size(0),
+                (const uint16_t*)type.data_ptr(), type.size(0), (const uint16_t*)position.data_ptr(), position.size(0),
+                (const uint16_t*)weight.data_ptr(), (const uint16_t*)bias.data_ptr(), (float)eps, (int)hidden,
+                (uint16_t*)o.out.data_ptr(), feature_major ? (uint16_t*)o.padded.data_ptr() : nullptr, stream),
           "spatha_embed_layernorm_f16");
     return o.tuple();
 }

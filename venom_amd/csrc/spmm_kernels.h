@@ -134,8 +134,8 @@ struct EmbeddingTables {
     int hidden;
 };
 hipError_t launch_embed_layernorm_f16(const EmbeddingTables& tables, const int64_t* ids, const int64_t* types, int64_t types_stride,
-                                      const int64_t* positions, int batch, int seq, const uint16_t* gamma, const uint16_t* beta, float eps,
-                                      uint16_t* out, uint16_t* out_t, hipStream_t stream);
+                                      int64_t types_row, const int64_t* positions, int batch, int seq, const uint16_t* gamma,
+                                      const uint16_t* beta, float eps, uint16_t* out, uint16_t* out_t, hipStream_t stream);
 
 // softmax(scale Q K^T) V per sequence and head of 64 features, result feature-major (attention.hip)
 hipError_t launch_attention_f16(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t pitch, int batch, int seq, int heads,
