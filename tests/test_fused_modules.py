@@ -156,3 +156,53 @@ def test_the_embedding_goes_with_the_default_build_only(monkeypatch):
     monkeypatch.setattr(spatha, "_extension", lambda: pytest.fail("the extension was asked"))
     with torch.no_grad():
         fused_embeddings()(input_ids=torch.arange(6)[None])
+
+
+def merged(cols, rows):
+    """A _MergedProjections without matrices: its product is x times the number of the call."""
+
+    class Merged(bert._MergedProjections):
+        def __init__(self):
+            self.starts, self.rows, self._last, self.calls = [0], rows, (None, None, None), 0
+
+        def product(self, flat):
+            self.calls += 1
+            return flat[:, :rows] * self.calls
+
+    return Merged
+
+
+def test_a_product_of_another_thread_is_not_taken():
+    """Between keeping a product and answering from it another thread may keep its own."""
+    mine, others = torch.randn(6, 8), torch.randn(4, 8)
+
+    class Raced(merged(8, 4)):
+        def __setattr__(self, name, value):
+            super().__setattr__(name, value)
+            if name == "_last" and value[0] is not None:
+                self.__dict__["_last"] = (bert._activation_key(others), others, others[:, :4])
+
+    group = Raced()
+    assert torch.equal(group.output(0, 4, mine), mine[:, :4])
+    assert torch.equal(group.output(0, 4, mine), mine[:, :4] * 2)          # (what is kept is the other thread's: computed again)
+
+
+def test_a_transposed_copy_of_another_thread_is_not_taken():
+    mine, others = torch.randn(6, 8), torch.randn(4, 8)
+    entries = [(bert._activation_key(mine), mine, mine.t().contiguous())]
+
+    class Raced(type(bert.SrnmSpmm)):
+        @property
+        def _last_rhs(cls):
+            seen = entries[-1]
+            entries.append((bert._activation_key(others), others, others.t().contiguous()))         # between two looks
+            return seen
+
+        @_last_rhs.setter
+        def _last_rhs(cls, value):
+            entries.append(value)
+
+    class Layer(bert.SrnmSpmm, metaclass=Raced):
+        pass
+
+    assert torch.equal(Layer._transposed(mine), mine.t())

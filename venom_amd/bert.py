@@ -78,9 +78,9 @@ class SrnmSpmm(torch.nn.Module):
     def _transposed(cls, flat):
         if flat.stride(0) == 1 and flat.stride(1) == flat.shape[0]:
             return flat.T              # feature-major already (the output of a fused feed-forward layer): no copy
-        key = _activation_key(flat)
-        if cls._last_rhs[0] == key:
-            return cls._last_rhs[2].contiguous()       # (a copy for a ragged token count has padded rows)
+        key, last = _activation_key(flat), cls._last_rhs       # (looked at once: another thread may leave its own copy there)
+        if last[0] == key:
+            return last[2].contiguous()       # (a copy for a ragged token count has padded rows)
         if flat.is_cuda and flat.dtype == torch.float16:
             rhs = spatha.transpose(flat.contiguous())
         else:
@@ -174,11 +174,11 @@ class _MergedProjections:
 
     def output(self, index, nrows, input):
         flat = torch.flatten(input, start_dim=0, end_dim=-2)
-        key = _activation_key(flat)
-        if self._last[0] != key:
-            self._last = (key, flat, self.product(flat))
+        key, last = _activation_key(flat), self._last          # (as above)
+        if last[0] != key:
+            last = self._last = (key, flat, self.product(flat))
         start = self.starts[index]
-        return self._last[2][:, start:start + nrows].reshape(*input.shape[:-1], nrows)
+        return last[2][:, start:start + nrows].reshape(*input.shape[:-1], nrows)
 
 
 def merge_qkv(model):
